@@ -20,6 +20,7 @@ import math
 import numpy as np
 import torch
 import torch.nn as nn
+import torch.nn.functional as F
 
 import dace_onnx_amd.onnx as donnx
 from dace_onnx_amd.onnx.proto import TensorProto, helper, numpy_helper
@@ -93,25 +94,31 @@ def draw(rng):
 
 
 class _Graph:
-    """Nodes and initializers of an ONNX graph under construction."""
+    """Nodes and initializers of an ONNX graph under construction, kept plain: ``exact`` reads them too."""
 
     def __init__(self, opset):
-        self.nodes, self.weights, self.opset = [], [], opset
+        self.nodes, self.weights, self.opset = [], {}, opset
 
     def node(self, op, inputs, **attributes):
         out = f"{op.lower()}_{len(self.nodes)}"
-        self.nodes.append(helper.make_node(op, inputs, [out], name=f"n{len(self.nodes)}", **attributes))
+        self.nodes.append((op, inputs, out, attributes))
         return out
 
     def weight(self, value, dtype=np.float32):
         name = f"w{len(self.weights)}"
-        self.weights.append(numpy_helper.from_array(np.ascontiguousarray(value, dtype=dtype), name))
+        self.weights[name] = np.ascontiguousarray(value, dtype=dtype)
         return name
 
-    def model(self, name, inputs, outputs):
-        infos = [helper.make_tensor_value_info(n, t, list(s)) for n, t, s in inputs]
-        outs = [helper.make_tensor_value_info(n, t, list(s)) for n, t, s in outputs]
-        graph = helper.make_graph(self.nodes, name, infos, outs, initializer=self.weights)
+    def finish(self, name, inputs, outputs):
+        self.name, self.inputs, self.outputs = name, inputs, outputs
+        return self
+
+    def model(self):
+        infos = [helper.make_tensor_value_info(n, t, list(s)) for n, t, s in self.inputs]
+        outs = [helper.make_tensor_value_info(n, t, list(s)) for n, t, s in self.outputs]
+        nodes = [helper.make_node(op, inputs, [out], name=f"n{i}", **attributes) for i, (op, inputs, out, attributes) in enumerate(self.nodes)]
+        weights = [numpy_helper.from_array(value, name) for name, value in self.weights.items()]
+        graph = helper.make_graph(nodes, self.name, infos, outs, initializer=weights)
         return helper.make_model(graph, opset_imports=[helper.make_opsetid("", self.opset)])
 
 
@@ -119,7 +126,7 @@ def _normal(rng, *shape, scale=1.0):
     return rng.standard_normal(shape, dtype=np.float32) * np.float32(scale)
 
 
-def _encoder_model(case, rng):
+def _encoder_graph(case, rng):
     batch, seq, hidden = case["batch"], case["seq"], case["hidden"]
     size, heads, inner = 64, case["hidden"] // 64, 4 * case["hidden"]
     g = _Graph(12 if case["exported"] else 20)
@@ -157,7 +164,7 @@ def _encoder_model(case, rng):
     out = dense(gelu(dense(attended, hidden, inner)), inner, hidden)
     out = layer_norm(g.node("Add", [out, attended]))
     inputs = [("x", F32, (batch, seq, hidden))] + ([("mask", F32, (batch, 1, 1, seq))] if case["masked"] else [])
-    return g.model("encoder", inputs, [(out, F32, (batch, seq, hidden))])
+    return g.finish("encoder", inputs, [(out, F32, (batch, seq, hidden))])
 
 
 def _convolved(extent, kernel, stride, pad):
@@ -181,7 +188,7 @@ def _convnet_layers(case):
 CONVNET_CLASSES = 1000
 
 
-def _convnet_model(case, rng):
+def _convnet_graph(case, rng):
     g = _Graph(12)
 
     def conv(x, c_in, c_out, kernel, stride):
@@ -200,73 +207,87 @@ def _convnet_model(case, rng):
         x, channels = g.node("Relu", [g.node("Add", [y, skip])]), width
     x = g.node("Flatten", [g.node("GlobalAveragePool", [x])], axis=1)
     x = g.node("Gemm", [x, g.weight(_normal(rng, CONVNET_CLASSES, 512, scale=0.05)), g.weight(_normal(rng, CONVNET_CLASSES, scale=0.05))], transB=1)
-    return g.model("convnet", [("x", F32, (case["batch"], 3, case["size"], case["size"]))], [(x, F32, (case["batch"], CONVNET_CLASSES))])
+    return g.finish("convnet", [("x", F32, (case["batch"], 3, case["size"], case["size"]))], [(x, F32, (case["batch"], CONVNET_CLASSES))])
 
 
-def _head_model(case, rng):
+def _head_graph(case, rng):
     g = _Graph(12)
     y = g.node("MatMul", ["x", g.weight(_normal(rng, case["hidden"], case["classes"], scale=0.05))])
     y = g.node("Add", [y, g.weight(_normal(rng, case["classes"], scale=0.05))])
     y = g.node("LogSoftmax", [y], axis=1)
-    return g.model("head", [("x", F32, (case["rows"], case["hidden"]))], [(y, F32, (case["rows"], case["classes"]))])
+    return g.finish("head", [("x", F32, (case["rows"], case["hidden"]))], [(y, F32, (case["rows"], case["classes"]))])
 
 
-def _quantised_model(case, rng):
+def _quantised_graph(case, rng):
     g = _Graph(12)
     a_type = np.uint8 if case["unsigned"] else np.int8
     weights = g.weight(rng.integers(-128, 128, (case["inner"], case["columns"]), dtype=np.int8), np.int8)
     a_zero = g.weight(121 if case["unsigned"] else 3, a_type)
     b_zero = g.weight(rng.integers(-8, 8, case["columns"], dtype=np.int8) if case["per_column"] else -2, np.int8)
     y = g.node("MatMulInteger", ["a", weights, a_zero, b_zero])
-    return g.model("quantised", [("a", TensorProto.UINT8 if case["unsigned"] else TensorProto.INT8, (case["rows"], case["inner"]))],
+    return g.finish("quantised", [("a", TensorProto.UINT8 if case["unsigned"] else TensorProto.INT8, (case["rows"], case["inner"]))],
                    [(y, TensorProto.INT32, (case["rows"], case["columns"]))])
 
 
-def _scores_model(case, rng):
+def _scores_graph(case, rng):
     g = _Graph(12)
     shape = (case["rows"], case["columns"])
     probabilities = g.node("Softmax", ["x"], axis=1)
     largest = g.node("ReduceMax", ["x"], axes=[1], keepdims=0)
-    return g.model("scores", [("x", F32, shape)], [(probabilities, F32, shape), (largest, F32, shape[:1])])
+    return g.finish("scores", [("x", F32, shape)], [(probabilities, F32, shape), (largest, F32, shape[:1])])
 
 
 # ------------------------------------------------------------------------------------------------ the contract
 
 
-def prepare(case, seed):
-    rng = np.random.default_rng(seed)
+_GRAPHS = {"encoder": _encoder_graph, "convnet": _convnet_graph, "head": _head_graph, "quantised": _quantised_graph, "scores": _scores_graph}
+
+
+def _inputs(case, rng):
+    """The arrays that a call gets; drawn after the weights."""
     kind = case["kind"]
-    if kind == "mlp":
-        sizes = [case["inputs"], case["width"], case["width"], case["classes"]]
-        layers = []
-        for n_in, n_out in zip(sizes, sizes[1:]):
-            linear = nn.utils.skip_init(nn.Linear, n_in, n_out)
-            with torch.no_grad():
-                linear.weight.copy_(torch.from_numpy(_normal(rng, n_out, n_in, scale=1 / math.sqrt(n_in))))
-                linear.bias.copy_(torch.from_numpy(_normal(rng, n_out, scale=0.05)))
-            layers += [linear, nn.ReLU()]
-        module = nn.Sequential(*layers[:-1], nn.Softmax(dim=1)).cuda().eval()
-        x = torch.from_numpy(_normal(rng, case["batch"], case["inputs"])).cuda()
-        model = DaceModule(module, dummy_inputs=(x,), sdfg_name="mlp")
-        return {"model": model, "inputs": [x]}
-    build = {"encoder": _encoder_model, "convnet": _convnet_model, "head": _head_model, "quantised": _quantised_model, "scores": _scores_model}[kind]
-    model = donnx.ONNXModel(kind, build(case, rng), use_hip_graph=bool(case.get("replayed", False)))
     if kind == "encoder":
         inputs = [_normal(rng, case["batch"], case["seq"], case["hidden"])]
         if case["masked"]:
             lengths = rng.integers((case["seq"] + 1) // 2, case["seq"] + 1, size=case["batch"])
             padding = np.arange(case["seq"])[None, :] >= lengths[:, None]
             inputs.append((padding * np.float32(-10000.0)).astype(np.float32).reshape(case["batch"], 1, 1, case["seq"]))
-    elif kind == "convnet":
-        inputs = [_normal(rng, case["batch"], 3, case["size"], case["size"])]
-    elif kind == "head":
-        inputs = [_normal(rng, case["rows"], case["hidden"])]
-    elif kind == "quantised":
+        return inputs
+    if kind == "convnet":
+        return [_normal(rng, case["batch"], 3, case["size"], case["size"])]
+    if kind == "mlp":
+        return [_normal(rng, case["batch"], case["inputs"])]
+    if kind == "head":
+        return [_normal(rng, case["rows"], case["hidden"])]
+    if kind == "quantised":
         low, high, dtype = (0, 256, np.uint8) if case["unsigned"] else (-128, 128, np.int8)
-        inputs = [rng.integers(low, high, (case["rows"], case["inner"]), dtype=dtype)]
-    else:
-        inputs = [_normal(rng, case["rows"], case["columns"], scale=2.0)]
-    return {"model": model, "inputs": [torch.from_numpy(a).cuda() for a in inputs]}
+        return [rng.integers(low, high, (case["rows"], case["inner"]), dtype=dtype)]
+    return [_normal(rng, case["rows"], case["columns"], scale=2.0)]
+
+
+def _mlp_layers(case, rng):
+    """(weight, bias) of the three dense layers."""
+    sizes = [case["inputs"], case["width"], case["width"], case["classes"]]
+    return [(_normal(rng, n_out, n_in, scale=1 / math.sqrt(n_in)), _normal(rng, n_out, scale=0.05)) for n_in, n_out in zip(sizes, sizes[1:])]
+
+
+def prepare(case, seed):
+    rng = np.random.default_rng(seed)
+    kind = case["kind"]
+    if kind == "mlp":
+        layers = []
+        for weight, bias in _mlp_layers(case, rng):
+            linear = nn.utils.skip_init(nn.Linear, weight.shape[1], weight.shape[0])
+            with torch.no_grad():
+                linear.weight.copy_(torch.from_numpy(weight))
+                linear.bias.copy_(torch.from_numpy(bias))
+            layers += [linear, nn.ReLU()]
+        module = nn.Sequential(*layers[:-1], nn.Softmax(dim=1)).cuda().eval()
+        x = torch.from_numpy(_inputs(case, rng)[0]).cuda()
+        model = DaceModule(module, dummy_inputs=(x,), sdfg_name="mlp")
+        return {"model": model, "inputs": [x]}
+    model = donnx.ONNXModel(kind, _GRAPHS[kind](case, rng).model(), use_hip_graph=bool(case.get("replayed", False)))
+    return {"model": model, "inputs": [torch.from_numpy(a).cuda() for a in _inputs(case, rng)]}
 
 
 def run(state):
@@ -298,6 +319,60 @@ def work(case):
         rows, inner, columns = case["rows"], case["inner"], case["columns"]
         return {"bytes": float(rows * inner + inner * columns + 4 * rows * columns), "flops": 2.0 * rows * inner * columns}
     return {"bytes": 4.0 * case["rows"] * (2 * case["columns"] + 1), "flops": 5.0 * case["rows"] * case["columns"]}
+
+
+# Sums over a window and the running sums of a matrix product are taken in float64, whole numbers too: below 2**53 they are exact.
+
+
+def _exact_conv(x, w, kernel_shape, pads, strides):
+    columns = F.unfold(x, kernel_shape, padding=pads[0], stride=strides[0])
+    rows, cols = (_convolved(x.shape[axis], kernel_shape[0], strides[0], pads[0]) for axis in (2, 3))
+    return torch.stack([w.reshape(w.shape[0], -1) @ image for image in columns]).reshape(x.shape[0], w.shape[0], rows, cols)
+
+
+def _exact_batch_norm(x, scale, shift, mean, variance, epsilon):
+    scale, shift, mean, variance = (v.reshape(1, -1, 1, 1) for v in (scale, shift, mean, variance))
+    return (x - mean) / torch.sqrt(variance + epsilon) * scale + shift
+
+
+def _exact_layer_norm(x, gamma, beta, axis, epsilon):
+    centred = x - x.mean(dim=axis, keepdim=True)
+    return centred / torch.sqrt((centred * centred).mean(dim=axis, keepdim=True) + epsilon) * gamma + beta
+
+
+_EXACT = {
+    "MatMul": torch.matmul, "Add": torch.add, "Sub": torch.sub, "Mul": torch.mul, "Div": torch.div, "Pow": torch.pow, "Sqrt": torch.sqrt,
+    "Erf": torch.erf, "Relu": torch.relu, "Gelu": F.gelu, "LayerNormalization": _exact_layer_norm, "BatchNormalization": _exact_batch_norm,
+    "Reshape": lambda x, shape: x.reshape([int(n) for n in shape]), "Transpose": lambda x, perm: x.permute(perm).contiguous(),
+    "Softmax": lambda x, axis: torch.softmax(x, axis), "LogSoftmax": lambda x, axis: torch.log_softmax(x, axis),
+    "ReduceMean": lambda x, axes, keepdims: x.mean(dim=axes, keepdim=bool(keepdims)),
+    "ReduceMax": lambda x, axes, keepdims: x.amax(dim=axes, keepdim=bool(keepdims)),
+    "Conv": _exact_conv, "MaxPool": lambda x, kernel_shape, pads, strides: F.max_pool2d(x, kernel_shape, strides, pads[0]),
+    "GlobalAveragePool": lambda x: x.mean(dim=(2, 3), keepdim=True), "Flatten": lambda x, axis: x.flatten(axis),
+    "Gemm": lambda x, w, b, transB: x @ w.t() + b, "MatMulInteger": lambda a, b, a_zero, b_zero: (a - a_zero) @ (b - b_zero),
+}
+
+
+def exact(case, seed):
+    rng = np.random.default_rng(seed)
+    device = "cuda" if torch.cuda.is_available() else "cpu"
+    wide = lambda a: torch.from_numpy(a).to(device, torch.float64)  # noqa: E731
+    if case["kind"] == "mlp":
+        layers = _mlp_layers(case, rng)
+        x = wide(_inputs(case, rng)[0])
+        for i, (weight, bias) in enumerate(layers):
+            x = x @ wide(weight).t() + wide(bias)
+            x = torch.relu(x) if i + 1 < len(layers) else torch.softmax(x, 1)
+        return x
+    graph = _GRAPHS[case["kind"]](case, rng)
+    values = {name: wide(value) for name, value in graph.weights.items()}
+    values.update({name: wide(array) for (name, _, _), array in zip(graph.inputs, _inputs(case, rng))})
+    for op, inputs, out, attributes in graph.nodes:
+        values[out] = _EXACT[op](*(values[name] for name in inputs), **attributes)
+    outputs = [values[name] for name, _, _ in graph.outputs]
+    if case["kind"] == "quantised":
+        outputs = [outputs[0].to(torch.int32)]
+    return outputs[0] if len(outputs) == 1 else tuple(outputs)
 
 
 def tolerance(case):
