@@ -68,6 +68,30 @@ __global__ __launch_bounds__(256) void reduce_rows(const float* __restrict__ X, 
     if (lane == 0) Y[row] = KIND == MI355X_REDUCE_MEAN ? s * (1.0f / (float)cols) : s;
 }
 
+// Many rows of up to 64 * NV columns: a wave takes UNR rows, all their loads first, so that a short row's trip to memory
+// and its six combining steps overlap the other rows' (one row per wave is that chain and nothing else: ReduceMax
+// [18912, 197] 6.2 -> 5.4 us).
+template <int KIND, int NV, int UNR>
+__global__ __launch_bounds__(256) void reduce_rows_short(const float* __restrict__ X, float* __restrict__ Y, int64_t rows, int cols) {
+    using R = Reducer<KIND, float>;
+    const int lane = threadIdx.x % WAVE;
+    const int64_t row0 = ((int64_t)blockIdx.x * (256 / WAVE) + threadIdx.x / WAVE) * UNR;
+    float v[UNR][NV];
+#pragma unroll
+    for (int u = 0; u < UNR; ++u)
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+            v[u][j] = row0 + u < rows && lane + j * WAVE < cols ? X[(row0 + u) * cols + lane + j * WAVE] : R::identity();
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) {
+        float s = v[u][0];
+#pragma unroll
+        for (int j = 1; j < NV; ++j) s = R::combine(s, v[u][j]);
+        s = wave_combine<KIND>(s);
+        if (lane == 0 && row0 + u < rows) Y[row0 + u] = KIND == MI355X_REDUCE_MEAN ? s * (1.0f / (float)cols) : s;
+    }
+}
+
 template <int KIND>
 __global__ __launch_bounds__(256) void reduce_strided(const float* __restrict__ X, float* __restrict__ Y,
                                                       int64_t outer, int64_t axis_len, int64_t inner) {
@@ -131,6 +155,13 @@ static int launch_reduce(const float* X, float* Y, int64_t outer, int64_t axis_l
     if (inner == 1) {
         const int64_t blocks = ceil_div(outer, (int64_t)(256 / WAVE));
         MI355X_REQUIRE(blocks < ((int64_t)1 << 31), "reduce: grid too large");
+        // (from 4096 rows on there are enough waves to fill the part with four rows each)
+        if (axis_len <= 256 && outer >= 4096) {
+            const dim3 grid((unsigned)ceil_div(outer, (int64_t)(256 / WAVE) * 4));
+            if (axis_len <= 64) hipLaunchKernelGGL((reduce_rows_short<KIND, 1, 4>), grid, dim3(256), 0, st, X, Y, outer, (int)axis_len);
+            else hipLaunchKernelGGL((reduce_rows_short<KIND, 4, 4>), grid, dim3(256), 0, st, X, Y, outer, (int)axis_len);
+            return check_launch("reduce_rows_short");
+        }
         const bool vec = axis_len % 4 == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;
         if (vec) hipLaunchKernelGGL((reduce_rows<KIND, true>), dim3((unsigned)blocks), dim3(256), 0, st, X, Y, outer, axis_len);
         else hipLaunchKernelGGL((reduce_rows<KIND, false>), dim3((unsigned)blocks), dim3(256), 0, st, X, Y, outer, axis_len);

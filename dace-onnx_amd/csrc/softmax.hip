@@ -14,8 +14,11 @@
 //       reductions are DPP row operations, no LDS. Each group handles UNR rows
 //       with all loads issued before the first reduction to keep HBM requests
 //       in flight.
-//   softmax_rows_loop   last axis, any cols: one wave per row, three sweeps
-//       (max, sum, write); sweeps two and three hit in L2.
+//   softmax_rows_any<THREADS, NV>  last axis, any cols <= THREADS*NV, no alignment asked
+//       of a row: the row in the registers of one wave (THREADS = 64) or of one workgroup,
+//       NV single floats per thread.
+//   softmax_rows_loop   last axis, longer rows: one workgroup of 1024 per row, three
+//       sweeps (max, sum, write).
 //   softmax_strided     axis is not last: one thread per (outer, inner) column,
 //       lanes adjacent along `inner` so every access is coalesced.
 #include "common.h"
@@ -102,23 +105,71 @@ __global__ __launch_bounds__(256) void softmax_rows_reg(const float* __restrict_
     }
 }
 
-template <bool LOG>
-__global__ __launch_bounds__(256) void softmax_rows_loop(const float* __restrict__ X,
-                                                         float* __restrict__ Y,
-                                                         int64_t rows, int64_t cols) {
-    const int lane = threadIdx.x % WAVE;
-    const int64_t row = (int64_t)blockIdx.x * (256 / WAVE) + threadIdx.x / WAVE;
-    if (row >= rows) return;  // whole wave leaves together
+// Reduction over a workgroup of THREADS (the wave itself where THREADS is 64): `part` holds one value per wave.
+template <int THREADS, bool MAX>
+__device__ __forceinline__ float block_reduce(float v, float* part) {
+    v = MAX ? wave_max(v) : wave_sum(v);
+    if constexpr (THREADS == WAVE) return v;
+    constexpr int WAVES = THREADS / WAVE;
+    __syncthreads();   // the previous reduction's values have been read
+    if (threadIdx.x % WAVE == 0) part[threadIdx.x / WAVE] = v;
+    __syncthreads();
+    v = part[0];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) v = MAX ? fmaxf(v, part[w]) : v + part[w];
+    return v;
+}
+
+// Bound by HBM: one read and one write. Rows of any length start at any multiple of four bytes, so lanes take single
+// floats (a wave's load is 256 contiguous bytes, at most one cache line more than an aligned one). All of a row's
+// loads are issued before the first reduction; a row stays with one wave up to 512 columns (no barrier, eight loads in
+// flight per lane) and takes as many waves as keep the loads per thread at 32 or fewer above that. Against three
+// sweeps by one wave per row: LogSoftmax [1024, 30522] 442 -> 58 us (4.3 TB/s), Softmax [18912, 197] 12.7 -> 8.3 us.
+template <int THREADS, int NV, bool LOG>
+__global__ __launch_bounds__(THREADS == WAVE ? 256 : THREADS) void softmax_rows_any(const float* __restrict__ X, float* __restrict__ Y,
+                                                                                    int64_t rows, int cols) {
+    constexpr int ROWS = THREADS == WAVE ? 4 : 1;   // rows per workgroup
+    __shared__ float part[THREADS / WAVE];
+    const int t = threadIdx.x % THREADS;
+    const int64_t row = (int64_t)blockIdx.x * ROWS + threadIdx.x / THREADS;
+    if (row >= rows) return;  // a whole wave, and only where no barrier follows (ROWS > 1)
     const float* x = X + row * cols;
     float* y = Y + row * cols;
+    float v[NV];
     float m = -INFINITY;
-    for (int64_t c = lane; c < cols; c += WAVE) m = fmaxf(m, x[c]);
-    m = wave_max(m);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) v[j] = t + j * THREADS < cols ? __builtin_nontemporal_load(x + t + j * THREADS) : -INFINITY;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) m = fmaxf(m, v[j]);
+    m = block_reduce<THREADS, true>(m, part);
     float s = 0.0f;
-    for (int64_t c = lane; c < cols; c += WAVE) s += expf(x[c] - m);
-    s = wave_sum(s);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {   // columns beyond the row hold -inf: exp(-inf - m) adds nothing
+        v[j] -= m;
+        const float e = expf(v[j]);
+        s += e;
+        if constexpr (!LOG) v[j] = e;
+    }
+    s = block_reduce<THREADS, false>(s, part);
     const float inv = 1.0f / s, log_s = LOG ? logf(s) : 0.0f;
-    for (int64_t c = lane; c < cols; c += WAVE) y[c] = LOG ? (x[c] - m) - log_s : expf(x[c] - m) * inv;
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+        if (t + j * THREADS < cols) __builtin_nontemporal_store(LOG ? v[j] - log_s : v[j] * inv, y + t + j * THREADS);
+}
+
+template <bool LOG>
+__global__ __launch_bounds__(1024) void softmax_rows_loop(const float* __restrict__ X, float* __restrict__ Y, int64_t cols) {
+    __shared__ float part[1024 / WAVE];
+    const float* x = X + (int64_t)blockIdx.x * cols;
+    float* y = Y + (int64_t)blockIdx.x * cols;
+    float m = -INFINITY;
+    for (int64_t c = threadIdx.x; c < cols; c += 1024) m = fmaxf(m, x[c]);
+    m = block_reduce<1024, true>(m, part);
+    float s = 0.0f;
+    for (int64_t c = threadIdx.x; c < cols; c += 1024) s += expf(x[c] - m);
+    s = block_reduce<1024, false>(s, part);
+    const float inv = 1.0f / s, log_s = LOG ? logf(s) : 0.0f;
+    for (int64_t c = threadIdx.x; c < cols; c += 1024) y[c] = LOG ? (x[c] - m) - log_s : expf(x[c] - m) * inv;
 }
 
 template <bool LOG>
@@ -154,6 +205,13 @@ static void launch_reg(const float* X, float* Y, int64_t rows, int cols, hipStre
     const int64_t blocks = ceil_div(rows, rows_per_block);
     hipLaunchKernelGGL((softmax_rows_reg<L, NV, UNR, LOG>), dim3((unsigned)blocks), dim3(256), 0, st,
                        X, Y, rows, cols);
+}
+
+template <int THREADS, int NV, bool LOG>
+static void launch_any(const float* X, float* Y, int64_t rows, int64_t cols, hipStream_t st) {
+    constexpr int ROWS = THREADS == WAVE ? 4 : 1;
+    hipLaunchKernelGGL((softmax_rows_any<THREADS, NV, LOG>), dim3((unsigned)ceil_div(rows, (int64_t)ROWS)), dim3(THREADS * ROWS), 0, st,
+                       X, Y, rows, (int)cols);
 }
 
 // Rows per lane group. Inputs of a few MB are one round trip to memory per CU and finish sooner the more
@@ -192,9 +250,14 @@ static int softmax_dispatch(const float* X, float* Y, int64_t outer, int64_t axi
         else if (vec_ok && cols <= 512) launch_reg_unr<64, 2, LOG>(X, Y, rows, (int)cols, st);
         else if (vec_ok && cols <= 1024) launch_reg_unr<64, 4, LOG>(X, Y, rows, (int)cols, st);
         else if (vec_ok && cols <= 2048) launch_reg_unr<64, 8, LOG>(X, Y, rows, (int)cols, st);
-        else
-            hipLaunchKernelGGL(softmax_rows_loop<LOG>, dim3((unsigned)ceil_div(rows, 256 / WAVE)),
-                               dim3(256), 0, st, X, Y, rows, cols);
+        else if (cols <= 64) launch_any<64, 1, LOG>(X, Y, rows, cols, st);
+        else if (cols <= 128) launch_any<64, 2, LOG>(X, Y, rows, cols, st);
+        else if (cols <= 256) launch_any<64, 4, LOG>(X, Y, rows, cols, st);
+        else if (cols <= 512) launch_any<64, 8, LOG>(X, Y, rows, cols, st);
+        else if (cols <= 2048) launch_any<256, 8, LOG>(X, Y, rows, cols, st);
+        else if (cols <= 8192) launch_any<512, 16, LOG>(X, Y, rows, cols, st);
+        else if (cols <= 32768) launch_any<1024, 32, LOG>(X, Y, rows, cols, st);
+        else hipLaunchKernelGGL(softmax_rows_loop<LOG>, dim3((unsigned)rows), dim3(1024), 0, st, X, Y, cols);
         return check_launch("softmax_rows");
     }
     const int64_t n = outer * inner;
