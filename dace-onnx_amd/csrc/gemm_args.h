@@ -27,4 +27,9 @@ bool launch_gemm_f32_nt(GemmArgs p, int cus, hipStream_t stream);
 // GEMM with both operands contiguous along k whose eight waves split K (gemm_f32_ksplit.hip): 32 x 96 tiles.
 bool launch_gemm_f32_ksplit(GemmArgs p, int cus, hipStream_t stream);
 
+// GEMM with A contiguous along k and B along k (b_kc) or n, on the bf16 matrix unit with every value split in three
+// (gemm_f32_split.hip). `other_cost`: nanoseconds per k the caller's own kernel takes; nothing is launched where no form of
+// this one is below it.
+bool launch_gemm_f32_split(GemmArgs p, bool b_kc, double other_cost, int cus, hipStream_t stream);
+
 }  // namespace mi355x

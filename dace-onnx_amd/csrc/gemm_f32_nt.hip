@@ -34,16 +34,6 @@
 
 namespace mi355x {
 
-template <int N, class F, int... I>
-__device__ __forceinline__ void nt_static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-// f(integral_constant<0>) ... f(integral_constant<N-1>): indices usable for register arrays
-template <int N, class F>
-__device__ __forceinline__ void nt_static_for(F&& f) {
-    nt_static_for_impl<N>(static_cast<F&&>(f), std::make_integer_sequence<int, N>{});
-}
-
 constexpr int NT_BK = 32, NT_THREADS = 512, NT_RING = 6, NT_STAGES = 3;
 
 // TN: 16-column MFMA tiles per wave (BN = 16 TN). WAVES_M wave rows of 16 rows each
@@ -236,7 +226,7 @@ __global__ __launch_bounds__(WAVES_M * KSPLIT * WAVE, PER_CU) void gemm_f32_nt_k
     // write LDS buffers nobody reads any more), so the step body stays branch-free
     // and the compiler's s_waitcnt counts stay exact from the first tile to the last.
     for (int kt0 = 0; kt0 < ktiles; kt0 += UNROLL) {
-        nt_static_for<UNROLL>([&](auto u_tag) {
+        static_for<UNROLL>([&](auto u_tag) {
             const int kt = kt0 + decltype(u_tag)::value;
             if (kt < ktiles)  // uniform; only the last group can be partial
                 tile_step(u_tag, std::true_type{}, std::true_type{}, std::true_type{}, std::true_type{}, kt);
@@ -332,6 +322,13 @@ bool launch_gemm_f32_nt(GemmArgs p, int cus, hipStream_t stream) {
             best_cost = cost;
         }
     }
+    // The bf16 form takes over where its own sweep says it is faster (gemm_f32_split.hip). 4.7e-3 ns per k and unit of cost is
+    // what these kernels measure (3.8 to 5.1 over outputs of 256 to 4096 tiles), less 8 % so that a tie stays here: 8192 x 768 x
+    // 768 64 against 85 us, 8192 x 3072 x 768 215 against 288, 4096 x 1024 x 768 48 against 60; 1024 x 3072 x 768 (42 against 40)
+    // and everything smaller stays.
+    const bool forced = force || tune.gemm_nt_bk || tune.gemm_nt_per_cu || tune.gemm_nt_waves || tune.gemm_group_m;
+    if (tune.gemm_split > 0 || (!forced && p.K >= 256))
+        if (launch_gemm_f32_split(p, true, 4.7e-3 * 0.92 * best_cost, cus, stream)) return true;
     p.tiles_m = ceil_div(p.M, cands[best].bm);
     p.tiles_n = ceil_div(p.N, cands[best].bn);
     p.nwg = p.batch * p.tiles_m * p.tiles_n;

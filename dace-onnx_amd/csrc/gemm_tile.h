@@ -5,10 +5,23 @@
 
 #include "common.h"
 
+#include <type_traits>
+#include <utility>
+
 namespace mi355x {
 
 constexpr int NUM_XCD = 8;
 constexpr int LDS_PAD = 4;
+
+template <int N, class F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+// f(integral_constant<0>) ... f(integral_constant<N-1>): indices usable for register arrays
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+    static_for_impl<N>(static_cast<F&&>(f), std::make_integer_sequence<int, N>{});
+}
 
 // Hardware places workgroup w on XCD w % 8. Give XCD x the contiguous logical
 // range it would own if the tile space were cut into eight slabs.

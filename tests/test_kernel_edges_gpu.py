@@ -56,3 +56,70 @@ def test_reductions_of_many_short_rows(kind, reference, rows, cols):
     assert torch.isnan(y).nonzero().flatten().tolist() == [3]
     x[3], y[3] = 0, 0
     assert worst(reference(x.double()), y) < (1e-6 if kind < 2 else 1e-12)
+
+
+def split_gemm(a, b, kc, bias=None, res=None, epi=0, alpha=1.0, batch=1):
+    """C = a @ b through mi355x_gemm_f32; ``b`` is [N, K] if ``kc`` else [K, N]; a batch shares b."""
+    M, K = a.shape[-2:]
+    N = b.shape[0] if kc else b.shape[1]
+    c = torch.full((batch, M, N), np.nan, device="cuda")
+    i64 = _lib.i64_array
+    call("mi355x_gemm_f32", a.data_ptr(), b.data_ptr(), c.data_ptr(), bias.data_ptr() if bias is not None else None,
+         res.data_ptr() if res is not None else None, 1, batch, M, N, K, i64([0, M * K, K, 1]), i64([0, 0] + ([1, K] if kc else [N, 1])),
+         i64([0, M * N, N]), i64([0, M * N, N]), alpha, epi)
+    return c
+
+
+@pytest.mark.parametrize("kc", [True, False])
+@pytest.mark.parametrize("rows", [64, 128, 256])
+@pytest.mark.parametrize("batch, M, N, K, epi", [(1, 1, 1, 32, 0), (1, 63, 65, 64, 1), (1, 64, 64, 96, 9), (2, 129, 127, 160, 13), (1, 257, 130, 32, 3),
+                                                 (1, 255, 258, 768, 9), (3, 512, 128, 1056, 8)])
+def test_gemm_of_values_split_in_three(tuning, rows, kc, batch, M, N, K, epi):
+    """Every form of the bf16 kernel at the edges of its tiles. A sum of K products: at most one rounding (2^-23, truncation
+    included) for each of the K / 32 steps, and three of 2^-24 for the products left out and the two sets of sums."""
+    tuning(MI355X_GEMM_SPLIT=rows)
+    rng = np.random.default_rng(M + N + K)
+    a = gpu(rng.standard_normal((batch, M, K), dtype=np.float32))
+    b = gpu(rng.standard_normal((N, K) if kc else (K, N), dtype=np.float32))
+    bias, res = gpu(rng.standard_normal(N, dtype=np.float32)), gpu(rng.standard_normal((batch, M, N), dtype=np.float32))
+    got = split_gemm(a, b, kc, bias, res, epi, 0.5, batch)
+    wide = b.double().t() if kc else b.double()
+    expected = 0.5 * (a.double() @ wide) + (bias.double() if epi & 1 else 0)
+    if epi & 2:
+        expected = expected.relu()
+    if epi & 4:
+        expected = torch.nn.functional.gelu(expected)
+    if epi & 8:
+        expected = expected + res.double()
+    bound = (a.double().abs() @ wide.abs() + 1) * (K // 32 + 8) * 2.0**-23
+    assert bool(((expected - got.double()).abs() <= 1.2 * bound).all())   # 1.13 is Gelu's steepest slope
+
+
+@pytest.mark.parametrize("kc", [True, False])
+@pytest.mark.parametrize("rows", [64, 128, 256])
+def test_split_gemm_keeps_infinities_nan_and_the_largest_values(tuning, rows, kc):
+    tuning(MI355X_GEMM_SPLIT=rows)
+    a = torch.randn(1, 300, 96, device="cuda")
+    b = torch.rand(200, 96, device="cuda") + 0.5
+    a[0, 3, 5], a[0, 70, 95], a[0, 130, 0], a[0, 131, 1:3] = float("inf"), -float("inf"), float("nan"), torch.tensor([float("inf"), -float("inf")])
+    a[0, 200], a[0, 200, 7], a[0, 290, 9] = 0, 3.4e38, 3.3999e38   # rounds up to infinity in bf16
+    b[:, 7] = 0.75
+    b[11, 9], b[150, 9], b[150, 60] = 0, 0.5, float("inf")   # (0.5: no product of its own overflows next to the infinite one)
+    expected = a[0].double() @ b.double().t()
+    got = split_gemm(a, b if kc else b.t().contiguous(), kc)[0]
+    single = expected.float()
+    assert torch.equal(torch.isnan(single), torch.isnan(got)) and torch.equal(torch.isinf(single), torch.isinf(got))
+    fine = torch.isfinite(single)
+    assert torch.equal(single[~fine].nan_to_num(nan=0), got[~fine].nan_to_num(nan=0))
+    assert bool(((expected - got.double()).abs()[fine] <= 1e-5 * (a[0].double().abs().nan_to_num(0, 0) @ b.double().abs().nan_to_num(0, 0, 0).t())[fine]).all())
+
+
+def test_gemm_picks_the_same_result_whatever_kernel(tuning):
+    """Sizes on both sides of the rules that pick the bf16 kernel, against the kernels it takes over from."""
+    for M, N, K, kc in ((512, 3072, 512, False), (2048, 3072, 512, False), (1024, 3072, 768, True), (4096, 1024, 768, True), (2048, 1001, 256, True),
+                        (64, 1002, 768, False), (64, 1002, 96, False), (64, 1002, 100, False), (3000, 2000, 776, True)):
+        a, b = torch.randn(1, M, K, device="cuda"), torch.randn(*((N, K) if kc else (K, N)), device="cuda")
+        tuning(MI355X_GEMM_SPLIT=None)
+        chosen = split_gemm(a, b, kc)
+        tuning(MI355X_GEMM_SPLIT=0)
+        assert worst(split_gemm(a, b, kc).double(), chosen) < 5e-6   # two roundings of 2^-24 sqrt(K) each, five sigma
