@@ -52,6 +52,8 @@ SIGNATURES: typing.Dict[str, typing.Tuple[typing.Any, typing.List[typing.Any]]] 
     "mi355x_softmax_f32": (_int, [_vp, _vp, _i64, _i64, _i64, _vp]),
     "mi355x_attention_f32": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,
                                     _c_i64_p, _c_i64_p, _c_i64_p, _c_i64_p, _f32, _vp]),
+    "mi355x_attention_masked_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,
+                                           _c_i64_p, _c_i64_p, _c_i64_p, _c_i64_p, _c_i64_p, _f32, _vp]),
     "mi355x_layernorm_f32": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _f32, _vp]),
     "mi355x_reduce_mean_f32": (_int, [_vp, _vp, _i64, _i64, _i64, _vp]),
     "mi355x_maxpool2d_f32": (_int, [_vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _c_i64_p, _c_i64_p, _c_i64_p, _vp]),

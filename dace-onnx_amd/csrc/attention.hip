@@ -33,6 +33,7 @@ struct AttnArgs {
     int64_t batch1, Sq, Sk, q_blocks, nwg;
     int64_t q_sb0, q_sb1, q_sr, k_sb0, k_sb1, k_sr, v_sb0, v_sb1, v_sr, o_sb0, o_sb1, o_sr;
     float scale;
+    const float* mask; int64_t m_sb0, m_sb1, m_sr;   // masked form: added to scale * Q K^T, keys contiguous, 0 strides broadcast
 };
 
 __device__ __forceinline__ float quad_lanes_max(float v) {  // over lanes li, li+16, li+32, li+48
@@ -170,6 +171,13 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(AttnArgs p) {
 // the end). Keys beyond Sk in the last block are loaded from the last valid row and their scores set to
 // -inf. Every wave takes part in the barriers of every block, so there is no early exit for query rows
 // beyond Sq: they are computed on the clamped last row and not stored.
+//
+// MASKED: scale * Q K^T + mask, the padding mask of a batch of unequal sentences (or any mask of the scores' shape up to
+// broadcasting). The scores stay in natural units then and the difference to the maximum is scaled by log2(e): a mask of the
+// type's lowest value times log2(e) would overflow, and a row of such keys only is a uniform softmax, as node by node. A block
+// whose keys are all -inf leaves the running sums alone; a row of them only is NaN at the end (0 / 0), also as node by node.
+// The nodes one at a time (two products, the addition, the softmax) took 406 us on 16 x 12 slices of 512 x 512 scores.
+template <bool MASKED>
 __global__ __launch_bounds__(256) void attention_f32_blocks_kernel(AttnArgs p) {
     constexpr int SK = AT_SK, D = AT_D, PITCH = AT_PITCH, NJ = SK / 16, NC = D / 16;
     __shared__ __attribute__((aligned(16))) float lds_k[SK * PITCH];
@@ -199,7 +207,13 @@ __global__ __launch_bounds__(256) void attention_f32_blocks_kernel(AttnArgs p) {
 #pragma unroll
     for (int t = 0; t < 4; ++t) out[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY, l_run = 0.f;   // of query row q0 + li (the same value in its four lanes)
-    const float c = p.scale * 1.44269504088896340736f;   // scores in units of log2: exp(scale s - m) = 2^(c s - m')
+    constexpr float LOG2E = 1.44269504088896340736f;
+    const float c = MASKED ? p.scale : p.scale * LOG2E;   // unmasked: scores in units of log2, exp(scale s - m) = 2^(c s - m')
+    const float* __restrict__ mask = nullptr;             // the mask's row of query q0 + li
+    if constexpr (MASKED) {
+        const int64_t qrow = q0 + li < p.Sq ? q0 + li : p.Sq - 1;
+        mask = p.mask + b0 * p.m_sb0 + b1 * p.m_sb1 + qrow * p.m_sr;
+    }
 
     for (int64_t key0 = 0; key0 < p.Sk; key0 += SK) {
         f32x4 rk[8], rv[8];
@@ -240,23 +254,34 @@ __global__ __launch_bounds__(256) void attention_f32_blocks_kernel(AttnArgs p) {
         float m_blk = -INFINITY;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
+            const int64_t key = key0 + 16 * j + 4 * lq;
             acc[j] *= c;
+            if constexpr (MASKED) {
+                f32x4 add;
+                if (!ragged) __builtin_memcpy(&add, mask + key, sizeof add);
+                else
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) add[r] = mask[key + r < p.Sk ? key + r : p.Sk - 1];
+                acc[j] += add;
+            }
             if (ragged) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    if (key0 + 16 * j + 4 * lq + r >= p.Sk) acc[j][r] = -INFINITY;
+                    if (key + r >= p.Sk) acc[j][r] = -INFINITY;
             }
             m_blk = fmaxf(m_blk, fmaxf(fmaxf(acc[j].x, acc[j].y), fmaxf(acc[j].z, acc[j].w)));
         }
         const float m_new = fmaxf(m_run, quad_lanes_max(m_blk));
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);    // 0 for the first block
+        const float m_ref = MASKED && m_new == -INFINITY ? 0.f : m_new;   // nothing but -inf so far: 2^(-inf - 0) = 0
+        auto power = [&](float v) { return __builtin_amdgcn_exp2f(MASKED ? (v - m_ref) * LOG2E : v - m_ref); };
+        const float alpha = power(m_run);    // 0 for the first block
         float sum = 0.f;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            acc[j].x = __builtin_amdgcn_exp2f(acc[j].x - m_new);
-            acc[j].y = __builtin_amdgcn_exp2f(acc[j].y - m_new);
-            acc[j].z = __builtin_amdgcn_exp2f(acc[j].z - m_new);
-            acc[j].w = __builtin_amdgcn_exp2f(acc[j].w - m_new);
+            acc[j].x = power(acc[j].x);
+            acc[j].y = power(acc[j].y);
+            acc[j].z = power(acc[j].z);
+            acc[j].w = power(acc[j].w);
             sum += (acc[j].x + acc[j].y) + (acc[j].z + acc[j].w);
         }
         l_run = l_run * alpha + quad_lanes_sum(sum);
@@ -294,12 +319,12 @@ __global__ __launch_bounds__(256) void attention_f32_blocks_kernel(AttnArgs p) {
 
 }  // namespace mi355x
 
-extern "C" int mi355x_attention_f32(const float* Q, const float* K, const float* V, float* O,
-                                    int64_t batch0, int64_t batch1, int64_t Sq, int64_t Sk, int64_t D,
-                                    const int64_t* q_strides, const int64_t* k_strides,
-                                    const int64_t* v_strides, const int64_t* o_strides,
-                                    float scale, void* stream) {
-    using namespace mi355x;
+namespace mi355x {
+
+// mask == nullptr: the unmasked product
+static int launch_attention(const float* Q, const float* K, const float* V, float* O, const float* mask, int64_t batch0,
+                            int64_t batch1, int64_t Sq, int64_t Sk, int64_t D, const int64_t* q_strides, const int64_t* k_strides,
+                            const int64_t* v_strides, const int64_t* o_strides, const int64_t* mask_strides, float scale, void* stream) {
     MI355X_REQUIRE(batch0 >= 0 && batch1 >= 0 && Sq >= 0, "attention: negative extent");
     MI355X_REQUIRE(Sk >= 1 && D == AT_D, "attention: head size 64 and at least one key are required (got %lld keys x %lld)",
                    (long long)Sk, (long long)D);
@@ -322,6 +347,12 @@ extern "C" int mi355x_attention_f32(const float* Q, const float* K, const float*
     p.v_sb0 = v_strides[0]; p.v_sb1 = v_strides[1]; p.v_sr = v_strides[2];
     p.o_sb0 = o_strides[0]; p.o_sb1 = o_strides[1]; p.o_sr = o_strides[2];
     p.scale = scale;
+    p.mask = mask;
+    p.m_sb0 = mask ? mask_strides[0] : 0; p.m_sb1 = mask ? mask_strides[1] : 0; p.m_sr = mask ? mask_strides[2] : 0;
+    if (mask) {
+        hipLaunchKernelGGL(attention_f32_blocks_kernel<true>, dim3((unsigned)p.nwg), dim3(256), 0, static_cast<hipStream_t>(stream), p);
+        return check_launch("attention_f32_blocks_kernel");
+    }
     if (Sk == AT_SK) {
         // MI355X_ATTN_WAVES = 2 / 3: 32 / 48 query rows per workgroup instead of 64 (measured on 8 x 12 slices of 128 rows:
         // 384 / 288 workgroups instead of 192 -- no faster, the time is one wave's chain of loads, 256 MFMAs and stores)
@@ -336,6 +367,26 @@ extern "C" int mi355x_attention_f32(const float* Q, const float* K, const float*
         else hipLaunchKernelGGL(attention_f32_kernel<4>, g, dim3(256), 0, st, p);
         return check_launch("attention_f32_kernel");
     }
-    hipLaunchKernelGGL(attention_f32_blocks_kernel, dim3((unsigned)p.nwg), dim3(256), 0, static_cast<hipStream_t>(stream), p);
+    hipLaunchKernelGGL(attention_f32_blocks_kernel<false>, dim3((unsigned)p.nwg), dim3(256), 0, static_cast<hipStream_t>(stream), p);
     return check_launch("attention_f32_blocks_kernel");
+}
+
+}  // namespace mi355x
+
+extern "C" int mi355x_attention_f32(const float* Q, const float* K, const float* V, float* O,
+                                    int64_t batch0, int64_t batch1, int64_t Sq, int64_t Sk, int64_t D,
+                                    const int64_t* q_strides, const int64_t* k_strides,
+                                    const int64_t* v_strides, const int64_t* o_strides,
+                                    float scale, void* stream) {
+    return mi355x::launch_attention(Q, K, V, O, nullptr, batch0, batch1, Sq, Sk, D, q_strides, k_strides, v_strides, o_strides, nullptr, scale, stream);
+}
+
+extern "C" int mi355x_attention_masked_f32(const float* Q, const float* K, const float* V, float* O, const float* mask,
+                                           int64_t batch0, int64_t batch1, int64_t Sq, int64_t Sk, int64_t D,
+                                           const int64_t* q_strides, const int64_t* k_strides,
+                                           const int64_t* v_strides, const int64_t* o_strides, const int64_t* mask_strides,
+                                           float scale, void* stream) {
+    using namespace mi355x;
+    MI355X_REQUIRE(batch0 * batch1 == 0 || Sq == 0 || (mask && mask_strides), "attention: null mask");
+    return launch_attention(Q, K, V, O, mask, batch0, batch1, Sq, Sk, D, q_strides, k_strides, v_strides, o_strides, mask_strides, scale, stream);
 }

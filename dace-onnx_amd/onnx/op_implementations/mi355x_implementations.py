@@ -643,7 +643,7 @@ class MI355XLogSoftmax(ONNXForward):
 
 @op_implementation(op="FusedAttention", name=IMPLEMENTATION_NAME)
 class MI355XFusedAttention(ONNXForward):
-    """``softmax(scale * Q K^T) V`` in one launch; scores stay in registers. The
+    """``softmax(scale * Q K^T [+ mask]) V`` in one launch; scores stay in registers. The
     operands are the arrays on the edges or the (shape, strides, offset) views the
     fusion pass attached (``_q_view`` ... ``_o_view``): head split / merge of a
     [B, S, H*D] projection is addressing, not a copy."""
@@ -687,15 +687,50 @@ class MI355XFusedAttention(ONNXForward):
         return ext[0], ext[1], Sq, Sk, D, strides
 
     @staticmethod
+    def _mask_strides(mask, batch, Sq, Sk):
+        """{b0, b1, row} strides of a contiguous mask broadcast to [*batch, Sq, Sk], or None where its keys are not contiguous
+        or it is larger than the scores. ``batch`` are the batch extents of the scores, ones included."""
+        if not _is_f32(mask) or not _contig(mask) or not mask.shape or mask.shape[-1] != Sk:
+            return None
+        extents = list(batch) + [Sq]
+        shape, strides = list(mask.shape[:-1]), list(mask.strides[:-1])
+        lead = len(shape) - len(extents)
+        if lead > 0 and any(e != 1 for e in shape[:lead]):
+            return None
+        shape, strides = [1] * -lead + shape[max(lead, 0):], [0] * -lead + strides[max(lead, 0):]
+        if any(e not in (1, want) for e, want in zip(shape, extents)):
+            return None
+        strides = [0 if e == 1 else st for e, st in zip(shape, strides)]
+        outer = [st for st, e in zip(strides[:-1], batch) if e != 1]   # the batch dimensions _plan keeps, in its order
+        return [0] * (2 - len(outer)) + outer + [strides[-1]]
+
+    @staticmethod
+    def _mask(node, state, sdfg):
+        """(has a mask, its strides)."""
+        if not any(e.dst_conn == "mask" for e in state.in_edges(node)):
+            return False, None
+        Q, K = (d for d, _ in MI355XFusedAttention._operands(node, state, sdfg)[:2])
+        return True, MI355XFusedAttention._mask_strides(in_desc_with_name(node, state, sdfg, "mask"), Q.shape[:-2], Q.shape[-2], K.shape[-2])
+
+    @staticmethod
     def forward_can_be_applied(node, state: SDFGState, sdfg: SDFG) -> bool:
         plan = MI355XFusedAttention._plan(MI355XFusedAttention._operands(node, state, sdfg))
-        return MI355XFusedAttention.supports(plan)
+        if not MI355XFusedAttention.supports(plan):
+            return False
+        masked, strides = MI355XFusedAttention._mask(node, state, sdfg)
+        return not masked or strides is not None
 
     @staticmethod
     def forward(node, state: SDFGState, sdfg: SDFG):
         descs = MI355XFusedAttention._operands(node, state, sdfg)
         b0, b1, Sq, Sk, D, strides = MI355XFusedAttention._plan(descs)
         offs = [o for _, o in descs]
+        masked, mask_strides = MI355XFusedAttention._mask(node, state, sdfg)
+        if masked:
+            return kernel_call_for_node(node, state, "mi355x_attention_masked_f32", [
+                Ptr("Q", offs[0]), Ptr("K", offs[1]), Ptr("V", offs[2]), Ptr("O", offs[3]), Ptr("mask"), b0, b1, Sq, Sk, D,
+                I64Array(strides[0]), I64Array(strides[1]), I64Array(strides[2]), I64Array(strides[3]), I64Array(mask_strides),
+                float(node.scale if node.scale is not None else 1.0), Stream()])
         return kernel_call_for_node(node, state, "mi355x_attention_f32", [
             Ptr("Q", offs[0]), Ptr("K", offs[1]), Ptr("V", offs[2]), Ptr("O", offs[3]), b0, b1, Sq, Sk, D,
             I64Array(strides[0]), I64Array(strides[1]), I64Array(strides[2]), I64Array(strides[3]),

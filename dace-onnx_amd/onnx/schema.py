@@ -144,11 +144,13 @@ SCHEMAS: typing.List[ONNXSchema] = [
                [ONNXParameter("output", "T")], [ONNXAttribute("mode", _A.String, "constant")],
                [ONNXTypeConstraint("T", _NUMERIC), ONNXTypeConstraint("tensor(int64)", [dace.int64])],
                "Pad `data` by `pads` = [begin_0, ..., begin_n, end_0, ..., end_n]."),
-    # Not an ONNX operator: the node the fusion pass puts in place of MatMul -> scale -> Softmax -> MatMul.
+    # Not an ONNX operator: the node the fusion pass puts in place of MatMul -> scale (-> Add of a mask) -> Softmax -> MatMul.
     ONNXSchema("FusedAttention", 1,
-               [ONNXParameter("Q", "T"), ONNXParameter("K", "T"), ONNXParameter("V", "T")], [ONNXParameter("O", "T")],
+               [ONNXParameter("Q", "T"), ONNXParameter("K", "T"), ONNXParameter("V", "T"), ONNXParameter("mask", "T", _O)],
+               [ONNXParameter("O", "T")],
                [ONNXAttribute("scale", _A.Float, 1.0)], [ONNXTypeConstraint("T", [dace.float32])],
-               "softmax(scale * Q K^T) V per batch entry; Q, O are [..., Sq, D], K, V are [..., Sk, D]."),
+               "softmax(scale * Q K^T + mask) V per batch entry; Q, O are [..., Sq, D], K, V are [..., Sk, D], the mask broadcasts to "
+               "[..., Sq, Sk]."),
     # Not an ONNX operator: a group of elementwise nodes merged by the fusion pass into one launch.
     ONNXSchema("FusedElementwise", 1, [ONNXParameter("X", "T", ONNXParameterType.Variadic)], [ONNXParameter("Y", "T")],
                [ONNXAttribute("program", _A.Ints), ONNXAttribute("immediates", _A.Floats), ONNXAttribute("kinds", _A.Ints)],

@@ -772,8 +772,8 @@ def _fuse_decomposed_gelu(sdfg: SDFG, state: SDFGState) -> int:
 
 # ----------------------------------------------------------------------------- attention
 def _fuse_attention(sdfg: SDFG, state: SDFGState) -> int:
-    """scores = alpha * (Q K^T); probs = Softmax(scores, last axis); ctx = probs V, every
-    intermediate single-use, becomes one FusedAttention node that reads Q, K, V and
+    """scores = alpha * (Q K^T) [+ mask]; probs = Softmax(scores, last axis); ctx = probs V, every
+    intermediate single-use, becomes one FusedAttention node that reads Q, K, V (and the mask) and
     writes ctx through the views the two MatMuls already carry. Runs after the view
     folds (so K^T and the head split are strides) and before the projections are
     widened (which only rebases those views)."""
@@ -792,6 +792,20 @@ def _fuse_attention(sdfg: SDFG, state: SDFGState) -> int:
             continue
         prod1 = _producer(state, scores)
         use2 = _next_op(sdfg, state, probs, "MatMul")
+        add, mask_e = None, None
+        if prod1 is not None and _is_op(prod1.src, "Add"):   # the scores plus a mask: the product behind it is what the node reads
+            add = prod1.src
+            for conn, other in (("A", "B"), ("B", "A")):
+                e, m = _in_edge(state, add, conn), _in_edge(state, add, other)
+                if e is None or m is None or not isinstance(e.src, AccessNode) or not isinstance(m.src, AccessNode):
+                    continue
+                behind = _producer(state, e.src)
+                if behind is not None and _is_op(behind.src, "MatMul") and _next_op(sdfg, state, e.src, "Add") is not None and \
+                        list(sdfg.arrays[e.src.data].shape) == list(sdfg.arrays[scores.data].shape):
+                    prod1, mask_e = behind, m
+                    break
+            else:
+                continue
         if prod1 is None or not _is_op(prod1.src, "MatMul") or use2 is None or use2.dst_conn != "A":
             continue
         mm1, mm2 = prod1.src, use2.dst
@@ -820,16 +834,22 @@ def _fuse_attention(sdfg: SDFG, state: SDFGState) -> int:
         plan = MI355XFusedAttention._plan([(Array(f32, v[0], v[1]), v[2]) for v in (qv, kv, vv, ov)])
         if not MI355XFusedAttention.supports(plan):
             continue
+        if mask_e is not None and MI355XFusedAttention._mask_strides(sdfg.arrays[mask_e.src.data], qv[0][:-2], plan[2], plan[3]) is None:
+            continue
         node = get_onnx_node("FusedAttention")(mm1.label + "_attention", scale=float(getattr(mm1, "_alpha", 1.0)))
         state.add_node(node)
         for conn, edge, view in (("Q", q_e, qv), ("K", kt_e, kv), ("V", v_e, vv)):
             node.add_in_connector(conn)
             state.add_edge(edge.src, None, node, conn, sdfg.make_array_memlet(edge.src.data))
             setattr(node, "_" + conn.lower() + "_view", tuple(view))
+        if mask_e is not None:
+            node.add_in_connector("mask")
+            state.add_edge(mask_e.src, None, node, "mask", sdfg.make_array_memlet(mask_e.src.data))
         node.add_out_connector("O")
         node._o_view = tuple(ov)
         out_access = o_e.dst
-        _drop_chain(sdfg, state, [mm1, sm, mm2], [q_e.src, kt_e.src, v_e.src, out_access])
+        _drop_chain(sdfg, state, [mm1, sm, mm2] + ([add] if add is not None else []),
+                    [q_e.src, kt_e.src, v_e.src, out_access] + ([mask_e.src] if mask_e is not None else []))
         state.add_edge(node, "O", out_access, None, sdfg.make_array_memlet(out_access.data))
         fused += 1
     return fused

@@ -207,6 +207,17 @@ int mi355x_attention_f32(const float* Q, const float* K, const float* V, float* 
                          const int64_t* v_strides, const int64_t* o_strides,
                          float scale, void* stream);
 
+/* The same with a mask added to the scaled scores before the softmax:
+ *   O[b0,b1] = softmax(scale * Q[b0,b1] K[b0,b1]^T + mask[b0,b1], over keys) V[b0,b1]
+ * mask_strides = {batch0, batch1, query row} in elements, 0 where the mask broadcasts; its keys are contiguous (any
+ * alignment). Replaces MatMul -> (Div | Mul) -> Add -> Softmax -> MatMul, what a batch of padded sentences runs
+ * (pure_implementations.py:77-79 between the nodes above). */
+int mi355x_attention_masked_f32(const float* Q, const float* K, const float* V, float* O, const float* mask,
+                                int64_t batch0, int64_t batch1, int64_t Sq, int64_t Sk, int64_t D,
+                                const int64_t* q_strides, const int64_t* k_strides,
+                                const int64_t* v_strides, const int64_t* o_strides, const int64_t* mask_strides,
+                                float scale, void* stream);
+
 /* ONNX LayerNormalization over the last axis, fp32, X is [rows, cols]:
  *   y = (x - mean) / sqrt(var + eps) * gamma + beta, biased variance.
  * The reference has no such node (opset 12); it runs the exporter's

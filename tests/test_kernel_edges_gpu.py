@@ -123,3 +123,29 @@ def test_gemm_picks_the_same_result_whatever_kernel(tuning):
         chosen = split_gemm(a, b, kc)
         tuning(MI355X_GEMM_SPLIT=0)
         assert worst(split_gemm(a, b, kc).double(), chosen) < 5e-6   # two roundings of 2^-24 sqrt(K) each, five sigma
+
+
+@pytest.mark.parametrize("sk", [1, 3, 127, 128, 129, 173, 300])
+@pytest.mark.parametrize("fill", [-10000.0, float(np.finfo(np.float32).min), -float("inf")])
+def test_masked_attention(sk, fill):
+    """The mask per key, per query row and per head; whole blocks and whole rows masked; a mask at an odd address."""
+    b0, b1, sq = 2, 3, 70
+    q, k, v = (torch.randn(b0, b1, n, 64, device="cuda") for n in (sq, sk, sk))
+    strides = lambda t: _lib.i64_array([t.stride(0), t.stride(1), t.stride(2)])   # noqa: E731
+    for shape in ((b0, 1, 1, sk), (1, 1, sq, sk), (b0, b1, sq, sk), (1, 1, 1, sk)):
+        buffer = torch.where(torch.rand(int(np.prod(shape)) + 1, device="cuda") < 0.3, fill, 0.0)
+        mask = buffer[1:].view(shape)
+        mask[..., :max(0, sk - 3)] = mask[..., :max(0, sk - 3)] if sk < 200 else fill   # a first block without one valid key
+        mask[0, 0, 0] = fill                                                            # a row without one (all of them if it is broadcast)
+        wide = mask.expand(b0, b1, sq, sk)
+        out = torch.full((b0, b1, sq, 64), np.nan, device="cuda")
+        call("mi355x_attention_masked_f32", q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), mask.data_ptr(), b0, b1, sq, sk, 64,
+             strides(q), strides(k), strides(v), strides(out),
+             _lib.i64_array([st if e > 1 else 0 for st, e in zip(mask.stride()[:3], shape)]), 0.125)
+        # the scores in fp32 as the nodes compute them: a mask of the type's lowest value absorbs them there
+        scores = (0.125 * (q.double() @ k.double().transpose(-1, -2).contiguous())).float() + wide
+        expected = torch.softmax(scores.double(), -1) @ v.double()
+        nan = torch.isnan(expected)
+        assert torch.equal(nan, torch.isnan(out))
+        # fp32 scores of up to 10 in magnitude: 2^-21 relative on a probability; -10000 leaves 2^-11 of rounding in a row of masked keys only
+        assert float((expected - out.double()).abs().nan_to_num(0).max()) < (2e-5 if fill != -10000.0 else 5e-3)
