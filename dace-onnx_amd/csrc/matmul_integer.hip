@@ -59,21 +59,59 @@ __device__ __forceinline__ int32_t b_zero_point(const MMIArgs& p, int64_t n) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Any shape and alignment: 128 x 128 tile, register-staged loads, B transposed with byte permutes.
-//   * A [M,K] is k-contiguous: 16-byte global loads, LDS tile [128][64+16 B],
+// Any shape and alignment: register-staged loads, B transposed with byte permutes.
+//   * A [M,K] is k-contiguous: 16-byte global loads at any address, LDS tile [rows][BK+16 B],
 //     a lane's MFMA operand (16 consecutive k of one row) is one 16-byte read.
 //   * B [K,N] is n-contiguous but the MFMA wants 16 k of one COLUMN per lane.
 //     The loader transposes 4x4 byte blocks in registers (v_perm_b32) once per
 //     workgroup and stores LDS words holding 4 consecutive k of one column,
 //     laid out [k/4][n]: writes are 16 bytes per lane, contiguous; a lane then
-//     reads columns (2j, 2j+1) of four k-quads as 8-byte reads, contiguous
-//     across lanes. The k order inside an operand is the same for A and B, which
-//     is all an exact integer dot product needs.
-//   * A wave owns 64 x 64 of Y as 2 x 2 MFMA tiles; tile t holds columns 2j+t,
-//     so a lane stores (col 2j, col 2j+1) of one row as 8 bytes.
-constexpr int MMI_BM = 128, MMI_BN = 128, MMI_BK = 64;
-constexpr int MMI_A_PITCH = MMI_BK + 16;         // bytes per A row in LDS
-constexpr int MMI_B_PITCH = MMI_BN + 4;          // words per k-quad row in LDS
+//     reads columns T j .. T j + T - 1 of four k-quads, contiguous across lanes.
+//     The k order inside an operand is the same for A and B, which is all an exact
+//     integer dot product needs.
+//   * 2 x 2 waves of (32 T) x (32 T) of Y. T = 2: 128 x 128 tiles in steps of 64 k; T = 1: 64 x 64 tiles in steps of 128 k (the
+//     same loads per thread and step, four times the workgroups), for outputs that would leave most of the chip idle.
+// What bounds it: the latency of a step (loads, transpose, LDS, barrier) in few workgroups. Loading byte by byte where K or N is
+// odd, as this kernel once did, cost 4 us per step. Whole vectors from unaligned addresses, clamped at the end of the matrix and
+// masked past the end of K, and loads two steps ahead (M x N x K, before and after): 197 x 1001 x 501 58 -> 8.8 us, 73 x 139 x 689
+// 72 -> 10.6, 1000 x 1000 x 1000 101 -> 13.2, 4096 x 3071 x 769 209 -> 75, 8192 x 2047 x 1531 537 -> 159; looking one step ahead
+// 197 x 1001 x 501 took 11.6 us, 8192 x 2047 x 1531 203.
+constexpr int mmi_bk(int t) { return t == 2 ? 64 : 128; }
+constexpr int mmi_tile(int t) { return 64 * t; }
+
+// 16 bytes from byte `off` of a matrix of `total` >= 16 bytes, whatever the alignment. Near its end the last 16 are loaded:
+// settle_bytes_16 then moves those from `off` on to the front.
+__device__ __forceinline__ u32x4 load_bytes_16(const int8_t* base, int64_t off, int64_t total) {
+    u32x4 v;
+    __builtin_memcpy(&v, base + (off < total - 16 ? off : total - 16), 16);
+    return v;
+}
+__device__ __forceinline__ u32x4 settle_bytes_16(u32x4 v, int64_t off, int64_t total) {
+    if (off <= total - 16) return v;
+    int d = (int)(off < total ? off - (total - 16) : 15);
+    uint64_t lo = v.x | (uint64_t)v.y << 32, hi = v.z | (uint64_t)v.w << 32;
+    if (d >= 8) { lo = hi; hi = 0; d -= 8; }
+    if (d > 0) { lo = lo >> (8 * d) | hi << (64 - 8 * d); hi >>= 8 * d; }
+    return u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+}
+// the first `bytes` bytes of v (any number, also <= 0 or >= 16), the others 0
+__device__ __forceinline__ u32x4 keep_bytes(u32x4 v, int64_t bytes) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const int64_t n = bytes - 4 * w;
+        v[w] &= n >= 4 ? ~0u : n <= 0 ? 0u : ~0u >> (32 - 8 * (int)n);
+    }
+    return v;
+}
+// the same with 4 bytes of a matrix of `total` >= 4
+__device__ __forceinline__ uint32_t load_bytes_4(const int8_t* base, int64_t off, int64_t total) {
+    uint32_t v;
+    __builtin_memcpy(&v, base + (off < total - 4 ? off : total - 4), 4);
+    return v;
+}
+__device__ __forceinline__ uint32_t settle_bytes_4(uint32_t v, int64_t off, int64_t total) {
+    return off <= total - 4 ? v : v >> (8 * (uint32_t)(off - (total - 4)) & 31u);
+}
 
 __device__ __forceinline__ uint32_t perm_b32(uint32_t hi, uint32_t lo, uint32_t sel) {
     return __builtin_amdgcn_perm(hi, lo, sel);
@@ -91,180 +129,186 @@ __device__ __forceinline__ void transpose_4x4_bytes(const uint32_t (&r)[4], uint
     o[3] = perm_b32(t23_hi, t01_hi, 0x07060302u);
 }
 
-template <bool VEC>
+// A needs 16 bytes and B four (launch precondition; smaller matrices are read byte by byte)
+template <int T, bool TINY>
 __global__ __launch_bounds__(256) void matmul_integer_i8_kernel(MMIArgs p) {
-    constexpr int BM = MMI_BM, BN = MMI_BN, BK = MMI_BK, NT = 256;
-    __shared__ __attribute__((aligned(16))) int8_t lds_a[2][BM * MMI_A_PITCH];
-    __shared__ __attribute__((aligned(16))) uint32_t lds_b[2][(BK / 4) * MMI_B_PITCH];
-    __shared__ int32_t lds_rowsum[4][64];
+    constexpr int BM = mmi_tile(T), BN = mmi_tile(T), BK = mmi_bk(T), NT = 256;
+    constexpr int A_PITCH = BK + 16, B_PITCH = BN + 4;   // bytes per A row, words per k-quad row in LDS
+    __shared__ __attribute__((aligned(16))) int8_t lds_a[2][BM * A_PITCH];
+    __shared__ __attribute__((aligned(16))) uint32_t lds_b[2][(BK / 4) * B_PITCH];
+    __shared__ int32_t lds_rowsum[4][32 * T];
 
     const int tid = threadIdx.x;
     const int lane = tid % WAVE, wave = tid / WAVE;
     const int lj = lane % 32, lg = lane / 32;
-    const int wm0 = (wave / 2) * 64, wn0 = (wave % 2) * 64;
+    const int wm0 = (wave / 2) * 32 * T, wn0 = (wave % 2) * 32 * T;
 
-    const int64_t logical = xcd_remap(blockIdx.x, p.nwg);
-    const int64_t m0 = (logical / p.tiles_n) * BM, n0 = (logical % p.tiles_n) * BN;
-    // unsigned bytes become signed ones (u ^ 0x80 = u - 128) as they are loaded; bytes outside the matrix stay 0,
+    const uint32_t logical = (uint32_t)xcd_remap(blockIdx.x, p.nwg), tiles_n = (uint32_t)p.tiles_n;
+    const int64_t m0 = (int64_t)(logical / tiles_n) * BM, n0 = (int64_t)(logical % tiles_n) * BN;
+    // unsigned bytes become signed ones (u ^ 0x80 = u - 128) as they are loaded; bytes past K are 0,
     // so a padded k adds 0 to the product and to both sums
     const uint32_t a_flip = p.a_unsigned ? 0x80808080u : 0u, b_flip = p.b_unsigned ? 0x80808080u : 0u;
+    const int64_t a_total = p.M * p.K, b_total = p.K * p.N;
 
     // ---- loaders ----------------------------------------------------------------
-    // A: 128 rows x 4 vectors of 16 bytes -> 2 vectors per thread
-    // B: 16 k-quads x 32 column groups of 4 -> 2 units (4 rows x 4 cols) per thread
-    i32x4 ra[2];
-    uint32_t rb[2][4];
-    auto load_tiles = [&](int64_t k0) {
+    // A: BM rows x BK / 16 vectors of 16 bytes -> 2 vectors per thread; rows past M repeat the last one and are not stored
+    // B: BK / 4 k-quads x BN / 4 column groups -> 2 units (4 rows x 4 cols) per thread; columns past N are not stored
+    int64_t a_off[2], b_off[2];
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+        const int idx = tid + it * NT;
+        const int64_t gm = m0 + idx / (BK / 16);
+        a_off[it] = (gm < p.M ? gm : p.M - 1) * p.K + 16 * (idx % (BK / 16));
+        b_off[it] = (int64_t)(4 * (idx / (BN / 4))) * p.N + n0 + 4 * (idx % (BN / 4));
+    }
+    struct Raw { u32x4 a[2]; uint32_t b[2][4]; };
+    // loads only: what they bring is looked at two steps later
+    auto load_tiles = [&](Raw& raw, int64_t k0) {
 #pragma unroll
         for (int it = 0; it < 2; ++it) {
-            const int idx = tid + it * NT;
-            const int row = idx / 4, c16 = idx % 4;
-            const int64_t gm = m0 + row, gk = k0 + 16 * c16;
-            i32x4 v = i32x4{0, 0, 0, 0};
-            if (gm < p.M) {
-                const int8_t* src = p.A + gm * p.K + gk;
-                if constexpr (VEC) {
-                    if (gk < p.K) v = *reinterpret_cast<const i32x4*>(src) ^ (int)a_flip;
-                } else {
-                    uint32_t w[4] = {0, 0, 0, 0};
-                    for (int e = 0; e < 16; ++e)
-                        if (gk + e < p.K) w[e / 4] |= (uint32_t)((uint8_t)src[e] ^ (uint8_t)a_flip) << (8 * (e % 4));
-                    v = i32x4{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
-                }
+            if constexpr (TINY) {
+                raw.a[it] = u32x4{0u, 0u, 0u, 0u};
+                for (int e = 0; e < 16; ++e)
+                    if (a_off[it] + k0 + e < a_total) raw.a[it][e / 4] |= (uint32_t)(uint8_t)p.A[a_off[it] + k0 + e] << (8 * (e % 4));
+            } else {
+                raw.a[it] = load_bytes_16(p.A, a_off[it] + k0, a_total);
             }
-            ra[it] = v;
-        }
-#pragma unroll
-        for (int it = 0; it < 2; ++it) {
-            const int idx = tid + it * NT;
-            const int kq = idx / 32, cg = idx % 32;
-            const int64_t gn = n0 + 4 * cg;
-            uint32_t rows[4];
 #pragma unroll
             for (int rr = 0; rr < 4; ++rr) {
-                const int64_t gk = k0 + 4 * kq + rr;
-                uint32_t w = 0;
-                if (gk < p.K) {
-                    const int8_t* src = p.B + gk * p.N + gn;
-                    if constexpr (VEC) {
-                        if (gn < p.N) w = *reinterpret_cast<const uint32_t*>(src) ^ b_flip;
-                    } else {
-                        for (int e = 0; e < 4; ++e)
-                            if (gn + e < p.N) w |= (uint32_t)((uint8_t)src[e] ^ (uint8_t)b_flip) << (8 * e);
-                    }
+                const int64_t off = b_off[it] + (k0 + rr) * p.N;
+                if constexpr (TINY) {
+                    raw.b[it][rr] = 0u;
+                    for (int e = 0; e < 4; ++e)
+                        if (off + e < b_total) raw.b[it][rr] |= (uint32_t)(uint8_t)p.B[off + e] << (8 * e);
+                } else {
+                    raw.b[it][rr] = load_bytes_4(p.B, off, b_total);
                 }
-                rows[rr] = w;
             }
-            transpose_4x4_bytes(rows, rb[it]);
         }
     };
-    auto store_tiles = [&](int buf) {
+    auto store_tiles = [&](const Raw& raw, int buf, int64_t k0) {
+        const bool ragged = k0 + BK > p.K;   // uniform
 #pragma unroll
         for (int it = 0; it < 2; ++it) {
             const int idx = tid + it * NT;
-            const int row = idx / 4, c16 = idx % 4;
-            *reinterpret_cast<i32x4*>(lds_a[buf] + row * MMI_A_PITCH + 16 * c16) = ra[it];
-        }
+            const int c16 = idx % (BK / 16), kq = idx / (BN / 4);
+            u32x4 v = TINY ? raw.a[it] : settle_bytes_16(raw.a[it], a_off[it] + k0, a_total);
+            v ^= a_flip;
+            if (ragged) v = keep_bytes(v, p.K - k0 - 16 * c16);
+            *reinterpret_cast<u32x4*>(lds_a[buf] + idx / (BK / 16) * A_PITCH + 16 * c16) = v;
+            uint32_t rows[4], cols[4];
 #pragma unroll
-        for (int it = 0; it < 2; ++it) {
-            const int idx = tid + it * NT;
-            const int kq = idx / 32, cg = idx % 32;
-            *reinterpret_cast<i32x4*>(lds_b[buf] + kq * MMI_B_PITCH + 4 * cg) =
-                i32x4{(int)rb[it][0], (int)rb[it][1], (int)rb[it][2], (int)rb[it][3]};
+            for (int rr = 0; rr < 4; ++rr) {
+                rows[rr] = (TINY ? raw.b[it][rr] : settle_bytes_4(raw.b[it][rr], b_off[it] + (k0 + rr) * p.N, b_total)) ^ b_flip;
+                if (ragged && k0 + 4 * kq + rr >= p.K) rows[rr] = 0u;
+            }
+            transpose_4x4_bytes(rows, cols);
+            *reinterpret_cast<u32x4*>(lds_b[buf] + kq * B_PITCH + 4 * (idx % (BN / 4))) = u32x4{cols[0], cols[1], cols[2], cols[3]};
         }
     };
 
-    i32x16 acc[2][2];
+    i32x16 acc[T][T];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < T; ++i)
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < T; ++t)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][t][r] = 0;
-    int32_t rowsum[2] = {0, 0};  // partial: rows wm0+32i+lj, this lane's k half
-    int32_t colsum[2] = {0, 0};  // partial: cols wn0+2*lj+t, this lane's k half
+    int32_t rowsum[T] = {};  // partial: rows wm0+32i+lj, this lane's k half
+    int32_t colsum[T] = {};  // partial: cols wn0+T*lj+t, this lane's k half
 
-    const int64_t ktiles = (p.K + BK - 1) / BK;
-    load_tiles(0);
-    store_tiles(0);
-    __syncthreads();
-    for (int64_t kt = 0; kt < ktiles; ++kt) {
-        const int buf = (int)(kt & 1);
-        if (kt + 1 < ktiles) load_tiles((kt + 1) * BK);
+    auto multiply = [&](int buf) {
 #pragma unroll
         for (int ks = 0; ks < BK / 32; ++ks) {
             // lane (lj, lg): k-quads 8*ks + 4*lg + {0..3} of this 32-k step
-            i32x4 af[2], bf[2];
+            i32x4 af[T], bf[T];
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
-                af[i] = *reinterpret_cast<const i32x4*>(lds_a[buf] + (wm0 + 32 * i + lj) * MMI_A_PITCH +
-                                                        32 * ks + 16 * lg);
+            for (int i = 0; i < T; ++i)
+                af[i] = *reinterpret_cast<const i32x4*>(lds_a[buf] + (wm0 + 32 * i + lj) * A_PITCH + 32 * ks + 16 * lg);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const i32x2 w = *reinterpret_cast<const i32x2*>(
-                    lds_b[buf] + (8 * ks + 4 * lg + q) * MMI_B_PITCH + wn0 + 2 * lj);
-                bf[0][q] = w.x;
-                bf[1][q] = w.y;
+                const uint32_t* src = lds_b[buf] + (8 * ks + 4 * lg + q) * B_PITCH + wn0 + T * lj;
+                if constexpr (T == 2) {
+                    const i32x2 w = *reinterpret_cast<const i32x2*>(src);
+                    bf[0][q] = w.x;
+                    bf[T - 1][q] = w.y;
+                } else {
+                    bf[0][q] = (int)*src;
+                }
             }
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < T; ++i)
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
                     rowsum[i] = __builtin_amdgcn_sdot4(af[i][q], 0x01010101, rowsum[i], false);
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
+            for (int t = 0; t < T; ++t)
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
                     colsum[t] = __builtin_amdgcn_sdot4(bf[t][q], 0x01010101, colsum[t], false);
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < T; ++i)
 #pragma unroll
-                for (int t = 0; t < 2; ++t)
+                for (int t = 0; t < T; ++t)
                     acc[i][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bf[t], acc[i][t], 0, 0, 0);
         }
-        if (kt + 1 < ktiles) store_tiles(buf ^ 1);
+    };
+
+    // tile kt is multiplied while kt + 1 (loaded a step ago) goes to LDS and kt + 2 is on its way
+    const int64_t ktiles = (p.K + BK - 1) / BK;
+    Raw even, odd;
+    if (ktiles > 0) load_tiles(even, 0);
+    if (ktiles > 1) load_tiles(odd, BK);
+    if (ktiles > 0) store_tiles(even, 0, 0);
+    __syncthreads();
+    auto step = [&](int64_t kt, int buf, Raw& next, Raw& after) {
+        if (kt + 2 < ktiles) load_tiles(after, (kt + 2) * BK);
+        multiply(buf);
+        if (kt + 1 < ktiles) store_tiles(next, buf ^ 1, (kt + 1) * BK);
         __syncthreads();
+    };
+    for (int64_t kt = 0; kt < ktiles; kt += 2) {
+        step(kt, 0, odd, even);
+        if (kt + 1 < ktiles) step(kt + 1, 1, even, odd);
     }
 
     // ---- zero-point correction ---------------------------------------------------
     // combine the two k halves (lanes l and l^32)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) rowsum[i] += __shfl_xor(rowsum[i], 32, WAVE);
+    for (int i = 0; i < T; ++i) rowsum[i] += __shfl_xor(rowsum[i], 32, WAVE);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) colsum[t] += __shfl_xor(colsum[t], 32, WAVE);
+    for (int t = 0; t < T; ++t) colsum[t] += __shfl_xor(colsum[t], 32, WAVE);
     // a lane needs the row sums of the 16 rows its accumulator registers hold
-    if (lg == 0) {
-        lds_rowsum[wave][lj] = rowsum[0];
-        lds_rowsum[wave][32 + lj] = rowsum[1];
-    }
+#pragma unroll
+    for (int i = 0; i < T; ++i)
+        if (lg == 0) lds_rowsum[wave][32 * i + lj] = rowsum[i];
     __syncthreads();
 
-    // acc[i][t][r] = Y[m0+wm0+32i + 8*(r/4)+4*lg+(r%4)][n0+wn0+2*lj+t]
-    const int64_t n = n0 + wn0 + 2 * lj;
-    uint32_t zbn[2], c2[2];   // zero point of the lane's two columns; colsum - K zb
+    // acc[i][t][r] = Y[m0+wm0+32i + 8*(r/4)+4*lg+(r%4)][n0+wn0+T*lj+t]
+    const int64_t n = n0 + wn0 + T * lj;
+    if (n >= p.N) return;
+    uint32_t zbn[T], c2[T];   // zero point of the lane's columns; colsum - K zb
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < T; ++t) {
         zbn[t] = n + t < p.N ? (uint32_t)b_zero_point(p, n + t) : 0u;
         c2[t] = (uint32_t)colsum[t] - (uint32_t)p.K * zbn[t];
     }
+    const uint32_t za_one = (uint32_t)a_zero_point(p, 0);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < T; ++i) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int row_in_tile = 8 * (r / 4) + 4 * lg + (r % 4);
             const int64_t m = m0 + wm0 + 32 * i + row_in_tile;
-            if (m >= p.M || n >= p.N) continue;
+            if (m >= p.M) continue;
             const uint32_t rs = (uint32_t)lds_rowsum[wave][32 * i + row_in_tile];
-            const uint32_t zam = (uint32_t)a_zero_point(p, m);
-            const int32_t y0 = (int32_t)((uint32_t)acc[i][0][r] - zbn[0] * rs - zam * c2[0]);
-            const int32_t y1 = (int32_t)((uint32_t)acc[i][1][r] - zbn[1] * rs - zam * c2[1]);
+            const uint32_t zam = p.za_stride == 0 ? za_one : (uint32_t)a_zero_point(p, m);
             int32_t* dst = p.Y + m * p.N + n;
-            if constexpr (VEC) {
-                __builtin_nontemporal_store(i32x2{y0, y1}, reinterpret_cast<i32x2*>(dst));
-            } else {
-                dst[0] = y0;
-                if (n + 1 < p.N) dst[1] = y1;
-            }
+            int32_t y[T];
+#pragma unroll
+            for (int t = 0; t < T; ++t) y[t] = (int32_t)((uint32_t)acc[i][t][r] - zbn[t] * rs - zam * c2[t]);
+            if (T == 2 && n + 1 < p.N) __builtin_memcpy(dst, y, 4 * T);   // (8 bytes, 4-byte aligned)
+            else dst[0] = y[0];
         }
     }
 }
@@ -1008,8 +1052,8 @@ extern "C" int mi355x_matmul_integer(const void* A, const void* B, const void* a
     p.za_stride = a_zero_point && a_zero_point_count != 1 ? 1 : 0;
     p.zb_stride = b_zero_point && b_zero_point_count != 1 ? 1 : 0;
     p.a_unsigned = a_unsigned != 0; p.b_unsigned = b_unsigned != 0;
-    p.tiles_m = ceil_div(M, MMI_BM);
-    p.tiles_n = ceil_div(N, MMI_BN);
+    p.tiles_m = ceil_div(M, (int64_t)MMF_BM);
+    p.tiles_n = ceil_div(N, (int64_t)MMF_BN);
     p.nwg = p.tiles_m * p.tiles_n;
     MI355X_REQUIRE(p.nwg < ((int64_t)1 << 31), "matmul_integer: grid too large");
     auto al = [](const void* q, int a) { return (reinterpret_cast<uintptr_t>(q) & (a - 1)) == 0; };
@@ -1064,10 +1108,20 @@ extern "C" int mi355x_matmul_integer(const void* A, const void* B, const void* a
         else launch_stream<false>(p, grid, st);
         return check_launch("matmul_integer_i8_stream_kernel");
     }
-    // 16-byte A loads need K % 16 == 0; 4-byte B loads need N % 4 == 0; 8-byte Y stores need N % 2 == 0
-    const bool vec = (K % 16 == 0) && (N % 4 == 0) && al(A, 16) && al(B, 4) && al(Y, 8);
-    if (vec) hipLaunchKernelGGL(matmul_integer_i8_kernel<true>, dim3((unsigned)p.nwg), dim3(256), 0, st, p);
-    else hipLaunchKernelGGL(matmul_integer_i8_kernel<false>, dim3((unsigned)p.nwg), dim3(256), 0, st, p);
+    // Any other shape: 64 x 64 tiles up to three of them per CU (512 tiles on 256 CUs, 1024 x 2048 x 1000: 18.0 us against 26.9 us as
+    // 128 x 128; 1024 tiles, 2048 x 2000 x 777: 30.7 against 26.6 us; 197 x 1001 x 501: 8.8 against 16.8 us).
+    if (cus <= 0) return set_error(MI355X_ERR_NOT_INITIALIZED, "matmul_integer: no usable HIP device");
+    const int64_t small_nwg = ceil_div(M, (int64_t)mmi_tile(1)) * ceil_div(N, (int64_t)mmi_tile(1));
+    const bool tiny = M * K < 16 || K * N < 4;
+    const bool small = tiny || (tune.mmi_tile ? tune.mmi_tile == 64 : small_nwg <= 3 * (int64_t)cus);
+    p.tiles_m = ceil_div(M, (int64_t)mmi_tile(small ? 1 : 2));
+    p.tiles_n = ceil_div(N, (int64_t)mmi_tile(small ? 1 : 2));
+    p.nwg = p.tiles_m * p.tiles_n;
+    MI355X_REQUIRE(p.nwg < ((int64_t)1 << 31), "matmul_integer: grid too large");
+    const dim3 g((unsigned)p.nwg), b(256);
+    if (tiny) hipLaunchKernelGGL((matmul_integer_i8_kernel<1, true>), g, b, 0, st, p);
+    else if (small) hipLaunchKernelGGL((matmul_integer_i8_kernel<1, false>), g, b, 0, st, p);
+    else hipLaunchKernelGGL((matmul_integer_i8_kernel<2, false>), g, b, 0, st, p);
     return check_launch("matmul_integer_i8_kernel");
 }
 

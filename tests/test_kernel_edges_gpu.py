@@ -149,3 +149,25 @@ def test_masked_attention(sk, fill):
         assert torch.equal(nan, torch.isnan(out))
         # fp32 scores of up to 10 in magnitude: 2^-21 relative on a probability; -10000 leaves 2^-11 of rounding in a row of masked keys only
         assert float((expected - out.double()).abs().nan_to_num(0).max()) < (2e-5 if fill != -10000.0 else 5e-3)
+
+
+@pytest.mark.parametrize("tile", [0, 64, 128])
+@pytest.mark.parametrize("M, N, K", [(1, 1, 1), (3, 7, 5), (2, 9, 8), (5, 1, 3), (5, 1, 4), (1, 3, 300), (63, 65, 127), (64, 64, 112), (65, 129, 129),
+                                     (130, 66, 33), (128, 128, 144), (129, 127, 257), (200, 130, 385)])
+def test_matmul_integer_of_any_extent_and_address(tuning, tile, M, N, K):
+    """Whole vectors from any address, clamped at the end of a matrix: both operands end where their allocation's view ends, the
+    bytes around them are not theirs, and the result is exact."""
+    tuning(MI355X_MMI_TILE=tile)
+    rng = np.random.default_rng(M * N + K)
+    for a_unsigned, b_unsigned, shift in ((0, 0, 0), (1, 0, 1), (0, 1, 2), (1, 1, 3)):
+        a_low, b_low = (0 if a_unsigned else -128), (0 if b_unsigned else -128)
+        a, b = rng.integers(a_low, a_low + 256, (M, K)), rng.integers(b_low, b_low + 256, (K, N))
+        za, zb = rng.integers(a_low, a_low + 256, M if shift % 2 else 1), rng.integers(b_low, b_low + 256, N if shift % 2 == 0 else 1)
+        held = [np.full(shift + v.size + 5, 77, np.uint8) for v in (a, b)]
+        for memory, v in zip(held, (a, b)):
+            memory[shift:shift + v.size] = v.astype(np.int64).astype(np.uint8).reshape(-1)
+        ga, gb, gza, gzb = gpu(held[0]), gpu(held[1]), gpu(za.astype(np.int64) & 255).to(torch.uint8), gpu(zb.astype(np.int64) & 255).to(torch.uint8)
+        y = torch.full((M, N), -1, dtype=torch.int32, device="cuda")
+        call("mi355x_matmul_integer", ga.data_ptr() + shift, gb.data_ptr() + shift, gza.data_ptr(), gzb.data_ptr(), y.data_ptr(), M, N, K,
+             a_unsigned, b_unsigned, za.size, zb.size)
+        assert np.array_equal((a - za[:, None]) @ (b - zb[None, :]), y.cpu().numpy())
