@@ -32,4 +32,11 @@ bool launch_gemm_f32_ksplit(GemmArgs p, int cus, hipStream_t stream);
 // this one is below it.
 bool launch_gemm_f32_split(GemmArgs p, bool b_kc, double other_cost, int cus, hipStream_t stream);
 
+// Nanoseconds per k of its fastest form, 1e300 where it takes no such product.
+double gemm_f32_split_cost(const GemmArgs& p, int cus);
+
+// GEMM with A contiguous along k and B along k (b_kc) or n whose outputs are few tiles (gemm_f32_direct.hip): no staging, K split
+// over the waves of a workgroup. `other_cost`: nanoseconds the caller's own kernel takes; nothing is launched where it is not behind.
+bool launch_gemm_f32_direct(GemmArgs p, bool b_kc, double other_cost, int cus, hipStream_t stream);
+
 }  // namespace mi355x

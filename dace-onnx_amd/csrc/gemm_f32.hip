@@ -26,6 +26,8 @@
 #include "gemm_tile.h"
 #include "gemm_args.h"
 
+#include <algorithm>
+
 #include <stdlib.h>
 
 namespace mi355x {
@@ -245,6 +247,9 @@ extern "C" int mi355x_gemm_f32(const float* A, const float* B, float* C, const f
     // kernel's register ring is longer than their K, and 32 x 64 tiles of four waves fill the part better: 7.4 against
     // 9.1 us, 128 x 128 x 128 9.9 against 11.0 us, 128 x 128 x 32 6.1 against 8.2 us)
     const Tuning tune = tuning();
+    if (tune.gemm_direct > 0 && p.a_sk == 1 && (p.b_sk == 1 || p.b_sn == 1) &&
+        launch_gemm_f32_direct(p, p.b_sk == 1, 0, cus, static_cast<hipStream_t>(stream)))
+        return check_launch("gemm_f32_direct_kernel");
     const bool small_stack = batch > 1 && M <= 128 && N <= 128 && K <= 128 &&   // (a forced variant of that kernel is taken all the same)
                              tune.gemm_nt_bn == 0 && tune.gemm_nt_per_cu == 0 && tune.gemm_nt_bk == 0 && tune.gemm_nt_waves == 0 && tune.gemm_ksplit != 1;
     if (a_kc && b_kc && vec && tune.gemm_config < 0 && !small_stack) {
@@ -260,6 +265,15 @@ extern "C" int mi355x_gemm_f32(const float* A, const float* B, float* C, const f
     const bool split_a = p.a_sk == 1 && al16(A) && m4(p.a_sm) && m4(p.a_sb0) && m4(p.a_sb1);
     const bool split_kc = p.b_sk == 1 && al16(B) && m4(p.b_sn) && m4(p.b_sb0) && m4(p.b_sb1);
     const double generic_cost = vec ? 2.0 * (double)batch * (double)M * (double)N / 110e3 * 0.95 : 1e300;
+    // Few tiles: operands straight from memory into registers. The kernel below takes about 3 us and then 16 ns per k however small
+    // the product is (5 x 300 x 784 15.8 us, 5 x 10 x 300 9.6, without 16-byte accesses 33 x 1000 x 1503 44.7), or its throughput.
+    if (tune.gemm_config < 0 && tune.gemm_split < 0 && !small_stack && p.a_sk == 1 && (p.b_sk == 1 || p.b_sn == 1)) {
+        const bool split_fits = split_a && (split_kc || (p.b_sn == 1 && p.b_sk != 1)) && K >= 128;
+        const double generic = std::max(16.0 * (double)K, 2.0 * (double)batch * (double)M * (double)N * (double)K / (vec ? 110e3 : 60e3));
+        const double split = split_fits ? (double)K * gemm_f32_split_cost(p, cus) : 1e300;
+        const double other = 3000 + (vec || split == 1e300 ? std::min(generic, split) : split);   // (without 16-byte accesses the bf16 form is what follows)
+        if (launch_gemm_f32_direct(p, p.b_sk == 1, other, cus, static_cast<hipStream_t>(stream))) return check_launch("gemm_f32_direct_kernel");
+    }
     if (tune.gemm_config < 0 && split_a && (split_kc || (p.b_sn == 1 && p.b_sk != 1)) && (tune.gemm_split > 0 || K >= 128) &&
         launch_gemm_f32_split(p, split_kc, generic_cost, cus, static_cast<hipStream_t>(stream)))
         return check_launch("gemm_f32_split_kernel");

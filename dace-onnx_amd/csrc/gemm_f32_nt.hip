@@ -327,6 +327,13 @@ bool launch_gemm_f32_nt(GemmArgs p, int cus, hipStream_t stream) {
     // 768 64 against 85 us, 8192 x 3072 x 768 215 against 288, 4096 x 1024 x 768 48 against 60; 1024 x 3072 x 768 (42 against 40)
     // and everything smaller stays.
     const bool forced = force || tune.gemm_nt_bk || tune.gemm_nt_per_cu || tune.gemm_nt_waves || tune.gemm_group_m;
+    // Few tiles: the kernel that reads its operands straight from memory, where its sweep says it is ahead. In one round of
+    // workgroups these kernels take 2.8 us and per k 13.2 ns, 10.9 as sixteen waves (256, 768, 1024 x any of up to 256 tiles: 6.2,
+    // 13.1, 16.5 us; K = 3072 36.1 us).
+    const bool one_round = p.batch * ceil_div(p.M, (int64_t)64) * ceil_div(p.N, (int64_t)48) <= cus;
+    if (!forced && tune.gemm_split < 0 &&
+        launch_gemm_f32_direct(p, true, one_round ? 2800 + (double)p.K * (p.K >= 1280 ? 10.9 : 13.2) : 4.7e-3 * best_cost * (double)p.K, cus, stream))
+        return true;
     if (tune.gemm_split > 0 || (!forced && p.K >= 256))
         if (launch_gemm_f32_split(p, true, 4.7e-3 * 0.92 * best_cost, cus, stream)) return true;
     p.tiles_m = ceil_div(p.M, cands[best].bm);

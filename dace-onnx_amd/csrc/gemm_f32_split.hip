@@ -30,6 +30,8 @@
 #include "gemm_tile.h"
 #include "gemm_args.h"
 
+#include <algorithm>
+
 namespace mi355x {
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -302,12 +304,23 @@ static double split_cost(int form, int64_t nwg, int cus) {
     return 77.0 * (double)up;
 }
 
+static bool split_takes(const GemmArgs& p) {
+    // operands are addressed with 32-bit byte offsets from the start of a batch's matrix
+    return p.K % SP_BK == 0 && p.K > 0 && p.a_sm >= 0 && p.b_sn >= 0 && p.b_sk >= 0 && (p.M - 1) * p.a_sm + p.K < ((int64_t)1 << 29) &&
+           (p.N - 1) * p.b_sn + (p.K - 1) * p.b_sk + 1 < ((int64_t)1 << 29);
+}
+
+double gemm_f32_split_cost(const GemmArgs& p, int cus) {
+    double best = 1e300;
+    if (tuning().gemm_split == 0 || !split_takes(p)) return best;
+    for (int f = 0; f < 3; ++f)
+        best = std::min(best, split_cost(f, p.batch * ceil_div(p.M, (int64_t)kSplitForms[f].bm) * ceil_div(p.N, (int64_t)kSplitForms[f].bn), cus));
+    return best;
+}
+
 bool launch_gemm_f32_split(GemmArgs p, bool b_kc, double other_cost, int cus, hipStream_t stream) {
     const int force = tuning().gemm_split;
-    if (force == 0 || p.K % SP_BK != 0 || p.K == 0) return false;
-    // operands are addressed with 32-bit byte offsets from the start of a batch's matrix
-    if (p.a_sm < 0 || p.b_sn < 0 || p.b_sk < 0 || (p.M - 1) * p.a_sm + p.K >= ((int64_t)1 << 29) ||
-        (p.N - 1) * p.b_sn + (p.K - 1) * p.b_sk + 1 >= ((int64_t)1 << 29)) return false;
+    if (force == 0 || !split_takes(p)) return false;
     int best = -1;
     double best_cost = other_cost;
     for (int f = 0; f < 3; ++f) {

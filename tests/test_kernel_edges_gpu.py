@@ -114,14 +114,44 @@ def test_split_gemm_keeps_infinities_nan_and_the_largest_values(tuning, rows, kc
     assert bool(((expected - got.double()).abs()[fine] <= 1e-5 * (a[0].double().abs().nan_to_num(0, 0) @ b.double().abs().nan_to_num(0, 0, 0).t())[fine]).all())
 
 
+@pytest.mark.parametrize("form, kc", [(11, True), (12, True), (22, True), (14, False), (24, False)])
+@pytest.mark.parametrize("batch, M, N, K, epi", [(1, 1, 4, 4, 0), (1, 1, 5, 5, 1), (1, 15, 17, 15, 9), (2, 16, 16, 16, 0), (1, 17, 33, 18, 3), (3, 31, 63, 255, 13),
+                                                 (1, 33, 65, 257, 9), (1, 5, 10, 300, 1), (1, 40, 130, 1503, 8), (2, 7, 66, 3072, 9), (1, 64, 127, 4099, 0)])
+def test_gemm_straight_from_memory(tuning, form, kc, batch, M, N, K, epi):
+    """Every form at the edges of its tiles and of its waves' shares of K, from addresses that are only 4-byte aligned, between values
+    that would show; and an infinity stays in its row. Sums of K / 16 products by each wave, then sixteen: a rounding of 2^-24 each."""
+    tuning(MI355X_GEMM_DIRECT=form)
+    rng = np.random.default_rng(M + N + K)
+    held = [torch.full((n + 9,), np.nan, device="cuda") for n in (batch * M * K, N * K, N, batch * M * N)]
+    a, b, bias, res = (h[5:-4] for h in held)
+    for view in (a, b, bias, res):
+        view.copy_(gpu(rng.standard_normal(view.numel(), dtype=np.float32)))
+    a, b, res = a.view(batch, M, K), b.view(N, K) if kc else b.view(K, N), res.view(batch, M, N)
+    got = split_gemm(a, b, kc, bias, res, epi, 0.5, batch)
+    wide = b.double().t().contiguous() if kc else b.double()
+    expected = 0.5 * (a.double() @ wide) + (bias.double() if epi & 1 else 0)
+    if epi & 2:
+        expected = expected.relu()
+    if epi & 4:
+        expected = torch.nn.functional.gelu(expected)
+    if epi & 8:
+        expected = expected + res.double()
+    bound = (a.double().abs() @ wide.abs() + 1) * (K // 16 + 24) * 2.0**-24
+    assert bool(((expected - got.double()).abs() <= 1.2 * bound).all())   # 1.13 is Gelu's steepest slope
+    a[0, M - 1, K - 1] = float("inf")
+    got = split_gemm(a, b, kc, batch=batch)
+    assert bool(torch.isfinite(got).flatten()[:(M - 1) * N].all()) and bool(torch.isinf(got[0, M - 1]).all())
+
+
 def test_gemm_picks_the_same_result_whatever_kernel(tuning):
     """Sizes on both sides of the rules that pick the bf16 kernel, against the kernels it takes over from."""
     for M, N, K, kc in ((512, 3072, 512, False), (2048, 3072, 512, False), (1024, 3072, 768, True), (4096, 1024, 768, True), (2048, 1001, 256, True),
-                        (64, 1002, 768, False), (64, 1002, 96, False), (64, 1002, 100, False), (3000, 2000, 776, True)):
+                        (64, 1002, 768, False), (64, 1002, 96, False), (64, 1002, 100, False), (3000, 2000, 776, True),
+                        (16, 768, 3072, True), (128, 768, 768, True), (5, 300, 784, True), (33, 1000, 1503, True), (3, 1001, 512, False)):
         a, b = torch.randn(1, M, K, device="cuda"), torch.randn(*((N, K) if kc else (K, N)), device="cuda")
-        tuning(MI355X_GEMM_SPLIT=None)
+        tuning(MI355X_GEMM_SPLIT=None, MI355X_GEMM_DIRECT=None)
         chosen = split_gemm(a, b, kc)
-        tuning(MI355X_GEMM_SPLIT=0)
+        tuning(MI355X_GEMM_SPLIT=0, MI355X_GEMM_DIRECT=0)
         assert worst(split_gemm(a, b, kc).double(), chosen) < 5e-6   # two roundings of 2^-24 sqrt(K) each, five sigma
 
 
