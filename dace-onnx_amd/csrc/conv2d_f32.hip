@@ -18,64 +18,13 @@
 // L1, never from HBM: the activation tensor of a layer fits the 256 MB cache.
 #include "common.h"
 #include "gemm_tile.h"
+#include "conv_args.h"
 
 #include <stdlib.h>
 #include <type_traits>
 #include <utility>
 
 namespace mi355x {
-
-// n / d for 0 <= n < 2^31 as umulhi(n, mul) >> shr (d == 1 special-cased).
-struct FastDiv {
-    uint32_t d, mul, shr;
-};
-static FastDiv make_fastdiv(int64_t d) {
-    FastDiv f;
-    f.d = (uint32_t)d;
-    if (d == 1) { f.mul = 0; f.shr = 0; return f; }
-    uint32_t l = 0;
-    while ((1ull << l) < (uint64_t)d) ++l;  // ceil(log2 d)
-    const uint32_t p = 31 + l;
-    f.mul = (uint32_t)(((1ull << p) + (uint64_t)d - 1) / (uint64_t)d);
-    f.shr = p - 32;
-    return f;
-}
-__device__ __forceinline__ uint32_t fdiv(uint32_t n, const FastDiv& f) {
-    return f.d == 1 ? n : (__umulhi(n, f.mul) >> f.shr);
-}
-
-// The part of the epilogue after bias and activation: the residual (same layout as Y, hence the same
-// offset) and the activation that follows it (the last two steps of a ResNet block).
-__device__ __forceinline__ f32x4 conv_epilogue_tail4(f32x4 v, int epi, const float* residual, int64_t off) {
-    if (epi & MI355X_EPI_RESIDUAL) v += __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(residual + off));
-    if (epi & MI355X_EPI_RELU_AFTER) v = f32x4{fmaxf(v.x, 0.f), fmaxf(v.y, 0.f), fmaxf(v.z, 0.f), fmaxf(v.w, 0.f)};
-    return v;
-}
-__device__ __forceinline__ float conv_epilogue_tail1(float v, int epi, const float* residual, int64_t off) {
-    if (epi & MI355X_EPI_RESIDUAL) v += residual[off];
-    if (epi & MI355X_EPI_RELU_AFTER) v = fmaxf(v, 0.f);
-    return v;
-}
-
-struct ConvArgs {
-    const float* X; const float* W; const float* bias; float* Y;
-    const float* residual;   // laid out like Y; read only with MI355X_EPI_RESIDUAL
-    int N, C, H, Wd, M, KH, KW, OH, OW;
-    int pad_t, pad_l, stride_h, stride_w, dil_h, dil_w;
-    int K;          // C*KH*KW
-    int64_t P;      // N*OH*OW
-    int OHW;
-    FastDiv div_khw, div_kw, div_ohw, div_ow;
-    int64_t tiles_m, tiles_p, nwg;
-    int group_m;    // tile walk order, see tile_coords
-    int epi;
-    int vec_w;      // W tile may use 16-byte loads
-    int vec_y;      // Y may use 16-byte stores (OH*OW % 4 == 0, aligned)
-    int x_bytes;    // size of X (gather kernel only; below 2^31)
-    // gather kernel: the first full_tiles workgroups take whole tiles, the rest 16-position slices from p_full on
-    int64_t full_tiles, p_full;
-    MI355X_TRACE_MEMBER
-};
 
 template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, bool VEC_W>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void conv2d_f32_kernel(ConvArgs p) {
@@ -708,6 +657,13 @@ extern "C" int mi355x_conv2d_res_f32(const float* X, const float* W, const float
     if (K % CG_BK == 0 && K <= CG_MAX_K && KH * KW <= 32 && M * K < ((int64_t)1 << 29) && C * H * Wd < ((int64_t)1 << 27) &&
         N * C * H * Wd + pads[0] * Wd + pads[1] + H * Wd < ((int64_t)1 << 29) && al16(W) && tune.conv_config < 0) {
         p.x_bytes = (int)(N * C * H * Wd * 4);
+        // Few tiles: the kernel that reads its operands straight from memory, where its sweep says it is ahead. A round of 64 x 64
+        // tiles takes 15.3 ns per k and 6.5 us besides (8 to 200 tiles: K = 576 15 us, 1152 24, 2304 42, 4608 77), 1 x 1 filters
+        // 19 and 5.4 (K = 64 6.6, 128 7.8, 256 10.3).
+        if (tune.conv_gather_bn == 0 && tune.conv_per_cu == 0 && tune.conv_tail < 0 && tune.conv_static_taps == 1) {
+            const int64_t rounds = ceil_div(ceil_div(M, (int64_t)CG_BM) * ceil_div(P, (int64_t)64), (int64_t)cus);
+            if (launch_conv2d_f32_direct(p, KH * KW == 1 ? 5400 + 19.0 * (double)K * (double)rounds : 6500 + 15.3 * (double)K * (double)rounds, cus, st)) return check_launch("conv2d_f32_direct_kernel");
+        }
         // 64 x 64 tiles (three workgroups share a CU) or 64 x 128 (one per CU). Time goes with the tiles a CU has
         // to run times their width; the wide tile, alone on its CU, pays its first loads and last stores in the open
         // (32 x 64 x 56 x 56 -> 64: 101.5 us as 784 wide tiles, 73.2 us as 1568 narrow ones two to a CU), hence its factor.

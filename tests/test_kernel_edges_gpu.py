@@ -201,3 +201,34 @@ def test_matmul_integer_of_any_extent_and_address(tuning, tile, M, N, K):
         call("mi355x_matmul_integer", ga.data_ptr() + shift, gb.data_ptr() + shift, gza.data_ptr(), gzb.data_ptr(), y.data_ptr(), M, N, K,
              a_unsigned, b_unsigned, za.size, zb.size)
         assert np.array_equal((a - za[:, None]) @ (b - zb[None, :]), y.cpu().numpy())
+
+
+@pytest.mark.parametrize("form", [None, 11, 21, 22])
+@pytest.mark.parametrize("N, C, H, W, M, kernel, stride, pads, dilation", [(1, 32, 1, 1, 1, 1, 1, (0, 0, 0, 0), 1), (1, 32, 3, 3, 17, 3, 1, (1, 1, 1, 1), 1),
+                                                                           (2, 64, 5, 7, 33, 3, 2, (0, 2, 1, 0), 1), (1, 96, 9, 4, 16, 3, 1, (2, 1, 2, 3), 2),
+                                                                           (3, 544, 3, 3, 15, 3, 1, (1, 1, 1, 1), 1), (2, 32, 11, 6, 40, 1, 2, (0, 0, 0, 0), 1),
+                                                                           (1, 1056, 5, 5, 65, 1, 1, (1, 0, 0, 1), 1), (1, 512, 7, 7, 512, 3, 1, (1, 1, 1, 1), 1)])
+def test_convolution_of_few_tiles(tuning, form, N, C, H, W, M, kernel, stride, pads, dilation):
+    """Every form at the edges of its tiles and of its waves' shares of the channels, all steps of the epilogue, between values that
+    would show. Sums of K / 16 products by each wave, then sixteen: a rounding of 2^-24 each."""
+    tuning(MI355X_CONV_DIRECT=form)
+    rng = np.random.default_rng(N + C + M)
+    top, left, bottom, right = pads
+    rows, cols = ((e + a + b - dilation * (kernel - 1) - 1) // stride + 1 for e, a, b in ((H, top, bottom), (W, left, right)))
+    held = [torch.full((n + 12,), np.nan, device="cuda") for n in (N * C * H * W, M * C * kernel * kernel, M, N * M * rows * cols)]
+    x, w, bias, res = (h[4:-8] for h in held)
+    for view in (x, w, bias, res):
+        view.copy_(gpu(rng.standard_normal(view.numel(), dtype=np.float32)))
+    wide = torch.nn.functional.pad(x.view(N, C, H, W).double(), (left, right, top, bottom))
+    columns = torch.nn.functional.unfold(wide, kernel, dilation=dilation, stride=stride)
+    flat = w.view(M, -1).double()
+    product = torch.stack([flat @ c for c in columns]).view(N, M, rows, cols)
+    bound = torch.stack([flat.abs() @ c.abs() for c in columns]).view(N, M, rows, cols)
+    for epi in (0, 1 + 2, 1 + 8 + 16):   # bias and relu; bias, residual and relu after it
+        y = torch.full((N, M, rows, cols), np.nan, device="cuda")
+        call("mi355x_conv2d_res_f32", x.data_ptr(), w.data_ptr(), bias.data_ptr(), res.data_ptr(), y.data_ptr(), N, C, H, W, M, kernel, kernel,
+             _lib.i64_array(pads), _lib.i64_array([stride] * 2), _lib.i64_array([dilation] * 2), epi)
+        expected = product + (bias.double().view(1, M, 1, 1) if epi & 1 else 0) + (res.double().view(N, M, rows, cols) if epi & 8 else 0)
+        if epi:
+            expected = expected.relu()
+        assert bool(((expected - y.double()).abs() <= (bound + 8) * (C * kernel * kernel // 16 + 24) * 2.0**-24).all())
