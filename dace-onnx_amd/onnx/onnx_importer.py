@@ -13,6 +13,7 @@ The model is a :class:`dace_onnx_amd.onnx.proto.ModelProto`, a path to a
 uploaded once at construction.
 """
 import collections
+import functools
 import logging
 import re
 import copy
@@ -33,6 +34,7 @@ from .shape_inference import infer_shapes as _infer_shapes
 log = logging.getLogger(__name__)
 
 
+@functools.lru_cache(maxsize=4096)
 def clean_onnx_name(name: str) -> str:
     """Make an ONNX value name a valid array name (``daceml/onnx/converters.py:204-211``)."""
     if re.match("^[0-9]", name):

@@ -597,11 +597,14 @@ class CompiledSDFG:
                 raise RuntimeError(f"{n} was not expanded; call expand_library_nodes() first")
         self._lib = _lib.library()  # raises if the HIP library is not built
         self._external = [k for k, d in sdfg.arrays.items() if not d.transient]
+        self._torch_types = {k: sdfg.arrays[k].dtype.as_torch() for k in self._external}
+        self._returned = [k for k in self._external if k.startswith("__return")]
         self._written = self._find_written(sdfg)
         self._transients = {}   # flattened key -> descriptor
         self._transient_tensors = {}   # flattened key -> its allocation (made on first use, kept)
         self._plan = []         # ("call", node, connector -> key) | ("alias", src key, dst key, dst descriptor)
         self._bound_key = None
+        self._patches = None    # per launch, the pointer arguments that follow the caller's arrays (see _rebind)
         self._graph = None
         self._build(sdfg, prefix="", outer_map={})
 
@@ -651,11 +654,13 @@ class CompiledSDFG:
 
     # -- binding ---------------------------------------------------------------------
     def _bind(self, env):
-        """Resolve every pointer argument against ``env`` (key -> tensor). Transient tensors are allocated on the
-        first call and kept: binding again (the caller passed other buffers) only resolves pointers anew."""
+        """The launch list with every pointer argument resolved against ``env`` (key -> tensor), and the patches
+        :meth:`_rebind` needs for other buffers (``None`` if the list holds device copies). Transient tensors are
+        allocated on the first call and kept."""
         import torch
         env = dict(env)
-        launches = []
+        launches, patches = [], []
+        root = {k: k for k in self._external}   # key -> the caller's array it is (a view of)
         # A Reshape-like alias whose result is caller-owned memory: let the producer of its source write there
         # directly (the source, a transient, becomes a view of the caller's buffer). Walking the aliases backwards
         # carries this through chains of them. What cannot be redirected (the source is caller-owned too, or
@@ -680,6 +685,7 @@ class CompiledSDFG:
             _, src_key, dst_key, _ = item
             if dst_key in env and src_key not in env and src_key in self._transients and not read_before(position, dst_key):
                 env[src_key] = env[dst_key].reshape(self._transients[src_key].shape)
+                root[src_key] = root.get(dst_key)
                 redirected.add((src_key, dst_key))
         for item in self._plan:
             if item[0] == "alias":
@@ -689,12 +695,21 @@ class CompiledSDFG:
                 src = self._tensor(env, src_key)
                 if dst_key in env:
                     launches.append(("copy", env[dst_key], src))
+                    patches = None
                 else:
                     env[dst_key] = src.reshape(dst_desc.shape)  # contiguous -> view
+                    root[dst_key] = root.get(src_key)
                 continue
             _, node, conn_to_key = item
             fn = getattr(self._lib, node.function)
             args, keep, stream_slots = [], [], []
+            slots, arrays = [], []
+
+            def follow(connector, address):
+                """The caller's array behind a pointer and the byte offset into it; None for a transient."""
+                name = root.get(conn_to_key[connector])
+                return None if name is None else (name, address - env[name].data_ptr())
+
             for i, a in enumerate(node.args):
                 if isinstance(a, Ptr):
                     if a.connector is None:
@@ -702,6 +717,9 @@ class CompiledSDFG:
                     else:
                         t = self._tensor(env, conn_to_key[a.connector])
                         args.append(t.data_ptr() + a.offset * t.element_size())
+                        followed = follow(a.connector, args[-1])
+                        if followed:
+                            slots.append((i, *followed))
                 elif isinstance(a, Stream):
                     stream_slots.append(i)
                     args.append(None)
@@ -711,7 +729,9 @@ class CompiledSDFG:
                     args.append(arr)
                 elif isinstance(a, (U32Array, F32Array, PtrArray)):
                     if isinstance(a, PtrArray):
-                        arr = _lib.pointer_array([self._tensor(env, conn_to_key[c]).data_ptr() for c in a.connectors])
+                        addresses = [self._tensor(env, conn_to_key[c]).data_ptr() for c in a.connectors]
+                        arr = _lib.pointer_array(addresses)
+                        arrays.append((i, addresses, [follow(c, at) for c, at in zip(a.connectors, addresses)]))
                     else:
                         arr = (_lib.u32_array if isinstance(a, U32Array) else _lib.f32_array)(a.values)
                     keep.append(arr)
@@ -719,7 +739,23 @@ class CompiledSDFG:
                 else:
                     args.append(a)
             launches.append(("call", fn, node.function, args, stream_slots, keep, node))
-        return env, launches
+            if patches is not None:
+                patches.append((slots, arrays))
+        return launches, patches
+
+    def _rebind(self, launches, address):
+        """A launch list for other buffers of the caller (name -> address): the calls of ``launches`` with their
+        pointer arguments replaced. A call whose outputs are fresh tensors does this instead of resolving the plan
+        anew; the lists are copied because another thread may be walking the old ones."""
+        result = []
+        for item, (slots, arrays) in zip(launches, self._patches):
+            args = list(item[3])
+            for i, name, offset in slots:
+                args[i] = address[name] + offset
+            for i, addresses, followed in arrays:
+                args[i] = _lib.pointer_array([at if to is None else address[to[0]] + to[1] for at, to in zip(addresses, followed)])
+            result.append((*item[:3], args, *item[4:]))
+        return result
 
     def _tensor(self, env, key):
         """The tensor bound to ``key``; a transient that has none yet gets its allocation, made once per
@@ -749,13 +785,17 @@ class CompiledSDFG:
     def __call__(self, **kwargs):
         import torch
         sdfg = self.sdfg
-        unknown = set(kwargs) - set(sdfg.arrays)
-        if unknown:
+        if not kwargs.keys() <= sdfg.arrays.keys():
+            unknown = set(kwargs) - set(sdfg.arrays)
             raise TypeError(f"unknown arguments {sorted(unknown)} for SDFG {sdfg.name}")
         env, staged_back = {}, []
-        any_torch = any(isinstance(v, torch.Tensor) for v in kwargs.values())
         for name in self._external:
             desc = sdfg.arrays[name]
+            v = kwargs.get(name)
+            # (the checks below on the way that most arguments take: comparing descriptors took most of a call)
+            if isinstance(v, torch.Tensor) and v.dtype is self._torch_types[name] and v.shape == desc.shape and v.is_cuda and v.is_contiguous():
+                env[name] = v
+                continue
             if name not in kwargs:
                 if name == "__return" or name.startswith("__return"):
                     env[name] = torch.empty(desc.shape, dtype=desc.dtype.as_torch(), device=self.device)
@@ -784,20 +824,25 @@ class CompiledSDFG:
                 if name in self._written and isinstance(v, np.ndarray):
                     staged_back.append((v, d))
                 env[name] = d
-        key = tuple((n, env[n].data_ptr()) for n in self._external)
+        key = [env[n].data_ptr() for n in self._external]
         if key != self._bound_key:
-            self._env, self._launch_list = self._bind(env)
+            if self._bound_key is None or self._patches is None:
+                self._launch_list, self._patches = self._bind(env)
+            else:
+                self._launch_list = self._rebind(self._launch_list, dict(zip(self._external, key)))
+            self._env = env   # the caller's arrays live as long as the launch list points to them
             self._bound_key = key
             self._graph = None
-        self._run(self._launch_list)
+        launches = self._launch_list
+        self._run(launches)
         for host, dev in staged_back:
             if isinstance(host, np.ndarray):
                 host[...] = dev.cpu().numpy()
             else:
                 host.copy_(dev)
-        rets = [n for n in self._external if n.startswith("__return")]
-        if rets:
-            outs = [self._env[n] if any_torch else self._env[n].cpu().numpy() for n in rets]
+        if self._returned:
+            any_torch = any(isinstance(v, torch.Tensor) for v in kwargs.values())
+            outs = [env[n] if any_torch else env[n].cpu().numpy() for n in self._returned]
             return outs[0] if len(outs) == 1 else tuple(outs)
         return None
 
