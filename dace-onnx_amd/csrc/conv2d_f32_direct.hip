@@ -77,24 +77,23 @@ __global__ __launch_bounds__(WAVE * CD_WAVES) void conv2d_f32_direct_kernel(Conv
 
     float vw[RING][TM][STEPS], vx[RING][TP][STEPS];
     auto load = [&](int slot, int g) {
-        const uint32_t outside = g >= end ? 0x80000000u : 0u;
         const int w_g = (TAPS == 9 ? 144 : 64) * g, x_g = 4 * GROUP * hw * g;
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
 #pragma unroll
             for (int h = 0; h < STEPS / 4; ++h) {
-                const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, (int)((w_off[i] + 16u * h) | outside), w_g, 0));
+                const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, (int)(w_off[i] + 16u * h), w_g, 0));
 #pragma unroll
                 for (int e = 0; e < 4; ++e) vw[slot][i][4 * h + e] = v[e];
             }
-            if constexpr (STEPS == 9) vw[slot][i][8] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(w_rsrc, (int)((w_off[i] + 32u) | outside), w_g, 0));
+            if constexpr (STEPS == 9) vw[slot][i][8] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(w_rsrc, (int)(w_off[i] + 32u), w_g, 0));
         }
 #pragma unroll
         for (int j = 0; j < TP; ++j)
 #pragma unroll
             for (int s = 0; s < STEPS; ++s)
                 vx[slot][j][s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                    x_rsrc, (int)(x_off[j][TAPS == 9 ? s : 0] | outside), x_g + (TAPS == 9 ? 0 : 4 * s * hw), 0));
+                    x_rsrc, (int)x_off[j][TAPS == 9 ? s : 0], x_g + (TAPS == 9 ? 0 : 4 * s * hw), 0));
     };
     f32x4 acc[TM][TP];
 #pragma unroll
@@ -103,7 +102,8 @@ __global__ __launch_bounds__(WAVE * CD_WAVES) void conv2d_f32_direct_kernel(Conv
         for (int j = 0; j < TP; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
 #pragma unroll
-    for (int u = 0; u < RING; ++u) load(u, begin + u);
+    for (int u = 0; u < RING; ++u)
+        if (begin + u < end) load(u, begin + u);
     for (int g = begin; g < end; g += RING) {
         static_for<RING>([&](auto u) {
             if (g + u < end) {
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(WAVE * CD_WAVES) void conv2d_f32_direct_kernel(Conv
 #pragma unroll
                         for (int j = 0; j < TP; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vw[u][i][s], vx[u][j][s], acc[i][j], 0, 0, 0);
             }
-            load(u, g + u + RING);
+            if (g + u + RING < end) load(u, g + u + RING);   // (uniform; a load that is all out of range costs the address unit as much as any)
         });
     }
 
@@ -139,12 +139,13 @@ __global__ __launch_bounds__(WAVE * CD_WAVES) void conv2d_f32_direct_kernel(Conv
 
 // Nanoseconds: `fixed`, then per round of workgroups `round` and `per_k`, from the layers of a residual classifier over 1 to 16
 // images (weights not in the L2; 3 x 3 from K = 576 to 4608, 1 x 1 from 64 to 256). Bound by what a CU draws from its L2, the nine
-// 4-byte loads per four channels included: one image 64 x 56 x 56 -> 64 14.8 -> 9.3 us, 128 x 28 x 28 -> 128 23.5 -> 13.0,
-// 256 x 14 x 14 -> 256 41.4 -> 14.4, 512 x 7 x 7 -> 512 77.2 -> 22.5 (eight images 76.9 -> 41.8), 1 x 1 256 x 14 x 14 -> 512 10.0 -> 7.6;
-// eight images 256 x 14 x 14 -> 256 would be 43.2 against 41.7 and stay.
+// 4-byte loads per four channels included: one image 64 x 56 x 56 -> 64 14.8 -> 7.9 us, 128 x 28 x 28 -> 128 23.5 -> 10.7,
+// 256 x 14 x 14 -> 256 41.3 -> 12.4, 512 x 7 x 7 -> 512 77.0 -> 20.6, 1 x 1 256 x 14 x 14 -> 512 10.0 -> 4.1; four images
+// 512 x 7 x 7 -> 512 76.8 -> 32.5, 128 x 28 x 28 -> 128 23.8 -> 20.8, 64 x 56 x 56 -> 64 would be 22.5 against 15.4 and stay.
+// (Loads past a wave's share, which a branch now skips: 64 x 56 x 56 -> 64 9.0 us with them, 1 x 1 7.6.)
 struct ConvDirectForm { int taps, tm, tp; double fixed, round, per_k; };
-static const ConvDirectForm kConvDirectForms[] = {{9, 1, 1, 2500, 2200, 3.85}, {9, 2, 1, 3000, 2500, 6.2}, {9, 2, 2, 3000, 1900, 7.9},
-                                                  {1, 1, 1, 3000, 0, 18}, {1, 2, 1, 3000, 0, 25}, {1, 2, 2, 3000, 0, 42}};
+static const ConvDirectForm kConvDirectForms[] = {{9, 1, 1, 3000, 0, 3.8}, {9, 2, 1, 3200, 0, 6.2}, {9, 2, 2, 3200, 0, 7.8},
+                                                  {1, 1, 1, 2800, 750, 2.5}, {1, 2, 1, 2900, 850, 3.4}, {1, 2, 2, 3000, 1500, 3.5}};
 
 template <int TAPS>
 static void launch_direct(int form, const ConvArgs& p, hipStream_t st) {

@@ -76,7 +76,7 @@ __global__ __launch_bounds__(WAVE * GD_WAVES) void gemm_f32_direct_kernel(GemmAr
     auto load = [&](int slot, int c) {
         const int k = 16 * c + 4 * lq;
         const uint32_t kb = (uint32_t)min(k, K - 4);
-        const uint32_t outside = (c >= end || k >= K) ? 0x80000000u : 0u;
+        const uint32_t outside = k >= K ? 0x80000000u : 0u;
 #pragma unroll
         for (int i = 0; i < TM; ++i)
             va[slot][i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, (int)((a_row[i] + 4u * kb) | outside), 0, 0));
@@ -116,11 +116,12 @@ __global__ __launch_bounds__(WAVE * GD_WAVES) void gemm_f32_direct_kernel(GemmAr
     };
 
 #pragma unroll
-    for (int u = 0; u < RING; ++u) load(u, begin + u);
+    for (int u = 0; u < RING; ++u)
+        if (begin + u < end) load(u, begin + u);
     for (int c = begin; c < end; c += RING) {
         static_for<RING>([&](auto u) {
             if (c + u < end) multiply(u, c + u);
-            load(u, c + u + RING);
+            if (c + u + RING < end) load(u, c + u + RING);   // (uniform; a load that is all out of range costs the address unit as much as any)
         });
     }
 
@@ -144,13 +145,14 @@ __global__ __launch_bounds__(WAVE * GD_WAVES) void gemm_f32_direct_kernel(GemmAr
 
 // Nanoseconds, from sweeps over M of 1 to 512, N of 256 to 30522 and K of 256 to 3072 with weights that are not in the L2: a launch,
 // the first loads and the sum over the waves (`fixed`), then per k while every workgroup has a CU to itself (`alone`) or per
-// round of them. A CU draws 30 to 35 bytes a nanosecond whatever the form, which is the bound: 16 x 768 x 768 6.9 us (64 x 48 tiles
-// through LDS 13.1), 16 x 768 x 3072 14.8 (36.1), 128 x 768 x 768 8.8 (13.7), 128 x 768 x 3072 20.3 (36.3), 256 x 768 x 3072 26.7
-// (36.3), 33 x 1000 x 1503 10.0 (44.7), 16 x 30522 x 768 with B along n 21.6 (31.7); 128 x 2304 x 768 20.3 (14.1) stays where it was.
-// (32 x 16 tiles equal 16 x 32; 64 x 32 and 32 x 64 tiles are never ahead.)
+// round of them. A CU draws 30 to 40 bytes a nanosecond whatever the form, which is the bound: 16 x 768 x 768 5.7 us (64 x 48 tiles
+// through LDS 13.1), 16 x 768 x 3072 13.6 (36.1), 128 x 768 x 768 7.3 (13.7), 128 x 768 x 3072 19.0 (36.2), 256 x 768 x 3072 25.8
+// (36.4), 33 x 1000 x 1503 8.7 (44.6), 16 x 30522 x 768 with B along n 19.2 (31.6); 128 x 2304 x 768 17.1 (13.9) stays where it was.
+// (Loads past a wave's share, which a branch now skips, were up to half of the time: 16 x 768 x 768 6.9 us with them. 32 x 16
+// tiles equal 16 x 32; 64 x 32 and 32 x 64 tiles are never ahead; both halves of a 128-byte line by one pair of loads changes nothing.)
 struct DirectForm { int tm, tn; bool b_kc; double fixed, alone, round; };
-static const DirectForm kDirectForms[] = {{1, 1, true, 4200, 3.5, 4.9}, {1, 2, true, 5000, 5.0, 7.2}, {2, 2, true, 5900, 6.7, 9.4},
-                                          {1, 4, false, 4800, 6.5, 10.0}, {2, 4, false, 6500, 7.0, 12.5}};
+static const DirectForm kDirectForms[] = {{1, 1, true, 3100, 3.4, 3.6}, {1, 2, true, 3400, 5.0, 5.9}, {2, 2, true, 3800, 7.1, 8.5},
+                                          {1, 4, false, 3500, 5.8, 7.8}, {2, 4, false, 4000, 8.0, 11.5}};
 
 bool launch_gemm_f32_direct(GemmArgs p, bool b_kc, double other_cost, int cus, hipStream_t stream) {
     const int force = tuning().gemm_direct;
