@@ -1,20 +1,25 @@
 // fp32 GEMM on the bf16 matrix unit: every operand value is split into three bf16 numbers on its way into LDS.
 //
 // The fp32 MFMA of this part delivers 157 TFLOP/s, the bf16 one 2500. A float has 24 significant bits, a bf16 eight, so
-// x = hi + mid + lo exactly (round to nearest, subtract, round again; exact for |x| >= 2^-110, below that the last bits of lo
-// fall under the smallest bf16 subnormal). Of the nine products of two split values the six that reach 2^-24 of the result are
+// x = hi + mid + lo (round to nearest, subtract, round again), exactly: values are multiplied by 2^16 before they are split, so that
+// the last bit of the smallest float, 2^-149, is the smallest bf16 subnormal, 2^-133 (the MFMA takes subnormals as they are), and
+// sums by 2^-32 after. Split as they came, values below 2^-110 lost bits: against values that bring the sums back to ordinary size
+// 3.5e-5 (2-norm) at 2^-120 and everything below 2^-136, where 1.6e-7 is left now; the two multiplications of a pair cost 1 to 3 %.
+// Of the nine products of two split values the six that reach 2^-24 of the result are
 // multiplied, each exact in the fp32 accumulator of the MFMA: hi hi in one set of accumulators, the five small ones in a
 // second set, added at the end, so the long sum takes K / 32 roundings where the fp32 MFMA takes K / 4. Against float64 over
 // N(0, 1) operands the result is closer than the fp32 kernels': 1.6e-7 against 5.0e-7 (2-norm) at K = 768, 3.4e-7 against
-// 7.1e-7 at K = 3072; with one set of accumulators it was 4.2e-7 and 8.7e-7.
+// 7.1e-7 at K = 3072; with one set of accumulators it was 4.2e-7 and 8.7e-7. The three products left out show where a sum has few
+// terms: a single product is off by up to 1.0e-7, the rounded product of two floats by 6e-8.
 //
-// Infinities, NaN and values that round up to infinity in bf16 make a sum of the split form NaN or infinite whatever the exact
+// Infinities, NaN, values from 2^112 and sums from 2^96 on make a sum of the split form NaN or infinite whatever the exact
 // product is. A wave whose sums are not all finite computes its part of the tile again with the fp32 MFMA, straight from
 // global memory: the result of such inputs is that of the fp32 kernels, only slower.
 //
-// What bounds it: the LDS. Per 32-k step of a 256 x 128 tile the eight waves issue 3072 cycles of MFMA per SIMD, 192 fragment reads
-// (8 cycles each) and 72 plane writes (16 cycles each, whatever the width). Measured on 8192 x 1024 x 3072 (263 us): without
-// the writes 197 us, without the reads 208 us, without the global loads 238 us, without the splitting arithmetic 263 us.
+// What bounds it: MFMA and LDS traffic of about the same length that hardly overlap. Per 32-k step of a 256 x 128 tile a SIMD issues
+// 3072 cycles of MFMA, and the CU 192 fragment reads (8 cycles each) and 72 plane writes (16 cycles each, whatever the width), 2688
+// cycles of LDS; the sum of both is the time. Measured on 8192 x 1024 x 3072 (245 us, 211 TFLOP/s): without the reads 205 us,
+// without the writes 221 us, without the splitting arithmetic 238 us, without the global loads 240 us.
 //
 //   * operand tile in LDS: three planes of 16-byte units (eight k of one row) in the order the MFMA reads them. The eight k
 //     of a unit are {4 g .. 4 g + 3, 16 + 4 g .. 16 + 4 g + 3}: with that order four neighbouring lanes load 64 contiguous bytes
@@ -39,11 +44,13 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int SP_BK = 32, SP_PLANES = 3, SP_FRAGMENT = 1024;   // k extent of a tile; bytes of one plane of 16 rows
 
-// two floats -> their three bf16 parts, packed
+// two floats -> the three bf16 parts of SP_SCALE times them, packed
+constexpr float SP_SCALE = 65536.f, SP_UNSCALE = 1.f / (SP_SCALE * SP_SCALE);
 __device__ __forceinline__ void split_pair(float x, float y, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
     auto pack = [](float a, float b) { return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2)); };
     auto low = [](uint32_t v) { return __builtin_bit_cast(float, v << 16); };
     auto high = [](uint32_t v) { return __builtin_bit_cast(float, v & 0xffff0000u); };
+    x *= SP_SCALE; y *= SP_SCALE;
     hi = pack(x, y);
     x -= low(hi); y -= high(hi);
     mid = pack(x, y);
@@ -60,7 +67,7 @@ __device__ __forceinline__ int split_unit(int r, int g) {
 template <int ROWS, int THREADS, bool KC>
 struct SplitTile {
     static constexpr int PER_T = ROWS * (SP_BK / 8) / THREADS, PLANE = ROWS * SP_BK * 2;
-    static constexpr int LOADS = PER_T * (KC ? 2 : 8), WRITES = PER_T * SP_PLANES, VALU = PER_T * 44;   // per thread and tile
+    static constexpr int LOADS = PER_T * (KC ? 2 : 8), WRITES = PER_T * SP_PLANES, VALU = PER_T * 52;   // per thread and tile
     static_assert(ROWS * (SP_BK / 8) % THREADS == 0, "whole units per thread");
 
     f32x4 v[PER_T][2];
@@ -230,7 +237,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * WAVE, PER_SIMD) void gemm_f32_s
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            acc[i][j] += small[i][j];
+            acc[i][j] = (acc[i][j] + small[i][j]) * SP_UNSCALE;
 #pragma unroll
             for (int r = 0; r < 4; ++r) probe = fmaf(acc[i][j][r], 0.f, probe);
         }

@@ -114,6 +114,26 @@ def test_split_gemm_keeps_infinities_nan_and_the_largest_values(tuning, rows, kc
     assert bool(((expected - got.double()).abs()[fine] <= 1e-5 * (a[0].double().abs().nan_to_num(0, 0) @ b.double().abs().nan_to_num(0, 0, 0).t())[fine]).all())
 
 
+@pytest.mark.parametrize("kc", [True, False])
+@pytest.mark.parametrize("rows", [64, 128, 256])
+def test_split_gemm_keeps_small_values(tuning, rows, kc):
+    """Values down to the smallest subnormal against values that bring the sums back to ordinary size, on either side, and sums
+    close to the smallest normal number. Where the values are ordinary floats nothing may be lost to their size: the bound is that
+    of the split itself. A subnormal is exact as well, so its products are."""
+    tuning(MI355X_GEMM_SPLIT=rows)
+    M, N, K = 130, 140, 96
+    rng = np.random.default_rng(rows)
+    for low, high in ((-100, 90), (-105, 95), (-112, 100), (-120, 100), (-126, 105), (-134, 105), (-148, 105), (-60, -58), (-3, 90)):
+        small, large = (torch.from_numpy(np.ldexp(rng.uniform(1, 2, s) * rng.choice([-1, 1], s), e).astype(np.float32)) for s, e in (((M, K), low), ((N, K), high)))
+        small[::2, ::3] = torch.from_numpy(rng.uniform(1, 2, small[::2, ::3].shape).astype(np.float32)) * 2.0**min(low + 20, 0)   # two sizes in a row
+        for a, b in ((small, large), (torch.cat([large, large])[:M], torch.cat([small, small])[:N])):
+            a, b = a.cuda().contiguous(), b.cuda().contiguous()
+            got = split_gemm(a[None], b if kc else b.t().contiguous(), kc)[0]
+            expected = a.double() @ b.double().t().contiguous()
+            bound = (a.double().abs() @ b.double().abs().t().contiguous()) * (K // 32 + 8) * 2.0**-23 + 2.0**-149
+            assert bool(((expected - got.double()).abs() <= bound).all()), (low, high)
+
+
 @pytest.mark.parametrize("form, kc", [(11, True), (12, True), (22, True), (14, False), (24, False)])
 @pytest.mark.parametrize("batch, M, N, K, epi", [(1, 1, 4, 4, 0), (1, 1, 5, 5, 1), (1, 15, 17, 15, 9), (2, 16, 16, 16, 0), (1, 17, 33, 18, 3), (3, 31, 63, 255, 13),
                                                  (1, 33, 65, 257, 9), (1, 5, 10, 300, 1), (1, 40, 130, 1503, 8), (2, 7, 66, 3072, 9), (1, 64, 127, 4099, 0)])
