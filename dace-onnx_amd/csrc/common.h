@@ -21,6 +21,9 @@ int check_launch(const char* kernel_name);
 
 static inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// Threads of one launch: of a grid of 2^32 and more the runtime runs the remainder and reports nothing.
+constexpr int64_t MAX_GRID_THREADS = ((int64_t)1 << 32) - 1;
+
 // Kernel-variant overrides from the MI355X_* environment variables (0 / -1 / false: not set), parsed once
 // and again on mi355x_reload_tuning(); CU count of the current device, asked of the runtime once per device.
 struct Tuning {

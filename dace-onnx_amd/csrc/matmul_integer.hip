@@ -1113,13 +1113,13 @@ extern "C" int mi355x_matmul_integer(const void* A, const void* B, const void* a
     if (cus <= 0) return set_error(MI355X_ERR_NOT_INITIALIZED, "matmul_integer: no usable HIP device");
     const int64_t small_nwg = ceil_div(M, (int64_t)mmi_tile(1)) * ceil_div(N, (int64_t)mmi_tile(1));
     const bool tiny = M * K < 16 || K * N < 4;
-    const bool small = tiny || (tune.mmi_tile ? tune.mmi_tile == 64 : small_nwg <= 3 * (int64_t)cus);
+    const bool small = !tiny && (tune.mmi_tile ? tune.mmi_tile == 64 : small_nwg <= 3 * (int64_t)cus);
     p.tiles_m = ceil_div(M, (int64_t)mmi_tile(small ? 1 : 2));
     p.tiles_n = ceil_div(N, (int64_t)mmi_tile(small ? 1 : 2));
     p.nwg = p.tiles_m * p.tiles_n;
     MI355X_REQUIRE(p.nwg < ((int64_t)1 << 31), "matmul_integer: grid too large");
     const dim3 g((unsigned)p.nwg), b(256);
-    if (tiny) hipLaunchKernelGGL((matmul_integer_i8_kernel<1, true>), g, b, 0, st, p);
+    if (tiny) hipLaunchKernelGGL((matmul_integer_i8_kernel<2, true>), g, b, 0, st, p);
     else if (small) hipLaunchKernelGGL((matmul_integer_i8_kernel<1, false>), g, b, 0, st, p);
     else hipLaunchKernelGGL((matmul_integer_i8_kernel<2, false>), g, b, 0, st, p);
     return check_launch("matmul_integer_i8_kernel");

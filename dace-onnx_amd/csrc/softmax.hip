@@ -210,8 +210,12 @@ static void launch_reg(const float* X, float* Y, int64_t rows, int cols, hipStre
 template <int THREADS, int NV, bool LOG>
 static void launch_any(const float* X, float* Y, int64_t rows, int64_t cols, hipStream_t st) {
     constexpr int ROWS = THREADS == WAVE ? 4 : 1;
-    hipLaunchKernelGGL((softmax_rows_any<THREADS, NV, LOG>), dim3((unsigned)ceil_div(rows, (int64_t)ROWS)), dim3(THREADS * ROWS), 0, st,
-                       X, Y, rows, (int)cols);
+    constexpr int64_t MOST = (MAX_GRID_THREADS / (THREADS * ROWS)) * ROWS;   // rows of one launch
+    for (int64_t row = 0; row < rows; row += MOST) {
+        const int64_t n = rows - row < MOST ? rows - row : MOST;
+        hipLaunchKernelGGL((softmax_rows_any<THREADS, NV, LOG>), dim3((unsigned)ceil_div(n, (int64_t)ROWS)), dim3(THREADS * ROWS), 0, st,
+                           X + row * cols, Y + row * cols, n, (int)cols);
+    }
 }
 
 // Rows per lane group. Inputs of a few MB are one round trip to memory per CU and finish sooner the more

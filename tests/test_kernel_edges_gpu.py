@@ -46,6 +46,27 @@ def test_softmax_of_odd_rows_keeps_nan_and_infinities_in_their_row():
     assert torch.allclose(torch.softmax(x, 1), y, rtol=2e-6, atol=1e-9, equal_nan=True)
 
 
+@pytest.mark.parametrize("rows, cols", [((1 << 24) + 5, 513), ((1 << 26) + 9, 3)])
+def test_softmax_of_more_rows_than_a_grid_holds(rows, cols):
+    """2^32 threads and more are several launches; rows on both sides of the seam."""
+    x, y = torch.empty(rows, cols, device="cuda"), torch.empty(rows, cols, device="cuda")
+    seam = [0, 1, (1 << 24) - 2, (1 << 24) - 1, 1 << 24, rows - 2, rows - 1] + [r for r in ((1 << 26) - 5, (1 << 26) - 4, 1 << 26) if r < rows]
+    x[seam] = torch.randn(len(seam), cols, device="cuda")
+    y[seam] = float("nan")
+    call("mi355x_softmax_f32", x.data_ptr(), y.data_ptr(), rows, cols, 1)
+    assert worst(torch.softmax(x[seam].double(), 1), y[seam]) < 1e-6
+
+
+def test_gemm_of_more_small_products_than_a_grid_of_the_few_tile_kernel_holds():
+    """2^22 workgroups of 1024 threads are too many for a launch: another kernel takes them."""
+    batch, N, K = (1 << 22) + 3, 4, 160
+    a, b = torch.empty(batch, 1, K, device="cuda"), torch.randn(N, K, device="cuda")
+    ends = [0, 1, 1 << 22, batch - 1]
+    a[ends] = torch.randn(len(ends), 1, K, device="cuda")
+    got = split_gemm(a, b, True, batch=batch)[ends]
+    assert worst(a[ends].double() @ b.double().t(), got) < 2e-6   # K / 16 + 24 roundings of 2^-24 at most
+
+
 @pytest.mark.parametrize("kind, reference", [(0, lambda x: x.mean(1)), (1, lambda x: x.sum(1)), (2, lambda x: x.amax(1)), (3, lambda x: x.amin(1))])
 @pytest.mark.parametrize("rows, cols", [(4096, 1), (4099, 63), (4097, 64), (4098, 65), (5000, 197), (4111, 256), (4096, 257), (4095, 197)])
 def test_reductions_of_many_short_rows(kind, reference, rows, cols):
