@@ -341,7 +341,7 @@ static int launch_attention(const float* Q, const float* K, const float* V, floa
     p.batch1 = batch1; p.Sq = Sq; p.Sk = Sk;
     p.q_blocks = ceil_div(Sq, (int64_t)AT_BQ);
     p.nwg = batch0 * batch1 * p.q_blocks;
-    MI355X_REQUIRE(p.nwg < ((int64_t)1 << 31), "attention: grid too large");
+    MI355X_REQUIRE(grid_fits(p.nwg, 256), "attention: grid too large");
     p.q_sb0 = q_strides[0]; p.q_sb1 = q_strides[1]; p.q_sr = q_strides[2];
     p.k_sb0 = k_strides[0]; p.k_sb1 = k_strides[1]; p.k_sr = k_strides[2];
     p.v_sb0 = v_strides[0]; p.v_sb1 = v_strides[1]; p.v_sr = v_strides[2];
@@ -359,7 +359,7 @@ static int launch_attention(const float* Q, const float* K, const float* V, floa
         const int waves = tuning().attn_waves == 2 || tuning().attn_waves == 3 ? tuning().attn_waves : 4;
         p.q_blocks = ceil_div(Sq, (int64_t)16 * waves);
         p.nwg = batch0 * batch1 * p.q_blocks;
-        MI355X_REQUIRE(p.nwg < ((int64_t)1 << 31), "attention: grid too large");
+        MI355X_REQUIRE(grid_fits(p.nwg, 64 * waves), "attention: grid too large");
         const dim3 g((unsigned)p.nwg);
         hipStream_t st = static_cast<hipStream_t>(stream);
         if (waves == 2) hipLaunchKernelGGL(attention_f32_kernel<2>, g, dim3(128), 0, st, p);

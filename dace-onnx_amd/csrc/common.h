@@ -23,6 +23,7 @@ static inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Threads of one launch: of a grid of 2^32 and more the runtime runs the remainder and reports nothing.
 constexpr int64_t MAX_GRID_THREADS = ((int64_t)1 << 32) - 1;
+static inline bool grid_fits(int64_t workgroups, int64_t threads) { return workgroups <= MAX_GRID_THREADS / threads; }
 
 // Kernel-variant overrides from the MI355X_* environment variables (0 / -1 / false: not set), parsed once
 // and again on mi355x_reload_tuning(); CU count of the current device, asked of the runtime once per device.

@@ -700,7 +700,7 @@ extern "C" int mi355x_conv2d_res_f32(const float* X, const float* W, const float
             }
         }
         p.nwg = p.full_tiles + slices;
-        MI355X_REQUIRE(p.nwg < ((int64_t)1 << 31), "conv2d: grid too large");
+        MI355X_REQUIRE(grid_fits(p.nwg, CG_THREADS), "conv2d: grid too large");
         // 3 x 3 and 1 x 1 filters over whole windows of 32 channels: taps known at compile time
         const int taps = (C % 32 == 0 && (KH * KW == 9 || KH * KW == 1) && tune.conv_static_taps) ? (int)(KH * KW) : 0;
         const dim3 g((unsigned)p.nwg), b(CG_THREADS);
@@ -723,7 +723,7 @@ extern "C" int mi355x_conv2d_res_f32(const float* X, const float* W, const float
     p.tiles_m = ceil_div(M, kConvTiles[cfg].bm);
     p.tiles_p = ceil_div(P, kConvTiles[cfg].bn);
     p.nwg = p.tiles_m * p.tiles_p;
-    MI355X_REQUIRE(p.nwg < ((int64_t)1 << 31), "conv2d: grid too large");
+    MI355X_REQUIRE(grid_fits(p.nwg, 256), "conv2d: grid too large");
     switch (cfg) {
         case 0: launch_conv<64, 128, 16, 2, 2>(p, st); break;
         case 1: launch_conv<64, 64, 32, 2, 2>(p, st); break;

@@ -175,7 +175,7 @@ bool launch_conv2d_f32_direct(const ConvArgs& args, double other_cost, int cus, 
     p.tiles_m = ceil_div((int64_t)p.M, (int64_t)16 * kConvDirectForms[best].tm);
     p.tiles_p = ceil_div(p.P, (int64_t)16 * kConvDirectForms[best].tp);
     p.nwg = p.tiles_m * p.tiles_p;
-    if (p.nwg * WAVE * CD_WAVES > MAX_GRID_THREADS) return false;
+    if (!grid_fits(p.nwg, WAVE * CD_WAVES)) return false;
     if (taps9) launch_direct<9>(best % 3, p, stream);
     else launch_direct<1>(best % 3, p, stream);
     return true;

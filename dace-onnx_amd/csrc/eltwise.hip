@@ -352,7 +352,7 @@ extern "C" int mi355x_permute_b32(const void* X, void* Y, int ndim, const int64_
         const int64_t tiles_r = ceil_div(m.shape[rdim], 64), tiles_c = ceil_div(m.shape[m.ndim - 1], 64);
         int64_t blocks = tiles_r * tiles_c;
         for (int d = 0; d < m.ndim - 1; ++d) if (d != rdim) blocks *= m.shape[d];
-        MI355X_REQUIRE(blocks < ((int64_t)1 << 31), "permute: grid too large");
+        MI355X_REQUIRE(grid_fits(blocks, 256), "permute: grid too large");
         hipLaunchKernelGGL(permute_tiled, dim3((unsigned)blocks), dim3(256), 0, st, x, y, m, rdim, tiles_r, tiles_c);
     } else {
         hipLaunchKernelGGL(permute_generic, dim3(grid_for(n)), dim3(256), 0, st, x, y, n, m);

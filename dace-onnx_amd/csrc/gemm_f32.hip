@@ -282,7 +282,7 @@ extern "C" int mi355x_gemm_f32(const float* A, const float* B, float* C, const f
     p.tiles_m = ceil_div(M, tc.bm);
     p.tiles_n = ceil_div(N, tc.bn);
     p.nwg = batch * p.tiles_m * p.tiles_n;
-    MI355X_REQUIRE(p.nwg < ((int64_t)1 << 31), "gemm: grid too large (%lld workgroups)", (long long)p.nwg);
+    MI355X_REQUIRE(grid_fits(p.nwg, 256), "gemm: grid too large (%lld workgroups)", (long long)p.nwg);
     {   // about two workgroups of these tiles share a CU
         const int64_t per_xcd = ceil_div(p.nwg, (int64_t)NUM_XCD), resident = 2 * (cus / NUM_XCD);
         const int64_t per_batch = p.tiles_m * p.tiles_n;   // tiles are numbered batch entry by batch entry

@@ -173,7 +173,7 @@ bool launch_gemm_f32_direct(GemmArgs p, bool b_kc, double other_cost, int cus, h
     p.tiles_m = ceil_div(p.M, (int64_t)16 * kDirectForms[best].tm);
     p.tiles_n = ceil_div(p.N, (int64_t)16 * kDirectForms[best].tn);
     p.nwg = p.batch * p.tiles_m * p.tiles_n;
-    if (p.nwg * WAVE * GD_WAVES > MAX_GRID_THREADS) return false;
+    if (!grid_fits(p.nwg, WAVE * GD_WAVES)) return false;
     const dim3 grid((unsigned)p.nwg), block(WAVE * GD_WAVES);
     if (best == 0) hipLaunchKernelGGL((gemm_f32_direct_kernel<1, 1, true>), grid, block, 0, stream, p);
     else if (best == 1) hipLaunchKernelGGL((gemm_f32_direct_kernel<1, 2, true>), grid, block, 0, stream, p);

@@ -220,7 +220,7 @@ bool launch_gemm_f32_ksplit(GemmArgs p, int cus, hipStream_t stream) {
     p.tiles_m = ceil_div(p.M, (int64_t)KS_BM);
     p.tiles_n = ceil_div(p.N, (int64_t)96);
     p.nwg = p.batch * p.tiles_m * p.tiles_n;
-    if (p.nwg >= ((int64_t)1 << 31)) return false;
+    if (!grid_fits(p.nwg, KS_THREADS)) return false;
     const int64_t per_xcd = ceil_div(p.nwg, (int64_t)NUM_XCD), per_batch = p.tiles_m * p.tiles_n;
     p.group_m = choose_group_m(p.tiles_m, per_xcd < per_batch ? per_xcd : per_batch, cus / NUM_XCD, KS_BM, 96, p.K * 4);
     const Tuning tune = tuning();

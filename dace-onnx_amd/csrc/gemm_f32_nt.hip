@@ -339,7 +339,7 @@ bool launch_gemm_f32_nt(GemmArgs p, int cus, hipStream_t stream) {
     p.tiles_m = ceil_div(p.M, cands[best].bm);
     p.tiles_n = ceil_div(p.N, cands[best].bn);
     p.nwg = p.batch * p.tiles_m * p.tiles_n;
-    if (p.nwg >= ((int64_t)1 << 31)) return false;
+    if (!grid_fits(p.nwg, best == 2 ? 2 * NT_THREADS : NT_THREADS)) return false;
     // an XCD holds cus / 8 tiles at a time (twice that for the candidates that run in pairs)
     const int64_t per_xcd = ceil_div(p.nwg, (int64_t)NUM_XCD);
     const int64_t per_batch = p.tiles_m * p.tiles_n;   // tiles are numbered batch entry by batch entry

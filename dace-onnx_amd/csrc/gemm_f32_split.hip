@@ -340,7 +340,7 @@ bool launch_gemm_f32_split(GemmArgs p, bool b_kc, double other_cost, int cus, hi
     p.tiles_m = ceil_div(p.M, (int64_t)form.bm);
     p.tiles_n = ceil_div(p.N, (int64_t)form.bn);
     p.nwg = p.batch * p.tiles_m * p.tiles_n;
-    if (p.nwg >= ((int64_t)1 << 31)) return false;
+    if (!grid_fits(p.nwg, best == 2 ? 512 : 256)) return false;
     const int64_t per_xcd = ceil_div(p.nwg, (int64_t)NUM_XCD), per_batch = p.tiles_m * p.tiles_n;
     p.group_m = choose_group_m(p.tiles_m, per_xcd < per_batch ? per_xcd : per_batch, (int64_t)form.resident * (cus / NUM_XCD), form.bm, form.bn, p.K * 4);
     const dim3 grid((unsigned)p.nwg);

@@ -109,7 +109,7 @@ extern "C" int mi355x_layernorm_f32(const float* X, const float* gamma, const fl
                    (long long)rows, (long long)cols);
     if (rows == 0 || cols == 0) return MI355X_OK;
     MI355X_REQUIRE(X && Y && gamma, "layernorm: null pointer (X, Y and gamma are required)");
-    MI355X_REQUIRE(ceil_div(rows, 256 / WAVE) < ((int64_t)1 << 31), "layernorm: too many rows");
+    MI355X_REQUIRE(grid_fits(ceil_div(rows, 256 / WAVE), 256), "layernorm: too many rows");
     hipStream_t st = static_cast<hipStream_t>(stream);
     const dim3 grid((unsigned)ceil_div(rows, 256 / WAVE)), block(256);
     auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };

@@ -1117,7 +1117,7 @@ extern "C" int mi355x_matmul_integer(const void* A, const void* B, const void* a
     p.tiles_m = ceil_div(M, (int64_t)mmi_tile(small ? 1 : 2));
     p.tiles_n = ceil_div(N, (int64_t)mmi_tile(small ? 1 : 2));
     p.nwg = p.tiles_m * p.tiles_n;
-    MI355X_REQUIRE(p.nwg < ((int64_t)1 << 31), "matmul_integer: grid too large");
+    MI355X_REQUIRE(grid_fits(p.nwg, 256), "matmul_integer: grid too large");
     const dim3 g((unsigned)p.nwg), b(256);
     if (tiny) hipLaunchKernelGGL((matmul_integer_i8_kernel<2, true>), g, b, 0, st, p);
     else if (small) hipLaunchKernelGGL((matmul_integer_i8_kernel<1, false>), g, b, 0, st, p);

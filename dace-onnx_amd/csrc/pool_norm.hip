@@ -168,7 +168,7 @@ extern "C" int mi355x_maxpool2d_f32(const float* X, float* Y, int64_t N, int64_t
     while (band > 1 && rows_needed(band) * W > LDS_FLOATS) --band;
     const int64_t bands_per_plane = ceil_div(OH, band);
     const int64_t nwg = N * C * bands_per_plane;
-    if (rows_needed(band) * W <= LDS_FLOATS && nwg < ((int64_t)1 << 31) && total >= 65536) {
+    if (rows_needed(band) * W <= LDS_FLOATS && grid_fits(nwg, 256) && total >= 65536) {
         // 16-byte loads need every band's first input row at a 16-byte boundary: that holds when X is aligned
         // and W is a multiple of 4 (then any row offset is)
         const bool vec = W % 4 == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;

@@ -154,7 +154,7 @@ template <int KIND>
 static int launch_reduce(const float* X, float* Y, int64_t outer, int64_t axis_len, int64_t inner, hipStream_t st) {
     if (inner == 1) {
         const int64_t blocks = ceil_div(outer, (int64_t)(256 / WAVE));
-        MI355X_REQUIRE(blocks < ((int64_t)1 << 31), "reduce: grid too large");
+        MI355X_REQUIRE(grid_fits(blocks, 256), "reduce: grid too large");
         // (from 4096 rows on there are enough waves to fill the part with four rows each)
         if (axis_len <= 256 && outer >= 4096) {
             const dim3 grid((unsigned)ceil_div(outer, (int64_t)(256 / WAVE) * 4));
@@ -168,7 +168,7 @@ static int launch_reduce(const float* X, float* Y, int64_t outer, int64_t axis_l
         return check_launch("reduce_rows");
     }
     const int64_t blocks = ceil_div(outer * inner, (int64_t)256);
-    MI355X_REQUIRE(blocks < ((int64_t)1 << 31), "reduce: grid too large");
+    MI355X_REQUIRE(grid_fits(blocks, 256), "reduce: grid too large");
     hipLaunchKernelGGL(reduce_strided<KIND>, dim3((unsigned)blocks), dim3(256), 0, st, X, Y, outer, axis_len, inner);
     return check_launch("reduce_strided");
 }
@@ -218,7 +218,7 @@ extern "C" int mi355x_reduce_nd_f32(int kind, const float* X, float* Y, int ndim
     if (p.n_out == 0) return MI355X_OK;
     MI355X_REQUIRE(X && Y, "reduce_nd: null pointer");
     const int64_t blocks = ceil_div(p.n_out, (int64_t)(256 / WAVE));
-    MI355X_REQUIRE(blocks < ((int64_t)1 << 31), "reduce_nd: grid too large");
+    MI355X_REQUIRE(grid_fits(blocks, 256), "reduce_nd: grid too large");
     hipStream_t st = static_cast<hipStream_t>(stream);
     const dim3 grid((unsigned)blocks), block(256);
     switch (kind) {

@@ -202,15 +202,18 @@ __global__ __launch_bounds__(256) void softmax_strided(const float* __restrict__
 template <int L, int NV, int UNR, bool LOG>
 static void launch_reg(const float* X, float* Y, int64_t rows, int cols, hipStream_t st) {
     constexpr int rows_per_block = (256 / L) * UNR;
-    const int64_t blocks = ceil_div(rows, rows_per_block);
-    hipLaunchKernelGGL((softmax_rows_reg<L, NV, UNR, LOG>), dim3((unsigned)blocks), dim3(256), 0, st,
-                       X, Y, rows, cols);
+    constexpr int64_t MOST = MAX_GRID_THREADS / 256 * rows_per_block;   // rows of one launch
+    for (int64_t row = 0; row < rows; row += MOST) {
+        const int64_t n = rows - row < MOST ? rows - row : MOST;
+        hipLaunchKernelGGL((softmax_rows_reg<L, NV, UNR, LOG>), dim3((unsigned)ceil_div(n, (int64_t)rows_per_block)), dim3(256), 0, st,
+                           X + row * cols, Y + row * cols, n, cols);
+    }
 }
 
 template <int THREADS, int NV, bool LOG>
 static void launch_any(const float* X, float* Y, int64_t rows, int64_t cols, hipStream_t st) {
     constexpr int ROWS = THREADS == WAVE ? 4 : 1;
-    constexpr int64_t MOST = (MAX_GRID_THREADS / (THREADS * ROWS)) * ROWS;   // rows of one launch
+    constexpr int64_t MOST = MAX_GRID_THREADS / (THREADS * ROWS) * ROWS;   // rows of one launch
     for (int64_t row = 0; row < rows; row += MOST) {
         const int64_t n = rows - row < MOST ? rows - row : MOST;
         hipLaunchKernelGGL((softmax_rows_any<THREADS, NV, LOG>), dim3((unsigned)ceil_div(n, (int64_t)ROWS)), dim3(THREADS * ROWS), 0, st,
@@ -261,11 +264,12 @@ static int softmax_dispatch(const float* X, float* Y, int64_t outer, int64_t axi
         else if (cols <= 2048) launch_any<256, 8, LOG>(X, Y, rows, cols, st);
         else if (cols <= 8192) launch_any<512, 16, LOG>(X, Y, rows, cols, st);
         else if (cols <= 32768) launch_any<1024, 32, LOG>(X, Y, rows, cols, st);
+        else if (!grid_fits(rows, 1024)) return set_error(MI355X_ERR_INVALID_ARGUMENT, "softmax: too many rows (%lld)", (long long)rows);
         else hipLaunchKernelGGL(softmax_rows_loop<LOG>, dim3((unsigned)rows), dim3(1024), 0, st, X, Y, cols);
         return check_launch("softmax_rows");
     }
     const int64_t n = outer * inner;
-    MI355X_REQUIRE(ceil_div(n, 256) < ((int64_t)1 << 31), "softmax: grid too large");
+    MI355X_REQUIRE(grid_fits(ceil_div(n, 256), 256), "softmax: grid too large");
     hipLaunchKernelGGL(softmax_strided<LOG>, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, st, X, Y,
                        outer, axis_len, inner);
     return check_launch("softmax_strided");

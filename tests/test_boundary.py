@@ -63,6 +63,24 @@ def test_missing_library_fails_loudly(monkeypatch):
         _lib.library()
 
 
+@pytest.mark.parametrize("name, args", [
+    ("mi355x_reduce_f32", (2, 1 << 27, 300, 1)),
+    ("mi355x_reduce_f32", (1, 1 << 30, 4, 8)),
+    ("mi355x_layernorm_f32", (1 << 27, 8, 1e-5)),
+    ("mi355x_softmax_f32", (1 << 30, 4, 8)),
+    ("mi355x_softmax_f32", (1 << 22, 40000, 1)),
+    ("mi355x_permute_b32", (3, (1 << 24, 64, 64), (4096, 1, 64))),
+    ("mi355x_attention_f32", (1 << 12, 1 << 12, 128, 200, 64, (64, 64, 64), (64, 64, 64), (64, 64, 64), (64, 64, 64), 1.0)),
+])
+def test_more_threads_than_a_grid_holds_are_refused(name, args):
+    """Of a launch of 2^32 threads or more the runtime runs the remainder and reports no error (no GPU: refused before a launch)."""
+    args = [_lib.i64_array(a) if isinstance(a, tuple) else a for a in args]
+    pointers = {"mi355x_layernorm_f32": 4, "mi355x_attention_f32": 4}.get(name, 2)
+    at = 1 if name == "mi355x_reduce_f32" else 0
+    status = getattr(_lib.library(), name)(*args[:at], *[4096] * pointers, *args[at:], None)
+    assert status == 1 and re.search(b"too (large|many)", _lib.library().mi355x_last_error())
+
+
 # ----------------------------------------------------------------------------- registry / nodes
 def test_registry_and_binding():
     impls = dict(donnx.ONNXForward.registered_implementations("Conv"))
