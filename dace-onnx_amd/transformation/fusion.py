@@ -834,7 +834,8 @@ def _fuse_attention(sdfg: SDFG, state: SDFGState) -> int:
         plan = MI355XFusedAttention._plan([(Array(f32, v[0], v[1]), v[2]) for v in (qv, kv, vv, ov)])
         if not MI355XFusedAttention.supports(plan):
             continue
-        if mask_e is not None and MI355XFusedAttention._mask_strides(sdfg.arrays[mask_e.src.data], qv[0][:-2], plan[2], plan[3]) is None:
+        if mask_e is not None and (MI355XFusedAttention._mask_strides(sdfg.arrays[mask_e.src.data], qv[0][:-2], plan[2], plan[3]) is None
+                                   or not MI355XFusedAttention.masked_pays(plan, add is not None)):
             continue
         node = get_onnx_node("FusedAttention")(mm1.label + "_attention", scale=float(getattr(mm1, "_alpha", 1.0)))
         state.add_node(node)

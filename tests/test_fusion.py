@@ -421,3 +421,17 @@ def test_attention_with_a_mask_is_one_launch(mask, fused, mask_first):
         b0, b1, row = attention[0][14]
         i, j, r, key = 1, 7, 100, 31
         assert values.reshape(-1)[i * b0 + j * b1 + r * row + key] == np.broadcast_to(values, (2, heads, seq, seq))[i, j, r, key]
+
+
+@pytest.mark.parametrize("batch, heads, queries, keys, fused", [(2, 12, 128, 128, True), (2, 4, 1, 128, True), (16, 12, 512, 512, True), (2, 4, 1, 2048, False),
+                                                                (2, 2, 64, 8192, False), (2, 1, 1174, 1174, False), (2, 12, 504, 504, True)])
+def test_masked_attention_of_few_queries_over_many_keys_stays_three_products(batch, heads, queries, keys, fused):
+    """One launch walks all keys in as many workgroups as there are blocks of 64 queries; where those are few the products are ahead."""
+    n = H.make_node
+    nodes = [n("Transpose", ["k"], ["kt"], perm=[0, 1, 3, 2]), n("MatMul", ["q", "kt"], ["s"]), n("Add", ["s", "mask"], ["masked"]),
+             n("Softmax", ["masked"], ["p"], axis=-1), n("MatMul", ["p", "v"], ["o"])]
+    info = lambda name, *shape: H.make_tensor_value_info(name, proto.TensorProto.FLOAT, list(shape))   # noqa: E731
+    graph = H.make_graph(nodes, "few", [info("q", batch, heads, queries, 64), info("k", batch, heads, keys, 64), info("v", batch, heads, keys, 64),
+                                        info("mask", batch, 1, 1, keys)], [info("o", batch, heads, queries, 64)])
+    calls = [f for f, _ in _launches(donnx.ONNXModel("few", H.make_model(graph, opset_imports=[H.make_opsetid("", 13)])))]
+    assert ("mi355x_attention_masked_f32" in calls) == fused
