@@ -809,7 +809,11 @@ def _fuse_attention(sdfg: SDFG, state: SDFGState) -> int:
         if prod1 is None or not _is_op(prod1.src, "MatMul") or use2 is None or use2.dst_conn != "A":
             continue
         mm1, mm2 = prod1.src, use2.dst
-        if any(_in_edge(state, n, c) is not None for n in (mm1, mm2) for c in ("_bias", "_residual")) \
+        # the mask of a batch of one, or one of exactly the scores' shape, has become the first product's bias or residual
+        for folded in (_in_edge(state, mm1, "_bias"), _in_edge(state, mm1, "_residual")):
+            if folded is not None:
+                mask_e = folded if mask_e is None else False   # (False: two of them)
+        if mask_e is False or any(_in_edge(state, mm2, c) is not None for c in ("_bias", "_residual")) \
                 or any(getattr(n, "_activation", None) for n in (mm1, mm2)) \
                 or getattr(mm1, "_y_view", None) or getattr(mm2, "_a_view", None) or getattr(mm2, "_alpha", 1.0) != 1.0:
             continue

@@ -396,11 +396,12 @@ def test_softmax_without_axis_attribute_takes_the_default_of_the_models_opset(op
     assert tuple(calls[0][1][2:5]) == (1, 2, 24)
 
 
-@pytest.mark.parametrize("mask, fused", [((2, 1, 1, 128), True), ((1, 1, 128, 128), True), ((128, 128), True), ((2, 12, 1, 128), True),
-                                         ((1, 12, 128, 128), True), ((2, 1, 128, 1), False), ((1, ), False),
-                                         ((128, ), False)])   # (one dimension: it has become the bias of the first product)
+@pytest.mark.parametrize("batch, mask, fused", [(2, (2, 1, 1, 128), True), (2, (1, 1, 128, 128), True), (2, (128, 128), True), (2, (2, 12, 1, 128), True),
+                                                (2, (1, 12, 128, 128), True), (2, (2, 1, 128, 1), False), (2, (1, ), False),
+                                                (2, (128, ), True), (2, (2, 12, 128, 128), True),   # (the first product's bias, its residual)
+                                                (1, (1, 1, 1, 128), True), (1, (128, ), True), (1, (1, 1, 128, 128), True), (1, (1, 12, 128, 128), True)])
 @pytest.mark.parametrize("mask_first", [False, True])
-def test_attention_with_a_mask_is_one_launch(mask, fused, mask_first):
+def test_attention_with_a_mask_is_one_launch(batch, mask, fused, mask_first):
     """MatMul -> Mul -> Add(mask) -> Softmax -> MatMul in every broadcast form of the mask; what the kernel cannot read stays
     as nodes. The mask's strides index the same element as numpy's broadcast."""
     heads, size, seq = 12, 64, 128
@@ -409,9 +410,9 @@ def test_attention_with_a_mask_is_one_launch(mask, fused, mask_first):
     nodes = [n("Transpose", ["k"], ["kt"], perm=[0, 1, 3, 2]), n("MatMul", ["q", "kt"], ["s"]), n("Mul", ["s", "c"], ["scaled"]),
              n("Add", ["mask", "scaled"] if mask_first else ["scaled", "mask"], ["masked"]), n("Softmax", ["masked"], ["p"], axis=-1),
              n("MatMul", ["p", "v"], ["o"])]
-    out = (2, heads, seq, size)
+    out = (batch, heads, seq, size)
     info = lambda name, shape: H.make_tensor_value_info(name, proto.TensorProto.FLOAT, list(shape))   # noqa: E731
-    graph = H.make_graph(nodes, "masked", [info(x, (2, heads, seq, size)) for x in names] + [info("mask", mask)], [info("o", out)],
+    graph = H.make_graph(nodes, "masked", [info(x, (batch, heads, seq, size)) for x in names] + [info("mask", mask)], [info("o", out)],
                               initializer=[proto.numpy_helper.from_array(np.float32(0.125).reshape(()), "c")])
     calls = _launches(donnx.ONNXModel("masked", H.make_model(graph, opset_imports=[H.make_opsetid("", 13)])))
     attention = [a for f, a in calls if f == "mi355x_attention_masked_f32"]
@@ -419,8 +420,8 @@ def test_attention_with_a_mask_is_one_launch(mask, fused, mask_first):
     if fused:
         values = np.arange(np.prod(mask)).reshape(mask)
         b0, b1, row = attention[0][14]
-        i, j, r, key = 1, 7, 100, 31
-        assert values.reshape(-1)[i * b0 + j * b1 + r * row + key] == np.broadcast_to(values, (2, heads, seq, seq))[i, j, r, key]
+        i, j, r, key = batch - 1, 7, 100, 31
+        assert values.reshape(-1)[i * b0 + j * b1 + r * row + key] == np.broadcast_to(values, (batch, heads, seq, seq))[i, j, r, key]
 
 
 @pytest.mark.parametrize("batch, heads, queries, keys, fused", [(2, 12, 128, 128, True), (2, 4, 1, 128, True), (16, 12, 512, 512, True), (2, 4, 1, 2048, False),
