@@ -71,48 +71,33 @@ __device__ __forceinline__ int32_t b_zero_point(const MMIArgs& p, int64_t n) {
 //     integer dot product needs.
 //   * 2 x 2 waves of (32 T) x (32 T) of Y. T = 2: 128 x 128 tiles in steps of 64 k; T = 1: 64 x 64 tiles in steps of 128 k (the
 //     same loads per thread and step, four times the workgroups), for outputs that would leave most of the chip idle.
-// What bounds it: the latency of a step (loads, transpose, LDS, barrier) in few workgroups. Loading byte by byte where K or N is
-// odd, as this kernel once did, cost 4 us per step. Whole vectors from unaligned addresses, clamped at the end of the matrix and
-// masked past the end of K, and loads two steps ahead (M x N x K, before and after): 197 x 1001 x 501 58 -> 8.8 us, 73 x 139 x 689
-// 72 -> 10.6, 1000 x 1000 x 1000 101 -> 13.2, 4096 x 3071 x 769 209 -> 75, 8192 x 2047 x 1531 537 -> 159; looking one step ahead
-// 197 x 1001 x 501 took 11.6 us, 8192 x 2047 x 1531 203.
+// What bounds it: the latency of a step (loads, transpose, LDS, barrier) in few workgroups, so loads are two steps ahead and registers
+// leave room for two (T = 2) or three workgroups to a CU: offsets are 32 bits from the tile's own rows, and the ends of the matrices
+// (last 16 or 4 bytes loaded and moved down, bytes past K cleared) cost something in the steps that reach them only. With 64-bit offsets
+// and every load settled for the end T = 2 had one workgroup to a CU and aligned extents were slower than with their own aligned loads,
+// one step ahead (M x N x K, those loads, then with one workgroup, now): 8192 x 1000 x 768 34.9, 41.7, 23.1 us, 4096 x 3076 x 784 67.9,
+// 85.0, 44.1, 16384 x 1000 x 1024 82, 98, 51, 15240 x 1884 x 16 46, 54, 32; others (byte by byte, one workgroup, now): 4096 x 3071 x 769
+// 203, 71, 45, 8192 x 2047 x 1531 536, 150, 78, 1000 x 1000 x 1000 102, 13.3, 12.0, 122 x 193 x 593 68, 10.3, 9.2.
 constexpr int mmi_bk(int t) { return t == 2 ? 64 : 128; }
 constexpr int mmi_tile(int t) { return 64 * t; }
 
-// 16 bytes from byte `off` of a matrix of `total` >= 16 bytes, whatever the alignment. Near its end the last 16 are loaded:
-// settle_bytes_16 then moves those from `off` on to the front.
-__device__ __forceinline__ u32x4 load_bytes_16(const int8_t* base, int64_t off, int64_t total) {
-    u32x4 v;
-    __builtin_memcpy(&v, base + (off < total - 16 ? off : total - 16), 16);
-    return v;
-}
-__device__ __forceinline__ u32x4 settle_bytes_16(u32x4 v, int64_t off, int64_t total) {
-    if (off <= total - 16) return v;
-    int d = (int)(off < total ? off - (total - 16) : 15);
-    uint64_t lo = v.x | (uint64_t)v.y << 32, hi = v.z | (uint64_t)v.w << 32;
-    if (d >= 8) { lo = hi; hi = 0; d -= 8; }
-    if (d > 0) { lo = lo >> (8 * d) | hi << (64 - 8 * d); hi >>= 8 * d; }
-    return u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+// v moved down by d bytes, 16 and more: 0
+__device__ __forceinline__ u32x4 move_bytes_down(u32x4 v, uint32_t d) {
+    if (d & 8) v = u32x4{v.z, v.w, 0u, 0u};
+    if (d & 4) v = u32x4{v.y, v.z, v.w, 0u};
+    v = u32x4{__builtin_amdgcn_alignbyte(v.y, v.x, d), __builtin_amdgcn_alignbyte(v.z, v.y, d), __builtin_amdgcn_alignbyte(v.w, v.z, d),
+              __builtin_amdgcn_alignbyte(0u, v.w, d)};   // (by d % 4)
+    return d < 16 ? v : u32x4{0u, 0u, 0u, 0u};
 }
 // the first `bytes` bytes of v (any number, also <= 0 or >= 16), the others 0
-__device__ __forceinline__ u32x4 keep_bytes(u32x4 v, int64_t bytes) {
+__device__ __forceinline__ u32x4 keep_bytes(u32x4 v, int bytes) {
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
-        const int64_t n = bytes - 4 * w;
-        v[w] &= n >= 4 ? ~0u : n <= 0 ? 0u : ~0u >> (32 - 8 * (int)n);
+        const int n = bytes - 4 * w;
+        v[w] &= n >= 4 ? ~0u : n <= 0 ? 0u : ~0u >> (32 - 8 * n);
     }
     return v;
 }
-// the same with 4 bytes of a matrix of `total` >= 4
-__device__ __forceinline__ uint32_t load_bytes_4(const int8_t* base, int64_t off, int64_t total) {
-    uint32_t v;
-    __builtin_memcpy(&v, base + (off < total - 4 ? off : total - 4), 4);
-    return v;
-}
-__device__ __forceinline__ uint32_t settle_bytes_4(uint32_t v, int64_t off, int64_t total) {
-    return off <= total - 4 ? v : v >> (8 * (uint32_t)(off - (total - 4)) & 31u);
-}
-
 __device__ __forceinline__ uint32_t perm_b32(uint32_t hi, uint32_t lo, uint32_t sel) {
     return __builtin_amdgcn_perm(hi, lo, sel);
 }
@@ -129,9 +114,10 @@ __device__ __forceinline__ void transpose_4x4_bytes(const uint32_t (&r)[4], uint
     o[3] = perm_b32(t23_hi, t01_hi, 0x07060302u);
 }
 
-// A needs 16 bytes and B four (launch precondition; smaller matrices are read byte by byte)
-template <int T, bool TINY>
-__global__ __launch_bounds__(256) void matmul_integer_i8_kernel(MMIArgs p) {
+// A needs 16 bytes and B four (launch precondition; smaller matrices are read byte by byte). Off: what a lane's offset into the rows
+// of a tile or step fits in, 32 bits below 2^24 columns.
+template <int T, typename Off, bool TINY>
+__global__ __launch_bounds__(256, 2) void matmul_integer_i8_kernel(MMIArgs p) {
     constexpr int BM = mmi_tile(T), BN = mmi_tile(T), BK = mmi_bk(T), NT = 256;
     constexpr int A_PITCH = BK + 16, B_PITCH = BN + 4;   // bytes per A row, words per k-quad row in LDS
     __shared__ __attribute__((aligned(16))) int8_t lds_a[2][BM * A_PITCH];
@@ -148,59 +134,100 @@ __global__ __launch_bounds__(256) void matmul_integer_i8_kernel(MMIArgs p) {
     // unsigned bytes become signed ones (u ^ 0x80 = u - 128) as they are loaded; bytes past K are 0,
     // so a padded k adds 0 to the product and to both sums
     const uint32_t a_flip = p.a_unsigned ? 0x80808080u : 0u, b_flip = p.b_unsigned ? 0x80808080u : 0u;
-    const int64_t a_total = p.M * p.K, b_total = p.K * p.N;
 
     // ---- loaders ----------------------------------------------------------------
     // A: BM rows x BK / 16 vectors of 16 bytes -> 2 vectors per thread; rows past M repeat the last one and are not stored
     // B: BK / 4 k-quads x BN / 4 column groups -> 2 units (4 rows x 4 cols) per thread; columns past N are not stored
-    int64_t a_off[2], b_off[2];
+    const int rows_in = (int)(p.M - m0 < BM ? p.M - m0 : BM);
+    const int8_t* a_tile = p.A + m0 * p.K;
+    const int8_t* b_tile = p.B + n0;
+    const int64_t a_left = (p.M - m0) * p.K, b_left = p.K * p.N - n0;   // bytes from there to the end of the matrix
+    Off a_off[2], b_off[2];
 #pragma unroll
     for (int it = 0; it < 2; ++it) {
-        const int idx = tid + it * NT;
-        const int64_t gm = m0 + idx / (BK / 16);
-        a_off[it] = (gm < p.M ? gm : p.M - 1) * p.K + 16 * (idx % (BK / 16));
-        b_off[it] = (int64_t)(4 * (idx / (BN / 4))) * p.N + n0 + 4 * (idx % (BN / 4));
+        const int idx = tid + it * NT, row = idx / (BK / 16);
+        a_off[it] = (Off)(row < rows_in ? row : rows_in - 1) * (Off)p.K + (Off)(16 * (idx % (BK / 16)));
+        b_off[it] = (Off)(4 * (idx / (BN / 4))) * (Off)p.N + (Off)(4 * (idx % (BN / 4)));
     }
+    // Where a vector of this step reaches past the end of its matrix (uniform: the last rows of tiles, the last steps), the last 16 or 4
+    // bytes are loaded in its place, and moved down before they go to LDS.
+    auto a_ends = [&](int64_t k0) { return (int64_t)(rows_in - 1) * p.K + k0 + BK > a_left; };
+    auto b_ends = [&](int64_t k0) { return (k0 + BK - 1) * p.N + BN > b_left; };
     struct Raw { u32x4 a[2]; uint32_t b[2][4]; };
     // loads only: what they bring is looked at two steps later
     auto load_tiles = [&](Raw& raw, int64_t k0) {
+        const int8_t* a = a_tile + k0;
+        const int8_t* b = b_tile + k0 * p.N;
+        const bool a_end = a_ends(k0), b_end = b_ends(k0);
+        if constexpr (TINY) {
 #pragma unroll
-        for (int it = 0; it < 2; ++it) {
-            if constexpr (TINY) {
+            for (int it = 0; it < 2; ++it) {
                 raw.a[it] = u32x4{0u, 0u, 0u, 0u};
                 for (int e = 0; e < 16; ++e)
-                    if (a_off[it] + k0 + e < a_total) raw.a[it][e / 4] |= (uint32_t)(uint8_t)p.A[a_off[it] + k0 + e] << (8 * (e % 4));
-            } else {
-                raw.a[it] = load_bytes_16(p.A, a_off[it] + k0, a_total);
-            }
+                    if (a_off[it] + k0 + e < a_left) raw.a[it][e / 4] |= (uint32_t)(uint8_t)a[a_off[it] + e] << (8 * (e % 4));
 #pragma unroll
-            for (int rr = 0; rr < 4; ++rr) {
-                const int64_t off = b_off[it] + (k0 + rr) * p.N;
-                if constexpr (TINY) {
+                for (int rr = 0; rr < 4; ++rr) {
+                    const int64_t off = b_off[it] + rr * p.N;
                     raw.b[it][rr] = 0u;
                     for (int e = 0; e < 4; ++e)
-                        if (off + e < b_total) raw.b[it][rr] |= (uint32_t)(uint8_t)p.B[off + e] << (8 * e);
-                } else {
-                    raw.b[it][rr] = load_bytes_4(p.B, off, b_total);
+                        if (off + k0 * p.N + e < b_left) raw.b[it][rr] |= (uint32_t)(uint8_t)b[off + e] << (8 * e);
                 }
+            }
+            return;
+        }
+        // (the clamped offsets count from 16 or 4 bytes before: what is left can be fewer)
+        const Off a_rest = (Off)(a_left - k0), b_rest = (Off)(b_left - k0 * p.N);
+        const int8_t* a_row = a_end ? a - 16 : a;
+#pragma unroll
+        for (int it = 0; it < 2; ++it) {
+            Off off = a_off[it];
+            if (a_end) off = off + 16 < a_rest ? off + 16 : a_rest;
+            __builtin_memcpy(&raw.a[it], a_row + off, 16);
+        }
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) {
+            const int8_t* b_row = b_end ? b - 4 : b + rr * p.N;
+#pragma unroll
+            for (int it = 0; it < 2; ++it) {
+                Off off = b_off[it];
+                if (b_end) off = off + rr * (Off)p.N + 4 < b_rest ? off + rr * (Off)p.N + 4 : b_rest;
+                __builtin_memcpy(&raw.b[it][rr], b_row + off, 4);
             }
         }
     };
-    auto store_tiles = [&](const Raw& raw, int buf, int64_t k0) {
+    auto store_tiles = [&](Raw& raw, int buf, int64_t k0) {
+        if (!TINY && a_ends(k0)) {
+            const Off rest = (Off)(a_left - k0);
+#pragma unroll
+            for (int it = 0; it < 2; ++it) {
+                const Off end = a_off[it] + 16;
+                if (end > rest) raw.a[it] = move_bytes_down(raw.a[it], (uint32_t)(end - rest < 16 ? end - rest : 16));
+            }
+        }
+        if (!TINY && b_ends(k0)) {
+            const Off rest = (Off)(b_left - k0 * p.N);
+#pragma unroll
+            for (int it = 0; it < 2; ++it)
+#pragma unroll
+                for (int rr = 0; rr < 4; ++rr) {
+                    const Off end = b_off[it] + rr * (Off)p.N + 4;
+                    if (end > rest) raw.b[it][rr] >>= 8 * (uint32_t)(end - rest) & 31u;   // (four and more: past K or N)
+                }
+        }
         const bool ragged = k0 + BK > p.K;   // uniform
+        const int left = ragged ? (int)(p.K - k0) : BK;
 #pragma unroll
         for (int it = 0; it < 2; ++it) {
             const int idx = tid + it * NT;
             const int c16 = idx % (BK / 16), kq = idx / (BN / 4);
-            u32x4 v = TINY ? raw.a[it] : settle_bytes_16(raw.a[it], a_off[it] + k0, a_total);
-            v ^= a_flip;
-            if (ragged) v = keep_bytes(v, p.K - k0 - 16 * c16);
+            u32x4 v = raw.a[it] ^ a_flip;
+            if (ragged) v = keep_bytes(v, left - 16 * c16);
             *reinterpret_cast<u32x4*>(lds_a[buf] + idx / (BK / 16) * A_PITCH + 16 * c16) = v;
             uint32_t rows[4], cols[4];
 #pragma unroll
             for (int rr = 0; rr < 4; ++rr) {
-                rows[rr] = (TINY ? raw.b[it][rr] : settle_bytes_4(raw.b[it][rr], b_off[it] + (k0 + rr) * p.N, b_total)) ^ b_flip;
-                if (ragged && k0 + 4 * kq + rr >= p.K) rows[rr] = 0u;
+                rows[rr] = raw.b[it][rr] ^ b_flip;
+                if (ragged && 4 * kq + rr >= left) rows[rr] = 0u;
             }
             transpose_4x4_bytes(rows, cols);
             *reinterpret_cast<u32x4*>(lds_b[buf] + kq * B_PITCH + 4 * (idx % (BN / 4))) = u32x4{cols[0], cols[1], cols[2], cols[3]};
@@ -1108,20 +1135,21 @@ extern "C" int mi355x_matmul_integer(const void* A, const void* B, const void* a
         else launch_stream<false>(p, grid, st);
         return check_launch("matmul_integer_i8_stream_kernel");
     }
-    // Any other shape: 64 x 64 tiles up to three of them per CU (512 tiles on 256 CUs, 1024 x 2048 x 1000: 18.0 us against 26.9 us as
-    // 128 x 128; 1024 tiles, 2048 x 2000 x 777: 30.7 against 26.6 us; 197 x 1001 x 501: 8.8 against 16.8 us).
+    // Any other shape: 64 x 64 tiles up to three of them per CU (512 tiles on 256 CUs, 1024 x 2000 x 777: 14.4 us against 19.8 us as
+    // 128 x 128; 768 tiles, 2048 x 1500 x 1500: 23.6 against 29.6; 1024 tiles, 2048 x 2000 x 777: 22.6 against 21.1 us).
     if (cus <= 0) return set_error(MI355X_ERR_NOT_INITIALIZED, "matmul_integer: no usable HIP device");
     const int64_t small_nwg = ceil_div(M, (int64_t)mmi_tile(1)) * ceil_div(N, (int64_t)mmi_tile(1));
-    const bool tiny = M * K < 16 || K * N < 4;
-    const bool small = !tiny && (tune.mmi_tile ? tune.mmi_tile == 64 : small_nwg <= 3 * (int64_t)cus);
+    const bool tiny = M * K < 16 || K * N < 4, wide = N >= ((int64_t)1 << 24) || K >= ((int64_t)1 << 24);
+    const bool small = !tiny && !wide && (tune.mmi_tile ? tune.mmi_tile == 64 : small_nwg <= 3 * (int64_t)cus);
     p.tiles_m = ceil_div(M, (int64_t)mmi_tile(small ? 1 : 2));
     p.tiles_n = ceil_div(N, (int64_t)mmi_tile(small ? 1 : 2));
     p.nwg = p.tiles_m * p.tiles_n;
     MI355X_REQUIRE(grid_fits(p.nwg, 256), "matmul_integer: grid too large");
     const dim3 g((unsigned)p.nwg), b(256);
-    if (tiny) hipLaunchKernelGGL((matmul_integer_i8_kernel<2, true>), g, b, 0, st, p);
-    else if (small) hipLaunchKernelGGL((matmul_integer_i8_kernel<1, false>), g, b, 0, st, p);
-    else hipLaunchKernelGGL((matmul_integer_i8_kernel<2, false>), g, b, 0, st, p);
+    if (tiny) hipLaunchKernelGGL((matmul_integer_i8_kernel<2, int64_t, true>), g, b, 0, st, p);
+    else if (wide) hipLaunchKernelGGL((matmul_integer_i8_kernel<2, int64_t, false>), g, b, 0, st, p);
+    else if (small) hipLaunchKernelGGL((matmul_integer_i8_kernel<1, uint32_t, false>), g, b, 0, st, p);
+    else hipLaunchKernelGGL((matmul_integer_i8_kernel<2, uint32_t, false>), g, b, 0, st, p);
     return check_launch("matmul_integer_i8_kernel");
 }
 

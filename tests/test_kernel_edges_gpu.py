@@ -224,7 +224,8 @@ def test_masked_attention(sk, fill):
 
 @pytest.mark.parametrize("tile", [0, 64, 128])
 @pytest.mark.parametrize("M, N, K", [(1, 1, 1), (3, 7, 5), (2, 9, 8), (5, 1, 3), (5, 1, 4), (1, 3, 300), (63, 65, 127), (64, 64, 112), (65, 129, 129),
-                                     (130, 66, 33), (128, 128, 144), (129, 127, 257), (200, 130, 385)])
+                                     (130, 66, 33), (128, 128, 144), (129, 127, 257), (200, 130, 385), (129, 3, 20), (129, 130, 1), (1, 2, 70), (16, 1, 4),
+                                     (129, 129, 70), (130, 132, 80), (257, 100, 784)])
 def test_matmul_integer_of_any_extent_and_address(tuning, tile, M, N, K):
     """Whole vectors from any address, clamped at the end of a matrix: both operands end where their allocation's view ends, the
     bytes around them are not theirs, and the result is exact."""
@@ -242,6 +243,16 @@ def test_matmul_integer_of_any_extent_and_address(tuning, tile, M, N, K):
         call("mi355x_matmul_integer", ga.data_ptr() + shift, gb.data_ptr() + shift, gza.data_ptr(), gzb.data_ptr(), y.data_ptr(), M, N, K,
              a_unsigned, b_unsigned, za.size, zb.size)
         assert np.array_equal((a - za[:, None]) @ (b - zb[None, :]), y.cpu().numpy())
+
+
+@pytest.mark.parametrize("M, N, K", [(2, (1 << 24) - 1, 3), (2, (1 << 24) + 5, 3), (3, 2, (1 << 24) + 70)])
+def test_matmul_integer_of_rows_past_32_bit_offsets(M, N, K):
+    rng = np.random.default_rng(K)
+    a, b = rng.integers(-128, 128, (M, K), dtype=np.int8), rng.integers(-128, 128, (K, N), dtype=np.int8)
+    y = torch.full((M, N), -1, dtype=torch.int32, device="cuda")
+    call("mi355x_matmul_integer", gpu(a).data_ptr(), gpu(b).data_ptr(), None, None, y.data_ptr(), M, N, K, 0, 0, 1, 1)
+    a, b = a.astype(np.float64), b.astype(np.float64)   # sums below 2^14 K, exact
+    assert np.array_equal((a @ b).astype(np.int64).astype(np.int32), y.cpu().numpy())
 
 
 @pytest.mark.parametrize("form", [None, 11, 21, 22])
