@@ -70,7 +70,7 @@ __global__ __launch_bounds__(256) void reduce_rows(const float* __restrict__ X, 
 
 // Many rows of up to 64 * NV columns: a wave takes UNR rows, all their loads first, so that a short row's trip to memory
 // and its six combining steps overlap the other rows' (one row per wave is that chain and nothing else: ReduceMax
-// [18912, 197] 6.2 -> 5.4 us).
+// [18912, 197] 6.2 -> 5.4 us, [262144, 129] 61 -> 34 us).
 template <int KIND, int NV, int UNR>
 __global__ __launch_bounds__(256) void reduce_rows_short(const float* __restrict__ X, float* __restrict__ Y, int64_t rows, int cols) {
     using R = Reducer<KIND, float>;
@@ -155,14 +155,16 @@ static int launch_reduce(const float* X, float* Y, int64_t outer, int64_t axis_l
     if (inner == 1) {
         const int64_t blocks = ceil_div(outer, (int64_t)(256 / WAVE));
         MI355X_REQUIRE(grid_fits(blocks, 256), "reduce: grid too large");
-        // (from 4096 rows on there are enough waves to fill the part with four rows each)
-        if (axis_len <= 256 && outer >= 4096) {
+        const bool vec = axis_len % 4 == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;
+        // Four rows to a wave from where there are enough waves for them to be ahead (ReduceMax, four rows against one): [8192, 33] 4.2
+        // and 3.7 us, [12288, 33] 4.3 and 4.2, [16384, 33] 4.4 and 4.7; [12288, 79] 4.9 and 4.4, [16384, 79] 5.0 both, [16384, 197] 5.2
+        // and 5.7; where a row is whole vectors [16384, 256] 5.3 and 5.1, [20000, 256] 5.6 and 5.7; [262144, 129] 34 and 61.
+        if (axis_len <= 256 && outer >= (axis_len <= 64 ? 12288 : vec ? 18432 : 16384)) {
             const dim3 grid((unsigned)ceil_div(outer, (int64_t)(256 / WAVE) * 4));
             if (axis_len <= 64) hipLaunchKernelGGL((reduce_rows_short<KIND, 1, 4>), grid, dim3(256), 0, st, X, Y, outer, (int)axis_len);
             else hipLaunchKernelGGL((reduce_rows_short<KIND, 4, 4>), grid, dim3(256), 0, st, X, Y, outer, (int)axis_len);
             return check_launch("reduce_rows_short");
         }
-        const bool vec = axis_len % 4 == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;
         if (vec) hipLaunchKernelGGL((reduce_rows<KIND, true>), dim3((unsigned)blocks), dim3(256), 0, st, X, Y, outer, axis_len);
         else hipLaunchKernelGGL((reduce_rows<KIND, false>), dim3((unsigned)blocks), dim3(256), 0, st, X, Y, outer, axis_len);
         return check_launch("reduce_rows");

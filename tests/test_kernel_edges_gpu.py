@@ -68,7 +68,8 @@ def test_gemm_of_more_small_products_than_a_grid_of_the_few_tile_kernel_holds():
 
 
 @pytest.mark.parametrize("kind, reference", [(0, lambda x: x.mean(1)), (1, lambda x: x.sum(1)), (2, lambda x: x.amax(1)), (3, lambda x: x.amin(1))])
-@pytest.mark.parametrize("rows, cols", [(4096, 1), (4099, 63), (4097, 64), (4098, 65), (5000, 197), (4111, 256), (4096, 257), (4095, 197)])
+@pytest.mark.parametrize("rows, cols", [(4096, 1), (4099, 63), (4097, 64), (4098, 65), (5000, 197), (4111, 256), (4096, 257), (4095, 197),
+                                        (12287, 33), (12288, 33), (12291, 64), (16383, 65), (16385, 79), (18431, 256), (18433, 200)])
 def test_reductions_of_many_short_rows(kind, reference, rows, cols):
     x = gpu(np.random.default_rng(rows).standard_normal((rows, cols), dtype=np.float32))
     x[3, cols // 2] = float("nan")
