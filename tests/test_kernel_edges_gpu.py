@@ -185,6 +185,17 @@ def test_gemm_straight_from_memory(tuning, form, kc, batch, M, N, K, epi):
     assert bool(torch.isfinite(got).flatten()[:(M - 1) * N].all()) and bool(torch.isinf(got[0, M - 1]).all())
 
 
+@pytest.mark.parametrize("batch, M, N, K, kc, form", [(48, 1338, 457, 47, False, 24), (96, 275, 1303, 120, False, 24), (96, 14, 2720, 64, True, 12)])
+def test_gemm_of_many_rounds_of_workgroups_is_not_one_of_few_tiles(tuning, batch, M, N, K, kc, form):
+    """Which kernel ran shows in the order of the sums: the bits are those of the kernels through LDS, not of the few-tile form."""
+    a, b = torch.randn(batch, M, K, device="cuda"), torch.randn(*((N, K) if kc else (K, N)), device="cuda")
+    results = []
+    for forced in (None, 0, form):
+        tuning(MI355X_GEMM_DIRECT=forced)
+        results.append(split_gemm(a, b, kc, batch=batch))
+    assert torch.equal(results[0], results[1]) and not torch.equal(results[1], results[2])
+
+
 def test_gemm_picks_the_same_result_whatever_kernel(tuning):
     """Sizes on both sides of the rules that pick the bf16 kernel, against the kernels it takes over from."""
     for M, N, K, kc in ((512, 3072, 512, False), (2048, 3072, 512, False), (1024, 3072, 768, True), (4096, 1024, 768, True), (2048, 1001, 256, True),
