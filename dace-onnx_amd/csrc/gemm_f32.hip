@@ -132,14 +132,15 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_f32_kernel(GemmAr
 
 // ---- host side ----------------------------------------------------------------
 
-struct TileConfig { int bm, bn, bk; };
+// ragged_round: nanoseconds per k and round of one tile to a CU, without 16-byte accesses
+struct TileConfig { int bm, bn, bk; double ragged_round; };
 // index order must match the switch in launch_config()
 static const TileConfig kConfigs[] = {
-    {128, 128, 16},  // 0: large problems, highest reuse
-    {64, 64, 32},    // 1
-    {64, 48, 32},    // 2: N multiple of 48 (768, 2304, 3072) with few tiles
-    {32, 64, 32},    // 3: small batched products
-    {128, 64, 32},   // 4
+    {128, 128, 16, 110},  // 0: large problems, highest reuse
+    {64, 64, 32, 37},    // 1
+    {64, 48, 32, 28},    // 2: N multiple of 48 (768, 2304, 3072) with few tiles
+    {32, 64, 32, 25},    // 3: small batched products
+    {128, 64, 32, 72},   // 4
 };
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
 
@@ -266,11 +267,15 @@ extern "C" int mi355x_gemm_f32(const float* A, const float* B, float* C, const f
     const bool split_kc = p.b_sk == 1 && al16(B) && m4(p.b_sn) && m4(p.b_sb0) && m4(p.b_sb1);
     const double generic_cost = vec ? 2.0 * (double)batch * (double)M * (double)N / 110e3 * 0.95 : 1e300;
     // Few tiles: operands straight from memory into registers. The kernel below takes about 3 us and then 16 ns per k however small
-    // the product is (5 x 300 x 784 15.8 us, 5 x 10 x 300 9.6, without 16-byte accesses 33 x 1000 x 1503 44.7), or its throughput.
+    // the product is (5 x 300 x 784 15.8 us, 5 x 10 x 300 9.6), or its throughput; without 16-byte accesses what its tiles take in a
+    // round over the CUs (569 shapes; the lowest quarter of each tile's).
     if (tune.gemm_config < 0 && tune.gemm_split < 0 && !small_stack && p.a_sk == 1 && (p.b_sk == 1 || p.b_sn == 1)) {
         const bool split_fits = split_a && (split_kc || (p.b_sn == 1 && p.b_sk != 1)) && K >= 128;
-        const double generic = std::max(16.0 * (double)K, 2.0 * (double)batch * (double)M * (double)N * (double)K / (vec ? 110e3 : 60e3));
-        const double split = split_fits ? (double)K * gemm_f32_split_cost(p, cus) : 1e300;
+        const TileConfig& tile = kConfigs[choose_config(batch, M, N, K, cus)];
+        const int64_t rounds = ceil_div(batch * ceil_div(M, (int64_t)tile.bm) * ceil_div(N, (int64_t)tile.bn), (int64_t)cus);
+        const double generic = vec ? std::max(16.0 * (double)K, 2.0 * (double)batch * (double)M * (double)N * (double)K / 110e3)
+                                   : tile.ragged_round * (double)rounds * (double)K;
+        const double split = split_fits ? std::min((double)K * gemm_f32_split_cost(p, cus), 1e300) : 1e300;   // (1e300: not a form of it)
         const double other = 3000 + (vec || split == 1e300 ? std::min(generic, split) : split);   // (without 16-byte accesses the bf16 form is what follows)
         if (launch_gemm_f32_direct(p, p.b_sk == 1, other, cus, static_cast<hipStream_t>(stream))) return check_launch("gemm_f32_direct_kernel");
     }

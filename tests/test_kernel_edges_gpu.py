@@ -185,7 +185,8 @@ def test_gemm_straight_from_memory(tuning, form, kc, batch, M, N, K, epi):
     assert bool(torch.isfinite(got).flatten()[:(M - 1) * N].all()) and bool(torch.isinf(got[0, M - 1]).all())
 
 
-@pytest.mark.parametrize("batch, M, N, K, kc, form", [(48, 1338, 457, 47, False, 24), (96, 275, 1303, 120, False, 24), (96, 14, 2720, 64, True, 12)])
+@pytest.mark.parametrize("batch, M, N, K, kc, form", [(48, 1338, 457, 47, False, 24), (96, 275, 1303, 120, False, 24), (96, 14, 2720, 64, True, 12),
+                                                        (200, 168, 382, 144, False, 24), (200, 1461, 43, 148, False, 24)])
 def test_gemm_of_many_rounds_of_workgroups_is_not_one_of_few_tiles(tuning, batch, M, N, K, kc, form):
     """Which kernel ran shows in the order of the sums: the bits are those of the kernels through LDS, not of the few-tile form."""
     a, b = torch.randn(batch, M, K, device="cuda"), torch.randn(*((N, K) if kc else (K, N)), device="cuda")
