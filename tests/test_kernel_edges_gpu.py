@@ -262,8 +262,8 @@ def test_matmul_integer_of_any_extent_and_address(tuning, tile, M, N, K):
 def test_matmul_integer_of_rows_past_32_bit_offsets(M, N, K):
     rng = np.random.default_rng(K)
     a, b = rng.integers(-128, 128, (M, K), dtype=np.int8), rng.integers(-128, 128, (K, N), dtype=np.int8)
-    y = torch.full((M, N), -1, dtype=torch.int32, device="cuda")
-    call("mi355x_matmul_integer", gpu(a).data_ptr(), gpu(b).data_ptr(), None, None, y.data_ptr(), M, N, K, 0, 0, 1, 1)
+    ga, gb, y = gpu(a), gpu(b), torch.full((M, N), -1, dtype=torch.int32, device="cuda")
+    call("mi355x_matmul_integer", ga.data_ptr(), gb.data_ptr(), None, None, y.data_ptr(), M, N, K, 0, 0, 1, 1)
     a, b = a.astype(np.float64), b.astype(np.float64)   # sums below 2^14 K, exact
     assert np.array_equal((a @ b).astype(np.int64).astype(np.int32), y.cpu().numpy())
 
