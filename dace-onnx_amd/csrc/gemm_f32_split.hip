@@ -4,7 +4,8 @@
 // x = hi + mid + lo (round to nearest, subtract, round again), exactly: values are multiplied by 2^16 before they are split, so that
 // the last bit of the smallest float, 2^-149, is the smallest bf16 subnormal, 2^-133 (the MFMA takes subnormals as they are), and
 // sums by 2^-32 after. Split as they came, values below 2^-110 lost bits: against values that bring the sums back to ordinary size
-// 3.5e-5 (2-norm) at 2^-120 and everything below 2^-136, where 1.6e-7 is left now; the two multiplications of a pair cost 1 to 3 %.
+// 3.5e-5 (2-norm) at 2^-120 and everything below 2^-136, where 1.6e-7 is left now; the two multiplications of a pair cost
+// 1 to 4 %, and 12 % where 64 x 64 tiles come two to a CU (12 x (675 x 160 x 1472): 48.9 -> 54.8 us).
 // Of the nine products of two split values the six that reach 2^-24 of the result are
 // multiplied, each exact in the fp32 accumulator of the MFMA: hi hi in one set of accumulators, the five small ones in a
 // second set, added at the end, so the long sum takes K / 32 roundings where the fp32 MFMA takes K / 4. Against float64 over
@@ -297,8 +298,10 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * WAVE, PER_SIMD) void gemm_f32_s
 }
 
 // Time per k of each form in nanoseconds, from sweeps over M of 512 to 8192, N of 768 to 3072 and K of 256 to 3072 (and N of
-// 1001 to 30522 with B contiguous along n), `n` = tiles per CU. 64 x 64: 26 / 35 / 44 / 56 for up to 1 / 2 / 3 / 4, then 13.7 n
-// + 6; 128 x 64: 38 / 48 / 72, then 23 n + 8; 256 x 128: 77 per round. (128 x 128 tiles are never ahead by more than 2 %;
+// 1001 to 30522 with B contiguous along n), `n` = tiles per CU. 64 x 64: 26 / 37 / 44 / 56 for up to 1 / 2 / 3 / 4, then 13.7 n
+// + 6; 128 x 64: 40 / 48 / 72, then 23 n + 8; 256 x 128: 77 per round. (Over 224 shapes of K = 128 to 3200 the pick is behind the
+// kernels it takes over from by more than 2 % in one, 2.4 %, and 1.8 % behind the best form on average. 35 and 38 for the second and
+// the first entry, measured before values were scaled: 1237 x 1536 x 2592 96 us here, 89 there. 128 x 128 tiles are never ahead by more than 2 %;
 // 128 x 256 tiles equal 256 x 128 and lose 6 % with B contiguous along n.)
 struct SplitForm { int bm, bn, resident; };
 static const SplitForm kSplitForms[] = {{64, 64, 4}, {128, 64, 3}, {256, 128, 1}};
@@ -306,8 +309,8 @@ static const SplitForm kSplitForms[] = {{64, 64, 4}, {128, 64, 3}, {256, 128, 1}
 static double split_cost(int form, int64_t nwg, int cus) {
     const double n = (double)nwg / cus;
     const int64_t up = ceil_div(nwg, (int64_t)cus);
-    if (form == 0) return up <= 1 ? 26 : up == 2 ? 35 : up == 3 ? 44 : up == 4 ? 56 : 13.7 * n + 6;
-    if (form == 1) return up <= 1 ? 38 : up == 2 ? 48 : up == 3 ? 72 : 23 * n + 8;
+    if (form == 0) return up <= 1 ? 26 : up == 2 ? 37 : up == 3 ? 44 : up == 4 ? 56 : 13.7 * n + 6;
+    if (form == 1) return up <= 1 ? 40 : up == 2 ? 48 : up == 3 ? 72 : 23 * n + 8;
     return 77.0 * (double)up;
 }
 

@@ -197,6 +197,16 @@ def test_gemm_of_many_rounds_of_workgroups_is_not_one_of_few_tiles(tuning, batch
     assert torch.equal(results[0], results[1]) and not torch.equal(results[1], results[2])
 
 
+@pytest.mark.parametrize("batch, M, N, K", [(12, 675, 160, 1472), (1, 1237, 1536, 2592), (8, 1024, 256, 2816)])
+def test_gemm_of_two_tiles_to_a_cu_stays_on_the_fp32_unit(tuning, batch, M, N, K):
+    a, b = torch.randn(batch, M, K, device="cuda"), torch.randn(N, K, device="cuda")
+    results = []
+    for forced in (None, 0, 64):
+        tuning(MI355X_GEMM_SPLIT=forced)
+        results.append(split_gemm(a, b, True, batch=batch))
+    assert torch.equal(results[0], results[1]) and not torch.equal(results[1], results[2])
+
+
 def test_gemm_picks_the_same_result_whatever_kernel(tuning):
     """Sizes on both sides of the rules that pick the bf16 kernel, against the kernels it takes over from."""
     for M, N, K, kc in ((512, 3072, 512, False), (2048, 3072, 512, False), (1024, 3072, 768, True), (4096, 1024, 768, True), (2048, 1001, 256, True),
