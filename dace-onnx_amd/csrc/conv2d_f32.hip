@@ -658,11 +658,12 @@ extern "C" int mi355x_conv2d_res_f32(const float* X, const float* W, const float
         N * C * H * Wd + pads[0] * Wd + pads[1] + H * Wd < ((int64_t)1 << 29) && al16(W) && tune.conv_config < 0) {
         p.x_bytes = (int)(N * C * H * Wd * 4);
         // Few tiles: the kernel that reads its operands straight from memory, where its sweep says it is ahead. A round of 64 x 64
-        // tiles takes 15.3 ns per k and 6.5 us besides (8 to 200 tiles: K = 576 15 us, 1152 24, 2304 42, 4608 77), 1 x 1 filters
-        // 19 and 5.4 (K = 64 6.6, 128 7.8, 256 10.3).
+        // tiles takes 16.5 ns per k and 5.1 us besides (8 to 200 tiles: K = 576 15 us, 1152 24, 2304 42, 4608 77), 1 x 1 filters
+        // 16.3 and 4.8 (K = 64 6.6, 128 7.8, 256 10.3), further rounds a little less.
         if (tune.conv_gather_bn == 0 && tune.conv_per_cu == 0 && tune.conv_tail < 0 && tune.conv_static_taps == 1) {
-            const int64_t rounds = ceil_div(ceil_div(M, (int64_t)CG_BM) * ceil_div(P, (int64_t)64), (int64_t)cus);
-            if (launch_conv2d_f32_direct(p, KH * KW == 1 ? 5400 + 19.0 * (double)K * (double)rounds : 6500 + 15.3 * (double)K * (double)rounds, cus, st)) return check_launch("conv2d_f32_direct_kernel");
+            const double k = (double)K, more = (double)(ceil_div(ceil_div(M, (int64_t)CG_BM) * ceil_div(P, (int64_t)64), (int64_t)cus) - 1);
+            const double gather = KH * KW == 1 ? 4800 + 16.3 * k + more * (2250 + 13.0 * k) : 5100 + 16.5 * k + more * (650 + 16.5 * k);
+            if (launch_conv2d_f32_direct(p, gather, cus, st)) return check_launch("conv2d_f32_direct_kernel");
         }
         // 64 x 64 tiles (three workgroups share a CU) or 64 x 128 (one per CU). Time goes with the tiles a CU has
         // to run times their width; the wide tile, alone on its CU, pays its first loads and last stores in the open

@@ -137,15 +137,18 @@ __global__ __launch_bounds__(WAVE * CD_WAVES) void conv2d_f32_direct_kernel(Conv
         }
 }
 
-// Nanoseconds: `fixed`, then per round of workgroups `round` and `per_k`, from the layers of a residual classifier over 1 to 16
-// images (weights not in the L2; 3 x 3 from K = 576 to 4608, 1 x 1 from 64 to 256). Bound by what a CU draws from its L2, the nine
+// Nanoseconds: `fixed` and `per_k` for the first round of workgroups, `again` and `again_k` for each further one (331 layers of 16 to
+// 1024 channels, K = 16 to 9216, up to 40 rounds; weights not in the L2). Where a strided filter reads half of each line of more than
+// 96 channels the further rounds take a fifth more. The rule picks no kernel that is more than 3 % behind in these, and is 0.2 % behind
+// the best pick on average; with `again` left out it was 10 to 20 % behind in ten: 3 x 32 x 20 x 20 -> 512 10.7 -> 12.9 us, 1 x 1
+// 5 x 512 x 33 x 33 -> 100 14.9 -> 17.5, 3 x 1024 x 33 x 33 -> 200 23.6 -> 28.5. Bound by what a CU draws from its L2, the nine
 // 4-byte loads per four channels included: one image 64 x 56 x 56 -> 64 14.8 -> 7.9 us, 128 x 28 x 28 -> 128 23.5 -> 10.7,
 // 256 x 14 x 14 -> 256 41.3 -> 12.4, 512 x 7 x 7 -> 512 77.0 -> 20.6, 1 x 1 256 x 14 x 14 -> 512 10.0 -> 4.1; four images
 // 512 x 7 x 7 -> 512 76.8 -> 32.5, 128 x 28 x 28 -> 128 23.8 -> 20.8, 64 x 56 x 56 -> 64 would be 22.5 against 15.4 and stay.
 // (Loads past a wave's share, which a branch now skips: 64 x 56 x 56 -> 64 9.0 us with them, 1 x 1 7.6.)
-struct ConvDirectForm { int taps, tm, tp; double fixed, round, per_k; };
-static const ConvDirectForm kConvDirectForms[] = {{9, 1, 1, 3000, 0, 3.8}, {9, 2, 1, 3200, 0, 6.2}, {9, 2, 2, 3200, 0, 7.8},
-                                                  {1, 1, 1, 2800, 750, 2.5}, {1, 2, 1, 2900, 850, 3.4}, {1, 2, 2, 3000, 1500, 3.5}};
+struct ConvDirectForm { int taps, tm, tp; double fixed, again, per_k, again_k; };
+static const ConvDirectForm kConvDirectForms[] = {{9, 1, 1, 2900, 670, 4.15, 3.1}, {9, 2, 1, 3000, 1070, 6.2, 5.75}, {9, 2, 2, 3650, 1740, 7.3, 6.45},
+                                                  {1, 1, 1, 3100, 730, 2.5, 3.0}, {1, 2, 1, 3200, 840, 4.2, 5.2}, {1, 2, 2, 3500, 2000, 5.55, 7.35}};
 
 template <int TAPS>
 static void launch_direct(int form, const ConvArgs& p, hipStream_t st) {
@@ -168,7 +171,8 @@ bool launch_conv2d_f32_direct(const ConvArgs& args, double other_cost, int cus, 
         const ConvDirectForm& form = kConvDirectForms[f];
         if (form.taps != (taps9 ? 9 : 1)) continue;
         const int64_t rounds = ceil_div(ceil_div((int64_t)p.M, (int64_t)16 * form.tm) * ceil_div(p.P, (int64_t)16 * form.tp), (int64_t)cus);
-        const double cost = form.fixed + (double)rounds * (form.round + form.per_k * (double)p.K);
+        const double strided = (p.stride_h > 1 || p.stride_w > 1) && p.C >= 96 && rounds > 1 ? 1.2 : 1.0;
+        const double cost = form.fixed + form.again * (double)(rounds - 1) + strided * (double)p.K * (form.per_k + form.again_k * (double)(rounds - 1));
         if (force > 0 ? force == 10 * form.tm + form.tp : cost < best_cost) { best = f; best_cost = cost; }
     }
     if (best < 0) return false;

@@ -307,3 +307,18 @@ def test_convolution_of_few_tiles(tuning, form, N, C, H, W, M, kernel, stride, p
         if epi:
             expected = expected.relu()
         assert bool(((expected - y.double()).abs() <= (bound + 8) * (C * kernel * kernel // 16 + 24) * 2.0**-24).all())
+
+
+@pytest.mark.parametrize("N, C, H, M, kernel, stride, form", [(3, 32, 20, 512, 3, 1, 22), (5, 512, 33, 100, 1, 1, 22), (3, 1024, 33, 200, 1, 1, 22),
+                                                              (4, 1024, 56, 100, 1, 2, 22)])
+def test_convolution_of_more_rounds_is_not_one_of_few_tiles(tuning, N, C, H, M, kernel, stride, form):
+    """Which kernel ran shows in the order of the sums: the bits are those of the kernel through LDS, not of the few-tile form."""
+    x, w = torch.randn(N, C, H, H, device="cuda"), torch.randn(M, C, kernel, kernel, device="cuda")
+    size = (H - 1) // stride + 1
+    results = []
+    for forced in (None, 0, form):
+        tuning(MI355X_CONV_DIRECT=forced)
+        results.append(torch.full((N, M, size, size), np.nan, device="cuda"))
+        call("mi355x_conv2d_f32", x.data_ptr(), w.data_ptr(), None, results[-1].data_ptr(), N, C, H, H, M, kernel, kernel,
+             _lib.i64_array([kernel // 2] * 4), _lib.i64_array([stride] * 2), _lib.i64_array([1, 1]), 0)
+    assert torch.equal(results[0], results[1]) and not torch.equal(results[1], results[2])
