@@ -147,10 +147,13 @@ __global__ __launch_bounds__(WAVE * GD_WAVES) void gemm_f32_direct_kernel(GemmAr
 // the first loads and the sum over the waves (`fixed`), then per k while every workgroup has a CU to itself (`alone`). More
 // workgroups than CUs run in rounds (one workgroup fills a CU's LDS), each with first loads and a sum of its own (`again`) and `round`
 // per k. Without `again` stacks of products over a short K came here and took two or three times as long: 200 x (2666 x 141 x 11) 189
-// -> 599 us, 512 x (5 x 1600 x 32) 79 -> 148, 96 x (1849 x 840 x 238) 1179 -> 1415 (489 shapes of 1 to 1200 rounds and K of 4 to 4096:
-// the rule now picks a kernel that is more than 4 % behind in one of them, and is 1.5 % behind the best pick on average). A CU draws 30 to 40 bytes a nanosecond whatever the form, which is the bound: 16 x 768 x 768 5.7 us (64 x 48 tiles
-// through LDS 13.1), 16 x 768 x 3072 13.6 (36.1), 128 x 768 x 768 7.3 (13.7), 128 x 768 x 3072 19.0 (36.2), 256 x 768 x 3072 25.8
-// (36.4), 33 x 1000 x 1503 8.7 (44.6), 16 x 30522 x 768 with B along n 19.2 (31.6); 128 x 2304 x 768 17.1 (13.9) stays where it was.
+// -> 599 us, 512 x (5 x 1600 x 32) 79 -> 148, 96 x (1849 x 840 x 238) 1179 -> 1415. Beyond eight rounds the fit is up to 15 % low
+// where rows are at odd addresses (96 x (512 x 238 x 1347) 531 us as 128 x 64 tiles, 650 here), which the rule then adds. Over 459
+// shapes of 1 to 1200 rounds and K of 4 to 4096 it picks no kernel that is more than 4 % behind the one before this file, and is 1.6 %
+// behind the best pick on average.
+// A CU draws 30 to 40 bytes a nanosecond whatever the form, which is the bound: 16 x 768 x 768 5.7 us (64 x 48 tiles through LDS
+// 13.1), 16 x 768 x 3072 13.6 (36.1), 128 x 768 x 768 7.3 (13.7), 128 x 768 x 3072 19.0 (36.2), 256 x 768 x 3072 25.8 (36.4),
+// 33 x 1000 x 1503 8.7 (44.6), 16 x 30522 x 768 with B along n 19.2 (31.6); 128 x 2304 x 768 17.1 (13.9) stays where it was.
 // (Loads past a wave's share, which a branch now skips, were up to half of the time: 16 x 768 x 768 6.9 us with them. 32 x 16
 // tiles equal 16 x 32; 64 x 32 and 32 x 64 tiles are never ahead; both halves of a 128-byte line by one pair of loads changes nothing.)
 struct DirectForm { int tm, tn; bool b_kc; double fixed, alone, again, round; };
@@ -169,7 +172,8 @@ bool launch_gemm_f32_direct(GemmArgs p, bool b_kc, double other_cost, int cus, h
         if (form.b_kc != b_kc) continue;
         const int64_t nwg = p.batch * ceil_div(p.M, (int64_t)16 * form.tm) * ceil_div(p.N, (int64_t)16 * form.tn);
         const int64_t rounds = ceil_div(nwg, (int64_t)cus);
-        const double cost = form.fixed + (rounds <= 1 ? form.alone * (double)p.K : form.again * (double)(rounds - 1) + form.round * (double)p.K * (double)rounds);
+        const double many = rounds > 8 ? 1.15 : 1.0;
+        const double cost = form.fixed + (rounds <= 1 ? form.alone * (double)p.K : many * (form.again * (double)(rounds - 1) + form.round * (double)p.K * (double)rounds));
         if (force > 0 ? force == 10 * form.tm + form.tn : cost < best_cost) { best = f; best_cost = cost; }
     }
     if (best < 0) return false;
