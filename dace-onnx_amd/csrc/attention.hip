@@ -180,7 +180,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(AttnArgs p) {
 // products it replaces: 2 x 12 heads, 69 queries, 300 keys, scores of standard deviation 8 9.2e-7 -> 5.3e-7 (2-norm against float64;
 // 5.7e-7 as two products and a softmax), 16 x 12 of 512 4.6e-7 -> 2.3e-7 (4.6e-7). It costs 1 %.
 // The bare exponential of a rounded argument is not seen in these (with the low part of the product 4.58e-7 for 4.59e-7, 5 % slower).
-// The nodes one at a time (two products, the addition, the softmax) take 259 us on 16 x 12 slices of 512 x 512 scores, this 133.
+// The nodes one at a time (two products, the addition, the softmax) take 259 us on 16 x 12 slices of 512 x 512 scores, this 135.
 // 128 keys go through here too: 8 x 12 slices 10.0 us, the one-pass kernel above without a mask 8.5, the nodes 22.5.
 template <bool MASKED>
 __global__ __launch_bounds__(256) void attention_f32_blocks_kernel(AttnArgs p) {

@@ -17,7 +17,6 @@
 
 #include <stdlib.h>
 #include <type_traits>
-#include <utility>
 
 namespace mi355x {
 
@@ -33,16 +32,6 @@ struct MMIArgs {
 };
 
 typedef int i32x2 __attribute__((ext_vector_type(2)));
-
-template <class F, int... I>
-__device__ __forceinline__ void mmi_static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-// f(integral_constant<0>) ... f(integral_constant<N-1>)
-template <int N, class F>
-__device__ __forceinline__ void mmi_static_for(F&& f) {
-    mmi_static_for_impl(static_cast<F&&>(f), std::make_integer_sequence<int, N>{});
-}
 
 // zero point of row m of A / column n of B as the kernels use it: that of the signed bytes they multiply
 __device__ __forceinline__ int32_t a_zero_point(const MMIArgs& p, int64_t m) {
@@ -879,7 +868,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, WAVES_M * WAVES_N == 4 ? ((
     // (behind the operand transfers, so that a cold page never delays the first step; they are looked at after the
     // loop). Both as assembly, so that the number of memory operations in flight is what is written here: the waits
     // below count them.
-    mmi_static_for<NS - 1>([&](auto s_tag) {
+    static_for<NS - 1>([&](auto s_tag) {
         issue_loads(decltype(s_tag)::value, decltype(s_tag)::value);
         load_a(s_tag, decltype(s_tag)::value);
     });
@@ -919,13 +908,13 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, WAVES_M * WAVES_N == 4 ? ((
             __syncthreads();
         };
         for (int kt0 = 0; kt0 < ktiles; kt0 += NS) {
-            mmi_static_for<NS>([&](auto r_tag) {
+            static_for<NS>([&](auto r_tag) {
                 const int kt = kt0 + decltype(r_tag)::value;
                 if (kt < ktiles) step(r_tag, kt);   // uniform; only the last group can be partial
             });
         }
     };
-    mmi_static_for<NW>([&](auto w_tag) {
+    static_for<NW>([&](auto w_tag) {
         constexpr int w = decltype(w_tag)::value;
         if (wave == w) k_loop(std::integral_constant<int, w / WAVES_N>{}, std::integral_constant<int, w % WAVES_N>{});
     });
