@@ -2,6 +2,7 @@
 1 x 1 layers of a ResNet-50 at 8 and 32 images.
 
     python -m dace_onnx_amd.testing.conv_variants
+    python -m dace_onnx_amd.testing.conv_variants few     # layers of few tiles: 1 to 16 images, and 160 random ones
 
 Prints microseconds per launch (HIP events around graph-recorded launches after a warm-up by time, as bench.py measures
 its rows) for
@@ -10,20 +11,72 @@ its rows) for
 * ``six-deep``: the same tiles through the six-deep ring, two workgroups per CU (``MI355X_CONV_PER_CU=2``);
 * ``wide``: 128-position tiles, one workgroup per CU (``MI355X_CONV_GATHER_BN=128``).
 
-The three add up the same products in the same order: the results are compared bit for bit here as well.
+The three add up the same products in the same order: the results are compared bit for bit here as well. ``few`` has the library's
+choice, ``lds``, never the few-tile kernel (``MI355X_CONV_DIRECT=0``), and its tiles (``=11`` ...), with weights that are not in the L2.
 """
+import itertools
 import os
+import random
+import sys
 
 from .. import _lib
 from .profiling import graph_time_us
 
-VARIABLES = ("MI355X_CONV_PER_CU", "MI355X_CONV_GATHER_BN")
+VARIABLES = ("MI355X_CONV_PER_CU", "MI355X_CONV_GATHER_BN", "MI355X_CONV_DIRECT")
 FORMS = (("library", {}), ("six-deep", {"MI355X_CONV_PER_CU": "2"}), ("wide", {"MI355X_CONV_GATHER_BN": "128"}))
 LAYERS = ((64, 56, 64, 3), (128, 28, 128, 3), (256, 14, 256, 3), (512, 7, 512, 3), (64, 56, 256, 1), (256, 56, 64, 1), (256, 56, 128, 1),
           (512, 28, 128, 1), (1024, 14, 256, 1), (2048, 7, 512, 1), (512, 7, 2048, 1), (128, 28, 512, 1))   # C, H = W, M, k
 
 
+FEW = (("library", None), ("lds", "0"), ("16x16", "11"), ("32x16", "21"), ("32x32", "22"))
+
+
+def few_layers():
+    """images, C, H = W, M, k, stride"""
+    for N in (1, 2, 4, 8, 16):
+        for C, H, M in ((64, 56, 64), (128, 28, 128), (256, 14, 256), (512, 7, 512)):
+            yield N, C, H, M, 3, 1
+        for C, H, M, k in ((64, 56, 128, 3), (64, 56, 128, 1), (128, 28, 256, 3), (128, 28, 256, 1), (256, 14, 512, 3), (256, 14, 512, 1)):
+            yield N, C, H, M, k, 2
+    rng = random.Random("few")
+    for _ in range(160):
+        yield (rng.choice((1, 1, 2, 3, 5, 8)), rng.choice((32, 64, 96, 128, 192, 256, 512, 1024)), rng.choice((4, 7, 10, 14, 20, 28, 33, 56)),
+               rng.choice((16, 32, 48, 64, 96, 100, 128, 200, 256, 512)), rng.choice((1, 3, 3)), rng.choice((1, 1, 2)))
+
+
+def few():
+    import torch
+    lib, i64, behind = _lib.library(), _lib.i64_array, []
+    for N, C, H, M, k, stride in few_layers():
+        size = (H - 1) // stride + 1
+        x, b, y = torch.randn(N, C, H, H, device="cuda"), torch.randn(M, device="cuda"), torch.empty(N, M, size, size, device="cuda")
+        w = itertools.cycle([torch.randn(M, C, k, k, device="cuda") * 0.05 for _ in range(max(1, min(20, int(64e6 / (4 * M * C * k * k)))))])
+        launch = lambda: lib.mi355x_conv2d_f32(x.data_ptr(), next(w).data_ptr(), b.data_ptr(), y.data_ptr(), N, C, H, H, M, k, k, i64([k // 2] * 4),   # noqa: E731
+                                               i64([stride] * 2), i64([1, 1]), _lib.EPI_BIAS | _lib.EPI_RELU, _lib.current_stream())
+        times = []
+        for _, form in FEW:
+            os.environ.pop("MI355X_CONV_DIRECT", None)
+            if form is not None:
+                os.environ["MI355X_CONV_DIRECT"] = form
+            lib.mi355x_reload_tuning()
+            times.append(min(graph_time_us(launch, reps=20, warm_ms=20.0) for _ in range(2)))
+        behind.append((times[0] / times[1], times[0] / min(times[1:])))
+        print(f"{N:3d} x {C:4d} x {H:2d} x {H:2d} -> {M:4d}, {k} x {k}, stride {stride}   " + " ".join(f"{name} {t:7.2f}" for (name, _), t in zip(FEW, times)) +
+              f"   library / lds {behind[-1][0]:.3f}, / best {behind[-1][1]:.3f}", flush=True)
+    print(f"{len(behind)} layers: library / lds at most {max(b for b, _ in behind):.3f}, above 1.03 in {sum(b > 1.03 for b, _ in behind)}; "
+          f"library / best form {sum(b for _, b in behind) / len(behind):.3f} on average, at most {max(b for _, b in behind):.3f}")
+
+
 def main():
+    try:
+        few() if sys.argv[1:] == ["few"] else layers()
+    finally:
+        for name in VARIABLES:
+            os.environ.pop(name, None)
+        _lib.library().mi355x_reload_tuning()
+
+
+def layers():
     import torch
     lib = _lib.library()
     st = _lib.current_stream
@@ -47,20 +100,15 @@ def main():
         return min(graph_time_us(launch, reps=20) for _ in range(2)), y.clone()
 
     print(f"{'images x C x H x W -> M, filter':>34s} {'tiles':>6s} " + " ".join(f"{name:>9s}" for name, _ in FORMS) + "   TFLOP/s  library / best  same bits")
-    try:
-        for N in (8, 32):
-            for C, H, M, k in LAYERS:
-                results = [run(N, C, H, M, k, variables) for _, variables in FORMS]
-                times = [t for t, _ in results]
-                same = all(bool(torch.equal(results[0][1], y)) for _, y in results[1:])
-                tiles = ((M + 63) // 64) * ((N * H * H + 63) // 64)
-                flop = 2.0 * N * M * H * H * C * k * k
-                print(f"{N:3d} x {C:4d} x {H:2d} x {H:2d} -> {M:4d}, {k} x {k}    {tiles:6d} " + " ".join(f"{t:9.2f}" for t in times) +
-                      f"   {flop / times[0] / 1e6:7.1f}  {times[0] / min(times):14.3f}  {same}", flush=True)
-    finally:
-        for name in VARIABLES:
-            os.environ.pop(name, None)
-        lib.mi355x_reload_tuning()
+    for N in (8, 32):
+        for C, H, M, k in LAYERS:
+            results = [run(N, C, H, M, k, variables) for _, variables in FORMS]
+            times = [t for t, _ in results]
+            same = all(bool(torch.equal(results[0][1], y)) for _, y in results[1:])
+            tiles = ((M + 63) // 64) * ((N * H * H + 63) // 64)
+            flop = 2.0 * N * M * H * H * C * k * k
+            print(f"{N:3d} x {C:4d} x {H:2d} x {H:2d} -> {M:4d}, {k} x {k}    {tiles:6d} " + " ".join(f"{t:9.2f}" for t in times) +
+                  f"   {flop / times[0] / 1e6:7.1f}  {times[0] / min(times):14.3f}  {same}", flush=True)
 
 
 if __name__ == "__main__":

@@ -1,8 +1,10 @@
-"""The k-contiguous fp32 GEMM (activations x [N, K] weights, bias epilogue) through the library's own choice and through
-each forced form of the kernel, over a set of shapes.
+"""The fp32 GEMM (activations x weights, bias epilogue) through the library's own choice and through each forced form of its
+kernels, over a set of shapes.
 
     python -m dace_onnx_amd.testing.gemm_variants            # the four launches of the BERT-base layer and shapes around them
     python -m dace_onnx_amd.testing.gemm_variants rounds     # 3072-wide outputs of 512 to 3328 tiles of 128 x 48, K = 768 .. 4096
+    python -m dace_onnx_amd.testing.gemm_variants few        # outputs of few tiles, and 160 random products and stacks
+    python -m dace_onnx_amd.testing.gemm_variants split      # outputs of many tiles, and 160 random products and stacks
 
 Prints microseconds per launch (HIP events around graph-recorded launches after a warm-up by time, as bench.py measures
 its rows), the best of the forced forms and the ratio of the library's choice to it. The forms (``MI355X_GEMM_NT_*``):
@@ -12,15 +14,24 @@ its rows), the best of the forced forms and the ratio of the library's choice to
 * ``64`` / ``96`` / ``144``: 64 x 64, 128 x 96 (16 waves) and 64 x 144 tiles;
 * ``128 deep`` / ``128 lean``: 128 x 48 tiles with the six-deep ring (two workgroups per CU) / the three-deep one (three).
 
-Every form is checked against float64 in tests/test_configs_gpu.py::test_k_contiguous_gemm_tiles_and_epilogues.
+``few`` and ``split`` take weights [N, K] (``kc``) and [K, N] (``nc``), ``few`` weights that are not in the L2 (it rotates through
+64 MB of them). Their forms: ``lds``, never the few-tile kernel (``MI355X_GEMM_DIRECT=0``), and its tiles (``=11`` ...); ``fp32``, neither
+that nor the bf16 kernel (``MI355X_GEMM_SPLIT=0``), and the latter's tiles (``=64`` ...).
+
+Every form is checked against float64 in tests/test_configs_gpu.py::test_k_contiguous_gemm_tiles_and_epilogues and
+tests/test_kernel_edges_gpu.py.
 """
+import itertools
+import math
 import os
+import random
 import sys
 
 from .. import _lib
 from .profiling import graph_time_us
 
-VARIABLES = ("MI355X_GEMM_NT_BM", "MI355X_GEMM_NT_BN", "MI355X_GEMM_NT_PER_CU", "MI355X_GEMM_NT_WAVES", "MI355X_GEMM_NT_BK")
+VARIABLES = ("MI355X_GEMM_NT_BM", "MI355X_GEMM_NT_BN", "MI355X_GEMM_NT_PER_CU", "MI355X_GEMM_NT_WAVES", "MI355X_GEMM_NT_BK", "MI355X_GEMM_DIRECT",
+             "MI355X_GEMM_SPLIT")
 FORMS = (("library", {}),
          ("48 deep", {"MI355X_GEMM_NT_BN": "48", "MI355X_GEMM_NT_PER_CU": "2", "MI355X_GEMM_NT_WAVES": "8"}),
          ("48 lean", {"MI355X_GEMM_NT_BN": "48", "MI355X_GEMM_NT_PER_CU": "3", "MI355X_GEMM_NT_WAVES": "8"}),
@@ -28,6 +39,12 @@ FORMS = (("library", {}),
          ("64", {"MI355X_GEMM_NT_BN": "64"}), ("96", {"MI355X_GEMM_NT_BN": "96"}), ("144", {"MI355X_GEMM_NT_BN": "144"}),
          ("128 deep", {"MI355X_GEMM_NT_BM": "128", "MI355X_GEMM_NT_BN": "48", "MI355X_GEMM_NT_PER_CU": "2"}),
          ("128 lean", {"MI355X_GEMM_NT_BM": "128", "MI355X_GEMM_NT_BN": "48", "MI355X_GEMM_NT_PER_CU": "3"}))
+
+
+FEW = (("library", {}), ("lds", {"MI355X_GEMM_DIRECT": "0"}))
+FEW_TILES = {True: (("16x16", "11"), ("16x32", "12"), ("32x32", "22")), False: (("16x64", "14"), ("32x64", "24"))}
+SPLIT = (("library", {}), ("fp32", {"MI355X_GEMM_DIRECT": "0", "MI355X_GEMM_SPLIT": "0"})) + tuple(
+    (name, {"MI355X_GEMM_DIRECT": "0", "MI355X_GEMM_SPLIT": rows}) for name, rows in (("64x64", "64"), ("128x64", "128"), ("256x128", "256")))
 
 
 def shapes(which: str):
@@ -41,11 +58,72 @@ def shapes(which: str):
     return out
 
 
+def random_shapes(which: str, count: int):
+    """(batch, M, N, K, kc), extents spread over their logarithm."""
+    rng = random.Random(which)
+    log_int = lambda low, high: min(high, max(low, round(math.exp(rng.uniform(math.log(low), math.log(high))))))   # noqa: E731
+    while count:
+        batch, kc = rng.choice((1, 1, 1, 8, 48, 200)), rng.random() < 0.5
+        if which == "few":
+            M, N, K, step = log_int(1, 4096), log_int(4, 8192), log_int(4, 4096), 32
+            work = batch * -(-M // 16) * -(-N // 32) * (1 + K / 512) / 256
+        else:
+            M, N, K, step = log_int(16, 8192), log_int(16, 8192), 32 * log_int(4, 100), 64
+            work = batch * -(-M // 64) * -(-N // 64) / 10 / 256
+        if rng.random() < 0.5:
+            N, K = max(step, N // step * step), max(32, K // 32 * 32)
+        if work <= (300 if which == "few" else 4) and batch * max(M * N, M * K, N * K) < 2e8:
+            count -= 1
+            yield batch, M, N, K, kc
+
+
+def few_and_split(which: str):
+    import torch
+    lib = _lib.library()
+    if which == "few":
+        fixed = [(1, M, N, K, True) for M in (1, 16, 40, 128, 256, 512) for N, K in ((768, 768), (2304, 768), (3072, 768), (768, 3072))]
+        fixed += [(1, M, 30522, 768, False) for M in (1, 16, 64)] + [(1, 5, 300, 784, True), (1, 5, 10, 300, True), (1, 33, 1000, 1503, True)]
+    else:
+        fixed = [(1, M, N, K, kc) for kc in (True, False) for M in (512, 1024, 2048, 4096, 8192) for N, K in ((768, 768), (2304, 768), (3072, 768), (768, 3072))]
+        fixed += [(1, 1024, 30522, 768, False), (1, 4096, 4096, 4096, True)]
+    behind = []
+    for batch, M, N, K, kc in itertools.chain(fixed, random_shapes(which, 160)):
+        forms = SPLIT if which == "split" else FEW + tuple((name, {"MI355X_GEMM_DIRECT": form}) for name, form in FEW_TILES[kc])
+        copies = max(1, min(20, int(64e6 / (4 * batch * N * K)))) if which == "few" else 1
+        a, w = torch.randn(batch, M, K, device="cuda"), [torch.randn(batch * N * K, device="cuda") * 0.05 for _ in range(copies)]
+        bias, out = torch.randn(N, device="cuda"), torch.empty(batch, M, N, device="cuda")
+        i64, weights = _lib.i64_array, itertools.cycle(w)
+        launch = lambda: lib.mi355x_gemm_f32(a.data_ptr(), next(weights).data_ptr(), out.data_ptr(), bias.data_ptr(), None, 1, batch, M, N, K,   # noqa: E731
+                                             i64([0, M * K, K, 1]), i64([0, N * K, 1, K] if kc else [0, N * K, N, 1]), i64([0, M * N, N]),
+                                             None, 1.0, _lib.EPI_BIAS, _lib.current_stream())
+        times = []
+        for _, variables in forms:
+            for name in VARIABLES:
+                os.environ.pop(name, None)
+            os.environ.update(variables)
+            lib.mi355x_reload_tuning()
+            times.append(min(graph_time_us(launch, reps=20, warm_ms=20.0) for _ in range(2)))
+        behind.append((times[0] / times[1], times[0] / min(times[1:])))
+        print(f"{batch:4d} x {M:5d} x {N:5d} x {K:5d} {'kc' if kc else 'nc'} " + " ".join(f"{name} {t:9.2f}" for (name, _), t in zip(forms, times)) +
+              f"   library / {forms[1][0]} {behind[-1][0]:.3f}, / best {behind[-1][1]:.3f}", flush=True)
+    print(f"{len(behind)} shapes: library / {forms[1][0]} at most {max(b for b, _ in behind):.3f}, above 1.03 in {sum(b > 1.03 for b, _ in behind)}; "
+          f"library / best form {sum(b for _, b in behind) / len(behind):.3f} on average, at most {max(b for _, b in behind):.3f}")
+
+
 def main():
+    which = sys.argv[1] if len(sys.argv) > 1 else "layer"
+    try:
+        few_and_split(which) if which in ("few", "split") else tiles(which)
+    finally:
+        for name in VARIABLES:
+            os.environ.pop(name, None)
+        _lib.library().mi355x_reload_tuning()
+
+
+def tiles(which: str):
     import torch
     lib = _lib.library()
     st = _lib.current_stream
-    which = sys.argv[1] if len(sys.argv) > 1 else "layer"
 
     def run(M, N, K, variables):
         for name in VARIABLES:
@@ -60,17 +138,12 @@ def main():
         return min(graph_time_us(launch, reps=20) for _ in range(2))
 
     print(f"{'M x N x K':>18s} {'tiles 128x48':>12s} " + " ".join(f"{name:>9s}" for name, _ in FORMS) + "   library / best forced form")
-    try:
-        for M, N, K in shapes(which):
-            times = [run(M, N, K, variables) for _, variables in FORMS]
-            best = min(times[1:])
-            tiles = ((M + 127) // 128) * ((N + 47) // 48)
-            print(f"{M:6d}x{N:5d}x{K:5d} {tiles:12d} " + " ".join(f"{t:9.2f}" for t in times) +
-                  f"   {times[0] / best:5.3f} ({FORMS[1 + times[1:].index(best)][0]}; {2.0 * M * N * K / times[0] / 1e6:5.1f} TFLOP/s)", flush=True)
-    finally:
-        for name in VARIABLES:
-            os.environ.pop(name, None)
-        lib.mi355x_reload_tuning()
+    for M, N, K in shapes(which):
+        times = [run(M, N, K, variables) for _, variables in FORMS]
+        best = min(times[1:])
+        tiles = ((M + 127) // 128) * ((N + 47) // 48)
+        print(f"{M:6d}x{N:5d}x{K:5d} {tiles:12d} " + " ".join(f"{t:9.2f}" for t in times) +
+              f"   {times[0] / best:5.3f} ({FORMS[1 + times[1:].index(best)][0]}; {2.0 * M * N * K / times[0] / 1e6:5.1f} TFLOP/s)", flush=True)
 
 
 if __name__ == "__main__":
