@@ -659,10 +659,11 @@ extern "C" int mi355x_conv2d_res_f32(const float* X, const float* W, const float
         p.x_bytes = (int)(N * C * H * Wd * 4);
         // Few tiles: the kernel that reads its operands straight from memory, where its sweep says it is ahead. A round of 64 x 64
         // tiles takes 16.5 ns per k and 5.1 us besides (8 to 200 tiles: K = 576 15 us, 1152 24, 2304 42, 4608 77), 1 x 1 filters
-        // 16.3 and 4.8 (K = 64 6.6, 128 7.8, 256 10.3), further rounds a little less.
+        // 17.2 and 5.05 (K = 64 6.6, 128 7.8, 256 10.3), further rounds a little less; strided ones 1.1 us more (9 x 128 x 24 x 24 -> 256 8.6).
         if (tune.conv_gather_bn == 0 && tune.conv_per_cu == 0 && tune.conv_tail < 0 && tune.conv_static_taps == 1) {
             const double k = (double)K, more = (double)(ceil_div(ceil_div(M, (int64_t)CG_BM) * ceil_div(P, (int64_t)64), (int64_t)cus) - 1);
-            const double gather = KH * KW == 1 ? 4800 + 16.3 * k + more * (2250 + 13.0 * k) : 5100 + 16.5 * k + more * (650 + 16.5 * k);
+            const double strided = strides[0] > 1 || strides[1] > 1 ? 1100 : 0;
+            const double gather = strided + (KH * KW == 1 ? 5050 + 17.2 * k + more * (2370 + 13.7 * k) : 5100 + 16.5 * k + more * (650 + 16.5 * k));
             if (launch_conv2d_f32_direct(p, gather, cus, st)) return check_launch("conv2d_f32_direct_kernel");
         }
         // 64 x 64 tiles (three workgroups share a CU) or 64 x 128 (one per CU). Time goes with the tiles a CU has

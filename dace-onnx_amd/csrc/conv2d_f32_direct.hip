@@ -138,9 +138,9 @@ __global__ __launch_bounds__(WAVE * CD_WAVES) void conv2d_f32_direct_kernel(Conv
 }
 
 // Nanoseconds: `fixed` and `per_k` for the first round of workgroups, `again` and `again_k` for each further one (331 layers of 16 to
-// 1024 channels, K = 16 to 9216, up to 40 rounds; weights not in the L2). Where a strided filter reads half of each line of more than
-// 96 channels the further rounds take a fifth more. The rule picks no kernel that is more than 3 % behind in these, and is 0.2 % behind
-// the best pick on average; with `again` left out it was 10 to 20 % behind in ten: 3 x 32 x 20 x 20 -> 512 10.7 -> 12.9 us, 1 x 1
+// 1024 channels, K = 16 to 9216, up to 40 rounds; weights not in the L2). A strided filter, which reads half of each line, takes up to
+// 1.3 times as long over a long K. The rule picks no kernel that is more than 3 % behind in these, and is 0.1 % behind
+// the best pick on average (over 500 others 5 % in one); with `again` left out it was 10 to 20 % behind in ten: 3 x 32 x 20 x 20 -> 512 10.7 -> 12.9 us, 1 x 1
 // 5 x 512 x 33 x 33 -> 100 14.9 -> 17.5, 3 x 1024 x 33 x 33 -> 200 23.6 -> 28.5. Bound by what a CU draws from its L2, the nine
 // 4-byte loads per four channels included: one image 64 x 56 x 56 -> 64 14.8 -> 7.9 us, 128 x 28 x 28 -> 128 23.5 -> 10.7,
 // 256 x 14 x 14 -> 256 41.3 -> 12.4, 512 x 7 x 7 -> 512 77.0 -> 20.6, 1 x 1 256 x 14 x 14 -> 512 10.0 -> 4.1; four images
@@ -171,7 +171,7 @@ bool launch_conv2d_f32_direct(const ConvArgs& args, double other_cost, int cus, 
         const ConvDirectForm& form = kConvDirectForms[f];
         if (form.taps != (taps9 ? 9 : 1)) continue;
         const int64_t rounds = ceil_div(ceil_div((int64_t)p.M, (int64_t)16 * form.tm) * ceil_div(p.P, (int64_t)16 * form.tp), (int64_t)cus);
-        const double strided = (p.stride_h > 1 || p.stride_w > 1) && p.C >= 96 && rounds > 1 ? 1.2 : 1.0;
+        const double strided = (p.stride_h > 1 || p.stride_w > 1) && p.K >= 500 && rounds > 1 ? 1.3 : 1.0;
         const double cost = form.fixed + form.again * (double)(rounds - 1) + strided * (double)p.K * (form.per_k + form.again_k * (double)(rounds - 1));
         if (force > 0 ? force == 10 * form.tm + form.tp : cost < best_cost) { best = f; best_cost = cost; }
     }
