@@ -156,10 +156,13 @@ static int launch_reduce(const float* X, float* Y, int64_t outer, int64_t axis_l
         const int64_t blocks = ceil_div(outer, (int64_t)(256 / WAVE));
         MI355X_REQUIRE(grid_fits(blocks, 256), "reduce: grid too large");
         const bool vec = axis_len % 4 == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;
-        // Four rows to a wave from where there are enough waves for them to be ahead (ReduceMax, four rows against one): [8192, 33] 4.2
-        // and 3.7 us, [12288, 33] 4.3 and 4.2, [16384, 33] 4.4 and 4.7; [12288, 79] 4.9 and 4.4, [16384, 79] 5.0 both, [16384, 197] 5.2
-        // and 5.7; where a row is whole vectors [16384, 256] 5.3 and 5.1, [20000, 256] 5.6 and 5.7; [262144, 129] 34 and 61.
-        if (axis_len <= 256 && outer >= (axis_len <= 64 ? 12288 : vec ? 18432 : 16384)) {
+        // Four rows to a wave from where there are enough waves for them to be ahead. Sums and means: from 4096 rows on ([4096, 33] 2.9 us
+        // both, [8192, 129] 3.1 and 3.3, [8192, 256] 3.1 both, [20000, 175] 3.5 and 4.4). The combining steps of maxima and minima, which keep
+        // NaN, are twice as long a chain: [8192, 33] 4.2 and 3.7 us, [12288, 33] 4.3 and 4.2, [16384, 33] 4.4 and 4.7; [12288, 79] 4.9
+        // and 4.4, [16384, 79] 5.0 both, [16384, 197] 5.2 and 5.7; where a row is whole vectors [16384, 256] 5.3 and 5.1, [20000, 256]
+        // 5.6 and 5.7; [262144, 129] 34 and 61.
+        const int64_t four = KIND == MI355X_REDUCE_MEAN || KIND == MI355X_REDUCE_SUM ? 4096 : axis_len <= 64 ? 12288 : vec ? 18432 : 16384;
+        if (axis_len <= 256 && outer >= four) {
             const dim3 grid((unsigned)ceil_div(outer, (int64_t)(256 / WAVE) * 4));
             if (axis_len <= 64) hipLaunchKernelGGL((reduce_rows_short<KIND, 1, 4>), grid, dim3(256), 0, st, X, Y, outer, (int)axis_len);
             else hipLaunchKernelGGL((reduce_rows_short<KIND, 4, 4>), grid, dim3(256), 0, st, X, Y, outer, (int)axis_len);
