@@ -185,6 +185,41 @@ def test_gemm_straight_from_memory(tuning, form, kc, batch, M, N, K, epi):
     assert bool(torch.isfinite(got).flatten()[:(M - 1) * N].all()) and bool(torch.isinf(got[0, M - 1]).all())
 
 
+@pytest.mark.parametrize("variable, form", [("MI355X_GEMM_DIRECT", f) for f in (11, 12, 22, 14, 24)] + [("MI355X_GEMM_SPLIT", f) for f in (64, 128, 256)])
+@pytest.mark.parametrize("kc", [True, False])
+@pytest.mark.parametrize("M, N, K", [(37, 70, 64), (130, 131, 96), (1, 5, 160)])
+def test_gemm_forms_take_any_strides(tuning, variable, form, kc, M, N, K):
+    """Rows further apart than their length in every operand, two batch levels in either order and broadcast, a residual laid out
+    otherwise than the result; nothing between the rows of the result is written. The bound is that of the kernels through LDS."""
+    rng = np.random.default_rng(M + N + K + form)
+    B0, B1 = 2, 3
+    for order, share_a, share_b in (((0, 1), False, False), ((1, 0), True, False), ((0, 1), False, True)):
+        def laid_out(rows, cols, gap, shared):
+            pitch = cols + gap
+            strides = [0, 0] if shared else [rows * pitch * (B1 if order == (0, 1) else 1), rows * pitch * (1 if order == (0, 1) else B0)]
+            memory = torch.full(((1 if shared else B0 * B1) * rows * pitch,), np.nan, device="cuda")
+            view = torch.as_strided(memory, (B0, B1, rows, cols), (*strides, pitch, 1))
+            torch.as_strided(memory, (memory.numel() // (rows * pitch), rows, cols), (rows * pitch, pitch, 1)).copy_(
+                gpu(rng.standard_normal((memory.numel() // (rows * pitch), rows, cols), dtype=np.float32)))
+            return memory, view, [*strides, pitch]
+        (_, a, sa), (_, b, sb) = laid_out(M, K, 4, share_a), laid_out(N if kc else K, K if kc else N, 8, share_b)
+        (cm, c, sc), (_, r, sr) = laid_out(M, N, 5, False), laid_out(M, N, 3, False)
+        bias, before = gpu(rng.standard_normal(N, dtype=np.float32)), cm.clone()
+        i64, results = _lib.i64_array, []
+        for forced in (form, 0):
+            tuning(**{"MI355X_GEMM_DIRECT": 0, "MI355X_GEMM_SPLIT": 0, variable: forced})
+            cm.copy_(before)
+            call("mi355x_gemm_f32", a.data_ptr(), b.data_ptr(), c.data_ptr(), bias.data_ptr(), r.data_ptr(), B0, B1, M, N, K, i64([*sa, 1]),
+                 i64([*sb[:2], *([1, sb[2]] if kc else [sb[2], 1])]), i64(sc), i64(sr), 0.5, _lib.EPI_BIAS | _lib.EPI_RESIDUAL)
+            results.append(c.clone())
+            assert torch.equal(torch.isnan(cm), torch.isnan(before))
+        wide = b.double().transpose(-1, -2).contiguous() if kc else b.double().contiguous()
+        expected = 0.5 * (a.double().contiguous() @ wide) + bias.double() + r.double()
+        bound = (a.double().abs().contiguous() @ wide.abs() + 2) * (K // 4 + 8) * 2.0**-24
+        for got in results:
+            assert bool(((expected - got.double()).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("batch, M, N, K, kc, form", [(48, 1338, 457, 47, False, 24), (96, 275, 1303, 120, False, 24), (96, 14, 2720, 64, True, 12),
                                                         (200, 168, 382, 144, False, 24), (200, 1461, 43, 148, False, 24)])
 def test_gemm_of_many_rounds_of_workgroups_is_not_one_of_few_tiles(tuning, batch, M, N, K, kc, form):
