@@ -139,9 +139,9 @@ __global__ __launch_bounds__(WAVE * CD_WAVES) void conv2d_f32_direct_kernel(Conv
 
 // Nanoseconds: `fixed` and `per_k` for the first round of workgroups, `again` and `again_k` for each further one (331 layers of 16 to
 // 1024 channels, K = 16 to 9216, up to 40 rounds; weights not in the L2). A strided filter, which reads half of each line, takes up to
-// 1.3 times as long over a long K. The rule picks no kernel that is more than 3 % behind in these, and is 0.1 % behind
-// the best pick on average (over 500 others 5 % in one); with `again` left out it was 10 to 20 % behind in ten: 3 x 32 x 20 x 20 -> 512 10.7 -> 12.9 us, 1 x 1
-// 5 x 512 x 33 x 33 -> 100 14.9 -> 17.5, 3 x 1024 x 33 x 33 -> 200 23.6 -> 28.5. Bound by what a CU draws from its L2, the nine
+// 1.3 times as long over a long K. The rule picks no kernel that is more than 3 % behind in these, and is 0.1 % behind the best pick on
+// average (over 500 others 5 % in one); with `again` left out it was 10 to 20 % behind in ten: 3 x 32 x 20 x 20 -> 512 10.7 -> 12.9 us,
+// 1 x 1 5 x 512 x 33 x 33 -> 100 14.9 -> 17.5, 3 x 1024 x 33 x 33 -> 200 23.6 -> 28.5. Bound by what a CU draws from its L2, the nine
 // 4-byte loads per four channels included: one image 64 x 56 x 56 -> 64 14.8 -> 7.9 us, 128 x 28 x 28 -> 128 23.5 -> 10.7,
 // 256 x 14 x 14 -> 256 41.3 -> 12.4, 512 x 7 x 7 -> 512 77.0 -> 20.6, 1 x 1 256 x 14 x 14 -> 512 10.0 -> 4.1; four images
 // 512 x 7 x 7 -> 512 76.8 -> 32.5, 128 x 28 x 28 -> 128 23.8 -> 20.8, 64 x 56 x 56 -> 64 would be 22.5 against 15.4 and stay.

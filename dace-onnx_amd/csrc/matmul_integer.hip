@@ -64,9 +64,9 @@ __device__ __forceinline__ int32_t b_zero_point(const MMIArgs& p, int64_t n) {
 // leave room for two (T = 2) or three workgroups to a CU: offsets are 32 bits from the tile's own rows, and the ends of the matrices
 // (last 16 or 4 bytes loaded and moved down, bytes past K cleared) cost something in the steps that reach them only. With 64-bit offsets
 // and every load settled for the end T = 2 had one workgroup to a CU and aligned extents were slower than with their own aligned loads,
-// one step ahead (M x N x K, those loads, then with one workgroup, now): 8192 x 1000 x 768 34.9, 41.7, 23.1 us, 4096 x 3076 x 784 67.9,
-// 85.0, 44.1, 16384 x 1000 x 1024 82, 98, 51, 15240 x 1884 x 16 46, 54, 32; others (byte by byte, one workgroup, now): 4096 x 3071 x 769
-// 203, 71, 45, 8192 x 2047 x 1531 536, 150, 78, 1000 x 1000 x 1000 102, 13.3, 12.0, 122 x 193 x 593 68, 10.3, 9.2.
+// one step ahead (M x N x K, those loads, then with one workgroup, now): 8192 x 1000 x 768 35.2, 42.1, 24.7 us, 4096 x 3076 x 784 68.6,
+// 85.7, 46.2, 16384 x 1000 x 1024 82, 98, 53, 15240 x 1884 x 16 46, 54, 32; others (byte by byte, one workgroup, now): 4096 x 3071 x 769
+// 203, 71, 44, 8192 x 2047 x 1531 536, 149, 81, 1000 x 1000 x 1000 102, 13.3, 12.0, 122 x 193 x 593 68, 10.3, 9.2.
 constexpr int mmi_bk(int t) { return t == 2 ? 64 : 128; }
 constexpr int mmi_tile(int t) { return 64 * t; }
 
