@@ -260,7 +260,7 @@ extern "C" int mi355x_gemm_f32(const float* A, const float* B, float* C, const f
         if (launch_gemm_f32_nt(p, cus, static_cast<hipStream_t>(stream))) return check_launch("gemm_f32_nt_kernel");
     }
     // What is left has B contiguous along n, or an N or alignment without 16-byte accesses. Without them the kernel below runs at
-    // 40 to 80 TFLOP/s and the bf16 form is never behind from K = 128 on (1024 x 30522 x 768: 268 against 626 us, 64 x 1002 x 768
+    // 40 to 80 TFLOP/s and the bf16 form is never behind from K = 128 on (1024 x 30522 x 768: 274 against 640 us, 64 x 1002 x 768
     // 22 against 27); with them it reaches 110 where it fills the chip (2048 x 3072 x 512: 71 us, the bf16 form 49; 512 x 3072 x 512:
     // 24 us both).
     const bool split_a = p.a_sk == 1 && al16(A) && m4(p.a_sm) && m4(p.a_sb0) && m4(p.a_sb1);

@@ -324,7 +324,7 @@ bool launch_gemm_f32_nt(GemmArgs p, int cus, hipStream_t stream) {
     }
     // The bf16 form takes over where its own sweep says it is faster (gemm_f32_split.hip). 4.7e-3 ns per k and unit of cost is
     // what these kernels measure (3.8 to 5.1 over outputs of 256 to 4096 tiles), less 8 % so that a tie stays here: 8192 x 768 x
-    // 768 64 against 85 us, 8192 x 3072 x 768 215 against 288, 4096 x 1024 x 768 48 against 60; 1024 x 3072 x 768 (42 against 40)
+    // 768 64 against 78 us, 8192 x 3072 x 768 209 against 279, 2048 x 3072 x 768 64 against 78; 1024 x 3072 x 768 (40.2 against 39.4)
     // and everything smaller stays.
     const bool forced = force || tune.gemm_nt_bk || tune.gemm_nt_per_cu || tune.gemm_nt_waves || tune.gemm_group_m;
     // Few tiles: the kernel that reads its operands straight from memory, where its sweep says it is ahead. In one round of
