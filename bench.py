@@ -31,6 +31,7 @@ if ROOT not in sys.path:
 WARM_MS = 40.0   # untimed repetitions before every measurement, see dace_onnx_amd/testing/profiling.py
 # published MI355X peaks (dense)
 PEAK_FP32_MFMA_TFLOPS = 157.3
+PEAK_SPLIT_MFMA_TFLOPS = 2516.6 / 6   # six bf16 products for one of fp32
 PEAK_INT8_MFMA_TOPS = 5000.0
 PEAK_HBM_GBS = 8000.0
 # L2 <-> fabric bytes of the four GEMM launches of one layer, from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of
@@ -42,6 +43,8 @@ GEMM_TRAFFIC_SOURCE = "profiles/bert_layer_gemm_traffic.txt (rocprofv3 --pmc FET
 
 def algorithmic_work(name, args):
     """(flops, bytes) of one launch from its C-ABI arguments (fp32 unless stated)."""
+    if name == "mi355x_gemm_packed_f32":   # the same arguments with the packed copy of B after A
+        return algorithmic_work("mi355x_gemm_f32", args[:1] + args[2:])
     if name == "mi355x_gemm_f32":
         b0, b1, M, N, K = args[5:10]
         epi = args[15]
@@ -190,7 +193,7 @@ def main():
 
     # ---- per-kernel durations, HIP events on the launch stream -----------------------------
     kernels = []
-    gemm_flops = gemm_us = gemm_bytes = layer_us = 0.0
+    gemm_flops = gemm_us = gemm_floor_us = gemm_bytes = layer_us = 0.0
     if not args.no_kernels:
         for node, relaunch in compiled.bound_launches():
             name = node.function
@@ -198,12 +201,16 @@ def main():
             flops, nbytes = algorithmic_work(name, plain)
             us = graph_time_us(relaunch)
             layer_us += us   # sum of the layer's kernel durations, to hold against ms_per_step
-            if name == "mi355x_gemm_f32":
+            if name in ("mi355x_gemm_f32", "mi355x_gemm_packed_f32"):
+                packed = name == "mi355x_gemm_packed_f32"
+                if packed:
+                    plain = plain[:1] + plain[2:]
                 gemm_flops += flops
                 gemm_bytes += nbytes
                 gemm_us += us
-                label = "gemm_f32 b{}x{} {}x{}x{} epi={}".format(*plain[5:10], plain[15])
-                kernels.append(kernel_row(label, us, flops, nbytes, "mfma"))
+                gemm_floor_us += flops / 1e6 / (PEAK_SPLIT_MFMA_TFLOPS if packed else PEAK_FP32_MFMA_TFLOPS)
+                label = "gemm_f32{} b{}x{} {}x{}x{} epi={}".format("_packed" if packed else "", *plain[5:10], plain[15])
+                kernels.append(kernel_row(label, us, flops, nbytes, "mfma", PEAK_SPLIT_MFMA_TFLOPS if packed else None))
             elif name == "mi355x_attention_f32":
                 label = "attention_f32 b{}x{} q{} k{} d{}".format(*plain[4:9])
                 kernels.append(kernel_row(label, us, flops, nbytes, "mfma"))
@@ -318,12 +325,13 @@ def main():
     roofline = None
     if gemm_us > 0:
         achieved = gemm_flops / gemm_us / 1e6
-        roofline = {"bound": "mfma", "achieved": round(achieved, 2), "peak": PEAK_FP32_MFMA_TFLOPS, "unit": "TFLOP/s",
-                    "frac": round(achieved / PEAK_FP32_MFMA_TFLOPS, 4), "traffic": GEMM_TRAFFIC_BYTES_PER_LAYER,
+        peak = gemm_flops / gemm_floor_us / 1e6   # of the matrix units the launches run on
+        roofline = {"bound": "mfma", "achieved": round(achieved, 2), "peak": round(peak, 1), "unit": "TFLOP/s",
+                    "frac": round(achieved / peak, 4), "traffic": GEMM_TRAFFIC_BYTES_PER_LAYER,
                     "traffic_source": GEMM_TRAFFIC_SOURCE,
                     "algorithmic_bytes_per_layer": gemm_bytes,
-                    "kernel": "gemm_f32_nt_kernel (all mi355x_gemm_f32 launches of one layer: QKV, output projection, FFN1, "
-                              "FFN2; the attention core runs in its own fused kernel, listed under kernels)",
+                    "kernel": "gemm_f32_packed_kernel / gemm_f32_nt_kernel (all GEMM launches of one layer: QKV, output projection, FFN1, "
+                              "FFN2; fp32 products as six bf16 ones where the weights are packed; the attention core runs in its own fused kernel, listed under kernels)",
                     "flop_per_layer": gemm_flops, "us_per_layer": round(gemm_us, 2)}
 
     # ---- CPU baseline: the oracle's layer on this box's host cores ---------------------------

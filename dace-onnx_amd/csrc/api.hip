@@ -58,6 +58,7 @@ static void parse_tuning(Tuning& t) {
     t.gemm_group_m = env_int("MI355X_GEMM_GROUP_M", 0);
     t.gemm_ksplit = env_int("MI355X_GEMM_KSPLIT", -1);
     t.gemm_split = env_int("MI355X_GEMM_SPLIT", -1);
+    t.gemm_packed = env_int("MI355X_GEMM_PACKED", -1);
     t.gemm_direct = env_int("MI355X_GEMM_DIRECT", -1);
     c = getenv("MI355X_CONV_CONFIG");
     t.conv_config = c && c[0] >= '0' && c[0] <= '9' ? c[0] - '0' : -1;

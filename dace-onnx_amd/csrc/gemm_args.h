@@ -24,6 +24,9 @@ struct GemmArgs {
 // the problem is outside what that kernel handles (nothing launched).
 bool launch_gemm_f32_nt(GemmArgs p, int cus, hipStream_t stream);
 
+// Nanoseconds that kernel takes, 1e300 where it takes no such product.
+double gemm_f32_nt_cost(const GemmArgs& p, int cus);
+
 // GEMM with both operands contiguous along k whose eight waves split K (gemm_f32_ksplit.hip): 32 x 96 tiles.
 bool launch_gemm_f32_ksplit(GemmArgs p, int cus, hipStream_t stream);
 
@@ -38,5 +41,8 @@ double gemm_f32_split_cost(const GemmArgs& p, int cus);
 // GEMM with A contiguous along k and B along k (b_kc) or n whose outputs are few tiles (gemm_f32_direct.hip): no staging, K split
 // over the waves of a workgroup. `other_cost`: nanoseconds the caller's own kernel takes; nothing is launched where it is not behind.
 bool launch_gemm_f32_direct(GemmArgs p, bool b_kc, double other_cost, int cus, hipStream_t stream);
+
+// Nanoseconds of its fastest form, 1e300 where it takes no such product.
+double gemm_f32_direct_cost(const GemmArgs& p, bool b_kc, int cus);
 
 }  // namespace mi355x

@@ -160,13 +160,12 @@ struct DirectForm { int tm, tn; bool b_kc; double fixed, alone, again, round; };
 static const DirectForm kDirectForms[] = {{1, 1, true, 3100, 3.4, 980, 2.4}, {1, 2, true, 3400, 5.0, 1400, 4.5}, {2, 2, true, 3800, 7.1, 2350, 6.8},
                                           {1, 4, false, 3500, 5.8, 1650, 5.6}, {2, 4, false, 4000, 8.0, 3050, 9.1}};
 
-bool launch_gemm_f32_direct(GemmArgs p, bool b_kc, double other_cost, int cus, hipStream_t stream) {
-    const int force = tuning().gemm_direct;
-    if (force == 0 || p.K < 4 || (!b_kc && p.N < 4)) return false;
+// The fastest form below `best_cost` (which becomes its time), -1 where there is none.
+static int choose_direct(const GemmArgs& p, bool b_kc, int force, int cus, double& best_cost) {
+    if (force == 0 || p.K < 4 || (!b_kc && p.N < 4)) return -1;
     if (p.a_sm < 0 || p.b_sn < 0 || p.b_sk < 0 || p.M >= ((int64_t)1 << 29) || p.N >= ((int64_t)1 << 29) ||
-        (p.M - 1) * p.a_sm + p.K >= ((int64_t)1 << 29) || (p.N - 1) * p.b_sn + (p.K - 1) * p.b_sk + 1 >= ((int64_t)1 << 29)) return false;
+        (p.M - 1) * p.a_sm + p.K >= ((int64_t)1 << 29) || (p.N - 1) * p.b_sn + (p.K - 1) * p.b_sk + 1 >= ((int64_t)1 << 29)) return -1;
     int best = -1;
-    double best_cost = 0.95 * other_cost;
     for (int f = 0; f < 5; ++f) {
         const DirectForm& form = kDirectForms[f];
         if (form.b_kc != b_kc) continue;
@@ -176,6 +175,18 @@ bool launch_gemm_f32_direct(GemmArgs p, bool b_kc, double other_cost, int cus, h
         const double cost = form.fixed + (rounds <= 1 ? form.alone * (double)p.K : many * (form.again * (double)(rounds - 1) + form.round * (double)p.K * (double)rounds));
         if (force > 0 ? force == 10 * form.tm + form.tn : cost < best_cost) { best = f; best_cost = cost; }
     }
+    return best;
+}
+
+double gemm_f32_direct_cost(const GemmArgs& p, bool b_kc, int cus) {
+    double cost = 1e300;
+    choose_direct(p, b_kc, -1, cus, cost);
+    return cost;
+}
+
+bool launch_gemm_f32_direct(GemmArgs p, bool b_kc, double other_cost, int cus, hipStream_t stream) {
+    double best_cost = 0.95 * other_cost;
+    const int best = choose_direct(p, b_kc, tuning().gemm_direct, cus, best_cost);
     if (best < 0) return false;
     p.tiles_m = ceil_div(p.M, (int64_t)16 * kDirectForms[best].tm);
     p.tiles_n = ceil_div(p.N, (int64_t)16 * kDirectForms[best].tn);

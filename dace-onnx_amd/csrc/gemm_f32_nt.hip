@@ -283,26 +283,22 @@ static bool deep_ring_rounds_fit(int64_t nwg, int cus, int64_t K) {
     return deep_empty * 8 <= deep && lean_empty * 10 >= 3 * lean;
 }
 
-// and N a multiple of 4. Additionally needed here: K a multiple of the 32-k tile.
-bool launch_gemm_f32_nt(GemmArgs p, int cus, hipStream_t stream) {
-    if (p.K % NT_BK != 0 || p.K == 0) return false;
-    // rows are addressed with 32-bit byte offsets from the start of a batch's matrix
-    if (p.a_sm < 0 || p.b_sn < 0 || (p.M - 1) * p.a_sm + p.K >= ((int64_t)1 << 29) || (p.N - 1) * p.b_sn + p.K >= ((int64_t)1 << 29)) return false;
-    // Candidates: 64x48, 64x64 and 64x144 tiles with two k-split groups, 128x48 and 128x96 tiles without.
-    // Cost ~ rounds of workgroups over the CUs x tile area. 128 x 48 tiles run two workgroups per CU (116 registers), and
-    // two workgroups that share a CU drift apart: one's first loads, last stores and barrier waits run under the other's
-    // MFMAs. Measured against 128 x 96 tiles, one workgroup per CU: 1024 x 3072 x 768 (with Gelu) 42.5 against 43.7 us,
-    // 2048 x 3072 x 768 78.7 against 82.6 us, 4096 x 4096 x 1024 261.8 against 297.5 us (131 TFLOP/s). A 128 x 48 tile
-    // that has a CU to itself loses to two 64 x 48 tiles (512 x 3072 x 768: 24.0 against 23.4 us), hence rounds counted in
-    // pairs for it. 128 x 96 stays selectable by hand (MI355X_GEMM_NT_BN=96).
-    struct Cand { int bm, bn, per_cu; double weight; };
-    // (1024 x 2304 x 768, measured: 768 tiles of 64 x 48, two workgroups sharing a CU, 35.2 us; 256 tiles of 64 x 144 36.1 us:
-    // the wide tile gets no discount)
-    const Cand cands[] = {{64, 48, 1, 1.0}, {64, 64, 1, 1.0}, {128, 96, 1, 0.8}, {64, 144, 1, 1.0}, {128, 48, 2, 0.78}};
+struct NtCandidate { int bm, bn, per_cu; double weight; };
+// Candidates: 64x48, 64x64 and 64x144 tiles with two k-split groups, 128x48 and 128x96 tiles without.
+// Cost ~ rounds of workgroups over the CUs x tile area. 128 x 48 tiles run two workgroups per CU (116 registers), and
+// two workgroups that share a CU drift apart: one's first loads, last stores and barrier waits run under the other's
+// MFMAs. Measured against 128 x 96 tiles, one workgroup per CU: 1024 x 3072 x 768 (with Gelu) 42.5 against 43.7 us,
+// 2048 x 3072 x 768 78.7 against 82.6 us, 4096 x 4096 x 1024 261.8 against 297.5 us (131 TFLOP/s). A 128 x 48 tile
+// that has a CU to itself loses to two 64 x 48 tiles (512 x 3072 x 768: 24.0 against 23.4 us), hence rounds counted in
+// pairs for it. 128 x 96 stays selectable by hand (MI355X_GEMM_NT_BN=96).
+// (1024 x 2304 x 768, measured: 768 tiles of 64 x 48, two workgroups sharing a CU, 35.2 us; 256 tiles of 64 x 144 36.1 us:
+// the wide tile gets no discount)
+static const NtCandidate cands[] = {{64, 48, 1, 1.0}, {64, 64, 1, 1.0}, {128, 96, 1, 0.8}, {64, 144, 1, 1.0}, {128, 48, 2, 0.78}};
+
+// The candidate for a product and its cost (`force`, `force_bm`: MI355X_GEMM_NT_BN and _BM, 0 where not set).
+static int choose_nt(const GemmArgs& p, int force, int force_bm, int cus, double& best_cost) {
     int best = 0;
-    double best_cost = 1e300;
-    const Tuning tune = tuning();
-    const int force = tune.gemm_nt_bn, force_bm = tune.gemm_nt_bm;
+    best_cost = 1e300;
     for (int c = 0; c < 5; ++c) {
         const int64_t nwg = p.batch * ceil_div(p.M, cands[c].bm) * ceil_div(p.N, cands[c].bn);
         double cost = (double)ceil_div(nwg, (int64_t)cus * cands[c].per_cu) * cands[c].per_cu * cands[c].bm * cands[c].bn * cands[c].weight;
@@ -322,6 +318,30 @@ bool launch_gemm_f32_nt(GemmArgs p, int cus, hipStream_t stream) {
             best_cost = cost;
         }
     }
+    return best;
+}
+
+// In one round of workgroups of 64 x 48 tiles: nanoseconds.
+static bool nt_one_round(const GemmArgs& p, int cus) { return p.batch * ceil_div(p.M, (int64_t)64) * ceil_div(p.N, (int64_t)48) <= cus; }
+static double nt_one_round_cost(const GemmArgs& p) { return 2800 + (double)p.K * (p.K >= 1280 ? 10.9 : 13.2); }
+
+double gemm_f32_nt_cost(const GemmArgs& p, int cus) {
+    if (p.K % NT_BK != 0 || p.K == 0) return 1e300;
+    if (nt_one_round(p, cus)) return nt_one_round_cost(p);
+    double cost;
+    choose_nt(p, 0, 0, cus, cost);
+    return 5000 + 4.7e-3 * cost * (double)p.K;
+}
+
+// and N a multiple of 4. Additionally needed here: K a multiple of the 32-k tile.
+bool launch_gemm_f32_nt(GemmArgs p, int cus, hipStream_t stream) {
+    if (p.K % NT_BK != 0 || p.K == 0) return false;
+    // rows are addressed with 32-bit byte offsets from the start of a batch's matrix
+    if (p.a_sm < 0 || p.b_sn < 0 || (p.M - 1) * p.a_sm + p.K >= ((int64_t)1 << 29) || (p.N - 1) * p.b_sn + p.K >= ((int64_t)1 << 29)) return false;
+    const Tuning tune = tuning();
+    const int force = tune.gemm_nt_bn;
+    double best_cost;
+    const int best = choose_nt(p, force, tune.gemm_nt_bm, cus, best_cost);
     // The bf16 form takes over where its own sweep says it is faster (gemm_f32_split.hip). 4.7e-3 ns per k and unit of cost is
     // what these kernels measure (3.8 to 5.1 over outputs of 256 to 4096 tiles), less 8 % so that a tie stays here: 8192 x 768 x
     // 768 64 against 78 us, 8192 x 3072 x 768 209 against 279, 2048 x 3072 x 768 64 against 78; 1024 x 3072 x 768 (40.2 against 39.4)
@@ -330,9 +350,8 @@ bool launch_gemm_f32_nt(GemmArgs p, int cus, hipStream_t stream) {
     // Few tiles: the kernel that reads its operands straight from memory, where its sweep says it is ahead. In one round of
     // workgroups these kernels take 2.8 us and per k 13.2 ns, 10.9 as sixteen waves (256, 768, 1024 x any of up to 256 tiles: 6.2,
     // 13.1, 16.5 us; K = 3072 36.1 us).
-    const bool one_round = p.batch * ceil_div(p.M, (int64_t)64) * ceil_div(p.N, (int64_t)48) <= cus;
     if (!forced && tune.gemm_split < 0 &&
-        launch_gemm_f32_direct(p, true, one_round ? 2800 + (double)p.K * (p.K >= 1280 ? 10.9 : 13.2) : 4.7e-3 * best_cost * (double)p.K, cus, stream))
+        launch_gemm_f32_direct(p, true, nt_one_round(p, cus) ? nt_one_round_cost(p) : 4.7e-3 * best_cost * (double)p.K, cus, stream))
         return true;
     if (tune.gemm_split > 0 || (!forced && p.K >= 256))
         if (launch_gemm_f32_split(p, true, 4.7e-3 * 0.92 * best_cost, cus, stream)) return true;

@@ -1,0 +1,462 @@
+// fp32 GEMM on the bf16 matrix unit with constant weights that were split beforehand.
+//
+// The arithmetic is that of gemm_f32_split.hip (three bf16 parts of every value, six products, two sets of accumulators). B, packed once
+// in fragment order (split_bf16.h), goes from memory straight into the registers of the MFMA; only A is split here, on its way into LDS.
+// That takes B's splitting, its LDS writes and its fragment reads out of the loop, and one MFMA of 32 x 32 x 16 does the work of
+// two of 16 x 16 x 32 at 1640 instead of 1415 TFLOP/s, the rate at which each runs with nothing else on the chip (273 and 236 TFLOP/s of
+// split products: the clock gives way before the issue slots do).
+//
+//   * WAVES_M x WAVES_N waves own (32 TM) x (32 TN) outputs each; WAVES_K such groups share K, step by step, and their sums meet in LDS
+//     once. A step is 32 k for each group: the tile is split into the stage the next step reads while this one is multiplied, one
+//     barrier a step, placed between the two halves so that the fragments of the half after it are read under MFMAs.
+//   * B's registers of a half are loaded again right after their last MFMA, for the half after the next.
+// What bounds it: the clock under MFMAs where tiles fill the chip several times over, a launch's first loads and last stores
+// (4 to 8 us, `fixed` below) where each CU has one tile. Against the kernels before it (MI355X_GEMM_PACKED=0): 8192 x 2304 x 768
+// 180 -> 144 us (201 TFLOP/s), 8192 x 768 x 768 65 -> 52, 8192 x 3072 x 768 222 -> 178, 8192 x 768 x 3072 228 -> 187,
+// 1024 x 30522 x 768 297 -> 235, 1500 x 1024 x 4096 135 -> 74, 1024 x 2304 x 768 36.5 -> 28.8, 1024 x 3072 x 768 42.4 -> 31.4,
+// 1024 x 768 x 3072 41.5 -> 37.5, 128 x 2304 x 768 12.3 -> 8.6, 373 x 1024 x 256 7.4 -> 6.1; 600 random products 0.81 of the time.
+// Its error against float64 is smaller than theirs: 0.8e-7 (2-norm) where the fp32 MFMA has 5.0e-7 and 16 x 16 x 32 1.6e-7 (K = 768).
+// Tried: B two steps ahead instead of one and A two (even), B's fragments through LDS, A packed beforehand too (its loads are half as
+// long again: even), loads and splits placed between the MFMAs by hand (even or behind).
+//   * An output register is 32 neighbouring columns of a row over 32 lanes: stores are whole 128-byte lines whatever N and the row
+//     stride are, and a lane has one bias value per 32 columns.
+#include "common.h"
+#include "gemm_tile.h"
+#include "gemm_args.h"
+#include "split_bf16.h"
+
+#include <algorithm>
+
+namespace mi355x {
+
+struct PackedGemmArgs {
+    GemmArgs g;
+    const char* packed;
+    int kt;   // steps of 32 k
+};
+
+template <int TM, int TN, int WAVES_M, int WAVES_N, int WAVES_K, int PER_SIMD>
+__global__ __launch_bounds__(WAVES_M * WAVES_N * WAVES_K * WAVE, PER_SIMD) void gemm_f32_packed_kernel(PackedGemmArgs pa) {
+    const GemmArgs& p = pa.g;
+    constexpr int WAVES = WAVES_M * WAVES_N * WAVES_K, THREADS = WAVES * WAVE, BM = 32 * TM * WAVES_M, BN = 32 * TN * WAVES_N;
+    constexpr int GROUP = BM / 32 * 2 * PK_FRAGMENT, STAGE = WAVES_K * GROUP;      // bytes of a 32-k tile of A; of all groups' tiles
+    constexpr int BLOCKS = BM * BN / 1024;                                        // 32 x 32 blocks of the workgroup's tile
+    constexpr int SUMS = WAVES_K > 1 ? WAVES_K * BLOCKS * 4096 : 0;
+    constexpr int UNITS = BM * 4 * WAVES_K, PER_T = UNITS / THREADS;
+    static_assert(UNITS % THREADS == 0 && THREADS % (4 * WAVE) == 0, "whole units per thread");
+    __shared__ __attribute__((aligned(16))) char lds[2 * STAGE > SUMS ? 2 * STAGE : SUMS];
+
+    const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int li = lane % 32, lh = lane / 32;
+    const int wm = wave % WAVES_M, wn = wave / WAVES_M % WAVES_N, wk = wave / (WAVES_M * WAVES_N);
+
+    const uint32_t logical = (uint32_t)xcd_remap(blockIdx.x, p.nwg), tiles_per_batch = (uint32_t)(p.tiles_m * p.tiles_n);
+    const uint32_t b = logical / tiles_per_batch, t = logical % tiles_per_batch;
+    const int64_t b0 = b / (uint32_t)p.batch1, b1 = b % (uint32_t)p.batch1;
+    int64_t tm, tn;
+    tile_coords(t, p.tiles_m, p.tiles_n, p.group_m, tm, tn);
+    const int64_t m0 = tm * BM, n0 = tn * BN;
+
+    // operands as raw buffers with 32-bit offsets (launch precondition); bit 31 makes a load return zero and drops a store
+    constexpr uint32_t OUT = 0x80000000u;
+    const float* A = p.A + b0 * p.a_sb0 + b1 * p.a_sb1;
+    const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(A), 0, 0x7fffffff, 0x00020000);
+    const __amdgpu_buffer_rsrc_t b_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(pa.packed), 0, 0x7fffffff, 0x00020000);
+
+    // A: (k group, row, unit) of this thread's units, four lanes to the 128 bytes of a row; rows beyond the matrix are its last one
+    uint32_t a_off[PER_T];
+    int a_at[PER_T];
+#pragma unroll
+    for (int it = 0; it < PER_T; ++it) {
+        const int idx = tid + it * THREADS, g = idx % 4, row = idx / 4 % BM, kg = idx / 4 / BM;
+        const int64_t r = m0 + row < p.M ? m0 + row : p.M - 1;
+        a_off[it] = (uint32_t)(r * p.a_sm + 32 * kg + 4 * g) * 4u;
+        // (rows xor-ed with 0, 4, 8, 12 for g = 0..3: neighbouring lanes write to different banks, and reads keep theirs)
+        a_at[it] = kg * GROUP + (row / 32 * 2 + g / 2) * PK_FRAGMENT + ((g & 1) * 32 + ((row % 32) ^ (4 * g))) * 16;
+    }
+    const int steps = (pa.kt + WAVES_K - 1) / WAVES_K;
+    f32x4 va[PER_T][2];
+    auto load_a = [&](int it, int st) {
+        uint32_t off = a_off[it];
+        if constexpr (WAVES_K > 1) {   // a group that has no tile in the last step multiplies zeros
+            const int kg = (tid + it * THREADS) / 4 / BM;
+            off = st * WAVES_K + kg < pa.kt ? off : OUT;
+        }
+        const int base = st * (32 * WAVES_K * 4);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) va[it][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, (int)(off + 64u * h), base, 0));
+    };
+    auto store_a = [&](char* stage, int it) {
+        u32x4 part[SP_PLANES];
+        split_unit8(va[it][0], va[it][1], part);
+#pragma unroll
+        for (int q = 0; q < SP_PLANES; ++q) *reinterpret_cast<u32x4*>(stage + a_at[it] + q * PK_PLANE) = part[q];
+    };
+    // B: one stream of fragments per 32 columns; columns beyond the matrix are its last block's
+    const int n_blocks = (int)((p.N + 31) / 32);
+    uint32_t b_off[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        const int block = min((int)(n0 / 32) + wn * TN + j, n_blocks - 1);
+        b_off[j] = (uint32_t)block * (uint32_t)pa.kt * (uint32_t)(2 * PK_FRAGMENT);
+    }
+    bf16x8 fa[2][TM][SP_PLANES], fb[2][TN][SP_PLANES];
+    auto load_b = [&](auto s_tag, int j, int st) {
+        constexpr int s = decltype(s_tag)::value;
+        const uint32_t at = b_off[j] + (uint32_t)(min(st * WAVES_K + wk, pa.kt - 1) * 2 + s) * (uint32_t)PK_FRAGMENT;
+#pragma unroll
+        for (int q = 0; q < SP_PLANES; ++q)
+            fb[s][j][q] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, lane * 16 + q * PK_PLANE, (int)at, 0));
+    };
+    int a_rd[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) a_rd[s] = wk * GROUP + (wm * TM * 2 + s) * PK_FRAGMENT + (lh * 32 + (li ^ (4 * (2 * s + lh)))) * 16;
+    auto read_a = [&](auto s_tag, const char* stage) {
+        constexpr int s = decltype(s_tag)::value;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int q = 0; q < SP_PLANES; ++q) fa[s][i][q] = *reinterpret_cast<const bf16x8*>(stage + a_rd[s] + i * 2 * PK_FRAGMENT + q * PK_PLANE);
+    };
+
+    f32x16 acc[TM][TN], small[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = small[i][j][r] = 0.f;
+    auto multiply = [&](auto s_tag, int next) {
+        constexpr int s = decltype(s_tag)::value;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+#pragma unroll
+            for (int u = 0; u < PK_PRODUCTS; ++u)
+#pragma unroll
+                for (int i = 0; i < TM; ++i) {
+                    f32x16& sum = u == 0 ? acc[i][j] : small[i][j];
+                    sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[s][i][PK_QA[u]], fb[s][j][PK_QB[u]], sum, 0, 0, 0);
+                }
+            load_b(s_tag, j, next);
+        }
+    };
+    auto sync = [&]() {   // LDS only: loads from memory stay in flight
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    };
+
+    constexpr std::integral_constant<int, 0> first{};
+    constexpr std::integral_constant<int, 1> second{};
+    const int last = steps - 1;   // look-aheads are clamped to the last step, not switched off
+#pragma unroll
+    for (int it = 0; it < PER_T; ++it) load_a(it, 0);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) load_b(first, j, 0);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) load_b(second, j, 0);
+#pragma unroll
+    for (int it = 0; it < PER_T; ++it) {
+        store_a(lds, it);
+        load_a(it, min(1, last));
+    }
+    sync();
+    read_a(first, lds);
+    for (int st = 0; st < steps; ++st) {
+        const int next = min(st + 1, last), after = min(st + 2, last);
+        const char* stage = lds + (st & 1) * STAGE;
+        char* other = lds + ((st + 1) & 1) * STAGE;
+        read_a(second, stage);
+#pragma unroll
+        for (int it = 0; it < PER_T; ++it) {
+            store_a(other, it);
+            load_a(it, after);
+        }
+        multiply(first, next);
+        sync();   // `other` is written, and everyone has read `stage`
+        read_a(first, other);
+        multiply(second, next);
+    }
+
+    // The sums of a block computed again with the fp32 MFMA, straight from global memory: for inputs that the split form cannot hold.
+    auto again = [&](int64_t bm, int64_t bn) __attribute__((always_inline)) {
+        f32x16 sum;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sum[r] = 0.f;
+        const int64_t m = bm + li, n = bn + li;
+        const float* ap = A + (m < p.M ? m : p.M - 1) * p.a_sm + lh;
+        const float* bp = p.B + (n < p.N ? n : p.N - 1) * p.b_sn + lh * p.b_sk;
+        for (int64_t k = 0; k < p.K; k += 2) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(ap[k], bp[k * p.b_sk], sum, 0, 0, 0);
+        return sum;
+    };
+
+    float* C = p.C + b0 * p.c_sb0 + b1 * p.c_sb1 + m0 * p.c_sm + n0;
+    const float* R = (p.epi & MI355X_EPI_RESIDUAL) ? p.residual + b0 * p.r_sb0 + b1 * p.r_sb1 + m0 * p.r_sm + n0 : p.C;
+    const __amdgpu_buffer_rsrc_t c_rsrc = __builtin_amdgcn_make_buffer_rsrc(C, 0, 0x7fffffff, 0x00020000);
+    const __amdgpu_buffer_rsrc_t r_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(R), 0, 0x7fffffff, 0x00020000);
+    const int rows = (int)min((int64_t)BM, p.M - m0), columns = (int)min((int64_t)BN, p.N - n0);
+    // `count` outputs of a column: rows m, m + 1, m + 2, m + 3, then eight rows on. No branch inside: loads and stores go out together.
+    auto finish = [&](auto count_tag, auto act_tag, auto res_tag, const float* v, int m, int n, float bias) __attribute__((always_inline)) {
+        constexpr int COUNT = decltype(count_tag)::value, ACT = decltype(act_tag)::value;
+        constexpr bool RES = decltype(res_tag)::value;
+        float res[COUNT];
+        uint32_t row[COUNT];
+#pragma unroll
+        for (int r = 0; r < COUNT; ++r) row[r] = (uint32_t)(m + 8 * (r / 4) + r % 4);
+        if constexpr (RES)
+#pragma unroll
+            for (int r = 0; r < COUNT; ++r) {
+                const uint32_t off = (row[r] * (uint32_t)p.r_sm + (uint32_t)n) * 4u;
+                res[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r_rsrc, (int)((int)row[r] < rows && n < columns ? off : OUT), 0, 0));
+            }
+#pragma unroll
+        for (int r = 0; r < COUNT; ++r) {
+            float o = apply_epilogue(fmaf(v[r], p.alpha, bias), ACT, 0.f);
+            if constexpr (RES) o += res[r];
+            const uint32_t off = (row[r] * (uint32_t)p.c_sm + (uint32_t)n) * 4u;
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, o), c_rsrc, (int)((int)row[r] < rows && n < columns ? off : OUT), 0, 0);
+        }
+    };
+    // f(activation, residual) with both known at compile time
+    auto with_epilogue = [&](auto&& f) __attribute__((always_inline)) {
+        auto act = [&](auto res) __attribute__((always_inline)) {
+            if (p.epi & MI355X_EPI_GELU) f(std::integral_constant<int, MI355X_EPI_GELU>{}, res);
+            else if (p.epi & MI355X_EPI_RELU) f(std::integral_constant<int, MI355X_EPI_RELU>{}, res);
+            else f(std::integral_constant<int, 0>{}, res);
+        };
+        if (p.epi & MI355X_EPI_RESIDUAL) act(std::true_type{});
+        else act(std::false_type{});
+    };
+    auto bias_of = [&](int n) { return (p.epi & MI355X_EPI_BIAS) && n < columns ? p.bias[n0 + n] : 0.f; };
+
+    if constexpr (WAVES_K == 1) {
+        float bias[TN], probe = 0.f;   // probe stays 0 while every sum is finite
+#pragma unroll
+        for (int j = 0; j < TN; ++j) bias[j] = bias_of(32 * (wn * TN + j) + li);
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                acc[i][j] = (acc[i][j] + small[i][j]) * SP_UNSCALE;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) probe = fmaf(acc[i][j][r], 0.f, probe);
+            }
+        if (__any(probe != 0.f)) {   // (NaN compares unequal)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) acc[i][j] = again(m0 + 32 * (wm * TM + i), n0 + 32 * (wn * TN + j));
+        }
+        with_epilogue([&](auto act, auto res) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    float v[16];
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) v[r] = acc[i][j][r];
+                    finish(std::integral_constant<int, 16>{}, act, res, v, 32 * (wm * TM + i) + 4 * lh, 32 * (wn * TN + j) + li, bias[j]);
+                }
+        });
+    } else {
+        // [group][block][register / 4][lane]: the quads of all groups are added up by the thread that stores them
+        constexpr int QUADS = BLOCKS * 256, PER = (QUADS + THREADS - 1) / THREADS;
+        f32x4* sums = reinterpret_cast<f32x4*>(lds);
+        __syncthreads();   // everyone has read its fragments
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                acc[i][j] = (acc[i][j] + small[i][j]) * SP_UNSCALE;
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    sums[((wk * BLOCKS + (wm * TM + i) * (TN * WAVES_N) + wn * TN + j) * 4 + q) * WAVE + lane] =
+                        f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+            }
+        float bias[PER];
+#pragma unroll
+        for (int it = 0; it < PER; ++it) {
+            const int v = it * THREADS + tid;
+            bias[it] = bias_of(32 * (v / 256 % (TN * WAVES_N)) + li);
+        }
+        __syncthreads();
+        f32x4 sum[PER];
+        float probe = 0.f;
+#pragma unroll
+        for (int it = 0; it < PER; ++it) {
+            const int v = min(it * THREADS + tid, QUADS - 1);
+            sum[it] = sums[v];
+#pragma unroll
+            for (int w = 1; w < WAVES_K; ++w) sum[it] += sums[w * QUADS + v];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) probe = fmaf(sum[it][r], 0.f, probe);
+        }
+        if (__syncthreads_or(probe != 0.f)) {
+            for (int block = wave; block < BLOCKS; block += WAVES) {
+                const f32x16 v = again(m0 + 32 * (block / (TN * WAVES_N)), n0 + 32 * (block % (TN * WAVES_N)));
+#pragma unroll
+                for (int q = 0; q < 4; ++q) sums[(block * 4 + q) * WAVE + lane] = f32x4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+            }
+            __syncthreads();
+#pragma unroll
+            for (int it = 0; it < PER; ++it) sum[it] = sums[min(it * THREADS + tid, QUADS - 1)];
+        }
+        with_epilogue([&](auto act, auto res) __attribute__((always_inline)) {
+#pragma unroll
+            for (int it = 0; it < PER; ++it) {
+                const int v = it * THREADS + tid, block = v / 256;
+                if (QUADS % THREADS && v >= QUADS) break;
+                const float s[4] = {sum[it][0], sum[it][1], sum[it][2], sum[it][3]};
+                finish(std::integral_constant<int, 4>{}, act, res, s, 32 * (block / (TN * WAVES_N)) + 8 * (v / WAVE % 4) + 4 * lh,
+                       32 * (block % (TN * WAVES_N)) + li, bias[it]);
+            }
+        });
+    }
+}
+
+// One unit (eight k of a row, a lane's share of a fragment) per thread: bound by the reads of B, once when a graph is prepared.
+__global__ void pack_f32_kernel(const float* w, u32x4* packed, int64_t rows, int64_t K, int64_t s_row, int64_t s_k, int64_t units) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= units) return;
+    const int l = (int)(i % WAVE), s = (int)(i / WAVE % 2), g = 2 * s + l / 32;
+    const int64_t steps = K / 32, step = i / (2 * WAVE) % steps, block = i / (2 * WAVE) / steps, row = block * 32 + l % 32;
+    f32x4 v[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[h][e] = row < rows ? w[row * s_row + (step * 32 + 16 * h + 4 * g + e) * s_k] : 0.f;
+    u32x4 part[SP_PLANES];
+    split_unit8(v[0], v[1], part);
+#pragma unroll
+    for (int q = 0; q < SP_PLANES; ++q) packed[((i / WAVE) * SP_PLANES + q) * WAVE + l] = part[q];
+}
+
+// Nanoseconds: `fixed` and `per_k` while every workgroup has a CU to itself, `again` and `again_k` for each further one on the same CU
+// (by halves from six on, where they no longer run in step). Fitted over 600 products of M = 8 to 16384, N = 64 to 32000 and
+// K = 64 to 4096; the pick is 1 % behind the fastest form or older kernel on average.
+struct PackedForm { int bm, bn, threads, resident; double fixed, per_k, again, again_k; };
+static const PackedForm kPackedForms[] = {
+    {128, 256, 512, 1, 8440, 56.0, 7580, 64.7}, {64, 256, 256, 2, 5220, 35.8, 3290, 30.8}, {64, 192, 512, 1, 7490, 25.8, 5920, 29.7},
+    {64, 128, 512, 1, 4900, 16.5, 2570, 17.5},  {64, 64, 512, 1, 5180, 8.85, 3530, 12.1},  {64, 64, 256, 3, 3870, 15.0, 860, 10.6},
+    {32, 64, 512, 1, 4260, 5.5, 1290, 6.25},    {32, 32, 512, 1, 4730, 3.69, 2050, 5.7},   {128, 128, 256, 2, 6040, 35.6, 3120, 31.7},
+    {64, 128, 256, 2, 3660, 21.0, 1900, 16.2}};
+constexpr int kNumPackedForms = sizeof(kPackedForms) / sizeof(kPackedForms[0]);
+
+static void launch_packed(int form, const PackedGemmArgs& p, hipStream_t st) {
+    const dim3 grid((unsigned)p.g.nwg), block(kPackedForms[form].threads);
+    switch (form) {
+        case 0: hipLaunchKernelGGL((gemm_f32_packed_kernel<2, 2, 2, 4, 1, 2>), grid, block, 0, st, p); break;
+        case 1: hipLaunchKernelGGL((gemm_f32_packed_kernel<2, 2, 1, 4, 1, 2>), grid, block, 0, st, p); break;
+        case 2: hipLaunchKernelGGL((gemm_f32_packed_kernel<1, 3, 2, 2, 2, 2>), grid, block, 0, st, p); break;
+        case 3: hipLaunchKernelGGL((gemm_f32_packed_kernel<2, 1, 1, 4, 2, 2>), grid, block, 0, st, p); break;
+        case 4: hipLaunchKernelGGL((gemm_f32_packed_kernel<2, 1, 1, 2, 4, 2>), grid, block, 0, st, p); break;
+        case 5: hipLaunchKernelGGL((gemm_f32_packed_kernel<1, 1, 2, 2, 1, 3>), grid, block, 0, st, p); break;
+        case 6: hipLaunchKernelGGL((gemm_f32_packed_kernel<1, 1, 1, 2, 4, 2>), grid, block, 0, st, p); break;
+        case 8: hipLaunchKernelGGL((gemm_f32_packed_kernel<2, 2, 2, 2, 1, 2>), grid, block, 0, st, p); break;
+        case 9: hipLaunchKernelGGL((gemm_f32_packed_kernel<2, 1, 1, 4, 1, 2>), grid, block, 0, st, p); break;
+        default: hipLaunchKernelGGL((gemm_f32_packed_kernel<1, 1, 1, 1, 8, 2>), grid, block, 0, st, p); break;
+    }
+}
+
+static double packed_cost(const PackedForm& f, int64_t nwg, int64_t K, int cus) {
+    const int64_t up = ceil_div(nwg, (int64_t)cus);
+    const double more = up <= 6 ? (double)(up - 1) : (double)nwg / cus - 0.5;
+    return f.fixed + f.per_k * (double)K + more * (f.again + f.again_k * (double)K);
+}
+
+// What mi355x_gemm_f32 takes, from the rules of its kernels (with what those leave out because it is the same on both of their sides:
+// a launch, first loads, last stores). Over the same products a median 7 % below what was measured.
+static double unpacked_cost(const GemmArgs& p, bool b_kc, int cus) {
+    double best = gemm_f32_direct_cost(p, b_kc, cus);
+    const bool nt = b_kc && p.N % 4 == 0;
+    if (nt) best = std::min(best, gemm_f32_nt_cost(p, cus));
+    const double split = gemm_f32_split_cost(p, cus);
+    if (split < 1e300 && p.K >= (nt ? 256 : 128)) best = std::min(best, (nt ? 6000 : 8000) + split * (double)p.K);
+    return best;
+}
+
+// Preconditions of the kernel besides pointer alignment
+static bool packed_takes(const GemmArgs& p) {
+    return p.K > 0 && p.K % 32 == 0 && p.a_sk == 1 && p.a_sm >= 0 && p.a_sm % 4 == 0 && p.a_sb0 % 4 == 0 && p.a_sb1 % 4 == 0 &&
+           p.b_sb0 == 0 && p.b_sb1 == 0 && (p.M - 1) * p.a_sm + p.K < ((int64_t)1 << 29) &&
+           ceil_div(p.N, (int64_t)32) * (p.K / 32) * (2 * PK_FRAGMENT) < ((int64_t)1 << 31) &&
+           p.c_sm >= 0 && p.c_sm < ((int64_t)1 << 22) && p.r_sm >= 0 && p.r_sm < ((int64_t)1 << 22);   // (rows of a tile of C, 32-bit byte offsets)
+}
+
+// The fastest form, -1 where mi355x_gemm_f32 is faster.
+static int choose_packed(const GemmArgs& p, int cus) {
+    double best_cost = unpacked_cost(p, p.b_sk == 1, cus);
+    int best = -1;
+    for (int f = 0; f < kNumPackedForms; ++f) {
+        const PackedForm& form = kPackedForms[f];
+        const double cost = packed_cost(form, p.batch * ceil_div(p.M, (int64_t)form.bm) * ceil_div(p.N, (int64_t)form.bn), p.K, cus);
+        if (cost < best_cost) { best = f; best_cost = cost; }
+    }
+    return best;
+}
+
+}  // namespace mi355x
+
+extern "C" int mi355x_pack_f32(const float* w, void* packed, int64_t rows, int64_t K, int64_t row_stride, int64_t k_stride, void* stream) {
+    using namespace mi355x;
+    MI355X_REQUIRE(rows >= 0 && K >= 0 && K % 32 == 0, "pack: %lld rows of %lld values, no multiple of 32", (long long)rows, (long long)K);
+    if (rows == 0 || K == 0) return MI355X_OK;
+    MI355X_REQUIRE(w && packed && (reinterpret_cast<uintptr_t>(packed) & 15) == 0, "pack: null or unaligned pointer");
+    const int64_t units = ceil_div(rows, (int64_t)32) * (K / 32) * 2 * WAVE;
+    MI355X_REQUIRE(grid_fits(ceil_div(units, (int64_t)256), 256), "pack: grid too large");
+    hipLaunchKernelGGL(pack_f32_kernel, dim3((unsigned)ceil_div(units, (int64_t)256)), dim3(256), 0, static_cast<hipStream_t>(stream), w,
+                       static_cast<u32x4*>(packed), rows, K, row_stride, k_stride, units);
+    return check_launch("pack_f32_kernel");
+}
+
+extern "C" int mi355x_gemm_packed_pays(int64_t batch, int64_t M, int64_t N, int64_t K, int b_kc) {
+    using namespace mi355x;
+    if (batch <= 0 || M <= 0 || N <= 0 || K <= 0) return 0;
+    GemmArgs p = {};
+    p.batch = batch; p.batch1 = 1; p.M = M; p.N = N; p.K = K;
+    p.a_sm = K; p.a_sk = 1; p.b_sk = b_kc ? 1 : N; p.b_sn = b_kc ? K : 1; p.c_sm = N;
+    const int cus = device_cus();
+    return packed_takes(p) && choose_packed(p, cus > 0 ? cus : 256) >= 0;
+}
+
+extern "C" int mi355x_gemm_packed_f32(const float* A, const void* packed, const float* B, float* C, const float* bias,
+                                      const float* residual, int64_t batch0, int64_t batch1, int64_t M, int64_t N, int64_t K,
+                                      const int64_t* a_strides, const int64_t* b_strides, const int64_t* c_strides,
+                                      const int64_t* r_strides, float alpha, int epilogue, void* stream) {
+    using namespace mi355x;
+    PackedGemmArgs pa;
+    GemmArgs& p = pa.g;
+    const int force = tuning().gemm_packed;
+    auto al16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+    if (A && B && C && packed && a_strides && b_strides && c_strides && batch0 > 0 && batch1 > 0 && M > 0 && N > 0 && K > 0 && force != 0 &&
+        (epilogue & ~(MI355X_EPI_BIAS | MI355X_EPI_RELU | MI355X_EPI_GELU | MI355X_EPI_RESIDUAL)) == 0 && (!(epilogue & MI355X_EPI_BIAS) || bias) &&
+        (!(epilogue & MI355X_EPI_RESIDUAL) || (residual && r_strides)) && (c_strides[2] >= N || M == 1) && al16(A) && al16(packed)) {
+        MI355X_TRACE_INIT(p);
+        p.A = A; p.B = B; p.C = C; p.bias = bias; p.residual = residual;
+        p.batch = batch0 * batch1; p.batch1 = batch1; p.M = M; p.N = N; p.K = K;
+        p.a_sb0 = a_strides[0]; p.a_sb1 = a_strides[1]; p.a_sm = a_strides[2]; p.a_sk = a_strides[3];
+        p.b_sb0 = b_strides[0]; p.b_sb1 = b_strides[1]; p.b_sk = b_strides[2]; p.b_sn = b_strides[3];
+        p.c_sb0 = c_strides[0]; p.c_sb1 = c_strides[1]; p.c_sm = c_strides[2];
+        const bool res = epilogue & MI355X_EPI_RESIDUAL;
+        p.r_sb0 = res ? r_strides[0] : 0; p.r_sb1 = res ? r_strides[1] : 0; p.r_sm = res ? r_strides[2] : 0;
+        p.alpha = alpha; p.epi = epilogue;
+        pa.packed = static_cast<const char*>(packed);
+        pa.kt = (int)(K / 32);
+        const int cus = device_cus();
+        if (cus <= 0) return set_error(MI355X_ERR_NOT_INITIALIZED, "gemm: no usable HIP device");
+        const int form = !packed_takes(p) ? -1 : force > 0 ? force - 1 : choose_packed(p, cus);
+        if (form >= 0 && form < kNumPackedForms) {
+            const PackedForm& f = kPackedForms[form];
+            p.tiles_m = ceil_div(M, (int64_t)f.bm);
+            p.tiles_n = ceil_div(N, (int64_t)f.bn);
+            p.nwg = p.batch * p.tiles_m * p.tiles_n;
+            if (grid_fits(p.nwg, f.threads)) {
+                const int64_t per_xcd = ceil_div(p.nwg, (int64_t)NUM_XCD), per_batch = p.tiles_m * p.tiles_n;
+                p.group_m = choose_group_m(p.tiles_m, per_xcd < per_batch ? per_xcd : per_batch, (int64_t)f.resident * (cus / NUM_XCD), f.bm, f.bn, K * 5);
+                launch_packed(form, pa, static_cast<hipStream_t>(stream));
+                return check_launch("gemm_f32_packed_kernel");
+            }
+        }
+    }
+    return mi355x_gemm_f32(A, B, C, bias, residual, batch0, batch1, M, N, K, a_strides, b_strides, c_strides, r_strides, alpha, epilogue, stream);
+}

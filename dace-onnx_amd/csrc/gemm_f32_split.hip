@@ -35,29 +35,13 @@
 #include "common.h"
 #include "gemm_tile.h"
 #include "gemm_args.h"
+#include "split_bf16.h"
 
 #include <algorithm>
 
 namespace mi355x {
 
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-constexpr int SP_BK = 32, SP_PLANES = 3, SP_FRAGMENT = 1024;   // k extent of a tile; bytes of one plane of 16 rows
-
-// two floats -> the three bf16 parts of SP_SCALE times them, packed
-constexpr float SP_SCALE = 65536.f, SP_UNSCALE = 1.f / (SP_SCALE * SP_SCALE);
-__device__ __forceinline__ void split_pair(float x, float y, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
-    auto pack = [](float a, float b) { return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2)); };
-    auto low = [](uint32_t v) { return __builtin_bit_cast(float, v << 16); };
-    auto high = [](uint32_t v) { return __builtin_bit_cast(float, v & 0xffff0000u); };
-    x *= SP_SCALE; y *= SP_SCALE;
-    hi = pack(x, y);
-    x -= low(hi); y -= high(hi);
-    mid = pack(x, y);
-    x -= low(mid); y -= high(mid);
-    lo = pack(x, y);
-}
+constexpr int SP_BK = 32, SP_FRAGMENT = 1024;   // k extent of a tile; bytes of one plane of 16 rows
 
 // byte offset of unit g (0..3) of row r (0..15) inside a fragment
 __device__ __forceinline__ int split_unit(int r, int g) {
@@ -102,14 +86,7 @@ struct SplitTile {
     }
     __device__ __forceinline__ void store(char* planes, int it) const {
         u32x4 part[SP_PLANES];
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                uint32_t hi, mid, lo;
-                split_pair(v[it][h][2 * s], v[it][h][2 * s + 1], hi, mid, lo);
-                part[0][2 * h + s] = hi; part[1][2 * h + s] = mid; part[2][2 * h + s] = lo;
-            }
+        split_unit8(v[it][0], v[it][1], part);
 #pragma unroll
         for (int q = 0; q < SP_PLANES; ++q) *reinterpret_cast<u32x4*>(planes + q * PLANE + lds[it]) = part[q];
     }

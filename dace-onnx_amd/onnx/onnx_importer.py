@@ -207,6 +207,7 @@ class ONNXModel:
                     self.state.add_edge(op_node, conn_name, access, None, memlet)
 
         self._compiled = None
+        self._packed = []   # packed copies of constant operands (transformation/packing.py)
         self._expanded = False
         self._static_io = None
 
@@ -355,6 +356,8 @@ class ONNXModel:
             if self.device.type != "cuda":
                 raise RuntimeError("ONNXModel executes on the MI355X only: no HIP device is visible")
             self.expand()
+            from ..transformation.packing import pack_constant_operands
+            self._packed = pack_constant_operands(self)
             self._compiled = self.sdfg.compile()
         return self._compiled
 
@@ -382,6 +385,8 @@ class ONNXModel:
                  input was a torch tensor, numpy arrays otherwise.
         """
         compiled = self.compile_and_init()
+        for copy_of_weight in self._packed:
+            copy_of_weight.refresh()
         inputs = self._call_args(args, kwargs)
         use_torch = any(isinstance(v, torch.Tensor) for v in inputs.values())
         call = {}

@@ -102,6 +102,24 @@ int mi355x_gemm_f32(const float* A, const float* B, float* C,
                     const int64_t* c_strides, const int64_t* r_strides,
                     float alpha, int epilogue, void* stream);
 
+/* The same product with a B that is constant, [K, N] without batch dimensions, and was packed beforehand for the bf16
+ * matrix unit (three bf16 parts of every value, in the order the kernel's registers take them; ONNX nodes do it once when the
+ * graph is prepared, transformation/packing.py, and the reference has no counterpart). `packed` holds, 6144 bytes each,
+ * ceil(N / 32) x K / 32 pairs of fragments (csrc/split_bf16.h); mi355x_pack_f32 writes them. B is the weight itself: it is read where a sum is not finite,
+ * and by mi355x_gemm_f32, which is called where the packed form does not apply (K not a multiple of 32, an A that is not
+ * contiguous along k or not on 16-byte boundaries, or a product for which it is not the faster one). */
+int mi355x_gemm_packed_f32(const float* A, const void* packed, const float* B, float* C, const float* bias,
+                           const float* residual, int64_t batch0, int64_t batch1, int64_t M, int64_t N, int64_t K,
+                           const int64_t* a_strides, const int64_t* b_strides, const int64_t* c_strides,
+                           const int64_t* r_strides, float alpha, int epilogue, void* stream);
+/* 1 where mi355x_gemm_packed_f32 takes `batch` products of M x N x K on the packed form (b_kc: B contiguous along k, else
+ * along n): what graph preparation asks before it packs. */
+int mi355x_gemm_packed_pays(int64_t batch, int64_t M, int64_t N, int64_t K, int b_kc);
+/* `rows` x K values (K a multiple of 32; strides in elements) packed, 16-byte aligned: for a [K, N] weight of contiguous rows
+ * rows = N, row_stride = 1, k_stride = N. */
+int mi355x_pack_f32(const float* w, void* packed, int64_t rows, int64_t K, int64_t row_stride, int64_t k_stride, void* stream);
+
+
 /* ONNX Conv, 2-D, NCHW, group 1, fp32, implicit GEMM on MFMA.
  *   Y[n,m,oy,ox] = epilogue(sum_{c,r,s} W[m,c,r,s] *
  *        X[n,c,oy*stride_h - pad_top + r*dil_h, ox*stride_w - pad_left + s*dil_w])

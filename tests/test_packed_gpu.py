@@ -1,0 +1,116 @@
+"""The kernels that multiply by packed constants, at the edges of their tiles and values, against float64."""
+import numpy as np
+import pytest
+import torch
+import torch.nn as nn
+
+from dace_onnx_amd import _lib
+from dace_onnx_amd.pytorch.module import DaceModule
+
+pytestmark = pytest.mark.gpu
+FORMS = range(1, 11)
+
+
+def call(name, *args):
+    _lib.check(getattr(_lib.library(), name)(*args, torch.cuda.current_stream().cuda_stream), name)
+
+
+def gpu(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def pack(w, rows, k, s_row, s_k):
+    packed = torch.empty(-(-rows // 32), k // 32, 2, 3, 64, 4, dtype=torch.int32, device="cuda")
+    call("mi355x_pack_f32", w.data_ptr(), packed.data_ptr(), rows, k, s_row, s_k)
+    return packed
+
+
+def packed_gemm(a, b, kc, bias=None, res=None, epi=0, alpha=1.0, batch=1, c_gap=0):
+    """C = a @ b; ``b`` is [N, K] if ``kc`` else [K, N]; rows of C ``c_gap`` apart, which stays as it was."""
+    M, K = a.shape[-2:]
+    N = b.shape[0] if kc else b.shape[1]
+    c = torch.full((batch, M, N + c_gap), -7.0, device="cuda")
+    i64 = _lib.i64_array
+    call("mi355x_gemm_packed_f32", a.data_ptr(), pack(b, N, K, *((K, 1) if kc else (1, N))).data_ptr(), b.data_ptr(), c.data_ptr(), _lib.ptr(bias),
+         _lib.ptr(res), 1, batch, M, N, K, i64([0, M * K, K, 1]), i64([0, 0] + ([1, K] if kc else [N, 1])), i64([0, M * (N + c_gap), N + c_gap]),
+         i64([0, M * N, N]), alpha, epi)
+    assert bool((c[..., N:] == -7).all())
+    return c[..., :N]
+
+
+def test_a_packed_operand_holds_every_bit():
+    w = gpu(np.random.default_rng(0).standard_normal((45, 96), dtype=np.float32) * np.float32(2.0)**np.arange(-140, 100, 2.5, dtype=np.float32))
+    parts = pack(w, 45, 96, 96, 1).cpu().view(torch.bfloat16).reshape(2, 3, 2, 3, 2, 32, 2, 4).double().sum(3)   # block, step, s, h, row, a, e
+    rows = parts.permute(0, 4, 1, 5, 2, 3, 6).reshape(64, 96) / 65536
+    assert torch.equal(rows[:45], w.cpu().double()) and not rows[45:].any()
+
+
+@pytest.mark.parametrize("kc", [True, False])
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("batch, M, N, K, epi", [(1, 1, 1, 32, 0), (1, 31, 33, 64, 1), (1, 64, 64, 96, 9), (2, 129, 127, 160, 13), (1, 257, 130, 32, 3),
+                                                 (1, 255, 258, 768, 9), (3, 96, 515, 1056, 8)])
+def test_gemm_by_a_packed_constant(tuning, form, kc, batch, M, N, K, epi):
+    """A sum of K products: at most one rounding (2^-23, truncation included) for each of the K / 16 steps, and three of 2^-24 for the
+    products left out and the sets of sums."""
+    tuning(MI355X_GEMM_PACKED=form)
+    rng = np.random.default_rng(M + N + K)
+    a = gpu(rng.standard_normal((batch, M, K), dtype=np.float32))
+    b = gpu(rng.standard_normal((N, K) if kc else (K, N), dtype=np.float32))
+    bias, res = gpu(rng.standard_normal(N, dtype=np.float32)), gpu(rng.standard_normal((batch, M, N), dtype=np.float32))
+    got = packed_gemm(a, b, kc, bias, res, epi, 0.5, batch, c_gap=3)
+    wide = b.double().t() if kc else b.double()
+    expected = 0.5 * (a.double() @ wide) + (bias.double() if epi & 1 else 0)
+    if epi & 2:
+        expected = expected.relu()
+    if epi & 4:
+        expected = torch.nn.functional.gelu(expected)
+    if epi & 8:
+        expected = expected + res.double()
+    bound = (a.double().abs() @ wide.abs() + 1) * (K // 16 + 8) * 2.0**-23
+    assert bool(((expected - got.double()).abs() <= 1.2 * bound).all())   # 1.13 is Gelu's steepest slope
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_gemm_by_a_packed_constant_keeps_infinities_nan_and_the_largest_values(tuning, form):
+    tuning(MI355X_GEMM_PACKED=form)
+    a = torch.randn(1, 300, 96, device="cuda")
+    b = torch.rand(200, 96, device="cuda") + 0.5
+    a[0, 3, 5], a[0, 70, 95], a[0, 130, 0], a[0, 131, 1:3] = float("inf"), -float("inf"), float("nan"), torch.tensor([float("inf"), -float("inf")])
+    a[0, 200], a[0, 200, 7], a[0, 290, 9] = 0, 3.4e38, 3.3999e38   # rounds up to infinity in bf16
+    b[:, 7] = 0.75
+    b[11, 9], b[150, 9], b[150, 60] = 0, 0.5, float("inf")   # (0.5: no product of its own overflows next to the infinite one)
+    expected = a[0].double() @ b.double().t()
+    single = expected.float()
+    fine = torch.isfinite(single)
+    for kc in (True, False):
+        got = packed_gemm(a, b if kc else b.t().contiguous(), kc)[0]
+        assert torch.equal(torch.isnan(single), torch.isnan(got)) and torch.equal(torch.isinf(single), torch.isinf(got))
+        assert torch.equal(single[~fine].nan_to_num(nan=0), got[~fine].nan_to_num(nan=0))
+        assert bool(((expected - got.double()).abs()[fine] <= 1e-5 * (a[0].double().abs().nan_to_num(0, 0) @ b.double().abs().nan_to_num(0, 0, 0).t())[fine]).all())
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("low, high", [(-100, 90), (-120, 100), (-148, 105), (-60, -58), (90, -3)])
+def test_gemm_by_a_packed_constant_keeps_small_values(tuning, form, low, high):
+    """Values down to the smallest subnormal against values that bring the sums back to ordinary size: exact products, so the bound is
+    that of ordinary ones."""
+    tuning(MI355X_GEMM_PACKED=form)
+    rng = np.random.default_rng(form)
+    a, b = (gpu(np.ldexp(rng.uniform(1, 2, s) * rng.choice([-1, 1], s), e).astype(np.float32)) for s, e in (((1, 70, 96), low), ((70, 96), high)))
+    got = packed_gemm(a, b, True)[0]
+    expected, size = a[0].double() @ b.double().t(), a[0].double().abs() @ b.double().abs().t()
+    assert bool(((expected - got.double()).abs() <= size * 14 * 2.0**-23 + 2.0**-149).all())
+
+
+def test_a_packed_copy_follows_its_weight():
+    """Parameters written in place after the first call: the next call multiplies by the new ones."""
+    linear = nn.Linear(768, 1024).cuda()
+    x = torch.randn(512, 768, device="cuda")
+    model = DaceModule(nn.Sequential(linear, nn.ReLU()), dummy_inputs=(x, ))
+    for _ in range(2):
+        with torch.no_grad():
+            linear.weight.mul_(0.5)
+            linear.weight[3] += 1
+        got, expected = model(x), torch.relu(x.double() @ linear.weight.double().t() + linear.bias.double()).detach()
+        assert float((got.double() - expected).norm() / expected.norm()) < 1e-6
+    assert [n.function for n, _ in model.dace_model.compile_and_init().bound_launches()] == ["mi355x_gemm_packed_f32"]
