@@ -573,6 +573,14 @@ static void launch_conv(const ConvArgs& p, hipStream_t st) {
     else hipLaunchKernelGGL((conv2d_f32_kernel<BM, BN, BK, WMs, WNs, false>), grid, block, 0, st, p);
 }
 
+// A round of 64 x 64 tiles takes 16.5 ns per k and 5.1 us besides (8 to 200 tiles: K = 576 15 us, 1152 24, 2304 42, 4608 77), 1 x 1
+// filters 17.2 and 5.05 (K = 64 6.6, 128 7.8, 256 10.3), further rounds a little less; strided ones 1.1 us more (9 x 128 x 24 x 24 -> 256 8.6).
+double conv2d_f32_gather_cost(const ConvArgs& p, int cus) {
+    const double k = (double)p.K, more = (double)(ceil_div(ceil_div((int64_t)p.M, (int64_t)CG_BM) * ceil_div(p.P, (int64_t)64), (int64_t)cus) - 1);
+    const double strided = p.stride_h > 1 || p.stride_w > 1 ? 1100 : 0;
+    return strided + (p.KH * p.KW == 1 ? 5050 + 17.2 * k + more * (2370 + 13.7 * k) : 5100 + 16.5 * k + more * (650 + 16.5 * k));
+}
+
 struct ConvTile { int bm, bn; };
 static const ConvTile kConvTiles[] = {{64, 128}, {64, 64}, {32, 64}, {16, 64}, {128, 64}};
 constexpr int kNumConvTiles = sizeof(kConvTiles) / sizeof(kConvTiles[0]);
@@ -657,15 +665,9 @@ extern "C" int mi355x_conv2d_res_f32(const float* X, const float* W, const float
     if (K % CG_BK == 0 && K <= CG_MAX_K && KH * KW <= 32 && M * K < ((int64_t)1 << 29) && C * H * Wd < ((int64_t)1 << 27) &&
         N * C * H * Wd + pads[0] * Wd + pads[1] + H * Wd < ((int64_t)1 << 29) && al16(W) && tune.conv_config < 0) {
         p.x_bytes = (int)(N * C * H * Wd * 4);
-        // Few tiles: the kernel that reads its operands straight from memory, where its sweep says it is ahead. A round of 64 x 64
-        // tiles takes 16.5 ns per k and 5.1 us besides (8 to 200 tiles: K = 576 15 us, 1152 24, 2304 42, 4608 77), 1 x 1 filters
-        // 17.2 and 5.05 (K = 64 6.6, 128 7.8, 256 10.3), further rounds a little less; strided ones 1.1 us more (9 x 128 x 24 x 24 -> 256 8.6).
-        if (tune.conv_gather_bn == 0 && tune.conv_per_cu == 0 && tune.conv_tail < 0 && tune.conv_static_taps == 1) {
-            const double k = (double)K, more = (double)(ceil_div(ceil_div(M, (int64_t)CG_BM) * ceil_div(P, (int64_t)64), (int64_t)cus) - 1);
-            const double strided = strides[0] > 1 || strides[1] > 1 ? 1100 : 0;
-            const double gather = strided + (KH * KW == 1 ? 5050 + 17.2 * k + more * (2370 + 13.7 * k) : 5100 + 16.5 * k + more * (650 + 16.5 * k));
-            if (launch_conv2d_f32_direct(p, gather, cus, st)) return check_launch("conv2d_f32_direct_kernel");
-        }
+        // Few tiles: the kernel that reads its operands straight from memory, where its sweep says it is ahead.
+        if (tune.conv_gather_bn == 0 && tune.conv_per_cu == 0 && tune.conv_tail < 0 && tune.conv_static_taps == 1 &&
+            launch_conv2d_f32_direct(p, conv2d_f32_gather_cost(p, cus), cus, st)) return check_launch("conv2d_f32_direct_kernel");
         // 64 x 64 tiles (three workgroups share a CU) or 64 x 128 (one per CU). Time goes with the tiles a CU has
         // to run times their width; the wide tile, alone on its CU, pays its first loads and last stores in the open
         // (32 x 64 x 56 x 56 -> 64: 101.5 us as 784 wide tiles, 73.2 us as 1568 narrow ones two to a CU), hence its factor.

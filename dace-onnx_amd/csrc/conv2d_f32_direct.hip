@@ -158,15 +158,15 @@ static void launch_direct(int form, const ConvArgs& p, hipStream_t st) {
     else hipLaunchKernelGGL((conv2d_f32_direct_kernel<2, 2, TAPS>), grid, block, 0, st, p);
 }
 
-bool launch_conv2d_f32_direct(const ConvArgs& args, double other_cost, int cus, hipStream_t stream) {
-    ConvArgs p = args;
+// The fastest form of these and its time; -1 where there is none.
+static int choose_direct(const ConvArgs& p, int cus, double& best_cost) {
     const int force = tuning().conv_direct;
     const bool taps9 = p.KH == 3 && p.KW == 3 && p.C % 4 == 0, taps1 = p.KH == 1 && p.KW == 1 && p.C % 16 == 0;
-    if (force == 0 || !(taps9 || taps1)) return false;
+    best_cost = 1e300;
+    if (force == 0 || !(taps9 || taps1)) return -1;
     // both operands are addressed with 32-bit byte offsets
-    if ((int64_t)p.M * p.K >= ((int64_t)1 << 29) || (int64_t)p.N * p.C * p.H * p.Wd >= ((int64_t)1 << 29)) return false;
+    if ((int64_t)p.M * p.K >= ((int64_t)1 << 29) || (int64_t)p.N * p.C * p.H * p.Wd >= ((int64_t)1 << 29)) return -1;
     int best = -1;
-    double best_cost = 0.95 * other_cost;
     for (int f = 0; f < 6; ++f) {
         const ConvDirectForm& form = kConvDirectForms[f];
         if (form.taps != (taps9 ? 9 : 1)) continue;
@@ -175,12 +175,25 @@ bool launch_conv2d_f32_direct(const ConvArgs& args, double other_cost, int cus, 
         const double cost = form.fixed + form.again * (double)(rounds - 1) + strided * (double)p.K * (form.per_k + form.again_k * (double)(rounds - 1));
         if (force > 0 ? force == 10 * form.tm + form.tp : cost < best_cost) { best = f; best_cost = cost; }
     }
-    if (best < 0) return false;
+    return best;
+}
+
+double conv2d_f32_direct_cost(const ConvArgs& p, int cus) {
+    double cost;
+    choose_direct(p, cus, cost);
+    return cost;
+}
+
+bool launch_conv2d_f32_direct(const ConvArgs& args, double other_cost, int cus, hipStream_t stream) {
+    ConvArgs p = args;
+    double cost;
+    const int best = choose_direct(p, cus, cost);
+    if (best < 0 || (tuning().conv_direct <= 0 && cost >= 0.95 * other_cost)) return false;
     p.tiles_m = ceil_div((int64_t)p.M, (int64_t)16 * kConvDirectForms[best].tm);
     p.tiles_p = ceil_div(p.P, (int64_t)16 * kConvDirectForms[best].tp);
     p.nwg = p.tiles_m * p.tiles_p;
     if (!grid_fits(p.nwg, WAVE * CD_WAVES)) return false;
-    if (taps9) launch_direct<9>(best % 3, p, stream);
+    if (kConvDirectForms[best].taps == 9) launch_direct<9>(best % 3, p, stream);
     else launch_direct<1>(best % 3, p, stream);
     return true;
 }

@@ -57,8 +57,12 @@ struct ConvArgs {
     MI355X_TRACE_MEMBER
 };
 
+// Nanoseconds of the gather kernel (conv2d_f32.hip).
+double conv2d_f32_gather_cost(const ConvArgs& p, int cus);
+
 // Convolution whose output is few tiles (conv2d_f32_direct.hip), 3 x 3 and 1 x 1 filters: no staging, the channels split over the
 // waves of a workgroup. `other_cost`: nanoseconds the caller's own kernel takes; nothing is launched where it is not behind.
+double conv2d_f32_direct_cost(const ConvArgs& p, int cus);   // nanoseconds of its fastest form, 1e300 where it has none
 bool launch_conv2d_f32_direct(const ConvArgs& p, double other_cost, int cus, hipStream_t stream);
 
 }  // namespace mi355x

@@ -10,6 +10,7 @@ are written into the tensors or arrays the caller passed.
 import numpy as np
 
 from ... import sdfg as dace
+from ...transformation.packing import pack_variable_filters
 from .node_utils import parse_variadic_param
 
 
@@ -53,5 +54,6 @@ def call_onnx_op(cls, **kwargs):
             state.add_edge(node, conn, state.add_write(arr), None, sdfg.make_array_memlet(arr))
             node.add_out_connector(conn)
     sdfg.expand_library_nodes()
+    pack_variable_filters(sdfg)
     sdfg.compile()(**call_args)
     return None

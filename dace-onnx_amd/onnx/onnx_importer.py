@@ -356,8 +356,9 @@ class ONNXModel:
             if self.device.type != "cuda":
                 raise RuntimeError("ONNXModel executes on the MI355X only: no HIP device is visible")
             self.expand()
-            from ..transformation.packing import pack_constant_operands
+            from ..transformation.packing import pack_constant_operands, pack_variable_filters
             self._packed = pack_constant_operands(self)
+            pack_variable_filters(self.sdfg)
             self._compiled = self.sdfg.compile()
         return self._compiled
 

@@ -1,4 +1,5 @@
-"""Constant operands of contractions, packed for the kernels of ``csrc/gemm_f32_packed.hip`` when a graph is compiled.
+"""Constant operands of contractions, packed for the kernels of ``csrc/gemm_f32_packed.hip`` and ``csrc/conv2d_f32_packed.hip`` when a
+graph is compiled.
 
 A packed copy holds three bf16 parts of every value in the order in which the matrix unit takes them (``csrc/split_bf16.h``); it is
 made once, on the GPU, and is a further weight of the model. The reference has no counterpart: its constants are handed to a BLAS
@@ -7,24 +8,23 @@ library as they are.
 import torch
 
 from .. import _lib
-from ..sdfg import AccessNode, KernelCall, Ptr, int32
+from ..sdfg import AccessNode, KernelCall, Ptr, Stream, int32
 
 
 class PackedOperand:
-    """A packed copy of ``rows`` x ``k`` values of a weight, at element strides ``row_stride`` and ``k_stride`` from ``offset``."""
+    """A packed copy of a weight, ``shape`` 32-bit words, written by the library's ``function`` from ``offset`` values on."""
 
-    def __init__(self, model, weight_name, rows, k, row_stride, k_stride, offset):
+    def __init__(self, model, weight_name, shape, function, geometry, offset):
         self.model, self.weight_name = model, weight_name
-        self.geometry = (rows, k, row_stride, k_stride)
-        self.offset = offset
-        self.packed = torch.empty([-(-rows // 32), k // 32, 2, 3, 64, 4], dtype=torch.int32, device=model.weights[weight_name].device)
+        self.function, self.geometry, self.offset = function, geometry, offset
+        self.packed = torch.empty(shape, dtype=torch.int32, device=model.weights[weight_name].device)
         self.pack()
 
     def pack(self):
         self.weight = self.model.weights[self.weight_name]
         self.version = self.weight._version
         start = self.weight.data_ptr() + 4 * self.offset
-        _lib.check(_lib.library().mi355x_pack_f32(start, self.packed.data_ptr(), *self.geometry, _lib.current_stream()), "mi355x_pack_f32")
+        _lib.check(getattr(_lib.library(), self.function)(start, self.packed.data_ptr(), *self.geometry, _lib.current_stream()), self.function)
 
     def refresh(self):
         """Pack again if the weight was replaced or written in place since (a wrapped module whose parameters were updated)."""
@@ -33,36 +33,91 @@ class PackedOperand:
             self.pack()
 
 
+def _packed_gemm(call, weight):
+    """(name suffix, shape, function, geometry, offset) of the copy that a GEMM multiplies by, and the call that does; None where it does not pay."""
+    lib = _lib.library()
+    offset = call.args[1].offset
+    batch0, batch1, M, N, K, a_strides, b_strides = call.args[5:12]
+    sb0, sb1, sk, sn = b_strides.values
+    if sb0 or sb1 or min(sk, sn) < 1 or a_strides.values[3] != 1 or a_strides.values[2] % 4 \
+            or not lib.mi355x_gemm_packed_pays(batch0 * batch1, M, N, K, int(sk == 1)):
+        return None
+    copy = (f"{N}_{K}_{sn}_{sk}_{offset}", [-(-N // 32), K // 32, 2, 3, 64, 4], "mi355x_pack_f32", (N, K, sn, sk), offset)
+    return copy, ("mi355x_gemm_packed_f32", [call.args[0], Ptr("_packed")] + call.args[1:])
+
+
+def _by_packed_filters(call, constant):
+    """(shape, geometry) of the copy that a convolution multiplies by, and the call that does; None where it does not pay."""
+    residual = [] if call.function == "mi355x_conv2d_res_f32" else [Ptr(None)]
+    args = [call.args[0], Ptr("_packed")] + call.args[1:3] + residual + call.args[3:]
+    N, C, H, Wd, M, KH, KW, pads, strides, dilations = args[6:16]
+    size = _lib.library().mi355x_conv2d_packed_pays(N, C, H, Wd, M, KH, KW, *(_lib.i64_array(a.values) for a in (pads, strides, dilations)), constant)
+    if not size or call.args[1].offset:
+        return None
+    return [size // 3072, 3, 64, 4], (M, C, KH, KW), ("mi355x_conv2d_packed_f32", args)
+
+
+def _packed_conv(call, weight):
+    """As :func:`_packed_gemm`, for a convolution."""
+    packed = _by_packed_filters(call, True)
+    if packed is None or tuple(weight.shape) != packed[1] or not weight.is_contiguous():
+        return None
+    shape, geometry, packed_call = packed
+    return ("filters", shape, "mi355x_pack_conv_f32", geometry, 0), packed_call
+
+
+def pack_variable_filters(sdfg):
+    """Pack the filters of the remaining convolutions on every call, where the library says that this pays too."""
+    for state in sdfg.nodes():
+        for call in state.nodes():
+            packed = _by_packed_filters(call, False) if isinstance(call, KernelCall) and _PACKED.get(call.function) is _packed_conv else None
+            if packed is None:
+                continue
+            shape, geometry, (function, args) = packed
+            filters = next(e for e in state.in_edges(call) if e.dst_conn == args[2].connector).src
+            clean = f"{filters.data}_packed_for_{state.node_id(call)}"
+            sdfg.add_transient(clean, shape, int32)
+            packed_call = KernelCall(call.label, function, args, list(call.in_connectors) + ["_packed"], list(call.out_connectors))
+            state.replace_node(call, packed_call, sdfg)
+            pack = KernelCall(f"{call.label}_pack", "mi355x_pack_conv_f32", [Ptr("W"), Ptr("_packed"), *geometry, Stream()], ["W"], ["_packed"])
+            access = state.add_access(clean)
+            state.add_edge(filters, None, pack, "W", sdfg.make_array_memlet(filters.data))
+            state.add_edge(pack, "_packed", access, None, sdfg.make_array_memlet(clean))
+            state.add_edge(access, None, packed_call, "_packed", sdfg.make_array_memlet(clean))
+
+
+_PACKED = {"mi355x_gemm_f32": _packed_gemm, "mi355x_conv2d_f32": _packed_conv, "mi355x_conv2d_res_f32": _packed_conv}
+
+
 def pack_constant_operands(model):
-    """Give every GEMM of ``model``'s expanded graph that multiplies by a constant, and for which the library says that it pays, a
-    packed copy of it. Returns the copies."""
+    """Give every GEMM and convolution of ``model``'s expanded graph that multiplies by a constant, and for which the library says that
+    it pays, a packed copy of it. Returns the copies."""
     from ..onnx.onnx_importer import clean_onnx_name
-    sdfg, lib = model.sdfg, _lib.library()
+    sdfg = model.sdfg
     by_clean = {clean_onnx_name(k): k for k in model.weights}
     copies = []
     for state in sdfg.nodes():
         written = {e.dst.data for e in state.edges() if isinstance(e.dst, AccessNode)}
         for call in state.nodes():
-            if not isinstance(call, KernelCall) or call.function != "mi355x_gemm_f32":
+            if not isinstance(call, KernelCall) or call.function not in _PACKED:
                 continue
-            b = call.args[1]
-            edge = next(e for e in state.in_edges(call) if e.dst_conn == b.connector)
-            batch0, batch1, M, N, K, a_strides, b_strides = call.args[5:12]
-            sb0, sb1, sk, sn = b_strides.values
-            if edge.src.data not in by_clean or edge.src.data in written or sb0 or sb1 or min(sk, sn) < 1:
+            edge = next(e for e in state.in_edges(call) if e.dst_conn == call.args[1].connector)
+            if edge.src.data not in by_clean or edge.src.data in written:
                 continue
             weight_name = by_clean[edge.src.data]
-            if model.weights[weight_name].dtype != torch.float32 or a_strides.values[3] != 1 or a_strides.values[2] % 4 \
-                    or not lib.mi355x_gemm_packed_pays(batch0 * batch1, M, N, K, int(sk == 1)):
+            if model.weights[weight_name].dtype != torch.float32:
                 continue
-            name = f"{weight_name}_packed_{N}_{K}_{sn}_{sk}_{b.offset}"
+            packed = _PACKED[call.function](call, model.weights[weight_name])
+            if packed is None:
+                continue
+            (suffix, *copy), (function, args) = packed
+            name = f"{weight_name}_packed_{suffix}"
             clean = clean_onnx_name(name)
             if name not in model.weights:
-                copies.append(PackedOperand(model, weight_name, N, K, sn, sk, b.offset))
+                copies.append(PackedOperand(model, weight_name, *copy))
                 model.weights[name] = copies[-1].packed
                 sdfg.add_array(clean, list(copies[-1].packed.shape), int32, transient=False)
-            args = [call.args[0], Ptr("_packed")] + call.args[1:]
-            packed_call = KernelCall(call.label, "mi355x_gemm_packed_f32", args, list(call.in_connectors) + ["_packed"], list(call.out_connectors))
+            packed_call = KernelCall(call.label, function, args, list(call.in_connectors) + ["_packed"], list(call.out_connectors))
             state.replace_node(call, packed_call, sdfg)
             state.add_edge(state.add_access(clean), None, packed_call, "_packed", sdfg.make_array_memlet(clean))
     if copies:

@@ -146,6 +146,22 @@ int mi355x_conv2d_res_f32(const float* X, const float* W, const float* bias, con
                           const int64_t* pads, const int64_t* strides,
                           const int64_t* dilations, int epilogue, void* stream);
 
+/* Filters W [M, C, KH, KW] as the three bf16 parts that mi355x_conv2d_packed_f32 multiplies by, written once if they are constant.
+ * mi355x_conv2d_packed_pays: bytes of the packed copy where the kernel (with the packing, unless constant) is ahead of
+ * mi355x_conv2d_f32 for this layer, 0 elsewhere
+ * (filters that are neither 3 x 3 nor 1 x 1 over a multiple of eight channels, nor 7 x 7 over at most four, among them).
+ * `packed` is 16-byte aligned. */
+int64_t mi355x_conv2d_packed_pays(int64_t N, int64_t C, int64_t H, int64_t Wd, int64_t M, int64_t KH, int64_t KW,
+                                  const int64_t* pads, const int64_t* strides, const int64_t* dilations, int constant);
+int mi355x_pack_conv_f32(const float* w, void* packed, int64_t M, int64_t C, int64_t KH, int64_t KW, void* stream);
+
+/* mi355x_conv2d_res_f32 by W and its packed copy (residual may be NULL without MI355X_EPI_RESIDUAL). */
+int mi355x_conv2d_packed_f32(const float* X, const void* packed, const float* W, const float* bias, const float* residual,
+                             float* Y, int64_t N, int64_t C, int64_t H, int64_t Wd,
+                             int64_t M, int64_t KH, int64_t KW,
+                             const int64_t* pads, const int64_t* strides,
+                             const int64_t* dilations, int epilogue, void* stream);
+
 /* ONNX MaxPool, 2-D, fp32, NCHW: Y[n,c,oh,ow] = max over the KH x KW window at
  * (oh * strides[0] - pads[0] + kh * dilations[0], ow * strides[1] - pads[1] + kw * dilations[1]);
  * positions in the padding do not take part. pads = {top, left, bottom, right}, floor output size
