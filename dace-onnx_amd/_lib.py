@@ -75,6 +75,8 @@ SIGNATURES: typing.Dict[str, typing.Tuple[typing.Any, typing.List[typing.Any]]] 
     "mi355x_eltwise_program_f32": (_int, [ctypes.POINTER(ctypes.c_void_p), _int, ctypes.POINTER(ctypes.c_void_p), _int, _vp,
                                           _i64, _i64, ctypes.POINTER(ctypes.c_uint32), _int,
                                           ctypes.POINTER(ctypes.c_float), _int, _vp]),
+    "mi355x_program_function": (_int, [ctypes.c_char_p]),
+    "mi355x_program_run": (_i64, [_vp, _i64, _i64, _vp, _i64, _vp, _vp]),
 }
 
 

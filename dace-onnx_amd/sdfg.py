@@ -21,8 +21,11 @@ Execution never leaves the GPU: arrays live in HBM as torch tensors, numpy
 arguments are staged in and out, and there is no host implementation of any
 node; a library node that was not expanded to kernels cannot run.
 """
+import array
 import collections
+import ctypes
 import itertools
+import struct
 import typing
 
 import numpy as np
@@ -578,6 +581,49 @@ class SDFG:
 # --------------------------------------------------------------------------- executor
 
 
+class _Program:
+    """A launch list as the words ``mi355x_program_run`` takes: one call into the library issues all launches, with the addresses of a
+    call's buffers put in place there."""
+
+    def __init__(self, lib, launches, patches, external):
+        words, bodies, moved = [], [], []   # calls; contents of pointer arrays, behind them; (word, source, offset)
+        sources = {name: i for i, name in enumerate(external)}
+        self._names = [item[2] for item in launches]
+        self._keep = launches   # arrays that words point to
+        for item, (slots, arrays) in zip(launches, patches):
+            _, fn, name, args, stream_slots, _, _ = item
+            function = lib.mi355x_program_function(name.encode())
+            if function < 0 or stream_slots != [len(args) - 1]:
+                raise RuntimeError(f"{name} cannot be part of a program")
+            first = len(words) + 1
+            words.append(function)
+            for argument, kind in zip(args[:-1], fn.argtypes):
+                if argument is None:
+                    words.append(0)
+                elif isinstance(argument, ctypes.Array):
+                    words.append(ctypes.addressof(argument))
+                elif kind is ctypes.c_float:
+                    words.append(struct.unpack("<I", struct.pack("<f", argument))[0])
+                else:
+                    words.append(int(argument))
+            moved += [(first + i, sources[source], offset) for i, source, offset in slots]
+            for i, addresses, followed in arrays:
+                bodies.append((first + i, addresses, followed))
+        for word, addresses, followed in bodies:
+            moved.append((word, -1, len(words)))
+            moved += [(len(words) + i, sources[to[0]], to[1]) for i, to in enumerate(followed) if to is not None]
+            words += addresses or [0]   # (an empty array has an address too)
+        self._words, self._moved = array.array("q", words), array.array("q", [v for m in moved for v in m])
+        self._run = lib.mi355x_program_run
+        self._fixed = (self._words.buffer_info()[0], len(words), len(launches), self._moved.buffer_info()[0], len(moved))
+
+    def run(self, addresses, stream):
+        addresses = array.array("q", addresses)
+        result = self._run(*self._fixed, addresses.buffer_info()[0], stream)
+        if result:
+            _lib.check(result & 0xff, self._names[result >> 8])
+
+
 class CompiledSDFG:
     """Executable form of an expanded SDFG: a flat list of kernel launches.
 
@@ -605,6 +651,8 @@ class CompiledSDFG:
         self._plan = []         # ("call", node, connector -> key) | ("alias", src key, dst key, dst descriptor)
         self._bound_key = None
         self._patches = None    # per launch, the pointer arguments that follow the caller's arrays (see _rebind)
+        self._program = None    # the launch list as one native call (None: it holds device copies)
+        self._launches, self._listed_key = [], None
         self._graph = None
         self._build(sdfg, prefix="", outer_map={})
 
@@ -757,6 +805,14 @@ class CompiledSDFG:
             result.append((*item[:3], args, *item[4:]))
         return result
 
+    @property
+    def _launch_list(self):
+        """The launches for the buffers of the last call (those of the program, which replaces addresses itself, are brought up to date)."""
+        if self._listed_key != self._bound_key:
+            self._launches = self._rebind(self._launches, dict(zip(self._external, self._bound_key)))
+            self._listed_key = self._bound_key
+        return self._launches
+
     def _tensor(self, env, key):
         """The tensor bound to ``key``; a transient that has none yet gets its allocation, made once per
         compiled SDFG and reused by every later binding."""
@@ -826,15 +882,18 @@ class CompiledSDFG:
                 env[name] = d
         key = [env[n].data_ptr() for n in self._external]
         if key != self._bound_key:
-            if self._bound_key is None or self._patches is None:
-                self._launch_list, self._patches = self._bind(env)
-            else:
-                self._launch_list = self._rebind(self._launch_list, dict(zip(self._external, key)))
+            if self._program is None:
+                self._launches, self._patches = self._bind(env)
+                self._listed_key = key
+                if self._patches is not None:
+                    self._program = _Program(self._lib, self._launches, self._patches, self._external)
             self._env = env   # the caller's arrays live as long as the launch list points to them
             self._bound_key = key
             self._graph = None
-        launches = self._launch_list
-        self._run(launches)
+        if self._program is None:
+            self._run(self._launches)
+        else:
+            self._program.run(key, torch.cuda.current_stream(self.device).cuda_stream)
         for host, dev in staged_back:
             if isinstance(host, np.ndarray):
                 host[...] = dev.cpu().numpy()

@@ -162,6 +162,15 @@ int mi355x_conv2d_packed_f32(const float* X, const void* packed, const float* W,
                              const int64_t* pads, const int64_t* strides,
                              const int64_t* dilations, int epilogue, void* stream);
 
+/* Several launches in one call. `program` holds `calls` calls one after the other, each the number of its function
+ * (mi355x_program_function of its name, -1 if it cannot be one) and its arguments but the stream in 64-bit words (a float in the
+ * low half), and anything behind them. On a copy of it, every patch {word, source, offset} puts addresses[source] + offset, or for
+ * source = -1 the address of word `offset` of the copy, in its place; then the calls are issued on `stream`. The first that fails
+ * ends the program: the result is its index << 8 | its status, otherwise MI355X_OK. */
+int mi355x_program_function(const char* name);
+int64_t mi355x_program_run(const int64_t* program, int64_t words, int64_t calls, const int64_t* patches, int64_t num_patches,
+                           const int64_t* addresses, void* stream);
+
 /* ONNX MaxPool, 2-D, fp32, NCHW: Y[n,c,oh,ow] = max over the KH x KW window at
  * (oh * strides[0] - pads[0] + kh * dilations[0], ow * strides[1] - pads[1] + kw * dilations[1]);
  * positions in the padding do not take part. pads = {top, left, bottom, right}, floor output size
