@@ -23,6 +23,9 @@
 //     and a lane ends up with four consecutive output columns of a row: 16-byte stores.
 #include "common.h"
 #include "gemm_tile.h"
+#include "split_bf16.h"
+
+#include <algorithm>
 
 namespace mi355x {
 
@@ -32,8 +35,8 @@ struct AttnArgs {
     const float* Q; const float* K; const float* V; float* O;
     int64_t batch1, Sq, Sk, q_blocks, nwg;
     int64_t q_sb0, q_sb1, q_sr, k_sb0, k_sb1, k_sr, v_sb0, v_sb1, v_sr, o_sb0, o_sb1, o_sr;
-    float scale;
     const float* mask; int64_t m_sb0, m_sb1, m_sr;   // masked form: added to scale * Q K^T, keys contiguous, 0 strides broadcast
+    float scale;   // (last: next to the mask's address the compiler keeps both in a local array and reads the mask through it)
 };
 
 __device__ __forceinline__ float quad_lanes_max(float v) {  // over lanes li, li+16, li+32, li+48
@@ -183,17 +186,11 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(AttnArgs p) {
 // The nodes one at a time (two products, the addition, the softmax) take 259 us on 16 x 12 slices of 512 x 512 scores, this 135.
 // 128 keys go through here too: 8 x 12 slices 10.0 us, the one-pass kernel above without a mask 8.5, the nodes 22.5.
 template <bool MASKED>
-__global__ __launch_bounds__(256) void attention_f32_blocks_kernel(AttnArgs p) {
+__device__ __forceinline__ void attention_blocks(const AttnArgs& p, int64_t slice, int64_t qb, float* lds_k, float* lds_v) {
     constexpr int SK = AT_SK, D = AT_D, PITCH = AT_PITCH, NJ = SK / 16, NC = D / 16, SETS = MASKED ? 2 : 1;
-    __shared__ __attribute__((aligned(16))) float lds_k[SK * PITCH];
-    __shared__ __attribute__((aligned(16))) float lds_v[SK * PITCH];
-
     const int tid = threadIdx.x;
     const int lane = tid % WAVE, wave = tid / WAVE;
     const int li = lane % 16, lq = lane / 16;
-
-    const int64_t logical = xcd_remap(blockIdx.x, p.nwg);
-    const int64_t slice = logical / p.q_blocks, qb = logical % p.q_blocks;
     const int64_t b0 = slice / p.batch1, b1 = slice % p.batch1;
     const float* __restrict__ Q = p.Q + b0 * p.q_sb0 + b1 * p.q_sb1;
     const float* __restrict__ K = p.K + b0 * p.k_sb0 + b1 * p.k_sb1;
@@ -269,12 +266,10 @@ __global__ __launch_bounds__(256) void attention_f32_blocks_kernel(AttnArgs p) {
             const int64_t key = key0 + 16 * j + 4 * lq;
             acc[j] *= c;
             if constexpr (MASKED) {
-                f32x4 add;
-                if (!ragged) __builtin_memcpy(&add, mask + key, sizeof add);
-                else
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) add[r] = mask[key + r < p.Sk ? key + r : p.Sk - 1];
-                acc[j] += add;
+                typedef f32x4 unaligned __attribute__((aligned(4)));
+                auto at = [&](int64_t k) { return mask[k < p.Sk ? k : p.Sk - 1]; };
+                if (!ragged) acc[j] += *reinterpret_cast<const unaligned*>(mask + key);
+                else acc[j] += f32x4{at(key), at(key + 1), at(key + 2), at(key + 3)};
             }
             if (ragged) {
 #pragma unroll
@@ -341,9 +336,247 @@ __global__ __launch_bounds__(256) void attention_f32_blocks_kernel(AttnArgs p) {
     }
 }
 
-}  // namespace mi355x
+template <bool MASKED>
+__global__ __launch_bounds__(256) void attention_f32_blocks_kernel(AttnArgs p) {
+    __shared__ __attribute__((aligned(16))) float lds_k[AT_SK * AT_PITCH];
+    __shared__ __attribute__((aligned(16))) float lds_v[AT_SK * AT_PITCH];
+    const int64_t logical = xcd_remap(blockIdx.x, p.nwg);
+    attention_blocks<MASKED>(p, logical / p.q_blocks, logical % p.q_blocks, lds_k, lds_v);
+}
 
-namespace mi355x {
+// Many rows: both products on the bf16 matrix unit, every value split in three (split_bf16.h; the six products in two sets of accumulators,
+// the second product block by block). A workgroup of four waves owns 128 query rows, 32 of them each, and walks the keys in blocks of 64:
+//   * S^T = K Q^T, Q split once into registers, K on its way into LDS in fragment order. A lane then holds half of a query's scores of the
+//     block, the lane 32 further on the other half: the maximum and the sum are register operations and one exchange.
+//   * O^T = V^T P^T takes the probabilities from the registers that they are in, split there; V is read a column per lane, so that the
+//     eight keys of a unit, in the order in which the scores lie, become one LDS write.
+//   * Query rows are the columns of O^T: their factors exp(old maximum - new maximum) are the lane's own.
+// Sums that are not finite (infinities, NaN, values past 2^112) send the workgroup through the fp32 kernel above.
+// What bounds it: a wave's chain of 6 us a block, half of it MFMAs and half splits and exponentials on the vector unit, which the waves of two
+// workgroups on a CU overlap to 3.4; 254 registers leave no room for a third. Against the kernels above, with a mask: 16 x 12 slices of
+// 512 x 512 135 -> 87 us, 32 x 12 of 256 73 -> 48, 20 x 12 of 200 50 -> 31, 32 x 12 of 64 15.1 -> 10.4; without: 121 -> 87, 65 -> 48, 44 -> 30,
+// 13.4 -> 10.0. 2-norm of the error against float64 5.9e-7 -> 4.0e-7 and 1.1e-6 -> 4.2e-7. Where a CU gets one workgroup or none its chain is the
+// longer one: 1 x 12 of 512 28.7 with the kernel above, 33.8 here.
+constexpr int AS_KEYS = 64, AS_ROWS = 128;
+
+template <bool MASKED>
+__global__ __launch_bounds__(256, 2) void attention_split_kernel(AttnArgs p) {
+    constexpr int D = AT_D, K_BYTES = AS_KEYS / 32 * (D / 16) * PK_FRAGMENT, BLOCKS_LDS = 2 * AT_SK * AT_PITCH * 4;
+    static_assert(2 * K_BYTES <= BLOCKS_LDS, "the fp32 form takes more");
+    __shared__ __attribute__((aligned(16))) char lds[BLOCKS_LDS];
+    char* const lds_k = lds;             // [32 keys][16 of D][part][lane]
+    char* const lds_v = lds + K_BYTES;   // [32 of D][16 keys][part][lane]
+
+    const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int li = lane % 32, lh = lane / 32;
+    const int64_t logical = xcd_remap(blockIdx.x, p.nwg);
+    const int64_t slice = logical / p.q_blocks, qb = logical % p.q_blocks;
+    const int64_t b0 = slice / p.batch1, b1 = slice % p.batch1;
+    // (a slice of K, of V and of the mask spans less than 2^31 bytes: launch precondition)
+    const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.K + b0 * p.k_sb0 + b1 * p.k_sb1), 0, 0x7fffffff, 0x00020000);
+    const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.V + b0 * p.v_sb0 + b1 * p.v_sb1), 0, 0x7fffffff, 0x00020000);
+    const int keys = (int)p.Sk, k_row = (int)p.k_sr * 4, v_row = (int)p.v_sr * 4;
+    const int64_t row = qb * AS_ROWS + 32 * wave + li, qrow = row < p.Sq ? row : p.Sq - 1;
+    const __amdgpu_buffer_rsrc_t m_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(MASKED ? p.mask + b0 * p.m_sb0 + b1 * p.m_sb1 : p.K), 0, 0x7fffffff, 0x00020000);
+    const int m_row = (int)(qrow * p.m_sr) * 4;
+
+    auto fragments = [](f32x4 a, f32x4 b, bf16x8 (&f)[SP_PLANES]) __attribute__((always_inline)) {
+        u32x4 part[SP_PLANES];
+        split_unit8(a, b, part);
+#pragma unroll
+        for (int q = 0; q < SP_PLANES; ++q) f[q] = __builtin_bit_cast(bf16x8, part[q]);
+    };
+    bf16x8 fq[D / 16][SP_PLANES];
+    {
+        const float* Q = p.Q + b0 * p.q_sb0 + b1 * p.q_sb1 + qrow * p.q_sr + 8 * lh;
+#pragma unroll
+        for (int c = 0; c < D / 16; ++c) fragments(*reinterpret_cast<const f32x4*>(Q + 16 * c), *reinterpret_cast<const f32x4*>(Q + 16 * c + 4), fq[c]);
+    }
+    f32x16 out[2];   // O^T: columns 32 db + 8 (r / 4) + 4 lh + r % 4 of query row li, times 2^32, not yet divided by the sum
+#pragma unroll
+    for (int db = 0; db < 2; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) out[db][r] = 0.f;
+    float m_run = -INFINITY, l_run = 0.f;
+    const float scale = p.scale * SP_UNSCALE;
+    constexpr float LOG2E = 1.44269504088896340736f;
+
+    f32x4 rk[2][2], rv[2][2];
+    auto load = [&](int key0) {   // keys beyond the last are the last one
+#pragma unroll
+        for (int it = 0; it < 2; ++it) {
+            const int idx = tid + it * 256, key = min(key0 + idx / 8, keys - 1);
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                rk[it][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(k_rsrc, key * k_row + 32 * (idx % 8) + 16 * h, 0, 0));
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {   // a wave's rows: keys 4 lh .. 4 lh + 3 and 8 further on, of the 16 of a step
+                const int at = min(key0 + 16 * (2 * it + wave / 2) + 8 * (e / 4) + 4 * (wave % 2) + e % 4, keys - 1);
+                rv[it][e / 4][e % 4] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(v_rsrc, 4 * lane, at * v_row, 0));
+            }
+        }
+    };
+    load(0);
+    for (int key0 = 0; key0 < keys; key0 += AS_KEYS) {
+        const bool ragged = key0 + AS_KEYS > keys;   // uniform
+        f32x4 add[2][4];   // the mask's values of the scores below
+        if constexpr (MASKED) {
+            if (!ragged) {
+#pragma unroll
+                for (int g = 0; g < 8; ++g)
+                    add[g / 4][g % 4] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(m_rsrc, m_row + 4 * (key0 + 8 * g + 4 * lh), 0, 0));
+            } else {
+                auto at = [&](int key) {
+                    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(m_rsrc, m_row + 4 * min(key, keys - 1), 0, 0));
+                };
+#pragma unroll
+                for (int g = 0; g < 8; ++g) {
+                    const int key = key0 + 8 * g + 4 * lh;
+                    add[g / 4][g % 4] = f32x4{at(key), at(key + 1), at(key + 2), at(key + 3)};
+                }
+            }
+        }
+        if (key0 > 0) __syncthreads();   // everyone has read the block before
+#pragma unroll
+        for (int it = 0; it < 2; ++it) {
+            const int idx = tid + it * 256;
+            u32x4 part[SP_PLANES];
+            split_unit8(rk[it][0], rk[it][1], part);
+            const int key = idx / 8, u = idx % 8;   // (rows xor-ed with 4 u: the eight units of a row go to different banks)
+#pragma unroll
+            for (int q = 0; q < SP_PLANES; ++q)
+                *reinterpret_cast<u32x4*>(lds_k + ((key / 32 * (D / 16) + u / 2) * SP_PLANES + q) * PK_PLANE + (u % 2 * 32 + ((key % 32) ^ (4 * u))) * 16) = part[q];
+            split_unit8(rv[it][0], rv[it][1], part);
+            const int step = idx / 128, half = idx / 64 % 2, d = idx % 64;
+#pragma unroll
+            for (int q = 0; q < SP_PLANES; ++q)
+                *reinterpret_cast<u32x4*>(lds_v + ((d / 32 * (AS_KEYS / 16) + step) * SP_PLANES + q) * PK_PLANE + (half * 32 + d % 32) * 16) = part[q];
+        }
+        __syncthreads();
+
+        // ---- the scores of this block: s[kb][r] of key 32 kb + 8 (r / 4) + 4 lh + r % 4
+        f32x16 s[2];
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            f32x16 sum, small;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sum[r] = small[r] = 0.f;
+#pragma unroll
+            for (int c = 0; c < D / 16; ++c) {
+                bf16x8 fk[SP_PLANES];
+#pragma unroll
+                for (int q = 0; q < SP_PLANES; ++q)
+                    fk[q] = *reinterpret_cast<const bf16x8*>(lds_k + ((kb * (D / 16) + c) * SP_PLANES + q) * PK_PLANE + (lh * 32 + (li ^ (4 * (2 * c + lh)))) * 16);
+#pragma unroll
+                for (int u = 0; u < PK_PRODUCTS; ++u) {
+                    f32x16& to = u == 0 ? sum : small;
+                    to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fk[PK_QA[u]], fq[c][PK_QB[u]], to, 0, 0, 0);
+                }
+            }
+            s[kb] = sum + small;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        load(key0 + AS_KEYS);   // in flight under the rest of the block
+        __builtin_amdgcn_sched_barrier(0);
+        float m_blk = -INFINITY;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                if constexpr (MASKED) s[kb][r] = fmaf(s[kb][r], scale, add[kb][r / 4][r % 4]);
+                else s[kb][r] *= scale;
+            }
+        if (ragged)
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (key0 + 32 * kb + 8 * (r / 4) + 4 * lh + r % 4 >= keys) s[kb][r] = -INFINITY;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) m_blk = fmaxf(m_blk, s[kb][r]);
+        const float m_new = fmaxf(m_run, fmaxf(m_blk, __shfl_xor(m_blk, 32, WAVE)));
+        const float m_ref = m_new == -INFINITY ? 0.f : m_new;   // nothing but -inf so far: 2^(-inf - 0) = 0
+        auto power = [&](float v) { return __builtin_amdgcn_exp2f((v - m_ref) * LOG2E); };
+        const float alpha = power(m_run);   // 0 for the first block
+        float part_sum[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                s[kb][r] = power(s[kb][r]);
+                part_sum[r % 4] += s[kb][r];
+            }
+        const float half_sum = (part_sum[0] + part_sum[1]) + (part_sum[2] + part_sum[3]);
+        l_run = l_run * alpha + (half_sum + __shfl_xor(half_sum, 32, WAVE));
+        m_run = m_new;
+
+        // ---- out = alpha out + V^T P^T
+        bf16x8 fp[AS_KEYS / 16][SP_PLANES];
+#pragma unroll
+        for (int step = 0; step < AS_KEYS / 16; ++step) {
+            f32x4 v[2];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e / 4][e % 4] = s[step / 2][8 * (step % 2) + e];
+            fragments(v[0], v[1], fp[step]);
+        }
+#pragma unroll
+        for (int db = 0; db < 2; ++db) {
+            f32x16 sum, small;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sum[r] = small[r] = 0.f;
+#pragma unroll
+            for (int step = 0; step < AS_KEYS / 16; ++step) {
+                bf16x8 fv[SP_PLANES];
+#pragma unroll
+                for (int q = 0; q < SP_PLANES; ++q)
+                    fv[q] = *reinterpret_cast<const bf16x8*>(lds_v + ((db * (AS_KEYS / 16) + step) * SP_PLANES + q) * PK_PLANE + lane * 16);
+#pragma unroll
+                for (int u = 0; u < PK_PRODUCTS; ++u) {
+                    f32x16& to = u == 0 ? sum : small;
+                    to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fv[PK_QA[u]], fp[step][PK_QB[u]], to, 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) out[db][r] = fmaf(out[db][r], alpha, sum[r] + small[r]);
+        }
+    }
+    // A score that is NaN or positive infinity makes the probabilities NaN and the sums with them; with all of them negative infinity the
+    // probabilities sum to 0.
+    float probe = 0.f;   // stays 0 while all sums are finite
+#pragma unroll
+    for (int db = 0; db < 2; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) probe = fmaf(out[db][r], 0.f, probe);
+    if (__syncthreads_or(probe != 0.f || !(l_run > 0.f))) {   // (NaN compares unequal)
+        for (int half = 0; half < AS_ROWS / AT_BQ; ++half) {
+            __syncthreads();
+            attention_blocks<MASKED>(p, slice, qb * (AS_ROWS / AT_BQ) + half, reinterpret_cast<float*>(lds), reinterpret_cast<float*>(lds) + AT_SK * AT_PITCH);
+        }
+        return;
+    }
+    if (row >= p.Sq) return;
+    const float inv = SP_UNSCALE / l_run;
+    float* O = p.O + b0 * p.o_sb0 + b1 * p.o_sb1 + row * p.o_sr + 4 * lh;
+#pragma unroll
+    for (int db = 0; db < 2; ++db)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<f32x4*>(O + 32 * db + 8 * g) =
+                f32x4{out[db][4 * g] * inv, out[db][4 * g + 1] * inv, out[db][4 * g + 2] * inv, out[db][4 * g + 3] * inv};
+}
+
+// Whether the split form is ahead. Nanoseconds of a workgroup with a CU to itself and of each further one on it, by blocks of keys: fitted over
+// 26 shapes of 12 to 512 slices, 33 to 512 keys, both forms measured on each; the form not taken is at most 4 % faster in these.
+static bool split_pays(int64_t slices, int64_t Sq, int64_t Sk, bool masked) {
+    const int cus = device_cus();
+    auto cost = [&](int64_t rows, int64_t keys, double fixed, double block, double again, double again_block) {
+        const double blocks = (double)ceil_div(Sk, keys), more = (double)(ceil_div(slices * ceil_div(Sq, rows), (int64_t)std::max(cus, 1)) - 1);
+        return fixed + blocks * block + more * (again + blocks * again_block);
+    };
+    return cost(AS_ROWS, AS_KEYS, 3400, 3800, 1500, 3000) < (masked ? 0.95 : 0.95 * 0.88) * cost(AT_BQ, AT_SK, 2400, 6600, 2000, 4900);
+}
 
 // mask == nullptr: the unmasked product
 static int launch_attention(const float* Q, const float* K, const float* V, float* O, const float* mask, int64_t batch0,
@@ -373,6 +606,15 @@ static int launch_attention(const float* Q, const float* K, const float* V, floa
     p.scale = scale;
     p.mask = mask;
     p.m_sb0 = mask ? mask_strides[0] : 0; p.m_sb1 = mask ? mask_strides[1] : 0; p.m_sr = mask ? mask_strides[2] : 0;
+    const int64_t split_blocks = ceil_div(Sq, (int64_t)AS_ROWS), split_nwg = batch0 * batch1 * split_blocks;
+    const int split = tuning().attn_split;
+    if (split != 0 && grid_fits(split_nwg, 256) && Sk < (1 << 24) && Sk * k_strides[2] < (1 << 29) && Sk * v_strides[2] < (1 << 29) && (!mask || (mask_strides[2] >= 0 && Sq * mask_strides[2] + Sk < (1 << 29))) && (split > 0 || (tuning().attn_waves == 0 && split_pays(batch0 * batch1, Sq, Sk, mask != nullptr)))) {
+        p.q_blocks = split_blocks;
+        p.nwg = split_nwg;
+        if (mask) hipLaunchKernelGGL(attention_split_kernel<true>, dim3((unsigned)p.nwg), dim3(256), 0, static_cast<hipStream_t>(stream), p);
+        else hipLaunchKernelGGL(attention_split_kernel<false>, dim3((unsigned)p.nwg), dim3(256), 0, static_cast<hipStream_t>(stream), p);
+        return check_launch("attention_split_kernel");
+    }
     if (mask) {
         hipLaunchKernelGGL(attention_f32_blocks_kernel<true>, dim3((unsigned)p.nwg), dim3(256), 0, static_cast<hipStream_t>(stream), p);
         return check_launch("attention_f32_blocks_kernel");

@@ -1,0 +1,82 @@
+"""Attention on the bf16 matrix unit, at the edges of its blocks and values: against float64, and against the fp32 kernel where sums are not finite."""
+import pytest
+import torch
+
+from dace_onnx_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+def attention(q, k, v, mask=None, scale=0.125):
+    (b0, b1, sq, _), sk = q.shape, k.shape[2]
+    rows = sq + 1
+    out = torch.full((b0, b1, rows, 64), -7.0, device="cuda")   # one row more than is written
+    strides = lambda t: _lib.i64_array([t.stride(0), t.stride(1), t.stride(2)])   # noqa: E731
+    args = [q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()]
+    geometry = [b0, b1, sq, sk, 64, strides(q), strides(k), strides(v), strides(out)]
+    if mask is None:
+        name, args = "mi355x_attention_f32", args + geometry
+    else:
+        broadcast = _lib.i64_array([st if e > 1 else 0 for st, e in zip(mask.stride()[:3], mask.shape)])
+        name, args = "mi355x_attention_masked_f32", args + [mask.data_ptr()] + geometry + [broadcast]
+    _lib.check(getattr(_lib.library(), name)(*args, scale, torch.cuda.current_stream().cuda_stream), name)
+    assert bool((out[:, :, sq:] == -7).all())
+    return out[:, :, :sq]
+
+
+def inputs(b0, b1, sq, sk, seed=0):
+    torch.manual_seed(sq + sk + seed)
+    return [torch.randn(b0, n, b1, 64, device="cuda").transpose(1, 2) for n in (sq, sk, sk)]   # heads side by side in a row
+
+
+@pytest.mark.parametrize("sq, sk", [(1, 1), (127, 63), (128, 64), (129, 65), (33, 130), (257, 200)])
+@pytest.mark.parametrize("shape", [None, "keys", "rows", "all"])
+def test_split_attention(tuning, sq, sk, shape):
+    """Scores of up to 8 in magnitude: 2^-24 of that, a few times, in the exponent of every probability; sums of up to 200 of them."""
+    tuning(MI355X_ATTN_SPLIT=1)
+    b0, b1 = 2, 3
+    q, k, v = inputs(b0, b1, sq, sk)
+    extents = {"keys": (b0, 1, 1, sk), "rows": (1, 1, sq, sk), "all": (b0, b1, sq, sk)}.get(shape)
+    mask = None
+    if extents:
+        memory = torch.where(torch.rand(b0 * b1 * sq * sk + 1, device="cuda") < 0.3, -10000.0, 0.0)[1:]   # (not 16-byte aligned)
+        mask = memory[:extents[0] * extents[1] * extents[2] * sk].view(extents)
+        mask[..., sk // 2] = 0
+    scores = 0.125 * (q.double() @ k.double().transpose(-1, -2).contiguous())
+    expected = torch.softmax(scores + mask.double() if extents else scores, -1) @ v.double()
+    got = attention(q, k, v, mask)
+    assert bool(((expected - got.double()).abs() <= 2.0**-19 * v.abs().max()).all())
+    assert float((expected - got.double()).norm() / expected.norm()) < 1e-6
+
+
+@pytest.mark.parametrize("fill", [-float("inf"), torch.finfo(torch.float32).min, -10000.0])
+@pytest.mark.parametrize("sk", [64, 150])
+def test_split_attention_over_masked_blocks_and_rows(tuning, sk, fill):
+    """A first block without a valid key and a row without one: as the fp32 kernel, NaN in the same places."""
+    q, k, v = inputs(2, 3, 70, sk)
+    mask = torch.zeros(2, 1, 70, sk, device="cuda")
+    mask[0, :, :40, :sk - 3], mask[1, :, 5] = fill, fill
+    results = []
+    for form in (0, 1):
+        tuning(MI355X_ATTN_SPLIT=form)
+        results.append(attention(q, k, v, mask))
+    assert torch.equal(torch.isnan(results[0]), torch.isnan(results[1])) and bool(torch.isnan(results[0]).any()) == (fill == -float("inf"))
+    masked_row = torch.zeros(2, 1, 70, 1, dtype=torch.bool, device="cuda")
+    masked_row[1, :, 5] = fill == -10000.0   # the scores there have lost all but 2^-11
+    difference = (results[0] - results[1]).abs().nan_to_num(0)
+    assert float(difference.masked_fill(masked_row, 0).max()) < 1e-5 and float(difference.max()) < 5e-3
+
+
+@pytest.mark.parametrize("masked", [False, True])
+def test_split_attention_keeps_infinities_nan_and_the_largest_values(tuning, masked):
+    mask = torch.zeros(1, 1, 1, 100, device="cuda") if masked else None
+    for place, value in ((0, float("inf")), (0, float("nan")), (1, -float("inf")), (1, float("nan")), (2, float("inf")), (2, float("nan")), (2, 3.0e38), (0, 1.0e36)):
+        tensors = inputs(2, 2, 150, 100, seed=place)
+        tensors[place][1, 0, 70, 9] = value
+        results = []
+        for form in (0, 1):
+            tuning(MI355X_ATTN_SPLIT=form)
+            results.append(attention(*tensors, mask))
+        assert torch.equal(torch.isnan(results[0]), torch.isnan(results[1])) and torch.equal(torch.isinf(results[0]), torch.isinf(results[1]))
+        fine = torch.isfinite(results[0])
+        assert bool(((results[0] - results[1]).abs()[fine] <= 1e-5 * results[0].abs()[fine].clamp(min=1)).all())
