@@ -49,11 +49,12 @@ def exact_conv(x, w, pads=(0, 0, 0, 0), strides=(1, 1), dilations=(1, 1)):
 
 
 # N, C, H, W, M, kernel, pads, strides, dilations, epilogue: one position; images that end inside a tile; odd extents and half a group of
-# channels; a stride and a dilation per axis; strips (48 and 64 columns); the residual block's end; few channels
+# channels; a stride and a dilation per axis; strips (48 and 64 columns) and none (47: patches of up to
+# 150 KB of LDS); the residual block's end; few channels
 LAYERS = [(1, 8, 3, 3, 1, 3, (0, 0, 0, 0), (1, 1), (1, 1), 0), (5, 16, 7, 7, 33, 3, (1, 1, 1, 1), (1, 1), (1, 1), 25),
           (2, 40, 13, 11, 70, 3, (1, 0, 2, 1), (1, 1), (1, 1), 3), (3, 24, 19, 17, 64, 3, (2, 1, 0, 3), (2, 1), (1, 2), 1),
           (2, 48, 9, 48, 96, 3, (1, 1, 1, 1), (1, 1), (1, 1), 9), (1, 136, 30, 64, 40, 3, (1, 1, 1, 1), (1, 1), (1, 1), 1),
-          (1, 64, 15, 17, 130, 3, (1, 1, 1, 1), (2, 2), (1, 1), 0), (2, 8, 5, 6, 31, 1, (0, 0, 0, 0), (1, 1), (1, 1), 1),
+          (1, 128, 9, 47, 33, 3, (1, 1, 1, 1), (1, 1), (1, 1), 1), (1, 64, 15, 17, 130, 3, (1, 1, 1, 1), (2, 2), (1, 1), 0), (2, 8, 5, 6, 31, 1, (0, 0, 0, 0), (1, 1), (1, 1), 1),
           (3, 72, 14, 15, 65, 1, (0, 1, 1, 0), (2, 3), (1, 1), 25), (1, 320, 20, 33, 128, 1, (0, 0, 0, 0), (1, 1), (1, 1), 3),
           (2, 3, 40, 33, 33, 7, (3, 3, 3, 3), (2, 2), (1, 1), 3), (1, 4, 21, 64, 70, 7, (0, 2, 5, 1), (1, 1), (1, 1), 9), (3, 1, 9, 8, 5, 7, (3, 3, 3, 3), (1, 2), (1, 1), 0),
           (4, 2, 17, 48, 31, 7, (0, 1, 1, 0), (1, 1), (1, 1), 25)]
