@@ -11,6 +11,11 @@ from .. import _lib
 from ..sdfg import AccessNode, KernelCall, Ptr, Stream, int32
 
 
+def _version(tensor):
+    """How often ``tensor`` was written in place, as far as torch counts it; tensors made under ``torch.inference_mode`` have no such count."""
+    return None if tensor.is_inference() else tensor._version
+
+
 class PackedOperand:
     """A packed copy of a weight, ``shape`` 32-bit words, written by the library's ``function`` from ``offset`` values on."""
 
@@ -22,14 +27,14 @@ class PackedOperand:
 
     def pack(self):
         self.weight = self.model.weights[self.weight_name]
-        self.version = self.weight._version
+        self.version = _version(self.weight)
         start = self.weight.data_ptr() + 4 * self.offset
         _lib.check(getattr(_lib.library(), self.function)(start, self.packed.data_ptr(), *self.geometry, _lib.current_stream()), self.function)
 
     def refresh(self):
         """Pack again if the weight was replaced or written in place since (a wrapped module whose parameters were updated)."""
         weight = self.model.weights[self.weight_name]
-        if weight is not self.weight or weight._version != self.version:
+        if weight is not self.weight or _version(weight) != self.version:
             self.pack()
 
 
