@@ -210,7 +210,8 @@ class ONNXModel:
         self._compiled = None
         self._packed = []   # packed copies of constant operands (transformation/packing.py)
         self._expanded = False
-        self._static_io = None
+        self._static_io = None         # use_hip_graph: inputs, outputs and weights that the recording is bound to
+        self._recorded_packed = None   # and which packed copies it uses
 
     # -- construction helpers ----------------------------------------------------------
     @staticmethod
@@ -363,6 +364,12 @@ class ONNXModel:
             self._compiled = self.sdfg.compile()
         return self._compiled
 
+    def _weight_args(self, weights, packed):
+        """``weights`` (by array name) as arguments of the compiled graph, each packed copy among them if ``packed`` says so, left out if not."""
+        for c, use in zip(self._packed, packed):
+            weights[c.array] = c.packed if use else None
+        return weights
+
     def _call_args(self, args, kwargs):
         if len(args) > len(self.inputs):
             raise TypeError(f"expected at most {len(self.inputs)} positional arguments, got {len(args)}")
@@ -387,8 +394,6 @@ class ONNXModel:
                  input was a torch tensor, numpy arrays otherwise.
         """
         compiled = self.compile_and_init()
-        for copy_of_weight in self._packed:
-            copy_of_weight.refresh()
         inputs = self._call_args(args, kwargs)
         use_torch = any(isinstance(v, torch.Tensor) for v in inputs.values())
         call = {}
@@ -402,6 +407,7 @@ class ONNXModel:
                 v = torch.from_numpy(np.ascontiguousarray(np.asarray(v, dtype=desc.dtype.np_dtype))).to(self.device)
             call[clean_onnx_name(n)] = v
         outputs = collections.OrderedDict()
+        packed = [c.current() for c in self._packed]
         if self.use_hip_graph:
             if self._static_io is None:
                 # private input/output buffers: the graph is bound to their addresses
@@ -410,13 +416,18 @@ class ONNXModel:
                 for n in self.outputs:
                     desc = self.sdfg.arrays[clean_onnx_name(n)]
                     s_out[clean_onnx_name(n)] = torch.empty(desc.shape, dtype=desc.dtype.as_torch(), device=self.device)
-                compiled(**s_in, **s_out, **self.clean_weights)  # eager run, binds the launch list
-                compiled.capture_graph()
-                self._static_io = (s_in, s_out)
+                self._static_io = (s_in, s_out, self.clean_weights)
             else:
-                s_in, s_out = self._static_io
+                s_in, s_out, _ = self._static_io
                 for k, v in call.items():
                     s_in[k].copy_(v)
+            if packed != self._recorded_packed:
+                # an eager run, which binds the launch list, for the recording. Weights are the tensors of the first call, written or
+                # not: a launch reads a weight that was written, or replaced, itself from here on.
+                compiled(**s_in, **s_out, **self._weight_args(self._static_io[2], packed))
+                compiled.capture_graph()
+                self._recorded_packed = packed
+            else:
                 compiled.replay()
             outputs = collections.OrderedDict((n, s_out[clean_onnx_name(n)].clone()) for n in self.outputs)
         else:
@@ -429,7 +440,7 @@ class ONNXModel:
                     desc = self.sdfg.arrays[k]
                     out_kwargs[k] = self.save_transients[k] = torch.empty(desc.shape, dtype=desc.dtype.as_torch(),
                                                                           device=self.device)
-            compiled(**call, **out_kwargs, **self.clean_weights)
+            compiled(**call, **out_kwargs, **self._weight_args(self.clean_weights, packed))
         results = [t if use_torch else t.cpu().numpy() for t in outputs.values()]
         return results[0] if len(results) == 1 else tuple(results)
 

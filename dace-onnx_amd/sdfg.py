@@ -152,6 +152,11 @@ class Scalar(Array):
         super().__init__(dtype, (), None, transient, storage)
 
 
+class PackedCopy(Array):
+    """Another argument in a kernel's own layout. A caller may leave it out (``None``): the launch gets a null pointer for it and reads
+    that argument itself."""
+
+
 class Memlet:
     """Data movement annotation. Only whole-array memlets occur on the ONNX path."""
 
@@ -645,6 +650,7 @@ class CompiledSDFG:
         self._external = [k for k, d in sdfg.arrays.items() if not d.transient]
         self._torch_types = {k: sdfg.arrays[k].dtype.as_torch() for k in self._external}
         self._returned = [k for k in self._external if k.startswith("__return")]
+        self._optional = {k for k in self._external if isinstance(sdfg.arrays[k], PackedCopy)}
         self._written = self._find_written(sdfg)
         self._transients = {}   # flattened key -> descriptor
         self._transient_tensors = {}   # flattened key -> its allocation (made on first use, kept)
@@ -764,6 +770,10 @@ class CompiledSDFG:
                         args.append(None)
                     else:
                         t = self._tensor(env, conn_to_key[a.connector])
+                        if t is None:   # a packed copy that was left out
+                            args.append(None)
+                            slots.append((i, conn_to_key[a.connector], 0))
+                            continue
                         args.append(t.data_ptr() + a.offset * t.element_size())
                         followed = follow(a.connector, args[-1])
                         if followed:
@@ -852,6 +862,9 @@ class CompiledSDFG:
             if isinstance(v, torch.Tensor) and v.dtype is self._torch_types[name] and v.shape == desc.shape and v.is_cuda and v.is_contiguous():
                 env[name] = v
                 continue
+            if v is None and name in self._optional:
+                env[name] = None
+                continue
             if name not in kwargs:
                 if name == "__return" or name.startswith("__return"):
                     env[name] = torch.empty(desc.shape, dtype=desc.dtype.as_torch(), device=self.device)
@@ -880,7 +893,7 @@ class CompiledSDFG:
                 if name in self._written and isinstance(v, np.ndarray):
                     staged_back.append((v, d))
                 env[name] = d
-        key = [env[n].data_ptr() for n in self._external]
+        key = [0 if t is None else t.data_ptr() for t in env.values()]
         if key != self._bound_key:
             if self._program is None:
                 self._launches, self._patches = self._bind(env)

@@ -8,7 +8,7 @@ library as they are.
 import torch
 
 from .. import _lib
-from ..sdfg import AccessNode, KernelCall, Ptr, Stream, int32
+from ..sdfg import AccessNode, KernelCall, PackedCopy, Ptr, Stream, int32
 
 
 def _version(tensor):
@@ -17,25 +17,23 @@ def _version(tensor):
 
 
 class PackedOperand:
-    """A packed copy of a weight, ``shape`` 32-bit words, written by the library's ``function`` from ``offset`` values on."""
+    """The packed copy ``array`` of a weight, ``shape`` 32-bit words, written by the library's ``function`` from ``offset`` values on.
 
-    def __init__(self, model, weight_name, shape, function, geometry, offset):
-        self.model, self.weight_name = model, weight_name
-        self.function, self.geometry, self.offset = function, geometry, offset
-        self.packed = torch.empty(shape, dtype=torch.int32, device=model.weights[weight_name].device)
-        self.pack()
+    Made once: the launches that multiply by it get the weight's address too, and read the weight itself where the copy is left out.
+    """
 
-    def pack(self):
-        self.weight = self.model.weights[self.weight_name]
+    def __init__(self, model, weight_name, array, shape, function, geometry, offset):
+        self.model, self.weight_name, self.array = model, weight_name, array
+        self.weight = model.weights[weight_name]
         self.version = _version(self.weight)
-        start = self.weight.data_ptr() + 4 * self.offset
-        _lib.check(getattr(_lib.library(), self.function)(start, self.packed.data_ptr(), *self.geometry, _lib.current_stream()), self.function)
+        self.packed = torch.empty(shape, dtype=torch.int32, device=self.weight.device)
+        start = self.weight.data_ptr() + 4 * offset
+        _lib.check(getattr(_lib.library(), function)(start, self.packed.data_ptr(), *geometry, _lib.current_stream()), function)
 
-    def refresh(self):
-        """Pack again if the weight was replaced or written in place since (a wrapped module whose parameters were updated)."""
-        weight = self.model.weights[self.weight_name]
-        if weight is not self.weight or _version(weight) != self.version:
-            self.pack()
+    def current(self):
+        """Whether the model's weight is still the tensor that was packed, and not written since."""
+        weight = self.model.weights.get(self.weight_name)
+        return weight is self.weight and _version(weight) == self.version
 
 
 def _packed_gemm(call, weight):
@@ -119,9 +117,9 @@ def pack_constant_operands(model):
             name = f"{weight_name}_packed_{suffix}"
             clean = clean_onnx_name(name)
             if name not in model.weights:
-                copies.append(PackedOperand(model, weight_name, *copy))
+                copies.append(PackedOperand(model, weight_name, clean, *copy))
                 model.weights[name] = copies[-1].packed
-                sdfg.add_array(clean, list(copies[-1].packed.shape), int32, transient=False)
+                sdfg.add_datadesc(clean, PackedCopy(int32, copies[-1].packed.shape))
             packed_call = KernelCall(call.label, function, args, list(call.in_connectors) + ["_packed"], list(call.out_connectors))
             state.replace_node(call, packed_call, sdfg)
             state.add_edge(state.add_access(clean), None, packed_call, "_packed", sdfg.make_array_memlet(clean))

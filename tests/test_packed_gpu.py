@@ -4,8 +4,11 @@ import pytest
 import torch
 import torch.nn as nn
 
+import dace_onnx_amd.onnx as donnx
 from dace_onnx_amd import _lib
 from dace_onnx_amd.pytorch.module import DaceModule
+from dace_onnx_amd.testing.graphs import bert_encoder_layer_model
+from oracle import pure_ops
 
 pytestmark = pytest.mark.gpu
 FORMS = range(1, 11)
@@ -103,7 +106,7 @@ def test_gemm_by_a_packed_constant_keeps_small_values(tuning, form, low, high):
 
 
 def test_a_packed_copy_follows_its_weight():
-    """Parameters written in place after the first call: the next call multiplies by the new ones."""
+    """Parameters written in place after the first call: the next call multiplies by the new ones (and not by the packed copy)."""
     linear = nn.Linear(768, 1024).cuda()
     x = torch.randn(512, 768, device="cuda")
     model = DaceModule(nn.Sequential(linear, nn.ReLU()), dummy_inputs=(x, ))
@@ -114,3 +117,54 @@ def test_a_packed_copy_follows_its_weight():
         got, expected = model(x), torch.relu(x.double() @ linear.weight.double().t() + linear.bias.double()).detach()
         assert float((got.double() - expected).norm() / expected.norm()) < 1e-6
     assert [n.function for n, _ in model.dace_model.compile_and_init().bound_launches()] == ["mi355x_gemm_packed_f32"]
+
+
+def encoder(**options):
+    weights = pure_ops.bert_layer_weights(np.random.default_rng(0))
+    torch.manual_seed(0)
+    return donnx.ONNXModel("encoder", bert_encoder_layer_model(weights, 8, 128, 12), **options), torch.randn(8, 128, 768, device="cuda")
+
+
+@pytest.mark.parametrize("where", ["cpu", "numpy", "cuda"])
+def test_a_replaced_weight_is_multiplied_by_wherever_it_lies(where):
+    model, x = encoder()
+    before = model(x)
+    packed = {c.weight_name: c for c in model._packed}
+    assert len(packed) == 4
+    for name, copy in packed.items():   # twice the weights of every product, elsewhere
+        moved = copy.weight * 2
+        model.weights[name] = moved.cpu().numpy() if where == "numpy" else moved.to(where)
+    replaced = model(x)
+    for name, copy in packed.items():   # the same in place, with the launches that read the weights themselves
+        model.weights[name] = copy.weight.mul_(2)
+    assert torch.equal(replaced, model(x)) and not torch.allclose(replaced, before)
+
+
+def test_a_replay_follows_weights_that_are_written():
+    model, x = encoder(use_hip_graph=True)
+    eager, _ = encoder()
+    for _ in range(3):
+        assert torch.equal(model(x), eager(x))
+    for m in (model, eager):
+        for copy in m._packed[1:3]:
+            copy.weight.mul_(0.5)
+    for _ in range(3):   # (a replay every time but the first)
+        assert torch.equal(model(x), eager(x))
+    model.weights[model._packed[3].weight_name] = model._packed[3].weight * 3
+    for _ in range(3):
+        got, expected = model(x), eager(x)
+        assert torch.allclose(got, expected, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("construction", [True, False])
+def test_a_model_made_or_first_called_under_inference_mode(construction):
+    expected, x = encoder()
+    expected = expected(x)
+    if construction:
+        with torch.inference_mode():
+            model, _ = encoder()
+    else:
+        model, _ = encoder()
+    with torch.inference_mode():
+        first = model(x)
+    assert torch.equal(first, expected) and torch.equal(model(x), expected) and model._packed

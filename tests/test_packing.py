@@ -7,6 +7,7 @@ import torch
 
 import dace_onnx_amd.onnx as donnx
 from dace_onnx_amd import _lib
+from dace_onnx_amd.sdfg import _Program
 from dace_onnx_amd.testing.graphs import bert_encoder_layer_model
 from dace_onnx_amd.transformation import packing
 from oracle import pure_ops
@@ -30,7 +31,7 @@ def pack_launches(monkeypatch):
     library = _Library(_lib.library(), launches)
     monkeypatch.setattr(packing._lib, "library", lambda: library)
     monkeypatch.setattr(packing._lib, "current_stream", lambda: 0)
-    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: type("Stream", (), {"synchronize": lambda self: None})())
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: type("Stream", (), {"synchronize": lambda self: None, "cuda_stream": 0})())
     return launches
 
 
@@ -48,6 +49,83 @@ def test_models_made_or_first_called_under_inference_mode_are_packed(pack_launch
         model.expand()
         copies = packing.pack_constant_operands(model)
     assert len(copies) == len(pack_launches) == 4 and all(c.weight.is_inference() for c in copies)
-    for copy in copies:   # nothing to do again, in the mode or out of it
-        copy.refresh()
-    assert len(pack_launches) == 4
+    assert all(c.current() for c in copies)
+
+
+@pytest.fixture
+def program_runs(monkeypatch):
+    """Calls of compiled graphs, recorded instead of issued."""
+    runs = []
+    monkeypatch.setattr(_Program, "run", lambda program, addresses, stream: runs.append(list(addresses)))
+    return runs
+
+
+def _ready(model):
+    """``model`` as its first call finds it, in host memory."""
+    model.expand()
+    model._packed = packing.pack_constant_operands(model)
+    model._compiled = model.sdfg.compile()
+    model._compiled.device = torch.device("cpu")
+    return model
+
+
+def _operands(model):
+    """(packed copy or None, weight) of each launch by a packed copy, as addresses."""
+    return [tuple(item[3][1:3]) for item in model._compiled._launch_list if item[2] == "mi355x_gemm_packed_f32"]
+
+
+def _packed_by(model):
+    return [(c.packed.data_ptr(), c.weight.data_ptr()) for c in model._packed]
+
+
+X = torch.zeros(8, 128, 768)
+
+
+def test_a_weight_that_was_written_or_replaced_is_read_itself(pack_launches, program_runs):
+    model = _ready(_encoder())
+    assert len(model._packed) == 4
+    model(X)
+    assert sorted(_operands(model)) == sorted(_packed_by(model))
+    first, second = model._packed[:2]
+    first.weight[0] += 1
+    model.weights[second.weight_name] = second.weight.clone()
+    model(X)
+    expected = {(0, first.weight.data_ptr()), (0, model.weights[second.weight_name].data_ptr())} | set(_packed_by(model)[2:])
+    assert {(p or 0, w) for p, w in _operands(model)} == expected
+    model.weights[second.weight_name] = second.weight
+    model(X)
+    assert _packed_by(model)[1] in _operands(model)
+    assert len(pack_launches) == 4 and len(program_runs) == 3
+
+
+@pytest.mark.parametrize("replace", [lambda w: w.double(), lambda w: w[:8].contiguous(), lambda w: w.t().contiguous().t(), lambda w: w.numpy()[:4]])
+def test_no_launch_reads_a_replaced_weight_that_the_call_refuses(pack_launches, program_runs, replace):
+    model = _ready(_encoder())
+    name = model._packed[0].weight_name
+    model.weights[name] = replace(model.weights[name])
+    with pytest.raises(TypeError):
+        model(X)
+    assert len(pack_launches) == 4 and not program_runs
+
+
+def test_recordings_keep_the_weights_they_were_made_with(pack_launches, program_runs, monkeypatch):
+    """A weight written in place takes effect at the next replay, one that is replaced does not, whether packed or not."""
+    model = _ready(_encoder())
+    model.use_hip_graph = True
+    replays = []
+    monkeypatch.setattr(model._compiled, "capture_graph", lambda: None)
+    monkeypatch.setattr(model._compiled, "replay", lambda: replays.append(1))
+    model(X)
+    model(X)
+    assert (len(program_runs), len(replays)) == (1, 1) and sorted(_operands(model)) == sorted(_packed_by(model))
+    first, second = model._packed[:2]
+    first.weight[0] += 1
+    model.weights[second.weight_name] = second.weight + 1
+    bias = next(n for n, w in model.weights.items() if w.dim() == 1 and w.dtype is torch.float32)
+    kept, model.weights[bias] = model.weights[bias], torch.ones_like(model.weights[bias])
+    model(X)
+    assert (len(program_runs), len(replays)) == (2, 1)
+    assert {(p or 0, w) for p, w in _operands(model)} == {(0, w) for _, w in _packed_by(model)[:2]} | set(_packed_by(model)[2:])
+    assert model.weights[bias].data_ptr() not in program_runs[-1] and kept.data_ptr() in program_runs[-1] + program_runs[0]
+    model(X)
+    assert (len(program_runs), len(replays)) == (2, 2) and len(pack_launches) == 4
