@@ -30,6 +30,7 @@ from .proto import ModelProto, TensorProto
 from .schema import ONNXParameterType
 from .nodes.onnx_op import get_onnx_node, has_onnx_node
 from .shape_inference import infer_shapes as _infer_shapes
+from .weights import Weights
 
 log = logging.getLogger(__name__)
 
@@ -153,7 +154,7 @@ class ONNXModel:
                 raise ValueError("Got input or output without name")
             self.value_infos.setdefault(value.name, value)
 
-        self.weights: typing.Dict[str, torch.Tensor] = {}  #: mapping from weight name to tensor
+        self.weights: typing.Dict[str, torch.Tensor] = Weights()  #: mapping from weight name to tensor
         for init in graph.initializer:
             self._add_constant_tensor(init, parent_pytorch_module)
 
@@ -319,12 +320,27 @@ class ONNXModel:
             if tensor.name in params:
                 weight = params[tensor.name].detach()
         if weight is None:
-            weight = torch.from_numpy(np.array(tensor.array, copy=True).reshape(tensor.dims))
-        self.weights[tensor.name] = weight.to(self.device).contiguous()
+            weight, owner = torch.from_numpy(np.array(tensor.array, copy=True).reshape(tensor.dims)), None
+        else:
+            owner = weight
+        weight = weight.to(self.device).contiguous()
+        if owner is None or weight.data_ptr() != owner.data_ptr():
+            self.weights.make(tensor.name, weight)
+        else:
+            self.weights[tensor.name] = weight   # the module's own memory
 
     @property
     def clean_weights(self):
+        """The weights by array name: arguments of the compiled graph."""
         return {clean_onnx_name(k): v for k, v in self.weights.items()}
+
+    def _own_weights(self):
+        """As :attr:`clean_weights`, for one call."""
+        return {clean_onnx_name(k): v for k, v in self.weights.peek_items()}
+
+    def weight_of(self, array):
+        """The weight behind the array of that name, None if there is none; read it only."""
+        return self._own_weights().get(array)
 
     # -- execution ------------------------------------------------------------------------
     def auto_optimize(self):
@@ -363,6 +379,24 @@ class ONNXModel:
             pack_variable_filters(self.sdfg)
             self._compiled = self.sdfg.compile()
         return self._compiled
+
+    def pack_weights(self):
+        """Pack the constant operands of the model's products as they are now.
+
+        Copies in the matrix unit's own layout are made when the graph is compiled, of weights that nobody but the model holds, and stay in
+        use until such a weight is read from :attr:`weights`, replaced or written. This makes them of all weights, those that a caller or
+        a wrapped module holds among them, and calls from here on multiply by them: a caller who writes such a weight in a way that torch
+        does not count (through ``.data``, from another library) calls it again after.
+        """
+        self.compile_and_init()
+        torch.cuda.synchronize(self.device)   # launches on any stream that still read the copies
+        for c in self._packed:
+            c.pack(declared=True)
+        torch.cuda.current_stream(self.device).synchronize()
+        self._static_io = self._recorded_packed = None
+
+    def _capturing(self):
+        return self.device.type == "cuda" and torch.cuda.is_current_stream_capturing()
 
     def _weight_args(self, weights, packed):
         """``weights`` (by array name) as arguments of the compiled graph, each packed copy among them if ``packed`` says so, left out if not."""
@@ -408,6 +442,9 @@ class ONNXModel:
             call[clean_onnx_name(n)] = v
         outputs = collections.OrderedDict()
         packed = [c.current() for c in self._packed]
+        if not self.use_hip_graph and any(use and not c.derived for c, use in zip(self._packed, packed)) and self._capturing():
+            # the caller's recording: its replays follow weights that are written after it
+            packed = [use and c.derived for c, use in zip(self._packed, packed)]
         if self.use_hip_graph:
             if self._static_io is None:
                 # private input/output buffers: the graph is bound to their addresses
@@ -416,7 +453,7 @@ class ONNXModel:
                 for n in self.outputs:
                     desc = self.sdfg.arrays[clean_onnx_name(n)]
                     s_out[clean_onnx_name(n)] = torch.empty(desc.shape, dtype=desc.dtype.as_torch(), device=self.device)
-                self._static_io = (s_in, s_out, self.clean_weights)
+                self._static_io = (s_in, s_out, self._own_weights())
             else:
                 s_in, s_out, _ = self._static_io
                 for k, v in call.items():
@@ -425,7 +462,7 @@ class ONNXModel:
                 # an eager run, which binds the launch list, for the recording. Weights are the tensors of the first call, written or
                 # not: a launch reads a weight that was written, or replaced, itself from here on.
                 compiled(**s_in, **s_out, **self._weight_args(self._static_io[2], packed))
-                compiled.capture_graph()
+                compiled.capture_graph(with_packed=True)
                 self._recorded_packed = packed
             else:
                 compiled.replay()
@@ -440,7 +477,7 @@ class ONNXModel:
                     desc = self.sdfg.arrays[k]
                     out_kwargs[k] = self.save_transients[k] = torch.empty(desc.shape, dtype=desc.dtype.as_torch(),
                                                                           device=self.device)
-            compiled(**call, **out_kwargs, **self._weight_args(self.clean_weights, packed))
+            compiled(**call, **out_kwargs, **self._weight_args(self._own_weights(), packed))
         results = [t if use_torch else t.cpu().numpy() for t in outputs.values()]
         return results[0] if len(results) == 1 else tuple(results)
 

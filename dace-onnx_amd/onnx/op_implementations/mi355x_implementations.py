@@ -1007,8 +1007,9 @@ class MI355XSlice(ONNXForward):
             edge = [e for e in state.in_edges(node) if e.dst_conn == name][0]
             if state.in_edges(edge.src):
                 return None             # computed by another node
-            if model is not None and edge.src.data in model.clean_weights:
-                idx.append([int(v) for v in model.clean_weights[edge.src.data].detach().cpu().reshape(-1).tolist()])
+            weight = None if model is None else model.weight_of(edge.src.data)
+            if weight is not None:
+                idx.append([int(v) for v in weight.detach().cpu().reshape(-1).tolist()])
             elif edge.src.data in getattr(sdfg, "_constant_inputs", {}):       # the call form donnx.ONNXSlice(...)
                 idx.append([int(v) for v in sdfg._constant_inputs[edge.src.data].reshape(-1)])
             else:

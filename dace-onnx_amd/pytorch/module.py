@@ -275,8 +275,9 @@ class DaceModule(nn.Module):
     :param exporter: "auto", "structural" or "torch": how the ONNX graph is obtained (see the module docstring).
 
     Parameters are read from ``module`` when the graph is built (first call): derived copies (k-contiguous,
-    concatenated, packed weights) are made then, so call :meth:`reset_sdfg` after changing parameters (a packed copy
-    goes out of use when its parameter is written in place, except through ``.data``, which torch does not count).
+    concatenated weights, and what is packed of them) are made then, so call :meth:`reset_sdfg` after changing parameters.
+    Parameters on the GPU that no such copy is made of are read where they lie on every call;
+    ``dace_model.pack_weights()`` packs them too, for a module whose parameters stay as they are.
     """
 
     def __init__(self, module: nn.Module, dummy_inputs: typing.Optional[typing.Tuple[torch.Tensor]] = None,

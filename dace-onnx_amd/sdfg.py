@@ -153,8 +153,12 @@ class Scalar(Array):
 
 
 class PackedCopy(Array):
-    """Another argument in a kernel's own layout. A caller may leave it out (``None``): the launch gets a null pointer for it and reads
-    that argument itself."""
+    """Another argument in a kernel's own layout. A caller may leave it out (or pass ``None``): the launch gets a null pointer for it and
+    reads that argument itself. ``derived``: of an argument that is a copy already, which nothing but the framework writes."""
+
+    def __init__(self, dtype, shape, derived):
+        super().__init__(dtype, shape)
+        self.derived = derived
 
 
 class Memlet:
@@ -919,17 +923,27 @@ class CompiledSDFG:
         return None
 
     # -- HIP graph -------------------------------------------------------------------
-    def capture_graph(self):
-        """Record the currently bound launch list into a HIP graph."""
+    def capture_graph(self, with_packed=False):
+        """Record the currently bound launch list into a HIP graph.
+
+        :param with_packed: record packed copies of arguments that a caller may write too; its replays do not follow that.
+        """
         import torch
         if self._bound_key is None:
             raise RuntimeError("call the compiled SDFG once before capturing it")
+        launches = self._launch_list
+        bound = dict(zip(self._external, self._bound_key))
+        left_out = [] if with_packed else [k for k in self._optional if bound[k] and not self.sdfg.arrays[k].derived]
+        if left_out and self._patches is not None:
+            launches = self._rebind(launches, {**bound, **dict.fromkeys(left_out, 0)})
+        elif left_out:
+            launches, _ = self._bind({**self._env, **dict.fromkeys(left_out)})
         # (a device copy left over from a Reshape into caller-owned memory is issued on the capture stream like
         # the kernels and becomes a node of the graph)
         g = torch.cuda.CUDAGraph()
         torch.cuda.synchronize()
         with torch.cuda.graph(g):
-            self._run(self._launch_list)
+            self._run(launches)
         self._graph = g
         return g
 
@@ -954,10 +968,11 @@ class CompiledSDFG:
         the order of ``__arrays``, the arrays whose device pointers the caller passes: the SDFG's non-transient
         arrays by name, then its transients by their flattened key (see :meth:`transient_descriptors`). A
         Reshape-like alias of a transient is a pointer assignment; one into caller-owned memory would need a
-        copy and is not supported here.
+        copy and is not supported here. Packed copies of arguments that a caller may write are left out.
         """
         name = name or self.sdfg.name
-        arrays = list(self._external) + [k for k in self._transients if k not in self._external]
+        left_out = {k for k in self._optional if not self.sdfg.arrays[k].derived}
+        arrays = [k for k in self._external if k not in left_out] + [k for k in self._transients if k not in self._external]
         index = {k: i for i, k in enumerate(arrays)}
         desc_of = {**{k: self.sdfg.arrays[k] for k in self._external}, **self._transients}
         lines = ['#include <stdint.h>', '#include <stdio.h>', '#include <stdlib.h>', '#include "mi355x_onnx.h"', '',
@@ -977,7 +992,8 @@ class CompiledSDFG:
             lines.append(f"    {{  // {node.label}")
             for conn, key in conn_to_key.items():
                 ctype = desc_of[key].dtype.ctype if key in desc_of else "float"
-                lines.append(f"        {ctype}* _{conn} = ({ctype}*)__arrays[{index[key]}];")
+                value = "nullptr" if key in left_out else f"({ctype}*)__arrays[{index[key]}]"
+                lines.append(f"        {ctype}* _{conn} = {value};")
                 lines.append(f"        (void)_{conn};")
             lines.extend("        " + ln for ln in node.as_cpp().splitlines())
             lines.append("    }")

@@ -92,7 +92,7 @@ def _constant_value(sdfg, name) -> typing.Optional[np.ndarray]:
     model = getattr(sdfg, "_parent_onnx_model", None)
     if model is None:
         return None
-    w = model.clean_weights.get(name)
+    w = model.weight_of(name)
     return None if w is None else w.detach().cpu().numpy()
 
 
@@ -209,7 +209,7 @@ def _fold_batchnorm_into_conv(sdfg: SDFG, state: SDFGState) -> int:
         e = _in_edge(state, node, conn)
         if e is None or not isinstance(e.src, AccessNode) or e.src.data not in by_clean or state.in_edges(e.src):
             return None
-        w = model.weights[by_clean[e.src.data]]
+        w = model.weights.peek(by_clean[e.src.data])
         return (e, w) if w.dtype == torch.float32 else None
 
     folded = 0
@@ -240,7 +240,8 @@ def _fold_batchnorm_into_conv(sdfg: SDFG, state: SDFGState) -> int:
         new_w = (w[1].double() * a.reshape(-1, *([1] * (w[1].dim() - 1)))).float().contiguous()
         new_b = (((bias[1].double() if bias is not None else torch.zeros_like(mean)) - mean) * a + beta).float().contiguous()
         w_name, b_name = by_clean[w[0].src.data] + "_bnfold_" + bn.label, by_clean[w[0].src.data] + "_bnfold_bias_" + bn.label
-        model.weights[w_name], model.weights[b_name] = new_w, new_b
+        model.weights.make(w_name, new_w, derived=True)
+        model.weights.make(b_name, new_b, derived=True)
         w_clean, b_clean = clean_onnx_name(w_name), clean_onnx_name(b_name)
         sdfg.add_array(w_clean, list(new_w.shape), sdfg.arrays[w[0].src.data].dtype, transient=False)
         sdfg.add_array(b_clean, [oc], sdfg.arrays[w[0].src.data].dtype, transient=False)
@@ -542,7 +543,8 @@ def _pretranspose_weights(sdfg: SDFG, state: SDFGState) -> int:
         t_name = b_e.src.data + "_kcontig"
         if t_name not in sdfg.arrays:
             sdfg.add_array(t_name, [n, k], desc.dtype, transient=False)
-            model.weights[by_clean[b_e.src.data] + "_kcontig"] = model.weights[by_clean[b_e.src.data]].t().contiguous()
+            w_name = by_clean[b_e.src.data]
+            model.weights.make(w_name + "_kcontig", model.weights.peek(w_name).t().contiguous(), derived=True)
         t_access = None
         for cand in state.nodes():
             if isinstance(cand, AccessNode) and cand.data == t_name:
@@ -1002,14 +1004,14 @@ def _fuse_shared_input_matmuls(sdfg: SDFG, state: SDFGState) -> int:
             continue
         # ---- constants: weights [K, sum N_i], biases [sum N_i]
         w_name = by_clean[first[2].src.data] + "_hcat"
-        model.weights[w_name] = torch.cat([model.weights[by_clean[m[2].src.data]] for m in members],
-                                          dim=0 if transposed else 1).contiguous()
+        wide_w = torch.cat([model.weights.peek(by_clean[m[2].src.data]) for m in members], dim=0 if transposed else 1).contiguous()
+        model.weights.make(w_name, wide_w, derived=True)
         w_clean = clean_onnx_name(w_name)
-        sdfg.add_array(w_clean, list(model.weights[w_name].shape), y0.dtype, transient=False)
+        sdfg.add_array(w_clean, list(wide_w.shape), y0.dtype, transient=False)
         b_clean = None
         if first[3] is not None:
             b_name = by_clean[first[3].src.data] + "_hcat"
-            model.weights[b_name] = torch.cat([model.weights[by_clean[m[3].src.data]].reshape(-1) for m in members]).contiguous()
+            model.weights.make(b_name, torch.cat([model.weights.peek(by_clean[m[3].src.data]).reshape(-1) for m in members]).contiguous(), derived=True)
             b_clean = clean_onnx_name(b_name)
             sdfg.add_array(b_clean, [n_total], y0.dtype, transient=False)
         wide = first[4].dst.data + "_hcat"

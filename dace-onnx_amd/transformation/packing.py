@@ -2,7 +2,7 @@
 graph is compiled.
 
 A packed copy holds three bf16 parts of every value in the order in which the matrix unit takes them (``csrc/split_bf16.h``); it is
-made once, on the GPU, and is a further weight of the model. The reference has no counterpart: its constants are handed to a BLAS
+made once, on the GPU. The reference has no counterpart: its constants are handed to a BLAS
 library as they are.
 """
 import torch
@@ -19,24 +19,38 @@ def _version(tensor):
 class PackedOperand:
     """The packed copy ``array`` of a weight, ``shape`` 32-bit words, written by the library's ``function`` from ``offset`` values on.
 
-    Made once: the launches that multiply by it get the weight's address too, and read the weight itself where the copy is left out.
+    The launches that multiply by it get the weight's address too, and read the weight itself where the copy is left out. It is made at
+    once of a weight that only the model holds (``onnx/weights.py``), and of others on request.
     """
 
-    def __init__(self, model, weight_name, array, shape, function, geometry, offset):
-        self.model, self.weight_name, self.array = model, weight_name, array
-        self.weight = model.weights[weight_name]
-        self.version = _version(self.weight)
-        self.packed = torch.empty(shape, dtype=torch.int32, device=self.weight.device)
-        start = self.weight.data_ptr() + 4 * offset
-        _lib.check(getattr(_lib.library(), function)(start, self.packed.data_ptr(), *geometry, _lib.current_stream()), function)
+    def __init__(self, model, weight_name, descriptor, array, shape, function, geometry, offset):
+        self.weights, self.weight_name, self.descriptor, self.array = model.weights, weight_name, descriptor, array
+        self.shape, self.function, self.geometry, self.offset = shape, function, geometry, offset
+        self.derived = model.weights.derived(weight_name)
+        self.device, self.weight, self.version, self.packed, self.declared = model.device, None, None, None, False
+        if model.weights.private(weight_name):
+            self.pack()
+
+    def pack(self, declared=False):
+        """``declared``: the caller answers for what is written into the weight from here on."""
+        weight = self.weights.peek(self.weight_name)
+        if not isinstance(weight, torch.Tensor) or weight.dtype != torch.float32 or tuple(weight.shape) != self.descriptor.shape \
+                or not weight.is_contiguous() or weight.device != self.device:
+            return
+        self.weight, self.version, self.declared = weight, _version(weight), declared
+        if self.packed is None:
+            self.packed = torch.empty(self.shape, dtype=torch.int32, device=self.device)
+        start = weight.data_ptr() + 4 * self.offset
+        _lib.check(getattr(_lib.library(), self.function)(start, self.packed.data_ptr(), *self.geometry, _lib.current_stream()), self.function)
 
     def current(self):
-        """Whether the model's weight is still the tensor that was packed, and not written since."""
-        weight = self.model.weights.get(self.weight_name)
-        return weight is self.weight and _version(weight) == self.version
+        """Whether the model's weight is still the tensor that was packed, and not written since as far as can be told."""
+        weight = self.weight
+        return weight is not None and self.weights.peek(self.weight_name) is weight and _version(weight) == self.version \
+            and (self.declared or self.weights.private(self.weight_name))
 
 
-def _packed_gemm(call, weight):
+def _packed_gemm(call, desc):
     """(name suffix, shape, function, geometry, offset) of the copy that a GEMM multiplies by, and the call that does; None where it does not pay."""
     lib = _lib.library()
     offset = call.args[1].offset
@@ -60,10 +74,10 @@ def _by_packed_filters(call, constant):
     return [size // 3072, 3, 64, 4], (M, C, KH, KW), ("mi355x_conv2d_packed_f32", args)
 
 
-def _packed_conv(call, weight):
+def _packed_conv(call, desc):
     """As :func:`_packed_gemm`, for a convolution."""
     packed = _by_packed_filters(call, True)
-    if packed is None or tuple(weight.shape) != packed[1] or not weight.is_contiguous():
+    if packed is None or desc.shape != packed[1] or not desc.is_contiguous():
         return None
     shape, geometry, packed_call = packed
     return ("filters", shape, "mi355x_pack_conv_f32", geometry, 0), packed_call
@@ -108,18 +122,20 @@ def pack_constant_operands(model):
             if edge.src.data not in by_clean or edge.src.data in written:
                 continue
             weight_name = by_clean[edge.src.data]
-            if model.weights[weight_name].dtype != torch.float32:
+            desc = sdfg.arrays[edge.src.data]
+            if desc.dtype.name != "float32":
                 continue
-            packed = _PACKED[call.function](call, model.weights[weight_name])
+            packed = _PACKED[call.function](call, desc)
             if packed is None:
                 continue
             (suffix, *copy), (function, args) = packed
             name = f"{weight_name}_packed_{suffix}"
             clean = clean_onnx_name(name)
-            if name not in model.weights:
-                copies.append(PackedOperand(model, weight_name, clean, *copy))
-                model.weights[name] = copies[-1].packed
-                sdfg.add_datadesc(clean, PackedCopy(int32, copies[-1].packed.shape))
+            if clean not in sdfg.arrays:
+                copies.append(PackedOperand(model, weight_name, desc, clean, *copy))
+                sdfg.add_datadesc(clean, PackedCopy(int32, copies[-1].shape, copies[-1].derived))
+                if copies[-1].derived:
+                    model.weights.make(name, copies[-1].packed, derived=True)
             packed_call = KernelCall(call.label, function, args, list(call.in_connectors) + ["_packed"], list(call.out_connectors))
             state.replace_node(call, packed_call, sdfg)
             state.add_edge(state.add_access(clean), None, packed_call, "_packed", sdfg.make_array_memlet(clean))

@@ -6,6 +6,7 @@ import torch.nn as nn
 
 import dace_onnx_amd.onnx as donnx
 from dace_onnx_amd import _lib
+from dace_onnx_amd.onnx.proto import TensorProto, helper, numpy_helper
 from dace_onnx_amd.pytorch.module import DaceModule
 from dace_onnx_amd.testing.graphs import bert_encoder_layer_model
 from oracle import pure_ops
@@ -168,3 +169,72 @@ def test_a_model_made_or_first_called_under_inference_mode(construction):
     with torch.inference_mode():
         first = model(x)
     assert torch.equal(first, expected) and torch.equal(model(x), expected) and model._packed
+
+
+def head(**options):
+    rng = np.random.default_rng(0)
+    weight = numpy_helper.from_array(rng.standard_normal((768, 3001), dtype=np.float32), "w")
+    info = lambda n, shape: helper.make_tensor_value_info(n, TensorProto.FLOAT, shape)   # noqa: E731
+    graph = helper.make_graph([helper.make_node("MatMul", ["x", "w"], ["y"])], "head", [info("x", [1024, 768])], [info("y", [1024, 3001])], initializer=[weight])
+    return donnx.ONNXModel("head", helper.make_model(graph, opset_imports=[helper.make_opsetid("", 13)]), **options), torch.randn(1024, 768, device="cuda")
+
+
+def close(got, x, w):
+    expected = x.double() @ w.double()
+    return float((got.double() - expected).norm() / expected.norm()) < 1e-6
+
+
+@pytest.mark.parametrize("replayed", [False, True])
+def test_writes_that_torch_does_not_count_take_effect_at_the_next_call(replayed):
+    model, x = head(use_hip_graph=replayed)
+    for _ in range(3):
+        model(x)
+    assert model._packed[0].current()
+    weight = model.weights["w"]
+    for _ in range(3):
+        weight.data.mul_(0.5)
+        assert close(model(x), x, weight)
+        model.weights["w"].data[3] += 1
+        assert close(model(x), x, weight)
+    model.pack_weights()
+    for _ in range(3):
+        assert model._packed[0].current() and close(model(x), x, weight)
+    weight.data.mul_(0.5)
+    model.pack_weights()
+    for _ in range(2):
+        assert close(model(x), x, weight)
+
+
+def test_writes_to_parameters_that_torch_does_not_count_take_effect_at_the_next_call():
+    linear, conv = nn.Linear(768, 1024).cuda(), nn.Conv2d(64, 64, 3, padding=1).cuda()
+    x, image = torch.randn(512, 768, device="cuda"), torch.randn(32, 64, 28, 28, device="cuda")
+    dense, convolution = DaceModule(linear, dummy_inputs=(x, )), DaceModule(conv, dummy_inputs=(image, ))
+    dense(x), convolution(image)
+    for _ in range(2):
+        linear.weight.data.mul_(0.5)
+        conv.weight.data.mul_(0.5)
+        with torch.no_grad():
+            assert close(dense(x) - linear.bias, x, linear.weight.t())
+            expected = torch.nn.functional.conv2d(image.cpu().double(), conv.weight.cpu().double(), conv.bias.cpu().double(), padding=1)
+            assert float((convolution(image).cpu().double() - expected).norm() / expected.norm()) < 1e-6
+
+
+def test_a_callers_recordings_follow_weights_that_are_written_after_them():
+    model, x = head()
+    model(x)
+    weight = model._packed[0].weight
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        recorded = model(x)
+    assert model._packed[0].current()
+    for _ in range(3):
+        weight.data.mul_(0.5)
+        graph.replay()
+        assert close(recorded, x, weight)
+    y = model(x)
+    compiled = model.compile_and_init()
+    compiled.capture_graph()   # of the call above
+    for _ in range(3):
+        weight.data.mul_(0.5)
+        compiled.replay()
+        assert close(y, x, weight)

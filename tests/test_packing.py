@@ -1,12 +1,16 @@
 """Packed copies of constant operands: which tensors they are made of and when they are used (no GPU: packing launches are recorded, not issued)."""
 import contextlib
+import copy
 
 import numpy as np
 import pytest
 import torch
+import torch.nn as nn
 
 import dace_onnx_amd.onnx as donnx
 from dace_onnx_amd import _lib
+from dace_onnx_amd.onnx.proto import TensorProto, helper, numpy_helper
+from dace_onnx_amd.pytorch.module import DaceModule
 from dace_onnx_amd.sdfg import _Program
 from dace_onnx_amd.testing.graphs import bert_encoder_layer_model
 from dace_onnx_amd.transformation import packing
@@ -113,7 +117,7 @@ def test_recordings_keep_the_weights_they_were_made_with(pack_launches, program_
     model = _ready(_encoder())
     model.use_hip_graph = True
     replays = []
-    monkeypatch.setattr(model._compiled, "capture_graph", lambda: None)
+    monkeypatch.setattr(model._compiled, "capture_graph", lambda with_packed: None)
     monkeypatch.setattr(model._compiled, "replay", lambda: replays.append(1))
     model(X)
     model(X)
@@ -129,3 +133,106 @@ def test_recordings_keep_the_weights_they_were_made_with(pack_launches, program_
     assert model.weights[bias].data_ptr() not in program_runs[-1] and kept.data_ptr() in program_runs[-1] + program_runs[0]
     model(X)
     assert (len(program_runs), len(replays)) == (2, 2) and len(pack_launches) == 4
+
+
+def _head(**options):
+    """A dense layer whose odd width leaves fusion nothing to derive: the product is by the initializer itself."""
+    rng = np.random.default_rng(0)
+    weight = numpy_helper.from_array(rng.standard_normal((768, 3001), dtype=np.float32), "w")
+    info = lambda n, shape: helper.make_tensor_value_info(n, TensorProto.FLOAT, shape)   # noqa: E731
+    graph = helper.make_graph([helper.make_node("MatMul", ["x", "w"], ["y"])], "head", [info("x", [1024, 768])], [info("y", [1024, 3001])], initializer=[weight])
+    return donnx.ONNXModel("head", helper.make_model(graph, opset_imports=[helper.make_opsetid("", 13)]), **options)
+
+
+HEAD_X = torch.zeros(1024, 768)
+
+
+@pytest.mark.parametrize("first", [True, False])
+@pytest.mark.parametrize("read", [lambda w: w["w"], lambda w: w.get("w"), lambda w: w.setdefault("w"), lambda w: dict(w)["w"], lambda w: {**w}["w"],
+                                  lambda w: list(w.values())[0], lambda w: [t for n, t in w.items() if n == "w"][0], lambda w: w.copy()["w"], lambda w: (w | {})["w"],
+                                  lambda w: ({} | w)["w"], lambda w: copy.copy(w)["w"], lambda w: w.pop("w")])
+def test_a_weight_that_was_handed_out_is_read_itself(pack_launches, program_runs, read, first):
+    """Whoever holds it can write it in ways that torch does not count."""
+    model = _head()
+    handed = read(model.weights) if first else None
+    if first and "w" not in model.weights:
+        model.weights["w"] = handed
+    _ready(model)
+    model(HEAD_X)
+    assert len(model._packed) == 1 and not model._packed[0].derived
+    packed = model._packed[0].packed
+    if first:
+        assert packed is None and not pack_launches
+    else:
+        assert _operands(model) == [(packed.data_ptr(), model._packed[0].weight.data_ptr())]
+        handed = read(model.weights)
+        if "w" not in model.weights:
+            model.weights["w"] = handed
+        model(HEAD_X)
+    assert _operands(model) == [(0 if not first else None, handed.data_ptr())]
+    compiled = model._compiled   # called without the model
+    compiled(x=HEAD_X, y=torch.zeros(1024, 3001), **model.clean_weights)
+    assert _operands(model)[0][0] in (0, None) and "_packed = nullptr" in compiled.program_source("head")[0]
+
+
+def test_names_and_sizes_hand_nothing_out(pack_launches):
+    model = _head()
+    assert list(model.weights) == ["w"] == list(model.weights.keys()) and "w" in model.weights and len(model.weights) == 1
+    assert len(packing.pack_constant_operands(model) if model.expand() else ()) == len(pack_launches) == 1
+
+
+def test_parameters_of_a_module_are_packed_on_request(pack_launches, program_runs, monkeypatch):
+    linear = nn.Linear(768, 1024)
+    model = _ready(DaceModule(nn.Sequential(linear, nn.ReLU()), dummy_inputs=(HEAD_X, )).dace_model)
+    model(HEAD_X)
+    assert not pack_launches and _operands(model) == [(None, linear.weight.data_ptr())]
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: None)
+    model.pack_weights()
+    model(HEAD_X)
+    assert len(pack_launches) == 1 and _operands(model) == _packed_by(model)
+    with torch.no_grad():
+        linear.weight.mul_(2)   # (torch counts this)
+    model(HEAD_X)
+    assert _operands(model) == [(0, linear.weight.data_ptr())]
+    model.pack_weights()
+    model(HEAD_X)
+    assert len(pack_launches) == 2 and _operands(model) == _packed_by(model)
+
+
+def test_weights_packed_on_request_are_those_that_the_call_takes(pack_launches, program_runs, monkeypatch):
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: None)
+    model = _ready(_head())
+    weight = model.weights["w"]
+    for replaced in (weight.double(), weight[:8], weight.t().contiguous().t(), weight.numpy()):
+        model.weights["w"] = replaced
+        model.pack_weights()
+    assert len(pack_launches) == 1 and not model._packed[0].current()
+
+
+def test_a_recording_is_made_again_when_a_weight_is_handed_out(pack_launches, program_runs, monkeypatch):
+    model = _ready(_head(use_hip_graph=True))
+    replays = []
+    monkeypatch.setattr(model._compiled, "capture_graph", lambda with_packed: None)
+    monkeypatch.setattr(model._compiled, "replay", lambda: replays.append(1))
+    model(HEAD_X)
+    model(HEAD_X)
+    assert _operands(model) == _packed_by(model) and (len(program_runs), len(replays)) == (1, 1)
+    handed = model.weights["w"]
+    model(HEAD_X)
+    model(HEAD_X)
+    assert _operands(model) == [(0, handed.data_ptr())] and (len(program_runs), len(replays)) == (2, 2)
+
+
+def test_a_callers_recording_reads_the_weights_themselves(pack_launches, program_runs, monkeypatch):
+    """Its replays follow weights that are written after it, which nobody is asked about then."""
+    model, recorded = _ready(_head()), []
+    model(HEAD_X)
+    monkeypatch.setattr(torch.cuda, "CUDAGraph", lambda: None)
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: None)
+    monkeypatch.setattr(torch.cuda, "graph", lambda g: contextlib.nullcontext())
+    monkeypatch.setattr(model._compiled, "_run", recorded.extend)
+    model._compiled.capture_graph()
+    assert [item[3][1] for item in recorded] == [0] and _operands(model) == _packed_by(model)
+    monkeypatch.setattr(model, "_capturing", lambda: True)
+    model(HEAD_X)
+    assert _operands(model) == [(0, model._packed[0].weight.data_ptr())]
