@@ -600,12 +600,9 @@ class _Program:
         self._names = [item[2] for item in launches]
         self._keep = launches   # arrays that words point to
         for item, (slots, arrays) in zip(launches, patches):
-            _, fn, name, args, stream_slots, _, _ = item
-            function = lib.mi355x_program_function(name.encode())
-            if function < 0 or stream_slots != [len(args) - 1]:
-                raise RuntimeError(f"{name} cannot be part of a program")
+            _, fn, name, args, _, _, _ = item
             first = len(words) + 1
-            words.append(function)
+            words.append(lib.mi355x_program_function(name.encode()))
             for argument, kind in zip(args[:-1], fn.argtypes):
                 if argument is None:
                     words.append(0)
@@ -625,6 +622,11 @@ class _Program:
         self._words, self._moved = array.array("q", words), array.array("q", [v for m in moved for v in m])
         self._run = lib.mi355x_program_run
         self._fixed = (self._words.buffer_info()[0], len(words), len(launches), self._moved.buffer_info()[0], len(moved))
+
+    @staticmethod
+    def takes(lib, launches):
+        """Whether all of ``launches`` are functions that the library can call so: those that take the stream last, and nowhere else."""
+        return all(lib.mi355x_program_function(name.encode()) >= 0 and slots == [len(args) - 1] for _, _, name, args, slots, _, _ in launches)
 
     def run(self, addresses, stream):
         addresses = array.array("q", addresses)
@@ -661,7 +663,7 @@ class CompiledSDFG:
         self._plan = []         # ("call", node, connector -> key) | ("alias", src key, dst key, dst descriptor)
         self._bound_key = None
         self._patches = None    # per launch, the pointer arguments that follow the caller's arrays (see _rebind)
-        self._program = None    # the launch list as one native call (None: it holds device copies)
+        self._program = None    # the launch list as one native call (None: it holds device copies, or functions that cannot be part of one)
         self._launches, self._listed_key = [], None
         self._graph = None
         self._build(sdfg, prefix="", outer_map={})
@@ -900,10 +902,13 @@ class CompiledSDFG:
         key = [0 if t is None else t.data_ptr() for t in env.values()]
         if key != self._bound_key:
             if self._program is None:
-                self._launches, self._patches = self._bind(env)
+                if self._bound_key is None or self._patches is None:
+                    self._launches, self._patches = self._bind(env)
+                    if self._patches is not None and _Program.takes(self._lib, self._launches):
+                        self._program = _Program(self._lib, self._launches, self._patches, self._external)
+                else:
+                    self._launches = self._rebind(self._launches, dict(zip(self._external, key)))
                 self._listed_key = key
-                if self._patches is not None:
-                    self._program = _Program(self._lib, self._launches, self._patches, self._external)
             self._env = env   # the caller's arrays live as long as the launch list points to them
             self._bound_key = key
             self._graph = None

@@ -2,8 +2,10 @@
 import array
 
 import pytest
+import torch
 
 from dace_onnx_amd import _lib
+from dace_onnx_amd import sdfg as dace
 
 
 def run(calls, patches=(), addresses=(), words=None, behind=()):
@@ -46,3 +48,50 @@ def test_addresses_take_their_place():
                                        dict(calls=[EMPTY], patches=[(1, -1, 6)]), dict(calls=[EMPTY], words=-1)])
 def test_what_is_no_program_is_refused(arguments):
     assert run(**arguments) & 0xff == 1
+
+
+def packing_sdfg(rows=40, k=64):
+    """A launch that cannot be part of a program, and one that can."""
+    sdfg = dace.SDFG("packing")
+    state = sdfg.add_state()
+    sdfg.add_array("w", [rows, k], dace.float32)
+    sdfg.add_array("largest", [rows], dace.float32)
+    sdfg.add_array("packed", [-(-rows // 32), k // 32, 2, 3, 64, 4], dace.int32)
+    pack = dace.KernelCall("pack", "mi355x_pack_f32", [dace.Ptr("w"), dace.Ptr("p"), rows, k, k, 1, dace.Stream()], ["w"], ["p"])
+    top = dace.KernelCall("largest", "mi355x_reduce_f32", [2, dace.Ptr("w"), dace.Ptr("y"), rows, k, 1, dace.Stream()], ["w"], ["y"])
+    empty = dace.KernelCall("empty", "mi355x_launch_empty_kernel", [dace.Stream()], [], [])
+    w = state.add_read("w")
+    for call, conn, name in ((pack, "p", "packed"), (top, "y", "largest")):
+        state.add_edge(w, None, call, "w", sdfg.make_array_memlet("w"))
+        state.add_edge(call, conn, state.add_write(name), None, sdfg.make_array_memlet(name))
+    state.add_node(empty)
+    return sdfg
+
+
+def test_functions_that_are_no_part_of_a_program_are_called_one_at_a_time(monkeypatch):
+    compiled = packing_sdfg().compile()
+    compiled.device = torch.device("cpu")
+    runs = []
+    monkeypatch.setattr(compiled, "_run", runs.append)
+    buffers = lambda: {k: torch.zeros(compiled.sdfg.arrays[k].shape, dtype=compiled._torch_types[k]) for k in compiled._external}  # noqa: E731
+    first, second = buffers(), buffers()
+    for arguments in (first, first, second):
+        compiled(**arguments)
+    assert compiled._program is None and len(runs) == 3 and runs[0] is runs[1]
+    for launches, arguments in zip(runs[1:], (first, second)):
+        args = {item[2]: item[3] for item in launches}
+        assert sorted(args) == ["mi355x_launch_empty_kernel", "mi355x_pack_f32", "mi355x_reduce_f32"]
+        w, packed, largest = (arguments[k].data_ptr() for k in ("w", "packed", "largest"))
+        assert args["mi355x_pack_f32"][:2] == [w, packed] and args["mi355x_reduce_f32"][1:3] == [w, largest]
+
+
+@pytest.mark.gpu
+def test_functions_that_are_no_part_of_a_program_run():
+    compiled = packing_sdfg().compile()
+    for _ in range(2):
+        w = torch.randn(40, 64, device="cuda")
+        packed, largest = torch.zeros(2, 2, 2, 3, 64, 4, dtype=torch.int32, device="cuda"), torch.zeros(40, device="cuda")
+        compiled(w=w, packed=packed, largest=largest)
+        parts = packed.cpu().view(torch.bfloat16).reshape(2, 2, 2, 3, 2, 32, 2, 4).double().sum(3)   # block, step, s, h, row, a, e
+        assert torch.equal(parts.permute(0, 4, 1, 5, 2, 3, 6).reshape(64, 64)[:40] / 65536, w.cpu().double())
+        assert torch.equal(largest.cpu(), w.cpu().amax(1))
