@@ -351,7 +351,7 @@ __global__ __launch_bounds__(256) void attention_f32_blocks_kernel(AttnArgs p) {
 //   * O^T = V^T P^T takes the probabilities from the registers that they are in, split there; V is read a column per lane, so that the
 //     eight keys of a unit, in the order in which the scores lie, become one LDS write.
 //   * Query rows are the columns of O^T: their factors exp(old maximum - new maximum) are the lane's own.
-// Sums that are not finite (infinities, NaN, values past 2^112) send the workgroup through the fp32 kernel above.
+// Sums that are not finite (infinities, NaN, values past 2^112, scores past 2^96) send the workgroup through the fp32 kernel above.
 // What bounds it: a wave's chain of 6 us a block, half of it MFMAs and half splits and exponentials on the vector unit, which the waves of two
 // workgroups on a CU overlap to 3.4; 254 registers leave no room for a third. Against the kernels above, with a mask: 16 x 12 slices of
 // 512 x 512 135 -> 87 us, 32 x 12 of 256 73 -> 48, 20 x 12 of 200 50 -> 31, 32 x 12 of 64 15.1 -> 10.4; without: 121 -> 87, 65 -> 48, 44 -> 30,
@@ -398,6 +398,7 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(AttnArgs p) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) out[db][r] = 0.f;
     float m_run = -INFINITY, l_run = 0.f;
+    bool infinite = false;   // a product of Q and K, of any lane of the wave
     const float scale = p.scale * SP_UNSCALE;
     constexpr float LOG2E = 1.44269504088896340736f;
 
@@ -478,7 +479,12 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(AttnArgs p) {
         __builtin_amdgcn_sched_barrier(0);
         load(key0 + AS_KEYS);   // in flight under the rest of the block
         __builtin_amdgcn_sched_barrier(0);
-        float m_blk = -INFINITY;
+        float m_blk = -INFINITY, largest = 0.f;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) largest = fmaxf(largest, fabsf(s[kb][r]));
+        infinite |= __any(largest == INFINITY) != 0;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -542,14 +548,14 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(AttnArgs p) {
             for (int r = 0; r < 16; ++r) out[db][r] = fmaf(out[db][r], alpha, sum[r] + small[r]);
         }
     }
-    // A score that is NaN or positive infinity makes the probabilities NaN and the sums with them; with all of them negative infinity the
-    // probabilities sum to 0.
+    // A score that is NaN or positive infinity makes the probabilities NaN and the sums with them. One that the split form made negative
+    // infinity would pass for a masked one. With all scores of a row masked that way 0 / 0 is the NaN that the fp32 kernel has there.
     float probe = 0.f;   // stays 0 while all sums are finite
 #pragma unroll
     for (int db = 0; db < 2; ++db)
 #pragma unroll
         for (int r = 0; r < 16; ++r) probe = fmaf(out[db][r], 0.f, probe);
-    if (__syncthreads_or(probe != 0.f || !(l_run > 0.f))) {   // (NaN compares unequal)
+    if (__syncthreads_or(probe != 0.f || infinite)) {   // (NaN compares unequal)
         for (int half = 0; half < AS_ROWS / AT_BQ; ++half) {
             __syncthreads();
             attention_blocks<MASKED>(p, slice, qb * (AS_ROWS / AT_BQ) + half, reinterpret_cast<float*>(lds), reinterpret_cast<float*>(lds) + AT_SK * AT_PITCH);

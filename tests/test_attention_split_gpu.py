@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from dace_onnx_amd import _lib
+from dace_onnx_amd.testing.profiling import graph_time_us
 
 pytestmark = pytest.mark.gpu
 
@@ -80,3 +81,33 @@ def test_split_attention_keeps_infinities_nan_and_the_largest_values(tuning, mas
         assert torch.equal(torch.isnan(results[0]), torch.isnan(results[1])) and torch.equal(torch.isinf(results[0]), torch.isinf(results[1]))
         fine = torch.isfinite(results[0])
         assert bool(((results[0] - results[1]).abs()[fine] <= 1e-5 * results[0].abs()[fine].clamp(min=1)).all())
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("scale", [0.125, -0.125])
+def test_split_attention_of_scores_that_only_the_split_form_cannot_hold(tuning, masked, scale):
+    """A score of 0 whose largest product is -1.5 x 2^96, past what sums of scaled values hold: the fp32 kernel's result, not a masked key."""
+    tuning(MI355X_ATTN_SPLIT=1)
+    q, k, v = inputs(2, 2, 150, 100)
+    mask = torch.zeros(1, 1, 1, 100, device="cuda") if masked else None
+    q[1, 0, 70, 0], q[1, 0, 70, 16:49:16] = 1.5 * 2.0**49, 2.0**48
+    k[..., 0::16], k[1, 0, 9] = 0, 0
+    k[1, 0, 9, 0], k[1, 0, 9, 16:49:16] = -2.0**47, 2.0**47
+    expected = torch.softmax(scale * (q.double() @ k.double().transpose(-1, -2).contiguous()), -1) @ v.double()
+    got = attention(q, k, v, mask, scale)
+    assert float((expected[1, 0, 70] - got[1, 0, 70].double()).norm() / expected[1, 0, 70].norm()) < 1e-6
+    assert float((expected - got.double()).norm() / expected.norm()) < 1e-6
+
+
+def test_sentences_without_a_valid_key_take_no_longer():
+    """Their rows are 0 / 0: nothing to compute again (twice the time and more where the fp32 kernel runs after)."""
+    q, k, v = inputs(32, 12, 64, 64)
+    mask, out = torch.zeros(32, 1, 1, 64, device="cuda"), torch.empty_like(q)
+    strides = lambda t: _lib.i64_array(t.stride()[:3])   # noqa: E731
+    launch = lambda: _lib.library().mi355x_attention_masked_f32(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), mask.data_ptr(), 32, 12, 64, 64, 64,   # noqa: E731
+                                                                strides(q), strides(k), strides(v), strides(out), _lib.i64_array([64, 0, 0]), 0.125, _lib.current_stream())
+    before = graph_time_us(launch)
+    mask[::2] = -float("inf")
+    assert graph_time_us(launch) < 1.5 * before
+    torch.cuda.synchronize()
+    assert bool(torch.isnan(out[::2]).all()) and bool(torch.isfinite(out[1::2]).all())
