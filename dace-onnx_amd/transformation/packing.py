@@ -20,15 +20,15 @@ class PackedOperand:
     """The packed copy ``array`` of a weight, ``shape`` 32-bit words, written by the library's ``function`` from ``offset`` values on.
 
     The launches that multiply by it get the weight's address too, and read the weight itself where the copy is left out. It is made at
-    once of a weight that only the model holds (``onnx/weights.py``), and of others on request.
+    once (``now``) of a weight that only the model holds (``onnx/weights.py``), and of others on request.
     """
 
-    def __init__(self, model, weight_name, descriptor, array, shape, function, geometry, offset):
+    def __init__(self, model, weight_name, descriptor, now, array, shape, function, geometry, offset):
         self.weights, self.weight_name, self.descriptor, self.array = model.weights, weight_name, descriptor, array
         self.shape, self.function, self.geometry, self.offset = shape, function, geometry, offset
         self.derived = model.weights.derived(weight_name)
         self.device, self.weight, self.version, self.packed, self.declared = model.device, None, None, None, False
-        if model.weights.private(weight_name):
+        if now and model.weights.private(weight_name):
             self.pack()
 
     def pack(self, declared=False):
@@ -108,11 +108,14 @@ _PACKED = {"mi355x_gemm_f32": _packed_gemm, "mi355x_conv2d_f32": _packed_conv, "
 
 def pack_constant_operands(model):
     """Give every GEMM and convolution of ``model``'s expanded graph that multiplies by a constant, and for which the library says that
-    it pays, a packed copy of it. Returns the copies."""
+    it pays, a packed copy of it. Returns the copies.
+
+    Under a caller's stream capture none is made: its launches are recorded, not run, and the weights that fusion derives hold nothing yet.
+    """
     from ..onnx.onnx_importer import clean_onnx_name
     sdfg = model.sdfg
     by_clean = {clean_onnx_name(k): k for k in model.weights}
-    copies = []
+    copies, now = [], not model._capturing()
     for state in sdfg.nodes():
         written = {e.dst.data for e in state.edges() if isinstance(e.dst, AccessNode)}
         for call in state.nodes():
@@ -132,13 +135,13 @@ def pack_constant_operands(model):
             name = f"{weight_name}_packed_{suffix}"
             clean = clean_onnx_name(name)
             if clean not in sdfg.arrays:
-                copies.append(PackedOperand(model, weight_name, desc, clean, *copy))
+                copies.append(PackedOperand(model, weight_name, desc, now, clean, *copy))
                 sdfg.add_datadesc(clean, PackedCopy(int32, copies[-1].shape, copies[-1].derived))
-                if copies[-1].derived:
+                if copies[-1].derived and copies[-1].packed is not None:
                     model.weights.make(name, copies[-1].packed, derived=True)
             packed_call = KernelCall(call.label, function, args, list(call.in_connectors) + ["_packed"], list(call.out_connectors))
             state.replace_node(call, packed_call, sdfg)
             state.add_edge(state.add_access(clean), None, packed_call, "_packed", sdfg.make_array_memlet(clean))
-    if copies:
+    if copies and now:
         torch.cuda.current_stream().synchronize()   # later calls may come on other streams
     return copies

@@ -238,3 +238,15 @@ def test_a_callers_recordings_follow_weights_that_are_written_after_them():
         weight.data.mul_(0.5)
         compiled.replay()
         assert close(y, x, weight)
+
+
+def test_a_first_call_under_stream_capture():
+    model, x = head()
+    graph, weight = torch.cuda.CUDAGraph(), dict.get(model.weights, "w")
+    with torch.cuda.graph(graph):
+        y = model(x)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        assert close(y, x, weight)
+    assert close(model(x), x, weight)

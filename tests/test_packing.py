@@ -236,3 +236,16 @@ def test_a_callers_recording_reads_the_weights_themselves(pack_launches, program
     monkeypatch.setattr(model, "_capturing", lambda: True)
     model(HEAD_X)
     assert _operands(model) == [(0, model._packed[0].weight.data_ptr())]
+
+
+@pytest.mark.parametrize("build", [_encoder, _head])
+def test_a_first_call_under_stream_capture_packs_nothing_and_waits_for_nothing(pack_launches, monkeypatch, build):
+    """A packing launch would be recorded instead of run, and a wait ends the capture: the launches read the weights themselves."""
+    model = build()
+    model.expand()
+    weights = list(model.weights.peek_items())
+    monkeypatch.setattr(model, "_capturing", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: pytest.fail("waits for a stream that is being captured"))
+    copies = packing.pack_constant_operands(model)
+    assert copies and not pack_launches and not any(c.current() for c in copies)
+    assert [(n, id(t)) for n, t in model.weights.peek_items()] == [(n, id(t)) for n, t in weights]
