@@ -178,15 +178,32 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * WAVES_K * WAVE, PER_SIMD) void 
         multiply(second, next);
     }
 
-    // The sums of a block computed again with the fp32 MFMA, straight from global memory: for inputs that the split form cannot hold.
-    auto again = [&](int64_t bm, int64_t bn) __attribute__((always_inline)) {
+    // The sums of a block over steps `from` to `to` computed again with the fp32 MFMA, straight from global memory: for inputs that the
+    // split form cannot hold. Only blocks that are not finite, with 32 k of loads in flight: bound by the fp32 MFMA. One row of NaN:
+    // 128 x 768 x 3072 235 -> 42 us (20 without, the kernel before 21), 1024 x 768 x 3072 379 -> 82 (38, 39), 8192 x 768 x 3072 1470 -> 321
+    // (186, the split kernel before 650).
+    auto again = [&](int64_t bm, int64_t bn, int from, int to) __attribute__((always_inline)) {
         f32x16 sum;
 #pragma unroll
         for (int r = 0; r < 16; ++r) sum[r] = 0.f;
         const int64_t m = bm + li, n = bn + li;
-        const float* ap = A + (m < p.M ? m : p.M - 1) * p.a_sm + lh;
-        const float* bp = p.B + (n < p.N ? n : p.N - 1) * p.b_sn + lh * p.b_sk;
-        for (int64_t k = 0; k < p.K; k += 2) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(ap[k], bp[k * p.b_sk], sum, 0, 0, 0);
+        const float* ap = A + (m < p.M ? m : p.M - 1) * p.a_sm + 16 * lh;
+        const float* bp = p.B + (n < p.N ? n : p.N - 1) * p.b_sn + 16 * lh * p.b_sk;
+        for (int st = from; st < to; ++st) {
+            typedef f32x4 unaligned __attribute__((aligned(4)));
+            f32x4 va[4], vb[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) va[c] = *reinterpret_cast<const f32x4*>(ap + 32 * st + 4 * c);
+            if (p.b_sk == 1) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) vb[c] = *reinterpret_cast<const unaligned*>(bp + 32 * st + 4 * c);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) vb[e / 4][e % 4] = bp[(32 * st + e) * p.b_sk];
+            }
+#pragma unroll
+            for (int e = 0; e < 16; ++e) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(va[e / 4][e % 4], vb[e / 4][e % 4], sum, 0, 0, 0);
+        }
         return sum;
     };
 
@@ -245,7 +262,12 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * WAVES_K * WAVE, PER_SIMD) void 
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) acc[i][j] = again(m0 + 32 * (wm * TM + i), n0 + 32 * (wn * TN + j));
+                for (int j = 0; j < TN; ++j) {
+                    float block = 0.f;
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) block = fmaf(acc[i][j][r], 0.f, block);
+                    if (__any(block != 0.f)) acc[i][j] = again(m0 + 32 * (wm * TM + i), n0 + 32 * (wn * TN + j), 0, pa.kt);
+                }
         }
         with_epilogue([&](auto act, auto res) __attribute__((always_inline)) {
 #pragma unroll
@@ -291,16 +313,27 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * WAVES_K * WAVE, PER_SIMD) void 
 #pragma unroll
             for (int r = 0; r < 4; ++r) probe = fmaf(sum[it][r], 0.f, probe);
         }
-        if (__syncthreads_or(probe != 0.f)) {
-            for (int block = wave; block < BLOCKS; block += WAVES) {
-                const f32x16 v = again(m0 + 32 * (block / (TN * WAVES_N)), n0 + 32 * (block % (TN * WAVES_N)));
+        if (__syncthreads_or(probe != 0.f))
+            for (int block = 0; block < BLOCKS; ++block) {   // each by all waves, a share of K each
+                float of_block = 0.f;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) sums[(block * 4 + q) * WAVE + lane] = f32x4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+                for (int it = 0; it < PER; ++it)
+                    if (min(it * THREADS + tid, QUADS - 1) / 256 == block)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) of_block = fmaf(sum[it][r], 0.f, of_block);
+                if (!__syncthreads_or(of_block != 0.f)) continue;   // (everyone has read the sums before)
+                const f32x16 v = again(m0 + 32 * (block / (TN * WAVES_N)), n0 + 32 * (block % (TN * WAVES_N)), pa.kt * wave / WAVES, pa.kt * (wave + 1) / WAVES);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) sums[(wave * 4 + q) * WAVE + lane] = f32x4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+                __syncthreads();
+#pragma unroll
+                for (int it = 0; it < PER; ++it) {
+                    const int u = min(it * THREADS + tid, QUADS - 1);
+                    if (u / 256 != block) continue;
+                    sum[it] = sums[u % 256];
+                    for (int w = 1; w < WAVES; ++w) sum[it] += sums[w * 256 + u % 256];
+                }
             }
-            __syncthreads();
-#pragma unroll
-            for (int it = 0; it < PER; ++it) sum[it] = sums[min(it * THREADS + tid, QUADS - 1)];
-        }
         with_epilogue([&](auto act, auto res) __attribute__((always_inline)) {
 #pragma unroll
             for (int it = 0; it < PER; ++it) {
