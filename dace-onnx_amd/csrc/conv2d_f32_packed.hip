@@ -246,62 +246,107 @@ __global__ __launch_bounds__(WAVES_M * WAVES_P * WAVES_K * WAVE, 2) void conv2d_
         if (WAVES_K > 1 && !late) sync();   // as many barriers for every wave
     }
 
-    // the sums of the groups, in order
+    // the sums of the groups, in order, into those of the first
+    auto add_groups = [&]() __attribute__((always_inline)) {
+        if constexpr (WAVES_K > 1) {
+            constexpr int WAVES_1 = WAVES_M * WAVES_P;
+            f32x4* sums = reinterpret_cast<f32x4*>(lds);
+            __syncthreads();
+            if (wk > 0)
+#pragma unroll
+                for (int j = 0; j < TP; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        sums[(((wave - WAVES_1) * TP + j) * 4 + q) * WAVE + lane] =
+                            f32x4{acc[j][4 * q], acc[j][4 * q + 1], acc[j][4 * q + 2], acc[j][4 * q + 3]};
+            __syncthreads();
+            if (wk == 0)
+#pragma unroll
+                for (int g = 0; g < WAVES_K - 1; ++g)
+#pragma unroll
+                    for (int j = 0; j < TP; ++j)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const f32x4 s = sums[(((g * WAVES_1 + wave) * TP + j) * 4 + q) * WAVE + lane];
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) acc[j][4 * q + e] += s[e];
+                        }
+        }
+    };
 #pragma unroll
     for (int j = 0; j < TP; ++j) acc[j] = (acc[j] + small[j]) * SP_UNSCALE;
-    if constexpr (WAVES_K > 1) {
-        constexpr int WAVES_1 = WAVES_M * WAVES_P;
-        f32x16* sums = reinterpret_cast<f32x16*>(lds);
-        __syncthreads();
-        if (wk > 0)
-#pragma unroll
-            for (int j = 0; j < TP; ++j)
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    reinterpret_cast<f32x4*>(lds)[(((wave - WAVES_1) * TP + j) * 4 + q) * WAVE + lane] =
-                        f32x4{acc[j][4 * q], acc[j][4 * q + 1], acc[j][4 * q + 2], acc[j][4 * q + 3]};
-        __syncthreads();
-        if (wk > 0) return;
-#pragma unroll
-        for (int g = 0; g < WAVES_K - 1; ++g)
-#pragma unroll
-            for (int j = 0; j < TP; ++j)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const f32x4 s = reinterpret_cast<const f32x4*>(sums)[(((g * WAVES_1 + wave) * TP + j) * 4 + q) * WAVE + lane];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[j][4 * q + e] += s[e];
-                }
-    }
+    add_groups();
     float probe = 0.f;   // stays 0 while every sum is finite
 #pragma unroll
     for (int j = 0; j < TP; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) probe = fmaf(acc[j][r], 0.f, probe);
     const int mb = m0 + 32 * wm;
-    if (__any(probe != 0.f)) {   // (NaN compares unequal) again with the fp32 MFMA, straight from memory: inputs that the split cannot hold
+    // (NaN compares unequal) Again with the fp32 MFMA, straight from memory: inputs that the split cannot hold. Of a wave's own blocks
+    // only those that are not finite; with several groups the whole tile, each over its share of the channels. One pixel of NaN: 32 x 128 x 28 x 28 -> 128 606 -> 156 us (44
+    // without, the kernel before 71), 32 x 512 x 7 x 7 -> 512 1319 -> 186 (48, 80), 1 x 512 x 7 x 7 601 -> 54 (17, 22).
+    if (WAVES_K > 1 ? __syncthreads_or(wk == 0 && probe != 0.f) : __any(probe != 0.f)) {
 #pragma unroll
         for (int j = 0; j < TP; ++j) {
+            float block = 0.f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) block = fmaf(acc[j][r], 0.f, block);
+            if (WAVES_K == 1 && !__any(block != 0.f)) continue;
             const int pp = min(p0 + 32 * (wp * TP + j) + li, (int)p.P - 1);
             uint32_t n, oy, ox;
             output_of(pp, n, oy, ox);
             const int y0 = (int)oy * p.stride_h - p.pad_t, x0 = (int)ox * p.stride_w - p.pad_l;
-            const float* w = p.W + (int64_t)min(mb + li, p.M - 1) * p.K;
+            const int m = min(mb + li, p.M - 1);
             f32x16 sum;
 #pragma unroll
             for (int r = 0; r < 16; ++r) sum[r] = 0.f;
-            for (int k = 0; k < p.K; k += 2) {
-                const int kk = min(k + lh, p.K - 1);
-                const uint32_t c = fdiv((uint32_t)kk, p.div_khw), t = (uint32_t)kk - c * (uint32_t)(p.KH * p.KW), ty = fdiv(t, p.div_kw);
-                const int y = y0 + (int)ty * p.dil_h, x = x0 + (int)(t - ty * (uint32_t)p.KW) * p.dil_w;
-                const bool in = (unsigned)y < (unsigned)p.H && (unsigned)x < (unsigned)p.Wd;
-                const float xv = in ? p.X[(((int64_t)n * p.C + c) * p.H + y) * p.Wd + x] : 0.f;
-                const bool counted = k + lh < p.K;
-                sum = __builtin_amdgcn_mfma_f32_32x32x2f32(counted ? w[kk] : 0.f, counted ? xv : 0.f, sum, 0, 0, 0);
+            if constexpr (PIXELS) {
+                const float* w = p.W + (int64_t)m * p.K;
+                for (int k = 0; k < p.K; k += 2) {
+                    const int kk = min(k + lh, p.K - 1);
+                    const uint32_t c = fdiv((uint32_t)kk, p.div_khw), t = (uint32_t)kk - c * (uint32_t)(p.KH * p.KW), ty = fdiv(t, p.div_kw);
+                    const int y = y0 + (int)ty * p.dil_h, x = x0 + (int)(t - ty * (uint32_t)p.KW) * p.dil_w;
+                    const bool in = (unsigned)y < (unsigned)p.H && (unsigned)x < (unsigned)p.Wd;
+                    const float xv = in ? p.X[(((int64_t)n * p.C + c) * p.H + y) * p.Wd + x] : 0.f;
+                    const bool counted = k + lh < p.K;
+                    sum = __builtin_amdgcn_mfma_f32_32x32x2f32(counted ? w[kk] : 0.f, counted ? xv : 0.f, sum, 0, 0, 0);
+                }
+            } else {
+                // All taps of CHANNELS channels at once, the upper lanes' CHANNELS further on: they are contiguous in a filter, and C is a
+                // multiple of eight. (Filters span less than 2^31 bytes: their packed copy does.)
+                constexpr int TAPS = FILTER::STEPS, CHANNELS = TAPS == 1 ? 16 : 4;
+                const __amdgpu_buffer_rsrc_t f_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.W), 0, 0x7fffffff, 0x00020000);
+                const uint32_t w_first = 4u * (uint32_t)(m * p.K + lh * CHANNELS * TAPS);
+                uint32_t x_first[TAPS];
+#pragma unroll
+                for (int t = 0; t < TAPS; ++t) {
+                    const int y = y0 + t / FILTER::PER_ROW * p.dil_h, x = x0 + t % FILTER::PER_ROW * p.dil_w;
+                    const bool in = (unsigned)y < (unsigned)p.H && (unsigned)x < (unsigned)p.Wd;
+                    x_first[t] = in ? 4u * (uint32_t)(((int)n * p.C * p.H + y) * p.Wd + x) + (uint32_t)(lh * CHANNELS) * (uint32_t)plane : OUT;
+                }
+                for (int c = 2 * CHANNELS * wk; c < p.C; c += 2 * CHANNELS * WAVES_K) {
+                    f32x4 wv[CHANNELS * TAPS / 4];
+                    float xv[CHANNELS * TAPS];
+#pragma unroll
+                    for (int g = 0; g < CHANNELS * TAPS / 4; ++g) {
+                        const bool counted = c + lh * CHANNELS + 4 * g / TAPS / 4 * 4 < p.C;
+                        wv[g] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(f_rsrc, (int)(counted ? w_first : OUT), (c * TAPS + 4 * g) * 4, 0));
+                    }
+#pragma unroll
+                    for (int i = 0; i < CHANNELS * TAPS; ++i) {
+                        const int e = i / TAPS;
+                        const bool counted = c + lh * CHANNELS + e / 4 * 4 < p.C;
+                        xv[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(x_rsrc, (int)(counted ? x_first[i % TAPS] : OUT), min(c + e, p.C - 1) * plane, 0));
+                    }
+#pragma unroll
+                    for (int i = 0; i < CHANNELS * TAPS; ++i) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[i / 4][i % 4], xv[i], sum, 0, 0, 0);
+                }
             }
             acc[j] = sum;
         }
+        add_groups();
     }
+    if (wk > 0) return;
 
     // acc[j][r]: filter 8 (r / 4) + 4 lh + r % 4 of the block, position li
     const __amdgpu_buffer_rsrc_t y_rsrc = __builtin_amdgcn_make_buffer_rsrc(p.Y, 0, 0x7fffffff, 0x00020000);
