@@ -35,7 +35,6 @@ from .weights import Weights
 log = logging.getLogger(__name__)
 
 
-@functools.lru_cache(maxsize=4096)
 @functools.lru_cache(maxsize=1 << 16)
 def clean_onnx_name(name: str) -> str:
     """Make an ONNX value name a valid array name (``daceml/onnx/converters.py:204-211``)."""

@@ -249,3 +249,13 @@ def test_a_first_call_under_stream_capture_packs_nothing_and_waits_for_nothing(p
     copies = packing.pack_constant_operands(model)
     assert copies and not pack_launches and not any(c.current() for c in copies)
     assert [(n, id(t)) for n, t in model.weights.peek_items()] == [(n, id(t)) for n, t in weights]
+
+
+def test_names_of_arrays_are_kept_once():
+    from dace_onnx_amd.onnx.onnx_importer import clean_onnx_name
+    assert not hasattr(clean_onnx_name.__wrapped__, "cache_info")
+    names = [f"{i}.a/b:c-d" for i in range(5000)]   # more than one large graph has
+    cleaned = [clean_onnx_name(n) for n in names]
+    misses = clean_onnx_name.cache_info().misses
+    assert [clean_onnx_name(n) for n in names] == cleaned and clean_onnx_name.cache_info().misses == misses
+    assert cleaned[7] == "ONNX_7DOTaSLASHbCOLONcDASHd"
