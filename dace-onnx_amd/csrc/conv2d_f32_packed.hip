@@ -580,7 +580,7 @@ static double unpacked_conv_cost(const ConvArgs& p, int cus, bool& summed_apart)
 // the gather kernel's estimate is up to a third too long for 1 x 1 filters, most for few of them). A form whose waves all sum the
 // same channels does not take over from the kernel that sums them apart: its error was up to 1.3 times as large there, everywhere else and
 // of the other forms it is 0.2 to 0.9 of the kernels' before.
-static int choose_packed_conv(PackedConvArgs& pa, int kind, int cus, double besides = 0) {
+static int choose_packed_conv(PackedConvArgs& pa, int kind, int cus, double besides) {
     const ConvArgs& p = pa.c;
     bool summed_apart;
     double best_cost = (kind != PC_1X1 ? 0.9 : p.M > 64 ? 0.85 : 0.7) * unpacked_conv_cost(p, cus, summed_apart) - besides;
@@ -605,6 +605,16 @@ static int choose_packed_conv(PackedConvArgs& pa, int kind, int cus, double besi
     return best;
 }
 
+// The form that takes a call, -1 where mi355x_conv2d_res_f32 does: the fastest, or the one that is forced (MI355X_CONV_PACKED) if its
+// patch fits. With its strips, its patch's pixels and its LDS.
+static int packed_conv_form(PackedConvArgs& pa, int kind, int cus, double besides, int& strip_w, int64_t& pixels, int& lds) {
+    const int force = tuning().conv_packed, form = force >= 0 ? force - 1 : choose_packed_conv(pa, kind, cus, besides);
+    if (form < 0 || form >= kNumPackedConvForms) return -1;
+    pixels = choose_strips(pa, kind, kPackedConvForms[form].bp, strip_w);
+    lds = packed_conv_lds(kind, kPackedConvForms[form], pixels);
+    return lds > 0 ? form : -1;
+}
+
 // Nanoseconds of mi355x_pack_conv_f32 before the convolution (512 x 256 filters of one tap 3.8 us, 768 x 512 of nine 16.5).
 constexpr double PACKING = 3000, PACKING_PER_WEIGHT = 0.004;
 
@@ -618,7 +628,9 @@ extern "C" int64_t mi355x_conv2d_packed_pays(int64_t N, int64_t C, int64_t H, in
     if (!pads || !strides || !dilations || !packed_conv_args(pa, kind, N, C, H, Wd, M, KH, KW, pads, strides, dilations)) return 0;
     const int cus = device_cus();
     const double packing = constant ? 0 : PACKING + PACKING_PER_WEIGHT * (double)M * pa.c.K;
-    if (choose_packed_conv(pa, kind, cus > 0 ? cus : 256, packing) < 0) return 0;
+    int strip_w, lds;
+    int64_t pixels;
+    if (packed_conv_form(pa, kind, cus > 0 ? cus : 256, packing, strip_w, pixels, lds) < 0) return 0;
     return ceil_div(M, (int64_t)32) * pa.groups * packed_conv_steps(kind) * PK_FRAGMENT;
 }
 
@@ -640,8 +652,7 @@ extern "C" int mi355x_conv2d_packed_f32(const float* X, const void* packed, cons
                                         float* Y, int64_t N, int64_t C, int64_t H, int64_t Wd, int64_t M, int64_t KH, int64_t KW,
                                         const int64_t* pads, const int64_t* strides, const int64_t* dilations, int epilogue, void* stream) {
     using namespace mi355x;
-    const int force = tuning().conv_packed;
-    if (X && W && Y && packed && pads && strides && dilations && force != 0 && (reinterpret_cast<uintptr_t>(packed) & 15) == 0 &&
+    if (X && W && Y && packed && pads && strides && dilations && (reinterpret_cast<uintptr_t>(packed) & 15) == 0 &&
         (epilogue & ~(MI355X_EPI_BIAS | MI355X_EPI_RELU | MI355X_EPI_RESIDUAL | MI355X_EPI_RELU_AFTER)) == 0 &&
         (!(epilogue & MI355X_EPI_BIAS) || bias) && (!(epilogue & MI355X_EPI_RESIDUAL) || residual)) {
         PackedConvArgs pa = {};
@@ -650,12 +661,11 @@ extern "C" int mi355x_conv2d_packed_f32(const float* X, const void* packed, cons
         if (packed_conv_args(pa, kind, N, C, H, Wd, M, KH, KW, pads, strides, dilations)) {
             const int cus = device_cus();
             if (cus <= 0) return set_error(MI355X_ERR_NOT_INITIALIZED, "conv2d: no usable HIP device");
-            const int form = force > 0 ? force - 1 : choose_packed_conv(pa, kind, cus);
-            if (form >= 0 && form < kNumPackedConvForms) {
+            int strip_w, lds;
+            int64_t pixels;
+            const int form = packed_conv_form(pa, kind, cus, 0, strip_w, pixels, lds);
+            if (form >= 0) {
                 const PackedConvForm& f = kPackedConvForms[form];
-                int strip_w;
-                const int64_t pixels = choose_strips(pa, kind, f.bp, strip_w);
-                const int lds = packed_conv_lds(kind, f, pixels);
                 p.X = X; p.W = W; p.bias = bias; p.residual = residual; p.Y = Y; p.epi = epilogue;
                 p.tiles_m = ceil_div(M, (int64_t)f.bm);
                 p.tiles_p = ceil_div(p.P, (int64_t)f.bp);
@@ -663,7 +673,7 @@ extern "C" int mi355x_conv2d_packed_f32(const float* X, const void* packed, cons
                 pa.packed = static_cast<const char*>(packed);
                 pa.stages = (int)packed_conv_stages(pa, kind, f);
                 hipStream_t st = static_cast<hipStream_t>(stream);
-                if (lds > 0 && grid_fits(p.nwg, f.waves * WAVE)) {
+                if (grid_fits(p.nwg, f.waves * WAVE)) {
                     set_strips(pa, kind, strip_w, pixels);
                     switch (kind) {
                         case PC_3X3: launch_packed_conv<PackedFilter<3, 3, false>, false, 1, 0>(form, pa, lds, st); break;

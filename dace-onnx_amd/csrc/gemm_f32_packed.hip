@@ -416,8 +416,11 @@ static bool packed_takes(const GemmArgs& p) {
            p.c_sm >= 0 && p.c_sm < ((int64_t)1 << 22) && p.r_sm >= 0 && p.r_sm < ((int64_t)1 << 22);   // (rows of a tile of C, 32-bit byte offsets)
 }
 
-// The fastest form, -1 where mi355x_gemm_f32 is faster.
+// The fastest form, -1 where mi355x_gemm_f32 is faster; or the one that is forced (MI355X_GEMM_PACKED).
 static int choose_packed(const GemmArgs& p, int cus) {
+    const int force = tuning().gemm_packed;
+    if (!packed_takes(p) || force == 0 || force > kNumPackedForms) return -1;
+    if (force > 0) return force - 1;
     double best_cost = unpacked_cost(p, p.b_sk == 1, cus);
     int best = -1;
     for (int f = 0; f < kNumPackedForms; ++f) {
@@ -449,7 +452,7 @@ extern "C" int mi355x_gemm_packed_pays(int64_t batch, int64_t M, int64_t N, int6
     p.batch = batch; p.batch1 = 1; p.M = M; p.N = N; p.K = K;
     p.a_sm = K; p.a_sk = 1; p.b_sk = b_kc ? 1 : N; p.b_sn = b_kc ? K : 1; p.c_sm = N;
     const int cus = device_cus();
-    return packed_takes(p) && choose_packed(p, cus > 0 ? cus : 256) >= 0;
+    return choose_packed(p, cus > 0 ? cus : 256) >= 0;
 }
 
 extern "C" int mi355x_gemm_packed_f32(const float* A, const void* packed, const float* B, float* C, const float* bias,
@@ -459,9 +462,8 @@ extern "C" int mi355x_gemm_packed_f32(const float* A, const void* packed, const 
     using namespace mi355x;
     PackedGemmArgs pa;
     GemmArgs& p = pa.g;
-    const int force = tuning().gemm_packed;
     auto al16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
-    if (A && B && C && packed && a_strides && b_strides && c_strides && batch0 > 0 && batch1 > 0 && M > 0 && N > 0 && K > 0 && force != 0 &&
+    if (A && B && C && packed && a_strides && b_strides && c_strides && batch0 > 0 && batch1 > 0 && M > 0 && N > 0 && K > 0 &&
         (epilogue & ~(MI355X_EPI_BIAS | MI355X_EPI_RELU | MI355X_EPI_GELU | MI355X_EPI_RESIDUAL)) == 0 && (!(epilogue & MI355X_EPI_BIAS) || bias) &&
         (!(epilogue & MI355X_EPI_RESIDUAL) || (residual && r_strides)) && (c_strides[2] >= N || M == 1) && al16(A) && al16(packed)) {
         MI355X_TRACE_INIT(p);
@@ -477,8 +479,8 @@ extern "C" int mi355x_gemm_packed_f32(const float* A, const void* packed, const 
         pa.kt = (int)(K / 32);
         const int cus = device_cus();
         if (cus <= 0) return set_error(MI355X_ERR_NOT_INITIALIZED, "gemm: no usable HIP device");
-        const int form = !packed_takes(p) ? -1 : force > 0 ? force - 1 : choose_packed(p, cus);
-        if (form >= 0 && form < kNumPackedForms) {
+        const int form = choose_packed(p, cus);
+        if (form >= 0) {
             const PackedForm& f = kPackedForms[form];
             p.tiles_m = ceil_div(M, (int64_t)f.bm);
             p.tiles_n = ceil_div(N, (int64_t)f.bn);

@@ -113,7 +113,7 @@ int mi355x_gemm_packed_f32(const float* A, const void* packed, const float* B, f
                            const int64_t* a_strides, const int64_t* b_strides, const int64_t* c_strides,
                            const int64_t* r_strides, float alpha, int epilogue, void* stream);
 /* 1 where mi355x_gemm_packed_f32 takes `batch` products of M x N x K on the packed form (b_kc: B contiguous along k, else
- * along n): what graph preparation asks before it packs. */
+ * along n): what graph preparation asks before it packs. (MI355X_GEMM_PACKED=n: whether its n-th form does.) */
 int mi355x_gemm_packed_pays(int64_t batch, int64_t M, int64_t N, int64_t K, int b_kc);
 /* `rows` x K values (K a multiple of 32; strides in elements) packed, 16-byte aligned: for a [K, N] weight of contiguous rows
  * rows = N, row_stride = 1, k_stride = N. */
@@ -150,7 +150,7 @@ int mi355x_conv2d_res_f32(const float* X, const float* W, const float* bias, con
  * mi355x_conv2d_packed_pays: bytes of the packed copy where the kernel (with the packing, unless constant) is ahead of
  * mi355x_conv2d_f32 for this layer, 0 elsewhere
  * (filters that are neither 3 x 3 nor 1 x 1 over a multiple of eight channels, nor 7 x 7 over at most four, among them).
- * `packed` is 16-byte aligned. */
+ * `packed` is 16-byte aligned. (MI355X_CONV_PACKED=n: where the n-th form takes the layer.) */
 int64_t mi355x_conv2d_packed_pays(int64_t N, int64_t C, int64_t H, int64_t Wd, int64_t M, int64_t KH, int64_t KW,
                                   const int64_t* pads, const int64_t* strides, const int64_t* dilations, int constant);
 int mi355x_pack_conv_f32(const float* w, void* packed, int64_t M, int64_t C, int64_t KH, int64_t KW, void* stream);

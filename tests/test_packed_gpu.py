@@ -34,6 +34,7 @@ def packed_gemm(a, b, kc, bias=None, res=None, epi=0, alpha=1.0, batch=1, c_gap=
     """C = a @ b; ``b`` is [N, K] if ``kc`` else [K, N]; rows of C ``c_gap`` apart, which stays as it was."""
     M, K = a.shape[-2:]
     N = b.shape[0] if kc else b.shape[1]
+    assert _lib.library().mi355x_gemm_packed_pays(batch, M, N, K, int(kc)) == 1   # (a form that does not take it would leave it to the kernels before)
     c = torch.full((batch, M, N + c_gap), -7.0, device="cuda")
     i64 = _lib.i64_array
     call("mi355x_gemm_packed_f32", a.data_ptr(), pack(b, N, K, *((K, 1) if kc else (1, N))).data_ptr(), b.data_ptr(), c.data_ptr(), _lib.ptr(bias),
