@@ -285,7 +285,18 @@ __global__ __launch_bounds__(WAVES_M * WAVES_P * WAVES_K * WAVE, 2) void conv2d_
     // (NaN compares unequal) Again with the fp32 MFMA, straight from memory: inputs that the split cannot hold. Of a wave's own blocks
     // only those that are not finite; with several groups the whole tile, each over its share of the channels. One pixel of NaN: 32 x 128 x 28 x 28 -> 128 606 -> 156 us (44
     // without, the kernel before 71), 32 x 512 x 7 x 7 -> 512 1319 -> 186 (48, 80), 1 x 512 x 7 x 7 601 -> 54 (17, 22).
-    if (WAVES_K > 1 ? __syncthreads_or(wk == 0 && probe != 0.f) : __any(probe != 0.f)) {
+    bool finite = !__any(probe != 0.f);
+    if constexpr (WAVES_K > 1) {
+        constexpr int PER_WAVE = TP * 4 * WAVE;   // a wave's sums of a group, which it has read: room for its word to all groups
+        uint32_t* said = reinterpret_cast<uint32_t*>(lds);
+        if (wk == 0) said[wave * PER_WAVE * 4] = finite;
+        __syncthreads();
+        uint32_t all = 1;
+#pragma unroll
+        for (int w = 0; w < WAVES_M * WAVES_P; ++w) all &= said[w * PER_WAVE * 4];
+        finite = __builtin_amdgcn_readfirstlane(all);
+    }
+    if (__builtin_expect(!finite, 0)) {
 #pragma unroll
         for (int j = 0; j < TP; ++j) {
             float block = 0.f;
