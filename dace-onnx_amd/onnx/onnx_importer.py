@@ -208,6 +208,7 @@ class ONNXModel:
                     self.state.add_edge(op_node, conn_name, access, None, memlet)
 
         self._compiled = None
+        self._array_names = ([], [])   # names of the weights, and of their arrays
         self._packed = []   # packed copies of constant operands (transformation/packing.py)
         self._expanded = False
         self._static_io = None         # use_hip_graph: inputs, outputs and weights that the recording is bound to
@@ -335,7 +336,11 @@ class ONNXModel:
 
     def _own_weights(self):
         """As :attr:`clean_weights`, for one call."""
-        return {clean_onnx_name(k): v for k, v in self.weights.peek_items()}
+        names, arrays = self._array_names
+        present = self.weights.peek_names()
+        if names != present:
+            names, arrays = self._array_names = present, [clean_onnx_name(n) for n in present]
+        return dict(zip(arrays, self.weights.peek_values()))
 
     def weight_of(self, array):
         """The weight behind the array of that name, None if there is none; read it only."""
@@ -397,6 +402,14 @@ class ONNXModel:
     def _capturing(self):
         return self.device.type == "cuda" and torch.cuda.is_current_stream_capturing()
 
+    def _packed_now(self):
+        """Which packed copies a call uses."""
+        packed = [c.current() for c in self._packed]
+        if not self.use_hip_graph and any(use and not c.derived for c, use in zip(self._packed, packed)) and self._capturing():
+            # the caller's recording: its replays follow weights that are written after it
+            packed = [use and c.derived for c, use in zip(self._packed, packed)]
+        return packed
+
     def _weight_args(self, weights, packed):
         """``weights`` (by array name) as arguments of the compiled graph, each packed copy among them if ``packed`` says so, left out if not."""
         for c, use in zip(self._packed, packed):
@@ -440,10 +453,7 @@ class ONNXModel:
                 v = torch.from_numpy(np.ascontiguousarray(np.asarray(v, dtype=desc.dtype.np_dtype))).to(self.device)
             call[clean_onnx_name(n)] = v
         outputs = collections.OrderedDict()
-        packed = [c.current() for c in self._packed]
-        if not self.use_hip_graph and any(use and not c.derived for c, use in zip(self._packed, packed)) and self._capturing():
-            # the caller's recording: its replays follow weights that are written after it
-            packed = [use and c.derived for c, use in zip(self._packed, packed)]
+        packed = self._packed_now() if self._packed else []
         if self.use_hip_graph:
             if self._static_io is None:
                 # private input/output buffers: the graph is bound to their addresses

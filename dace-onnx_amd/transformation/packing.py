@@ -11,11 +11,6 @@ from .. import _lib
 from ..sdfg import AccessNode, KernelCall, PackedCopy, Ptr, Stream, int32
 
 
-def _version(tensor):
-    """How often ``tensor`` was written in place, as far as torch counts it; tensors made under ``torch.inference_mode`` have no such count."""
-    return None if tensor.is_inference() else tensor._version
-
-
 class PackedOperand:
     """The packed copy ``array`` of a weight, ``shape`` 32-bit words, written by the library's ``function`` from ``offset`` values on.
 
@@ -37,7 +32,9 @@ class PackedOperand:
         if not isinstance(weight, torch.Tensor) or weight.dtype != torch.float32 or tuple(weight.shape) != self.descriptor.shape \
                 or not weight.is_contiguous() or weight.device != self.device:
             return
-        self.weight, self.version, self.declared = weight, _version(weight), declared
+        self.weight, self.declared = weight, declared
+        # how often it was written in place, as far as torch counts it; tensors made under torch.inference_mode have no such count
+        self.version = None if weight.is_inference() else weight._version
         if self.packed is None:
             self.packed = torch.empty(self.shape, dtype=torch.int32, device=self.device)
         start = weight.data_ptr() + 4 * self.offset
@@ -46,8 +43,8 @@ class PackedOperand:
     def current(self):
         """Whether the model's weight is still the tensor that was packed, and not written since as far as can be told."""
         weight = self.weight
-        return weight is not None and self.weights.peek(self.weight_name) is weight and _version(weight) == self.version \
-            and (self.declared or self.weights.private(self.weight_name))
+        return weight is not None and self.weights.peek(self.weight_name) is weight and (self.version is None or weight._version == self.version) \
+            and (self.derived or self.declared or self.weights.private(self.weight_name))
 
 
 def _packed_gemm(call, desc):

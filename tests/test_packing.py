@@ -243,12 +243,12 @@ def test_a_first_call_under_stream_capture_packs_nothing_and_waits_for_nothing(p
     """A packing launch would be recorded instead of run, and a wait ends the capture: the launches read the weights themselves."""
     model = build()
     model.expand()
-    weights = list(model.weights.peek_items())
+    weights = list(dict.items(model.weights))
     monkeypatch.setattr(model, "_capturing", lambda: True)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: pytest.fail("waits for a stream that is being captured"))
     copies = packing.pack_constant_operands(model)
     assert copies and not pack_launches and not any(c.current() for c in copies)
-    assert [(n, id(t)) for n, t in model.weights.peek_items()] == [(n, id(t)) for n, t in weights]
+    assert [(n, id(t)) for n, t in dict.items(model.weights)] == [(n, id(t)) for n, t in weights]
 
 
 def test_names_of_arrays_are_kept_once():
