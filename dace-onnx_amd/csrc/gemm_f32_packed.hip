@@ -369,7 +369,7 @@ __global__ void pack_f32_kernel(const float* w, u32x4* packed, int64_t rows, int
 
 // Nanoseconds: `fixed` and `per_k` while every workgroup has a CU to itself, `again` and `again_k` for each further one on the same CU
 // (by halves from six on, where they no longer run in step). Fitted over 600 products of M = 8 to 16384, N = 64 to 32000 and
-// K = 64 to 4096; the pick is 1 % behind the fastest form or older kernel on average.
+// K = 64 to 4096.
 struct PackedForm { int bm, bn, threads, resident; double fixed, per_k, again, again_k; };
 static const PackedForm kPackedForms[] = {
     {128, 256, 512, 1, 8440, 56.0, 7580, 64.7}, {64, 256, 256, 2, 5220, 35.8, 3290, 30.8}, {64, 192, 512, 1, 7490, 25.8, 5920, 29.7},
@@ -401,9 +401,11 @@ static double packed_cost(const PackedForm& f, int64_t nwg, int64_t K, int cus) 
 }
 
 // What mi355x_gemm_f32 takes, from the rules of its kernels (with what those leave out because it is the same on both of their sides:
-// a launch, first loads, last stores). Over the same products a median 7 % below what was measured.
+// a launch, first loads, last stores). Over the same products a median 7 % below what was measured; the few-tile kernel's is at times too
+// long, by up to a tenth where weights come from beyond the L2 (1245 x 96 x 1056 9.2 us, packed 10.1): its share below is what keeps
+// those there.
 static double unpacked_cost(const GemmArgs& p, bool b_kc, int cus) {
-    double best = gemm_f32_direct_cost(p, b_kc, cus);
+    double best = 0.91 * gemm_f32_direct_cost(p, b_kc, cus);
     const bool nt = b_kc && p.N % 4 == 0;
     if (nt) best = std::min(best, gemm_f32_nt_cost(p, cus));
     const double split = gemm_f32_split_cost(p, cus);
@@ -419,12 +421,19 @@ static bool packed_takes(const GemmArgs& p) {
            p.c_sm >= 0 && p.c_sm < ((int64_t)1 << 22) && p.r_sm >= 0 && p.r_sm < ((int64_t)1 << 22);   // (rows of a tile of C, 32-bit byte offsets)
 }
 
-// The fastest form, -1 where mi355x_gemm_f32 is faster; or the one that is forced (MI355X_GEMM_PACKED).
+// The fastest form, -1 where mi355x_gemm_f32 is faster; or the one that is forced (MI355X_GEMM_PACKED). Few rows are bound by the weights'
+// way into the CUs, of which the packed copy has half as many bytes again, and the estimates do not know it: with weights from beyond the
+// L2 1 x 20149 x 832 took 14.5 us and packed 19.0, 5 x 20736 x 2432 38.5 and 53.4, 8 x 4576 x 2080 13.4 and 15.7, 20 x 7232 x 2368 17.2 and
+// 20.0. Up to 16 rows (31 products, of which the packed form was ahead in 14, by 3 % on average behind) none is packed, up to 32 those that are
+// well ahead (28 x 13792 x 1280 23.6 -> 19.1). Over 413 products that nothing was fitted to the pick is at most 4 % behind the kernels before
+// and takes 0.88 of their time; against the fastest form it is 2.4 % behind over 187, up to 1.7 times where K is short and tiles are many
+// (5190 x 23059 x 192 282 us packed, 485 as picked: the estimate of the kernels before is low there).
 static int choose_packed(const GemmArgs& p, int cus) {
     const int force = tuning().gemm_packed;
     if (!packed_takes(p) || force == 0 || force > kNumPackedForms) return -1;
     if (force > 0) return force - 1;
-    double best_cost = unpacked_cost(p, p.b_sk == 1, cus);
+    if (p.M <= 16) return -1;
+    double best_cost = (p.M <= 32 ? 0.8 : 1) * unpacked_cost(p, p.b_sk == 1, cus);
     int best = -1;
     for (int f = 0; f < kNumPackedForms; ++f) {
         const PackedForm& form = kPackedForms[f];

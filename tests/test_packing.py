@@ -259,3 +259,15 @@ def test_names_of_arrays_are_kept_once():
     misses = clean_onnx_name.cache_info().misses
     assert [clean_onnx_name(n) for n in names] == cleaned and clean_onnx_name.cache_info().misses == misses
     assert cleaned[7] == "ONNX_7DOTaSLASHbCOLONcDASHd"
+
+
+@pytest.mark.parametrize("M, N, K, kc", [(1, 20149, 832, True), (5, 20736, 2432, True), (8, 4576, 2080, True), (16, 768, 3072, True), (20, 7232, 2368, False),
+                                         (25, 3776, 1568, True), (13, 4650, 800, False), (1245, 96, 1056, True)])
+def test_products_that_the_weights_bytes_bound_are_not_packed(M, N, K, kc):
+    """A packed copy has half as many bytes again: these took 1.07 to 1.39 times as long by it, with weights from beyond the L2."""
+    assert _lib.library().mi355x_gemm_packed_pays(1, M, N, K, int(kc)) == 0
+
+
+@pytest.mark.parametrize("M, N, K", [(128, 768, 3072), (128, 2304, 768), (865, 3072, 768), (1024, 768, 768), (8192, 768, 3072), (28, 13792, 1280)])
+def test_products_of_more_rows_are_packed(M, N, K):
+    assert _lib.library().mi355x_gemm_packed_pays(1, M, N, K, 1) == 1
