@@ -5,6 +5,7 @@ kernels, over a set of shapes.
     python -m dace_onnx_amd.testing.gemm_variants rounds     # 3072-wide outputs of 512 to 3328 tiles of 128 x 48, K = 768 .. 4096
     python -m dace_onnx_amd.testing.gemm_variants few        # outputs of few tiles, and 160 random products and stacks
     python -m dace_onnx_amd.testing.gemm_variants split      # outputs of many tiles, and 160 random products and stacks
+    python -m dace_onnx_amd.testing.gemm_variants packed     # by packed weights: the layer's products at 16 to 8192 rows, and 160 random ones
 
 Prints microseconds per launch (HIP events around graph-recorded launches after a warm-up by time, as bench.py measures
 its rows), the best of the forced forms and the ratio of the library's choice to it. The forms (``MI355X_GEMM_NT_*``):
@@ -14,9 +15,10 @@ its rows), the best of the forced forms and the ratio of the library's choice to
 * ``64`` / ``96`` / ``144``: 64 x 64, 128 x 96 (16 waves) and 64 x 144 tiles;
 * ``128 deep`` / ``128 lean``: 128 x 48 tiles with the six-deep ring (two workgroups per CU) / the three-deep one (three).
 
-``few`` and ``split`` take weights [N, K] (``kc``) and [K, N] (``nc``), ``few`` weights that are not in the L2 (it rotates through
+``few`` and ``split`` take weights [N, K] (``kc``) and [K, N] (``nc``), ``few`` and ``packed`` weights that are not in the L2 (they rotate through
 64 MB of them). Their forms: ``lds``, never the few-tile kernel (``MI355X_GEMM_DIRECT=0``), and its tiles (``=11`` ...); ``fp32``, neither
-that nor the bf16 kernel (``MI355X_GEMM_SPLIT=0``), and the latter's tiles (``=64`` ...).
+that nor the bf16 kernel (``MI355X_GEMM_SPLIT=0``), and the latter's tiles (``=64`` ...). ``packed``: ``before``, without the packed copy
+(``MI355X_GEMM_PACKED=0``), and the forms of the packed kernel by number, as in its table (``=1`` ...).
 
 Every form is checked against float64 in tests/test_configs_gpu.py::test_k_contiguous_gemm_tiles_and_epilogues and
 tests/test_kernel_edges_gpu.py.
@@ -31,7 +33,7 @@ from .. import _lib
 from .profiling import graph_time_us
 
 VARIABLES = ("MI355X_GEMM_NT_BM", "MI355X_GEMM_NT_BN", "MI355X_GEMM_NT_PER_CU", "MI355X_GEMM_NT_WAVES", "MI355X_GEMM_NT_BK", "MI355X_GEMM_DIRECT",
-             "MI355X_GEMM_SPLIT")
+             "MI355X_GEMM_SPLIT", "MI355X_GEMM_PACKED")
 FORMS = (("library", {}),
          ("48 deep", {"MI355X_GEMM_NT_BN": "48", "MI355X_GEMM_NT_PER_CU": "2", "MI355X_GEMM_NT_WAVES": "8"}),
          ("48 lean", {"MI355X_GEMM_NT_BN": "48", "MI355X_GEMM_NT_PER_CU": "3", "MI355X_GEMM_NT_WAVES": "8"}),
@@ -110,14 +112,60 @@ def few_and_split(which: str):
           f"library / best form {sum(b for _, b in behind) / len(behind):.3f} on average, at most {max(b for _, b in behind):.3f}")
 
 
+def set_variables(variables):
+    for name in VARIABLES:
+        os.environ.pop(name, None)
+    os.environ.update(variables)
+    _lib.library().mi355x_reload_tuning()
+
+
+def packed():
+    import torch
+    lib, i64, rng = _lib.library(), _lib.i64_array, random.Random("packed")
+    log_int = lambda low, high: min(high, max(low, round(math.exp(rng.uniform(math.log(low), math.log(high))))))   # noqa: E731
+    shapes = [(M, N, K, True) for M in (16, 128, 865, 1024, 2048, 8192) for N, K in ((768, 768), (2304, 768), (3072, 768), (768, 3072))]
+    shapes += [(1024, 30522, 768, False), (1500, 1024, 4096, True), (373, 1024, 256, True)]
+    while len(shapes) < 27 + 160:
+        M, N, K = log_int(8, 16384), log_int(64, 32000), 32 * log_int(2, 128)
+        if M * N * K < 2e11:
+            shapes.append((M, N // 32 * 32 if rng.random() < 0.5 else N, K, rng.random() < 0.5))
+    forms = (("library", {}), ("before", {"MI355X_GEMM_PACKED": "0"})) + tuple((str(f), {"MI355X_GEMM_PACKED": str(f)}) for f in range(1, 11))
+    ratios = []
+    for M, N, K, kc in shapes:
+        a, bias, out = (torch.randn(s, device="cuda") for s in ((M, K), (N, ), (M, N)))
+        operands = []
+        for _ in range(max(1, min(20, int(64e6 / (4 * N * K))))):
+            w, copy = torch.randn((N, K) if kc else (K, N), device="cuda"), torch.empty(-(-N // 32) * (K // 32) * 1536, dtype=torch.int32, device="cuda")
+            _lib.check(lib.mi355x_pack_f32(w.data_ptr(), copy.data_ptr(), N, K, *((K, 1) if kc else (1, N)), _lib.current_stream()), "pack")
+            operands.append((w, copy))
+        turns = itertools.cycle(operands)
+
+        def launch():
+            w, copy = next(turns)
+            return lib.mi355x_gemm_packed_f32(a.data_ptr(), copy.data_ptr(), w.data_ptr(), out.data_ptr(), bias.data_ptr(), None, 1, 1, M, N, K,
+                                              i64([0, M * K, K, 1]), i64([0, 0, 1, K] if kc else [0, 0, N, 1]), i64([0, M * N, N]), None, 1.0,
+                                              _lib.EPI_BIAS, _lib.current_stream())
+
+        times = []
+        for _, variables in forms:
+            set_variables(variables)
+            times.append(min(graph_time_us(launch, reps=20, replays=3, warm_ms=10.0) for _ in range(2)))
+        set_variables({})
+        ratios.append((times[0] / times[1], times[0] / min(times[1:])))
+        print(f"{M:5d} x {N:5d} x {K:4d} {'kc' if kc else 'nc'} {'packed' if lib.mi355x_gemm_packed_pays(1, M, N, K, int(kc)) else 'before':6s} " +
+              " ".join(f"{name} {t:.1f}" for (name, _), t in zip(forms, times)) +
+              f"   library / before {ratios[-1][0]:.3f}, / best {ratios[-1][1]:.3f}", flush=True)
+    for name, column in (("before", 0), ("best form", 1)):
+        r = [x[column] for x in ratios]
+        print(f"{len(r)} products: library / {name} {math.exp(sum(map(math.log, r)) / len(r)):.3f} on (geometric) average, at most {max(r):.3f}, above 1.03 in {sum(x > 1.03 for x in r)}")
+
+
 def main():
     which = sys.argv[1] if len(sys.argv) > 1 else "layer"
     try:
-        few_and_split(which) if which in ("few", "split") else tiles(which)
+        packed() if which == "packed" else few_and_split(which) if which in ("few", "split") else tiles(which)
     finally:
-        for name in VARIABLES:
-            os.environ.pop(name, None)
-        _lib.library().mi355x_reload_tuning()
+        set_variables({})
 
 
 def tiles(which: str):
