@@ -37,7 +37,7 @@ PEAK_HBM_GBS = 8000.0
 # L2 <-> fabric bytes of the four GEMM launches of one layer, from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of
 # this script scaled by a copy kernel of known size (profiles/bert_layer_gemm_traffic.txt); counters cannot be
 # read from inside the process, so the figure is carried here and re-measured whenever the GEMM kernels change
-GEMM_TRAFFIC_BYTES_PER_LAYER = 176060019
+GEMM_TRAFFIC_BYTES_PER_LAYER = 212352205
 GEMM_TRAFFIC_SOURCE = "profiles/bert_layer_gemm_traffic.txt (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of this script; not re-measured by this run)"
 
 
@@ -354,7 +354,7 @@ def main():
         "value": round(ms_per_step, 5), "unit": "ms", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "ms_per_step": round(ms_per_step, 5), "higher_is_better": False, "scaling": "weak", "vs_baseline": None,
         "dtype": "f32", "data": "synthetic",
-        "config": {"workload": "BASELINE.json configs[2]: BERT-base encoder layer, B=8 S=128 H=768 heads=12 FFN=3072, "
+        "config": {"workload": "BERT-base encoder layer, B=8 S=128 H=768 heads=12 FFN=3072, "
                                "ONNX graph of MatMul/Add/Reshape/Transpose/Div/Softmax/LayerNormalization/Gelu",
                    "launches_per_step": compiled.num_launches, "replay": "host_launches" if mode == "eager" else "hip_graph",
                    "warm_ms": WARM_MS, "warm_steps": warm_steps,
