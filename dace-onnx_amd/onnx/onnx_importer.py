@@ -208,7 +208,6 @@ class ONNXModel:
                     self.state.add_edge(op_node, conn_name, access, None, memlet)
 
         self._compiled = None
-        self._array_names = ([], [])   # names of the weights, and of their arrays
         self._packed = []   # packed copies of constant operands (transformation/packing.py)
         self._expanded = False
         self._static_io = None         # use_hip_graph: inputs, outputs and weights that the recording is bound to
@@ -336,11 +335,7 @@ class ONNXModel:
 
     def _own_weights(self):
         """As :attr:`clean_weights`, for one call."""
-        names, arrays = self._array_names
-        present = self.weights.peek_names()
-        if names != present:
-            names, arrays = self._array_names = present, [clean_onnx_name(n) for n in present]
-        return dict(zip(arrays, self.weights.peek_values()))
+        return {clean_onnx_name(k): v for k, v in self.weights.peek_items()}
 
     def weight_of(self, array):
         """The weight behind the array of that name, None if there is none; read it only."""
@@ -486,7 +481,8 @@ class ONNXModel:
                     desc = self.sdfg.arrays[k]
                     out_kwargs[k] = self.save_transients[k] = torch.empty(desc.shape, dtype=desc.dtype.as_torch(),
                                                                           device=self.device)
-            compiled(**call, **out_kwargs, **self._weight_args(self._own_weights(), packed))
+            weights = self._own_weights()
+            compiled(**call, **out_kwargs, **(self._weight_args(weights, packed) if packed else weights))
         results = [t if use_torch else t.cpu().numpy() for t in outputs.values()]
         return results[0] if len(results) == 1 else tuple(results)
 

@@ -24,11 +24,8 @@ class Weights(dict):
         """The tensor, for readers inside the package that do not keep it; None if there is none."""
         return dict.get(self, name)
 
-    def peek_names(self):
-        return list(dict.keys(self))
-
-    def peek_values(self):
-        return dict.values(self)
+    def peek_items(self):
+        return dict.items(self)
 
     def derived(self, name):
         return name in self._derived
