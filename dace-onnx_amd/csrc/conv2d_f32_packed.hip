@@ -422,7 +422,7 @@ __global__ void pack_conv_f32_kernel(const float* w, u32x4* packed, int M, int C
 // `per_step` (stages of the loop over channels, MFMA steps where there are few) and `per_pixel` (hundreds of a patch, times the stages) hold
 // while every workgroup has a CU to itself, the others for each further one on the same CU (by halves from six on, as in
 // gemm_f32_packed.hip). Fitted over 370 layers of 1 to 32 images, 5 to 256 columns, 1 to 512 channels and 16 to 768 filters, 3 % off on
-// average; the pick is 1 % behind the fastest form.
+// average; the pick is 2.5 % behind the fastest form over 144 others, up to 1.6 times for 1 x 1 and for few 7 x 7 filters.
 struct PackedConvCost { int per_t; double fixed, per_step, per_pixel, again, again_step, again_pixel; };
 struct PackedConvForm { int bm, bp, waves, waves_k; PackedConvCost kinds[3]; };
 constexpr PackedConvForm kPackedConvForms[] = {
@@ -587,7 +587,7 @@ static double unpacked_conv_cost(const ConvArgs& p, int cus, bool& summed_apart)
 }
 
 // The fastest form, -1 where mi355x_conv2d_res_f32 is faster than that and `besides` nanoseconds (or so close that the estimates do not tell: at 0.94 for every kind
-// 3 of 131 layers were 5 to 14 % slower, 32 x 256 x 56 x 56 -> 64, 1 x 1, 38.2 -> 43.5 us;
+// 3 of 131 layers were 5 to 14 % slower, 32 x 256 x 56 x 56 -> 64, 1 x 1, 38.2 -> 43.5 us; as it is 1 of 438, 4 x 1 x 244 x 244 -> 100, 63.6 -> 66.7;
 // the gather kernel's estimate is up to a third too long for 1 x 1 filters, most for few of them). A form whose waves all sum the
 // same channels does not take over from the kernel that sums them apart: its error was up to 1.3 times as large there, everywhere else and
 // of the other forms it is 0.2 to 0.9 of the kernels' before.

@@ -107,7 +107,7 @@ int mi355x_gemm_f32(const float* A, const float* B, float* C,
  * graph is prepared, transformation/packing.py, and the reference has no counterpart). `packed` holds, 6144 bytes each,
  * ceil(N / 32) x K / 32 pairs of fragments (csrc/split_bf16.h); mi355x_pack_f32 writes them. B is the weight itself: it is read where a sum is not finite,
  * and by mi355x_gemm_f32, which is called where the packed form does not apply (K not a multiple of 32, an A that is not
- * contiguous along k or not on 16-byte boundaries, or a product for which it is not the faster one). */
+ * contiguous along k or not on 16-byte boundaries, a product for which it is not the faster one, or a null `packed`). */
 int mi355x_gemm_packed_f32(const float* A, const void* packed, const float* B, float* C, const float* bias,
                            const float* residual, int64_t batch0, int64_t batch1, int64_t M, int64_t N, int64_t K,
                            const int64_t* a_strides, const int64_t* b_strides, const int64_t* c_strides,
@@ -155,7 +155,7 @@ int64_t mi355x_conv2d_packed_pays(int64_t N, int64_t C, int64_t H, int64_t Wd, i
                                   const int64_t* pads, const int64_t* strides, const int64_t* dilations, int constant);
 int mi355x_pack_conv_f32(const float* w, void* packed, int64_t M, int64_t C, int64_t KH, int64_t KW, void* stream);
 
-/* mi355x_conv2d_res_f32 by W and its packed copy (residual may be NULL without MI355X_EPI_RESIDUAL). */
+/* mi355x_conv2d_res_f32 by W and its packed copy, which may be NULL (residual may be NULL without MI355X_EPI_RESIDUAL). */
 int mi355x_conv2d_packed_f32(const float* X, const void* packed, const float* W, const float* bias, const float* residual,
                              float* Y, int64_t N, int64_t C, int64_t H, int64_t Wd,
                              int64_t M, int64_t KH, int64_t KW,
