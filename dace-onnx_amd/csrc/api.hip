@@ -73,6 +73,7 @@ static void parse_tuning(Tuning& t) {
     t.mmi_tile = env_int("MI355X_MMI_TILE", 0);
     t.attn_waves = env_int("MI355X_ATTN_WAVES", 0);
     t.attn_split = env_int("MI355X_ATTN_SPLIT", -1);
+    t.attn_few = env_int("MI355X_ATTN_FEW", -1);
 }
 
 Tuning tuning() {

@@ -30,6 +30,7 @@
 namespace mi355x {
 
 constexpr int AT_SK = 128, AT_D = 64, AT_BQ = 64, AT_PITCH = AT_D + LDS_PAD;
+constexpr int AF_ROWS = 16, AF_KEYS = 16;
 
 struct AttnArgs {
     const float* Q; const float* K; const float* V; float* O;
@@ -344,6 +345,219 @@ __global__ __launch_bounds__(256) void attention_f32_blocks_kernel(AttnArgs p) {
     attention_blocks<MASKED>(p, logical / p.q_blocks, logical % p.q_blocks, lds_k, lds_v);
 }
 
+// Few query blocks (a sentence, a small batch): 16 query rows to a workgroup, the keys in chunks of 16 shared by its waves, wave w taking
+// chunks w, w + WAVES, ... with a running maximum and sum of its own. No wave waits for another before the end, where their sums meet
+// in LDS; no operand passes through LDS: K and Q are read as the fragments of S = Q K^T lie (16 rows, 64 bytes of each), V as 16-byte vectors of
+// four rows, whole lines both, and the probabilities are the next product's operand as they stand.
+// Both products are those of the split form below, with MFMAs of 16 x 16 x 16, and so is the error (0.96 to 1.03 of it; 0.25 to 0.65 of the fp32
+// kernels'). A chunk whose sums are not finite is multiplied again with the fp32 MFMA, by its wave, from the registers it is in.
+// What bounds it: the chain of one wave (launch, first loads, splits, 48 MFMAs a chunk, two exchanges, the sum over the waves) while a CU has
+// one workgroup, the splits beyond, which the kernels of 64 and 128 query rows make once for all of them. 1 x 12 slices of 16 x 16
+// 7.1 -> 3.8 us, of 64 x 64 7.3 -> 4.5, of 128 x 128 7.8 -> 5.8, of 256 x 256 13.8 -> 7.9, 8 x 12 of 16 x 512 25 -> 11.5. (With fp32 MFMAs
+// 3.3, 4.2, 5.5, 7.4, 10.3, but 1.2 to 1.6 times the error of the split form.)
+template <bool MASKED, int WAVES>
+__global__ __launch_bounds__(WAVE * WAVES) void attention_few_kernel(AttnArgs p) {
+    constexpr int ROWS = AF_ROWS, KEYS = AF_KEYS, D = AT_D, NC = D / 16;
+    constexpr float LOG2E = 1.44269504088896340736f;
+    const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int li = lane % 16, lq = lane / 16;
+
+    const uint32_t logical = (uint32_t)xcd_remap(blockIdx.x, p.nwg);   // (grids are below 2^31)
+    const uint32_t slice = logical / (uint32_t)p.q_blocks, qb = logical % (uint32_t)p.q_blocks;
+    const int64_t b0 = slice / (uint32_t)p.batch1, b1 = slice % (uint32_t)p.batch1;
+    const float* __restrict__ Q = p.Q + b0 * p.q_sb0 + b1 * p.q_sb1;
+    const float* __restrict__ K = p.K + b0 * p.k_sb0 + b1 * p.k_sb1 + 4 * lq;
+    const float* __restrict__ V = p.V + b0 * p.v_sb0 + b1 * p.v_sb1 + 4 * li;
+    float* __restrict__ O = p.O + b0 * p.o_sb0 + b1 * p.o_sb1;
+    const int64_t q0 = (int64_t)qb * ROWS, qrow = q0 + li < p.Sq ? q0 + li : p.Sq - 1;   // clamped: computed, not stored
+    const float* __restrict__ mask = MASKED ? p.mask + b0 * p.m_sb0 + b1 * p.m_sb1 + qrow * p.m_sr : nullptr;
+
+    typedef short bf16x4 __attribute__((ext_vector_type(4)));
+    auto parts = [](float x, float y, float z, float w, bf16x4 (&f)[SP_PLANES]) __attribute__((always_inline)) {
+        uint32_t part[SP_PLANES][2];
+        split_pair(x, y, part[0][0], part[1][0], part[2][0]);
+        split_pair(z, w, part[0][1], part[1][1], part[2][1]);
+#pragma unroll
+        for (int q = 0; q < SP_PLANES; ++q) f[q] = __builtin_bit_cast(bf16x4, (u32x2{part[q][0], part[q][1]}));
+    };
+    // of any lane (the sum of finite values may overflow: that is more work, not another result)
+    auto not_finite = [](const f32x4& v) __attribute__((always_inline)) {
+        return __any(fmaf(v[0], 0.f, fmaf(v[1], 0.f, fmaf(v[2], 0.f, v[3] * 0.f))) != 0.f) != 0;   // (NaN compares unequal)
+    };
+    f32x4 rk[NC], rv[4], rm, rq[NC];
+    bf16x4 fq[NC][SP_PLANES];
+    auto load_k = [&](int64_t key0) {   // keys beyond the last are the last one
+        const float* row = K + (key0 + li < p.Sk ? key0 + li : p.Sk - 1) * p.k_sr;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) rk[c] = *reinterpret_cast<const f32x4*>(row + 16 * c);
+        if constexpr (MASKED) {
+            typedef f32x4 unaligned __attribute__((aligned(4)));
+            if (key0 + KEYS <= p.Sk) rm = *reinterpret_cast<const unaligned*>(mask + key0 + 4 * lq);
+            else
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int64_t key = key0 + 4 * lq + r;
+                    rm[r] = mask[key < p.Sk ? key : p.Sk - 1];
+                }
+        }
+    };
+    auto load_v = [&](int64_t key0) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int64_t key = key0 + 4 * lq + r;
+            rv[r] = *reinterpret_cast<const f32x4*>(V + (key < p.Sk ? key : p.Sk - 1) * p.v_sr);
+        }
+    };
+    const int64_t first = (int64_t)wave * KEYS;
+    if (first < p.Sk) {
+        load_k(first);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) rq[c] = *reinterpret_cast<const f32x4*>(Q + qrow * p.q_sr + 16 * c + 4 * lq);
+        load_v(first);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) parts(rq[c][0], rq[c][1], rq[c][2], rq[c][3], fq[c]);
+    }
+    f32x4 out[4];   // out[t][r] = O[q0 + 4 lq + r][4 li + t] of this wave's keys, not yet divided by the sum
+#pragma unroll
+    for (int t = 0; t < 4; ++t) out[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_run = -INFINITY, l_run = 0.f;   // of query row q0 + li (the same value in its four lanes)
+    for (int64_t key0 = first; key0 < p.Sk; key0 += WAVES * KEYS) {
+        const int64_t next = key0 + WAVES * KEYS;   // uniform
+        f32x4 s;   // S[q0 + li][key0 + 4 lq + r]
+        {
+            f32x4 sum[2], small[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) sum[h] = small[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                bf16x4 fk[SP_PLANES];
+                parts(rk[c][0], rk[c][1], rk[c][2], rk[c][3], fk);
+#pragma unroll
+                for (int u = 0; u < PK_PRODUCTS; ++u) {
+                    f32x4& to = u == 0 ? sum[c % 2] : small[c % 2];
+                    to = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(fk[PK_QA[u]], fq[c][PK_QB[u]], to, 0, 0, 0);
+                }
+            }
+            s = ((sum[0] + sum[1]) + (small[0] + small[1])) * SP_UNSCALE;
+        }
+        if (__builtin_expect(not_finite(s), 0)) {
+            f32x4 set[NC];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) set[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int c = 0; c < NC; ++c) set[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(rk[c][e], rq[c][e], set[c], 0, 0, 0);
+            s = (set[0] + set[1]) + (set[2] + set[3]);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if constexpr (MASKED) s[r] = fmaf(s[r], p.scale, rm[r]);
+            else s[r] *= p.scale;
+        }
+        if (next < p.Sk) load_k(next);
+        if (key0 + KEYS > p.Sk)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (key0 + 4 * lq + r >= p.Sk) s[r] = -INFINITY;
+        const float m_new = fmaxf(m_run, quad_lanes_max(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]))));
+        const float m_ref = m_new == -INFINITY ? 0.f : m_new;   // nothing but -inf so far: 2^(-inf - 0) = 0
+        auto power = [&](float v) { return __builtin_amdgcn_exp2f((v - m_ref) * LOG2E); };
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[r] = power(s[r]);
+        const float sum = quad_lanes_sum((s[0] + s[1]) + (s[2] + s[3]));
+        f32x4 product[4];
+        {
+            bf16x4 fp[SP_PLANES];
+            parts(s[0], s[1], s[2], s[3], fp);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                bf16x4 fv[SP_PLANES];
+                parts(rv[0][t], rv[1][t], rv[2][t], rv[3][t], fv);
+                f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f}, small = sum;
+#pragma unroll
+                for (int u = 0; u < PK_PRODUCTS; ++u) {
+                    f32x4& to = u == 0 ? sum : small;
+                    to = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(fp[PK_QA[u]], fv[PK_QB[u]], to, 0, 0, 0);
+                }
+                product[t] = (sum + small) * SP_UNSCALE;
+            }
+        }
+        if (__builtin_expect(not_finite((product[0] + product[1]) + (product[2] + product[3])), 0)) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) product[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) product[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[r], rv[r][t], product[t], 0, 0, 0);
+        }
+        if (next < p.Sk) load_v(next);
+        if (key0 == first) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) out[t] = product[t];
+            l_run = sum;
+        } else {
+            const float alpha = power(m_run);
+            l_run = fmaf(l_run, alpha, sum);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float a = __shfl(alpha, 4 * lq + r, WAVE);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) out[t][r] = fmaf(out[t][r], a, product[t][r]);
+            }
+        }
+        m_run = m_new;
+    }
+    if constexpr (WAVES == 1) {
+        const float inv = 1.0f / l_run;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float a = __shfl(inv, 4 * lq + r, WAVE);
+            if (q0 + 4 * lq + r < p.Sq)
+                *reinterpret_cast<f32x4*>(O + (q0 + 4 * lq + r) * p.o_sr + 4 * li) = f32x4{out[0][r] * a, out[1][r] * a, out[2][r] * a, out[3][r] * a};
+        }
+    } else {
+        // the sums of the waves, in their order: one with no key has a maximum of -inf and adds zeros
+        constexpr int PER = ROWS * D / (WAVE * WAVES);   // outputs of a thread, of one row
+        __shared__ __attribute__((aligned(16))) float part[WAVES][ROWS][D];
+        __shared__ float part_m[WAVES][ROWS], part_l[WAVES][ROWS];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            *reinterpret_cast<f32x4*>(&part[wave][4 * lq + r][4 * li]) = f32x4{out[0][r], out[1][r], out[2][r], out[3][r]};
+        if (lq == 0) {
+            part_m[wave][li] = m_run;
+            part_l[wave][li] = l_run;
+        }
+        __syncthreads();
+        const int row = tid / (D / PER), col = tid % (D / PER) * PER;
+        float m = part_m[0][row];
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) m = fmaxf(m, part_m[w][row]);
+        const float m_ref = m == -INFINITY ? 0.f : m;
+        float l = 0.f, sum[PER];
+#pragma unroll
+        for (int e = 0; e < PER; ++e) sum[e] = 0.f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            const float a = __builtin_amdgcn_exp2f((part_m[w][row] - m_ref) * LOG2E);
+            l = fmaf(part_l[w][row], a, l);
+#pragma unroll
+            for (int e = 0; e < PER; ++e) sum[e] = fmaf(part[w][row][col + e], a, sum[e]);
+        }
+        const float inv = 1.0f / l;
+        if (q0 + row < p.Sq) {
+            typedef float vec __attribute__((ext_vector_type(PER < 4 ? PER : 4)));
+#pragma unroll
+            for (int e = 0; e < PER; e += (PER < 4 ? PER : 4)) {
+                vec v;
+#pragma unroll
+                for (int i = 0; i < (PER < 4 ? PER : 4); ++i) v[i] = sum[e + i] * inv;
+                *reinterpret_cast<vec*>(O + (q0 + row) * p.o_sr + col + e) = v;
+            }
+        }
+    }
+}
+
 // Many rows: both products on the bf16 matrix unit, every value split in three (split_bf16.h; the six products in two sets of accumulators,
 // the second product block by block). A workgroup of four waves owns 128 query rows, 32 of them each, and walks the keys in blocks of 64:
 //   * S^T = K Q^T, Q split once into registers, K on its way into LDS in fragment order. A lane then holds half of a query's scores of the
@@ -573,15 +787,28 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(AttnArgs p) {
                 f32x4{out[db][4 * g] * inv, out[db][4 * g + 1] * inv, out[db][4 * g + 2] * inv, out[db][4 * g + 3] * inv};
 }
 
-// Whether the split form is ahead. Nanoseconds of a workgroup with a CU to itself and of each further one on it, by blocks of keys: fitted over
-// 26 shapes of 12 to 512 slices, 33 to 512 keys, both forms measured on each; the form not taken is at most 4 % faster in these.
-static bool split_pays(int64_t slices, int64_t Sq, int64_t Sk, bool masked) {
-    const int cus = device_cus();
-    auto cost = [&](int64_t rows, int64_t keys, double fixed, double block, double again, double again_block) {
-        const double blocks = (double)ceil_div(Sk, keys), more = (double)(ceil_div(slices * ceil_div(Sq, rows), (int64_t)std::max(cus, 1)) - 1);
-        return fixed + blocks * block + more * (again + blocks * again_block);
-    };
-    return cost(AS_ROWS, AS_KEYS, 3400, 3800, 1500, 3000) < (masked ? 0.95 : 0.95 * 0.88) * cost(AT_BQ, AT_SK, 2400, 6600, 2000, 4900);
+// Nanoseconds of a workgroup with a CU to itself and of each further one on it, by blocks of keys: fitted over 26 shapes of 12 to 512 slices, 33
+// to 512 keys, both forms measured on each; of the two the form not taken is at most 4 % faster in these.
+static double attention_cost(int64_t slices, int64_t Sq, int64_t Sk, int64_t rows, int64_t keys, double fixed, double block, double again, double again_block) {
+    const double blocks = (double)ceil_div(Sk, keys), more = (double)(ceil_div(slices * ceil_div(Sq, rows), (int64_t)std::max(device_cus(), 1)) - 1);
+    return fixed + blocks * block + more * (again + blocks * again_block);
+}
+static double split_cost(int64_t slices, int64_t Sq, int64_t Sk) { return attention_cost(slices, Sq, Sk, AS_ROWS, AS_KEYS, 3400, 3800, 1500, 3000); }
+static double blocks_cost(int64_t slices, int64_t Sq, int64_t Sk, bool masked) {
+    return (masked ? 1 : 0.88) * attention_cost(slices, Sq, Sk, AT_BQ, AT_SK, 2400, 6600, 2000, 4900);
+}
+static bool split_pays(int64_t slices, int64_t Sq, int64_t Sk, bool masked) { return split_cost(slices, Sq, Sk) < 0.95 * blocks_cost(slices, Sq, Sk, masked); }
+
+// How many waves share the keys in the form for few query blocks, 0 where another form is ahead. A wave to a chunk up to four of them (a workgroup
+// to a CU: up to eight); further workgroups on a CU cost what their chunks take. Over 100 shapes of 8 to 512 keys and 12 to 384 slices the pick is at
+// most 5 % behind the fastest form (4 x 12 x 100 and 5 x 12 x 173 with a mask: 15 % and 5 %) and never behind the forms before this one.
+static int few_waves(int64_t slices, int64_t Sq, int64_t Sk, bool masked) {
+    const int64_t chunks = ceil_div(Sk, (int64_t)AF_KEYS), up = ceil_div(slices * ceil_div(Sq, (int64_t)AF_ROWS), (int64_t)std::max(device_cus(), 1));
+    const int waves = chunks <= 1 ? 1 : chunks <= 2 ? 2 : chunks <= 4 || up > 1 ? 4 : 8;
+    const double fixed[] = {2400, 2500, 3000, 3950}, chunk[] = {1400, 1500, 1470, 1850};
+    const int form = waves == 1 ? 0 : waves == 2 ? 1 : waves == 4 ? 2 : 3;
+    const double cost = fixed[form] + chunk[form] * (double)ceil_div(chunks, (int64_t)waves) + (masked ? 1.1 : 1) * (double)(up - 1) * (850 + 210 * (double)chunks);
+    return cost < 0.95 * std::min(split_cost(slices, Sq, Sk), blocks_cost(slices, Sq, Sk, masked)) ? waves : 0;
 }
 
 // mask == nullptr: the unmasked product
@@ -612,9 +839,27 @@ static int launch_attention(const float* Q, const float* K, const float* V, floa
     p.scale = scale;
     p.mask = mask;
     p.m_sb0 = mask ? mask_strides[0] : 0; p.m_sb1 = mask ? mask_strides[1] : 0; p.m_sr = mask ? mask_strides[2] : 0;
+    const Tuning forced = tuning();
+    const int64_t few_nwg = batch0 * batch1 * ceil_div(Sq, (int64_t)AF_ROWS);
+    const int waves = forced.attn_few > 0 ? forced.attn_few : forced.attn_few < 0 && forced.attn_split < 0 && forced.attn_waves == 0 ? few_waves(batch0 * batch1, Sq, Sk, mask != nullptr) : 0;
+    if (waves > 0 && grid_fits(few_nwg, WAVE * 8)) {
+        p.q_blocks = ceil_div(Sq, (int64_t)AF_ROWS);
+        p.nwg = few_nwg;
+        auto launch = [&](auto count) {
+            constexpr int W = decltype(count)::value;
+            const dim3 grid((unsigned)p.nwg), block(WAVE * W);
+            if (mask) hipLaunchKernelGGL((attention_few_kernel<true, W>), grid, block, 0, static_cast<hipStream_t>(stream), p);
+            else hipLaunchKernelGGL((attention_few_kernel<false, W>), grid, block, 0, static_cast<hipStream_t>(stream), p);
+        };
+        if (waves == 1) launch(std::integral_constant<int, 1>{});
+        else if (waves == 2) launch(std::integral_constant<int, 2>{});
+        else if (waves <= 4) launch(std::integral_constant<int, 4>{});
+        else launch(std::integral_constant<int, 8>{});
+        return check_launch("attention_few_kernel");
+    }
     const int64_t split_blocks = ceil_div(Sq, (int64_t)AS_ROWS), split_nwg = batch0 * batch1 * split_blocks;
-    const int split = tuning().attn_split;
-    if (split != 0 && grid_fits(split_nwg, 256) && Sk < (1 << 24) && Sk * k_strides[2] < (1 << 29) && Sk * v_strides[2] < (1 << 29) && (!mask || (mask_strides[2] >= 0 && Sq * mask_strides[2] + Sk < (1 << 29))) && (split > 0 || (tuning().attn_waves == 0 && split_pays(batch0 * batch1, Sq, Sk, mask != nullptr)))) {
+    const int split = forced.attn_split;
+    if (split != 0 && grid_fits(split_nwg, 256) && Sk < (1 << 24) && Sk * k_strides[2] < (1 << 29) && Sk * v_strides[2] < (1 << 29) && (!mask || (mask_strides[2] >= 0 && Sq * mask_strides[2] + Sk < (1 << 29))) && (split > 0 || (forced.attn_waves == 0 && split_pays(batch0 * batch1, Sq, Sk, mask != nullptr)))) {
         p.q_blocks = split_blocks;
         p.nwg = split_nwg;
         if (mask) hipLaunchKernelGGL(attention_split_kernel<true>, dim3((unsigned)p.nwg), dim3(256), 0, static_cast<hipStream_t>(stream), p);
@@ -628,14 +873,14 @@ static int launch_attention(const float* Q, const float* K, const float* V, floa
     if (Sk == AT_SK) {
         // MI355X_ATTN_WAVES = 2 / 3: 32 / 48 query rows per workgroup instead of 64 (measured on 8 x 12 slices of 128 rows:
         // 384 / 288 workgroups instead of 192 -- no faster, the time is one wave's chain of loads, 256 MFMAs and stores)
-        const int waves = tuning().attn_waves == 2 || tuning().attn_waves == 3 ? tuning().attn_waves : 4;
-        p.q_blocks = ceil_div(Sq, (int64_t)16 * waves);
+        const int rows_waves = forced.attn_waves == 2 || forced.attn_waves == 3 ? forced.attn_waves : 4;
+        p.q_blocks = ceil_div(Sq, (int64_t)16 * rows_waves);
         p.nwg = batch0 * batch1 * p.q_blocks;
-        MI355X_REQUIRE(grid_fits(p.nwg, 64 * waves), "attention: grid too large");
+        MI355X_REQUIRE(grid_fits(p.nwg, 64 * rows_waves), "attention: grid too large");
         const dim3 g((unsigned)p.nwg);
         hipStream_t st = static_cast<hipStream_t>(stream);
-        if (waves == 2) hipLaunchKernelGGL(attention_f32_kernel<2>, g, dim3(128), 0, st, p);
-        else if (waves == 3) hipLaunchKernelGGL(attention_f32_kernel<3>, g, dim3(192), 0, st, p);
+        if (rows_waves == 2) hipLaunchKernelGGL(attention_f32_kernel<2>, g, dim3(128), 0, st, p);
+        else if (rows_waves == 3) hipLaunchKernelGGL(attention_f32_kernel<3>, g, dim3(192), 0, st, p);
         else hipLaunchKernelGGL(attention_f32_kernel<4>, g, dim3(256), 0, st, p);
         return check_launch("attention_f32_kernel");
     }

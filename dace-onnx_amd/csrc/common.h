@@ -32,7 +32,7 @@ struct Tuning {
     int conv_config = -1, conv_gather_bn = 0, conv_tail = -1, conv_static_taps = 1, conv_per_cu = 0, conv_direct = -1, conv_packed = -1;
     bool mmi_generic = false;
     int mmi_wgs_per_cu = 0, mmi_tile = 0;
-    int attn_waves = 0, attn_split = -1;
+    int attn_waves = 0, attn_split = -1, attn_few = -1;
 };
 Tuning tuning();   // a copy taken under the lock: a reload never changes what a launch in progress reads
 int device_cus();
@@ -79,6 +79,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
 

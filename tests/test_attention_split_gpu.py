@@ -111,3 +111,44 @@ def test_sentences_without_a_valid_key_take_no_longer():
     assert graph_time_us(launch) < 1.5 * before
     torch.cuda.synchronize()
     assert bool(torch.isnan(out[::2]).all()) and bool(torch.isfinite(out[1::2]).all())
+
+
+@pytest.mark.parametrize("waves", [1, 2, 4, 8])
+@pytest.mark.parametrize("sq, sk", [(1, 1), (16, 16), (17, 15), (33, 130), (5, 129), (64, 300)])
+@pytest.mark.parametrize("shape", [None, "keys", "rows", "all"])
+def test_attention_of_few_rows(tuning, waves, sq, sk, shape):
+    """Chunks of 16 keys shared by the waves, fewer and more of them than waves, ragged ones: bounds as for the split form."""
+    tuning(MI355X_ATTN_FEW=waves)
+    b0, b1 = 2, 3
+    q, k, v = inputs(b0, b1, sq, sk)
+    extents = {"keys": (b0, 1, 1, sk), "rows": (1, 1, sq, sk), "all": (b0, b1, sq, sk)}.get(shape)
+    mask = None
+    if extents:
+        memory = torch.where(torch.rand(b0 * b1 * sq * sk + 1, device="cuda") < 0.3, -10000.0, 0.0)[1:]   # (not 16-byte aligned)
+        mask = memory[:extents[0] * extents[1] * extents[2] * sk].view(extents)
+        mask[..., sk // 2] = 0
+    scores = 0.125 * (q.double() @ k.double().transpose(-1, -2).contiguous())
+    expected = torch.softmax(scores + mask.double() if extents else scores, -1) @ v.double()
+    got = attention(q, k, v, mask)
+    assert bool(((expected - got.double()).abs() <= 2.0**-19 * v.abs().max()).all())
+    assert float((expected - got.double()).norm() / expected.norm()) < 1e-6
+
+
+@pytest.mark.parametrize("waves", [1, 4, 8])
+@pytest.mark.parametrize("masked", [False, True])
+def test_attention_of_few_rows_keeps_infinities_nan_and_the_largest_values(tuning, waves, masked):
+    """Against the fp32 kernel; a mask of -inf over whole chunks and over a whole row among the values."""
+    mask = torch.zeros(1, 1, 20, 100, device="cuda") if masked else None
+    if masked:
+        mask[..., :40], mask[:, :, 7] = -float("inf"), -float("inf")
+    for place, value in ((0, float("inf")), (0, float("nan")), (1, -float("inf")), (1, float("nan")), (2, float("inf")), (2, float("nan")), (2, 3.0e38), (0, 1.0e36)):
+        tensors = inputs(2, 2, 20, 100, seed=place)
+        tensors[place][1, 0, 13 if place == 0 else 70, 9] = value
+        results = []
+        for form in (dict(MI355X_ATTN_SPLIT=0), dict(MI355X_ATTN_FEW=waves)):
+            tuning(MI355X_ATTN_SPLIT=None, MI355X_ATTN_FEW=None)
+            tuning(**form)
+            results.append(attention(*tensors, mask))
+        assert torch.equal(torch.isnan(results[0]), torch.isnan(results[1])) and torch.equal(torch.isinf(results[0]), torch.isinf(results[1]))
+        fine = torch.isfinite(results[0])
+        assert bool(((results[0] - results[1]).abs()[fine] <= 1e-5 * results[0].abs()[fine].clamp(min=1)).all())
