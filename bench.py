@@ -45,6 +45,12 @@ def algorithmic_work(name, args):
     """(flops, bytes) of one launch from its C-ABI arguments (fp32 unless stated)."""
     if name == "mi355x_gemm_packed_f32":   # the same arguments with the packed copy of B after A
         return algorithmic_work("mi355x_gemm_f32", args[:1] + args[2:])
+    if name == "mi355x_gemm_parts_f32":
+        parts, M, N, K = args[4:8]
+        return 2.0 * M * N * K, 4.0 * (M * K + K * N + parts * M * N)
+    if name == "mi355x_layernorm_parts_f32":   # sums, residual and result
+        parts, rows, cols = args[1], args[8], args[9]
+        return 0.0, 4.0 * (parts + 2) * rows * cols + 12.0 * cols
     if name == "mi355x_gemm_f32":
         b0, b1, M, N, K = args[5:10]
         epi = args[15]
@@ -211,6 +217,14 @@ def main():
                 gemm_floor_us += flops / 1e6 / (PEAK_SPLIT_MFMA_TFLOPS if packed else PEAK_FP32_MFMA_TFLOPS)
                 label = "gemm_f32{} b{}x{} {}x{}x{} epi={}".format("_packed" if packed else "", *plain[5:10], plain[15])
                 kernels.append(kernel_row(label, us, flops, nbytes, "mfma", PEAK_SPLIT_MFMA_TFLOPS if packed else None))
+            elif name == "mi355x_gemm_parts_f32":
+                packed = node.args[2].connector is not None
+                gemm_flops += flops
+                gemm_bytes += nbytes
+                gemm_us += us
+                gemm_floor_us += flops / 1e6 / (PEAK_SPLIT_MFMA_TFLOPS if packed else PEAK_FP32_MFMA_TFLOPS)
+                kernels.append(kernel_row("gemm_parts_f32{} {} parts {}x{}x{}".format("_packed" if packed else "", *plain[4:8]), us, flops, nbytes, "mfma",
+                                          PEAK_SPLIT_MFMA_TFLOPS if packed else None))
             elif name == "mi355x_attention_f32":
                 label = "attention_f32 b{}x{} q{} k{} d{}".format(*plain[4:9])
                 kernels.append(kernel_row(label, us, flops, nbytes, "mfma"))
@@ -218,6 +232,7 @@ def main():
                 label = name.replace("mi355x_", "") + " " + "x".join(str(v) for v in (plain[5] if name == "mi355x_eltwise_f32"
                                                                                      else plain[3] if name == "mi355x_permute_b32"
                                                                                      else plain[2:5] if name == "mi355x_softmax_f32"
+                                                                                     else [plain[1], *plain[8:10]] if name == "mi355x_layernorm_parts_f32"
                                                                                      else plain[4:6]))
                 kernels.append(kernel_row(label, us, 0.0, nbytes, "hbm"))
 

@@ -32,7 +32,8 @@ namespace mi355x {
 struct PackedGemmArgs {
     GemmArgs g;
     const char* packed;
-    int kt;   // steps of 32 k
+    int kt;          // steps of 32 k
+    int kt_stream;   // of 32 columns of the packed copy: as many, or those of all parts where a batch entry multiplies a part of K
 };
 
 template <int TM, int TN, int WAVES_M, int WAVES_N, int WAVES_K, int PER_SIMD>
@@ -97,11 +98,12 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * WAVES_K * WAVE, PER_SIMD) void 
     };
     // B: one stream of fragments per 32 columns; columns beyond the matrix are its last block's
     const int n_blocks = (columns_all + 31) / 32;
+    const uint32_t first_step = pa.kt_stream != pa.kt ? b * (uint32_t)pa.kt : 0u;
     uint32_t b_off[TN];
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
         const int block = min((int)(n0 / 32) + wn * TN + j, n_blocks - 1);
-        b_off[j] = (uint32_t)block * (uint32_t)pa.kt * (uint32_t)(2 * PK_FRAGMENT);
+        b_off[j] = ((uint32_t)block * (uint32_t)pa.kt_stream + first_step) * (uint32_t)(2 * PK_FRAGMENT);
     }
     bf16x8 fa[2][TM][SP_PLANES], fb[2][TN][SP_PLANES];
     auto load_b = [&](auto s_tag, int j, int st) {
@@ -191,7 +193,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * WAVES_K * WAVE, PER_SIMD) void 
         for (int r = 0; r < 16; ++r) sum[r] = 0.f;
         const int64_t m = bm + li, n = bn + li;
         const float* ap = A + (m < p.M ? m : p.M - 1) * p.a_sm + 16 * lh;
-        const float* bp = p.B + (n < p.N ? n : p.N - 1) * p.b_sn + 16 * lh * p.b_sk;
+        const float* bp = p.B + b0 * p.b_sb0 + (n < p.N ? n : p.N - 1) * p.b_sn + 16 * lh * p.b_sk;
         for (int st = from; st < to; ++st) {
             typedef f32x4 unaligned __attribute__((aligned(4)));
             f32x4 va[4], vb[4];
@@ -416,7 +418,7 @@ static double unpacked_cost(const GemmArgs& p, bool b_kc, int cus) {
 // Preconditions of the kernel besides pointer alignment
 static bool packed_takes(const GemmArgs& p) {
     return p.K > 0 && p.K % 32 == 0 && p.a_sk == 1 && p.a_sm >= 0 && p.a_sm % 4 == 0 && p.a_sb0 % 4 == 0 && p.a_sb1 % 4 == 0 &&
-           p.b_sb0 == 0 && p.b_sb1 == 0 && (p.M - 1) * p.a_sm + p.K < ((int64_t)1 << 29) &&
+           p.b_sb1 == 0 && (p.M - 1) * p.a_sm + p.K < ((int64_t)1 << 29) &&
            ceil_div(p.N, (int64_t)32) * (p.K / 32) * (2 * PK_FRAGMENT) < ((int64_t)1 << 31) &&
            p.c_sm >= 0 && p.c_sm < ((int64_t)1 << 22) && p.r_sm >= 0 && p.r_sm < ((int64_t)1 << 22);   // (rows of a tile of C, 32-bit byte offsets)
 }
@@ -428,19 +430,57 @@ static bool packed_takes(const GemmArgs& p) {
 // well ahead (28 x 13792 x 1280 23.6 -> 19.1). Over 413 products that nothing was fitted to the pick is at most 4 % behind the kernels before
 // and takes 0.88 of their time; against the fastest form it is 2.4 % behind over 187, up to 1.7 times where K is short and tiles are many
 // (5190 x 23059 x 192 282 us packed, 485 as picked: the estimate of the kernels before is low there).
-static int choose_packed(const GemmArgs& p, int cus) {
+// `best_cost`: of what is chosen, either way.
+static int choose_packed(const GemmArgs& p, int cus, double& best_cost) {
     const int force = tuning().gemm_packed;
-    if (!packed_takes(p) || force == 0 || force > kNumPackedForms) return -1;
-    if (force > 0) return force - 1;
-    if (p.M <= 16) return -1;
-    double best_cost = (p.M <= 32 ? 0.8 : 1) * unpacked_cost(p, p.b_sk == 1, cus);
+    best_cost = 0;
+    if (force > 0 && force <= kNumPackedForms && packed_takes(p)) return force - 1;
+    best_cost = unpacked_cost(p, p.b_sk == 1, cus);
+    if (!packed_takes(p) || force >= 0 || p.M <= 16) return -1;
+    if (p.M <= 32) best_cost *= 0.8;
     int best = -1;
     for (int f = 0; f < kNumPackedForms; ++f) {
         const PackedForm& form = kPackedForms[f];
         const double cost = packed_cost(form, p.batch * ceil_div(p.M, (int64_t)form.bm) * ceil_div(p.N, (int64_t)form.bn), p.K, cus);
         if (cost < best_cost) { best = f; best_cost = cost; }
     }
+    if (best < 0 && p.M <= 32) best_cost /= 0.8;
     return best;
+}
+
+static int choose_packed(const GemmArgs& p, int cus) {
+    double cost;
+    return choose_packed(p, cus, cost);
+}
+
+// The same for a product in parts (batch entries of p): the packed forms and the few-tile kernel, no other -- those before have up to twice their
+// error. -1: the few-tile kernel.
+static int choose_part(const GemmArgs& p, bool packed, int cus, double& best_cost) {
+    const int force = tuning().gemm_packed;
+    best_cost = 0;
+    if (force > 0 && force <= kNumPackedForms && packed && packed_takes(p)) return force - 1;
+    best_cost = 0.91 * gemm_f32_direct_cost(p, p.b_sk == 1, cus);
+    if (!packed || !packed_takes(p) || force >= 0 || p.M <= 16) return -1;
+    int best = -1;
+    for (int f = 0; f < kNumPackedForms; ++f) {
+        const PackedForm& form = kPackedForms[f];
+        const double cost = packed_cost(form, p.batch * ceil_div(p.M, (int64_t)form.bm) * ceil_div(p.N, (int64_t)form.bn), p.K, cus) * (p.M <= 32 ? 1.25 : 1);
+        if (cost < best_cost) { best = f; best_cost = cost; }
+    }
+    return best;
+}
+
+static int launch_chosen(PackedGemmArgs& pa, int form, int cus, hipStream_t stream) {
+    GemmArgs& p = pa.g;
+    const PackedForm& f = kPackedForms[form];
+    p.tiles_m = ceil_div(p.M, (int64_t)f.bm);
+    p.tiles_n = ceil_div(p.N, (int64_t)f.bn);
+    p.nwg = p.batch * p.tiles_m * p.tiles_n;
+    if (!grid_fits(p.nwg, f.threads)) return -1;
+    const int64_t per_xcd = ceil_div(p.nwg, (int64_t)NUM_XCD), per_batch = p.tiles_m * p.tiles_n;
+    p.group_m = choose_group_m(p.tiles_m, per_xcd < per_batch ? per_xcd : per_batch, (int64_t)f.resident * (cus / NUM_XCD), f.bm, f.bn, p.K * 5);
+    launch_packed(form, pa, stream);
+    return check_launch("gemm_f32_packed_kernel");
 }
 
 }  // namespace mi355x
@@ -477,7 +517,7 @@ extern "C" int mi355x_gemm_packed_f32(const float* A, const void* packed, const 
     auto al16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     if (A && B && C && packed && a_strides && b_strides && c_strides && batch0 > 0 && batch1 > 0 && M > 0 && N > 0 && K > 0 &&
         (epilogue & ~(MI355X_EPI_BIAS | MI355X_EPI_RELU | MI355X_EPI_GELU | MI355X_EPI_RESIDUAL)) == 0 && (!(epilogue & MI355X_EPI_BIAS) || bias) &&
-        (!(epilogue & MI355X_EPI_RESIDUAL) || (residual && r_strides)) && (c_strides[2] >= N || M == 1) && al16(A) && al16(packed)) {
+        (!(epilogue & MI355X_EPI_RESIDUAL) || (residual && r_strides)) && (c_strides[2] >= N || M == 1) && al16(A) && al16(packed) && b_strides[0] == 0) {
         MI355X_TRACE_INIT(p);
         p.A = A; p.B = B; p.C = C; p.bias = bias; p.residual = residual;
         p.batch = batch0 * batch1; p.batch1 = batch1; p.M = M; p.N = N; p.K = K;
@@ -488,22 +528,90 @@ extern "C" int mi355x_gemm_packed_f32(const float* A, const void* packed, const 
         p.r_sb0 = res ? r_strides[0] : 0; p.r_sb1 = res ? r_strides[1] : 0; p.r_sm = res ? r_strides[2] : 0;
         p.alpha = alpha; p.epi = epilogue;
         pa.packed = static_cast<const char*>(packed);
-        pa.kt = (int)(K / 32);
+        pa.kt = pa.kt_stream = (int)(K / 32);
         const int cus = device_cus();
         if (cus <= 0) return set_error(MI355X_ERR_NOT_INITIALIZED, "gemm: no usable HIP device");
         const int form = choose_packed(p, cus);
         if (form >= 0) {
-            const PackedForm& f = kPackedForms[form];
-            p.tiles_m = ceil_div(M, (int64_t)f.bm);
-            p.tiles_n = ceil_div(N, (int64_t)f.bn);
-            p.nwg = p.batch * p.tiles_m * p.tiles_n;
-            if (grid_fits(p.nwg, f.threads)) {
-                const int64_t per_xcd = ceil_div(p.nwg, (int64_t)NUM_XCD), per_batch = p.tiles_m * p.tiles_n;
-                p.group_m = choose_group_m(p.tiles_m, per_xcd < per_batch ? per_xcd : per_batch, (int64_t)f.resident * (cus / NUM_XCD), f.bm, f.bn, K * 5);
-                launch_packed(form, pa, static_cast<hipStream_t>(stream));
-                return check_launch("gemm_f32_packed_kernel");
-            }
+            const int status = launch_chosen(pa, form, cus, static_cast<hipStream_t>(stream));
+            if (status >= 0) return status;
         }
     }
     return mi355x_gemm_f32(A, B, C, bias, residual, batch0, batch1, M, N, K, a_strides, b_strides, c_strides, r_strides, alpha, epilogue, stream);
+}
+
+// Between one and eight parts, of at least 256 k each, by the estimates of the kernels and what the normalization takes longer to read them.
+// Over 49 products of 1 to 2048 rows the pick takes 0.82 of the time in one part, normalization included, and is nowhere more than 2 % behind it.
+// Both launches, weights from beyond the L2: 16 x 768 x 3072 16.0 us in one part, 8.9 in eight; 128 rows 21.7, 12.9 in four; 512 rows 28.9, 22.5 in
+// four; 865 rows 39.7, 30.3 in three; 1024 rows 40.3, 35.2 in four; 16 x 1024 x 4096 19.6, 9.9 in eight; 128 x 768 x 768 9.9, 9.3 in three.
+extern "C" int64_t mi355x_gemm_parts(int64_t M, int64_t N, int64_t K, int b_kc, int packed) {
+    using namespace mi355x;
+    if (M <= 0 || N <= 0 || K <= 0 || N % 4 || N > 1024) return 1;
+    int cus = device_cus();
+    if (cus <= 0) cus = 256;
+    GemmArgs p = {};
+    p.batch = p.batch1 = 1; p.M = M; p.N = N; p.K = K;
+    p.a_sm = K; p.a_sk = 1; p.b_sk = b_kc ? 1 : N; p.b_sn = b_kc ? K : 1; p.c_sm = N;
+    double best_cost;
+    if (packed) choose_packed(p, cus, best_cost);
+    else best_cost = unpacked_cost(p, p.b_sk == 1, cus);
+    best_cost *= 0.95;
+    int64_t best = 1;
+    for (const int64_t parts : {2, 3, 4, 6, 8}) {
+        if (K % (parts * 32) || K / parts < 256) continue;
+        p.batch = parts; p.K = K / parts;
+        double cost;
+        choose_part(p, packed, cus, cost);
+        cost += 200.0 + 50.0 * (double)parts + 4.0 * (double)parts * (double)M * (double)N / 10000.0;
+        if (cost < best_cost) { best = parts; best_cost = cost; }
+    }
+    return best;
+}
+
+extern "C" int mi355x_gemm_parts_packed_pays(int64_t parts, int64_t M, int64_t N, int64_t K, int b_kc) {
+    using namespace mi355x;
+    if (parts <= 0 || M <= 0 || N <= 0 || K <= 0 || K % (32 * parts)) return 0;
+    GemmArgs p = {};
+    p.batch = parts; p.batch1 = 1; p.M = M; p.N = N; p.K = K / parts;
+    p.a_sm = K; p.a_sk = 1; p.b_sk = b_kc ? 1 : N; p.b_sn = b_kc ? K : 1; p.c_sm = N;
+    const int cus = device_cus();
+    double cost;
+    return choose_part(p, ceil_div(N, (int64_t)32) * (K / 32) * (2 * PK_FRAGMENT) < ((int64_t)1 << 31), cus > 0 ? cus : 256, cost) >= 0;
+}
+
+extern "C" int mi355x_gemm_parts_f32(const float* A, const float* B, const void* packed, float* P, int64_t parts, int64_t M, int64_t N, int64_t K,
+                                     int64_t a_row_stride, int64_t b_k_stride, int64_t b_column_stride, float alpha, void* stream) {
+    using namespace mi355x;
+    MI355X_REQUIRE(parts > 0 && M >= 0 && N >= 0 && K >= 0 && K % parts == 0, "gemm_parts: K = %lld in %lld parts", (long long)K, (long long)parts);
+    const int64_t share = K / parts;
+    const int64_t a[4] = {share, 0, a_row_stride, 1}, b[4] = {share * b_k_stride, 0, b_k_stride, b_column_stride}, c[3] = {M * N, 0, N};
+    if (A && B && P && M > 0 && N > 0 && share > 0) {
+        PackedGemmArgs pa = {};
+        GemmArgs& p = pa.g;
+        MI355X_TRACE_INIT(p);
+        p.A = A; p.B = B; p.C = P;
+        p.batch = parts; p.batch1 = 1; p.M = M; p.N = N; p.K = share;
+        p.a_sb0 = a[0]; p.a_sm = a[2]; p.a_sk = 1;
+        p.b_sb0 = b[0]; p.b_sk = b[2]; p.b_sn = b[3];
+        p.c_sb0 = c[0]; p.c_sm = N;
+        p.alpha = alpha; p.epi = MI355X_EPI_NONE;
+        pa.packed = static_cast<const char*>(packed);
+        pa.kt = (int)(share / 32); pa.kt_stream = (int)(K / 32);
+        const int cus = device_cus();
+        if (cus <= 0) return set_error(MI355X_ERR_NOT_INITIALIZED, "gemm: no usable HIP device");
+        const bool takes = packed && share % 32 == 0 && ceil_div(N, (int64_t)32) * (K / 32) * (2 * PK_FRAGMENT) < ((int64_t)1 << 31) &&
+                           ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(packed)) & 15) == 0;
+        double cost;
+        const int form = choose_part(p, takes, cus, cost);
+        if (form >= 0) {
+            const int status = launch_chosen(pa, form, cus, static_cast<hipStream_t>(stream));
+            if (status >= 0) return status;
+        }
+        // (a copy that is left out in a product of many rows: a kernel of large tiles)
+        const bool b_kc = b_k_stride == 1;
+        if (form < 0 && (b_kc || b_column_stride == 1) && cost < 1.4 * unpacked_cost(p, b_kc, cus) &&
+            launch_gemm_f32_direct(p, b_kc, 1e300, cus, static_cast<hipStream_t>(stream)))
+            return check_launch("gemm_f32_direct_kernel");
+    }
+    return mi355x_gemm_f32(A, B, P, nullptr, nullptr, parts, 1, M, N, share, a, b, c, nullptr, alpha, MI355X_EPI_NONE, stream);
 }

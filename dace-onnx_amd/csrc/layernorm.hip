@@ -12,7 +12,10 @@
 //       NV float4 per lane (768 columns = 3 loads of 16 bytes per lane), DPP +
 //       readlane reductions, no LDS.
 //   layernorm_rows_loop     any cols: one wave per row, three sweeps.
+//   layernorm_parts_reg<NV, PARTS>  the first, over partial sums of the product before it.
 #include "common.h"
+
+#include <type_traits>
 
 namespace mi355x {
 
@@ -73,6 +76,61 @@ __global__ __launch_bounds__(256) void layernorm_rows_reg(const float* __restric
     }
 }
 
+// The same over the sums of a product that was computed in parts (mi355x_gemm_parts_f32): x = sum_s P[s] + bias + residual, in that order. One wave
+// per row, all of a row's loads in flight at once; values at any 4-byte boundary. Bound by the launch and one trip to memory for few rows (16 x 768 in
+// eight parts 3.2 us, layernorm_rows_reg 2.2), so up to 1024 rows a workgroup is one wave; by the bytes for many (2048 x 768 in four parts 5.3 us).
+template <int NV, int PARTS>
+__global__ __launch_bounds__(256) void layernorm_parts_reg(const float* __restrict__ P, const float* __restrict__ bias,
+                                                           const float* __restrict__ residual, int64_t r_sm,
+                                                           const float* __restrict__ gamma, const float* __restrict__ beta,
+                                                           float* __restrict__ Y, int64_t rows, int cols, float eps) {
+    typedef f32x4 unaligned __attribute__((aligned(4)));
+    const int lane = threadIdx.x % WAVE;
+    const int64_t row = (int64_t)blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
+    if (row >= rows) return;  // wave-uniform
+    const int cols4 = cols >> 2;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 v[PARTS][NV], r[NV], c[NV], g[NV], b[NV];
+#pragma unroll
+    for (int s = 0; s < PARTS; ++s) {
+        const f32x4* src = reinterpret_cast<const f32x4*>(P + (s * rows + row) * cols);
+#pragma unroll
+        for (int j = 0; j < NV; ++j) v[s][j] = lane + j * WAVE < cols4 ? src[lane + j * WAVE] : zero;
+    }
+    auto vectors = [&](f32x4 (&to)[NV], const float* from) {
+#pragma unroll
+        for (int j = 0; j < NV; ++j) to[j] = from != nullptr && lane + j * WAVE < cols4 ? f32x4(reinterpret_cast<const unaligned*>(from)[lane + j * WAVE]) : zero;
+    };
+    vectors(r, residual ? residual + row * r_sm : nullptr);
+    vectors(c, bias);
+    vectors(g, gamma);
+    vectors(b, beta);
+
+    float sum = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+#pragma unroll
+        for (int s = 1; s < PARTS; ++s) v[0][j] += v[s][j];
+        if (bias != nullptr) v[0][j] += c[j];
+        if (residual != nullptr) v[0][j] += r[j];
+        sum += (v[0][j].x + v[0][j].y) + (v[0][j].z + v[0][j].w);
+    }
+    const float inv_n = 1.0f / (float)cols;
+    const float mean = wave_sum(sum) * inv_n;
+    float q = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+        if (lane + j * WAVE < cols4) {
+            v[0][j] -= mean;
+            q += (v[0][j].x * v[0][j].x + v[0][j].y * v[0][j].y) + (v[0][j].z * v[0][j].z + v[0][j].w * v[0][j].w);
+        }
+    const float inv_std = 1.0f / sqrtf(wave_sum(q) * inv_n + eps);
+    unaligned* dst = reinterpret_cast<unaligned*>(Y + row * cols);
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+        if (lane + j * WAVE < cols4) dst[lane + j * WAVE] = (v[0][j] * inv_std) * g[j] + b[j];
+}
+
 __global__ __launch_bounds__(256) void layernorm_rows_loop(const float* __restrict__ X,
                                                            const float* __restrict__ gamma,
                                                            const float* __restrict__ beta,
@@ -124,4 +182,32 @@ extern "C" int mi355x_layernorm_f32(const float* X, const float* gamma, const fl
     else if (vec_ok && cols <= 4096) hipLaunchKernelGGL(layernorm_rows_reg<16>, grid, block, 0, st, X, gamma, beta, Y, rows, c, eps);
     else hipLaunchKernelGGL(layernorm_rows_loop, grid, block, 0, st, X, gamma, beta, Y, rows, cols, eps);
     return check_launch("layernorm_rows");
+}
+
+extern "C" int mi355x_layernorm_parts_f32(const float* P, int64_t parts, const float* bias, const float* residual, int64_t r_row_stride,
+                                          const float* gamma, const float* beta, float* Y, int64_t rows, int64_t cols, float eps, void* stream) {
+    using namespace mi355x;
+    MI355X_REQUIRE(rows >= 0 && cols >= 0 && cols % 4 == 0 && cols <= 1024 && (parts == 2 || parts == 3 || parts == 4 || parts == 6 || parts == 8),
+                   "layernorm_parts: %lld parts of %lld x %lld", (long long)parts, (long long)rows, (long long)cols);
+    if (rows == 0 || cols == 0) return MI355X_OK;
+    MI355X_REQUIRE(P && Y && gamma && (reinterpret_cast<uintptr_t>(P) & 15) == 0, "layernorm_parts: null or unaligned pointer");
+    const unsigned waves = rows <= 1024 ? 1 : 4;
+    MI355X_REQUIRE(grid_fits(ceil_div(rows, (int64_t)waves), waves * WAVE), "layernorm_parts: too many rows");
+    const dim3 grid((unsigned)ceil_div(rows, (int64_t)waves)), block(waves * WAVE);
+    auto launch = [&](auto nv, auto n) {
+        hipLaunchKernelGGL((layernorm_parts_reg<decltype(nv)::value, decltype(n)::value>), grid, block, 0, static_cast<hipStream_t>(stream), P, bias, residual,
+                           r_row_stride, gamma, beta, Y, rows, (int)cols, eps);
+    };
+    auto with_parts = [&](auto nv) {
+        if (parts == 2) launch(nv, std::integral_constant<int, 2>{});
+        else if (parts == 3) launch(nv, std::integral_constant<int, 3>{});
+        else if (parts == 4) launch(nv, std::integral_constant<int, 4>{});
+        else if (parts == 6) launch(nv, std::integral_constant<int, 6>{});
+        else launch(nv, std::integral_constant<int, 8>{});
+    };
+    if (cols <= 256) with_parts(std::integral_constant<int, 1>{});
+    else if (cols <= 512) with_parts(std::integral_constant<int, 2>{});
+    else if (cols <= 768) with_parts(std::integral_constant<int, 3>{});
+    else with_parts(std::integral_constant<int, 4>{});
+    return check_launch("layernorm_parts_reg");
 }

@@ -374,6 +374,8 @@ class ONNXModel:
                 raise RuntimeError("ONNXModel executes on the MI355X only: no HIP device is visible")
             self.expand()
             from ..transformation.packing import pack_constant_operands, pack_variable_filters
+            from ..transformation.partial_sums import split_products
+            split_products(self)
             self._packed = pack_constant_operands(self)
             pack_variable_filters(self.sdfg)
             self._compiled = self.sdfg.compile()

@@ -51,6 +51,12 @@ def _packed_gemm(call, desc):
     """(name suffix, shape, function, geometry, offset) of the copy that a GEMM multiplies by, and the call that does; None where it does not pay."""
     lib = _lib.library()
     offset = call.args[1].offset
+    if call.function == "mi355x_gemm_parts_f32":
+        parts, M, N, K, a_row, sk, sn = call.args[4:11]
+        if a_row % 4 or not lib.mi355x_gemm_parts_packed_pays(parts, M, N, K, int(sk == 1)):
+            return None
+        copy = (f"{N}_{K}_{sn}_{sk}_{offset}", [-(-N // 32), K // 32, 2, 3, 64, 4], "mi355x_pack_f32", (N, K, sn, sk), offset)
+        return copy, (call.function, call.args[:2] + [Ptr("_packed")] + call.args[3:])
     batch0, batch1, M, N, K, a_strides, b_strides = call.args[5:12]
     sb0, sb1, sk, sn = b_strides.values
     if sb0 or sb1 or min(sk, sn) < 1 or a_strides.values[3] != 1 or a_strides.values[2] % 4 \
@@ -100,7 +106,7 @@ def pack_variable_filters(sdfg):
             state.add_edge(access, None, packed_call, "_packed", sdfg.make_array_memlet(clean))
 
 
-_PACKED = {"mi355x_gemm_f32": _packed_gemm, "mi355x_conv2d_f32": _packed_conv, "mi355x_conv2d_res_f32": _packed_conv}
+_PACKED = {"mi355x_gemm_f32": _packed_gemm, "mi355x_gemm_parts_f32": _packed_gemm, "mi355x_conv2d_f32": _packed_conv, "mi355x_conv2d_res_f32": _packed_conv}
 
 
 def pack_constant_operands(model):

@@ -119,6 +119,17 @@ int mi355x_gemm_packed_pays(int64_t batch, int64_t M, int64_t N, int64_t K, int 
  * rows = N, row_stride = 1, k_stride = N. */
 int mi355x_pack_f32(const float* w, void* packed, int64_t rows, int64_t K, int64_t row_stride, int64_t k_stride, void* stream);
 
+/* The product alpha A B in `parts` sums over equal shares of K (which `parts` divides), P[s] = [M, N] contiguous: workgroups for a chip that the outputs
+ * alone leave idle. mi355x_layernorm_parts_f32 adds them up. A is contiguous along k; `packed` as for mi355x_gemm_packed_f32 (of all of K; NULL:
+ * B is read itself). */
+int mi355x_gemm_parts_f32(const float* A, const float* B, const void* packed, float* P, int64_t parts, int64_t M, int64_t N, int64_t K,
+                          int64_t a_row_stride, int64_t b_k_stride, int64_t b_column_stride, float alpha, void* stream);
+/* How many parts a product of M x N x K followed by a LayerNormalization of its rows is computed in (b_kc as for
+ * mi355x_gemm_packed_pays; `packed`: whether there is a packed copy); 1: in one. */
+int64_t mi355x_gemm_parts(int64_t M, int64_t N, int64_t K, int b_kc, int packed);
+/* 1 where mi355x_gemm_parts_f32 multiplies by the packed copy if it has one. */
+int mi355x_gemm_parts_packed_pays(int64_t parts, int64_t M, int64_t N, int64_t K, int b_kc);
+
 
 /* ONNX Conv, 2-D, NCHW, group 1, fp32, implicit GEMM on MFMA.
  *   Y[n,m,oy,ox] = epilogue(sum_{c,r,s} W[m,c,r,s] *
@@ -270,6 +281,10 @@ int mi355x_attention_masked_f32(const float* Q, const float* K, const float* V, 
 int mi355x_layernorm_f32(const float* X, const float* gamma, const float* beta,
                          float* Y, int64_t rows, int64_t cols, float eps,
                          void* stream);
+/* The same of sum_s P[s] + bias + residual, P[s] being the `parts` (2, 3, 4, 6 or 8) sums of mi355x_gemm_parts_f32. cols: a multiple of 4,
+ * at most 1024; bias, beta and residual (rows r_row_stride apart) may be NULL; P on a 16-byte boundary. */
+int mi355x_layernorm_parts_f32(const float* P, int64_t parts, const float* bias, const float* residual, int64_t r_row_stride,
+                               const float* gamma, const float* beta, float* Y, int64_t rows, int64_t cols, float eps, void* stream);
 
 /* ONNX ReduceMean along one axis, fp32. X viewed as [outer, axis_len, inner]
  * (C-contiguous); Y is [outer, inner] (keepdims only changes the shape the
