@@ -635,6 +635,27 @@ class _Program:
             _lib.check(result & 0xff, self._names[result >> 8])
 
 
+class _Recording:
+    """A HIP graph that is never destroyed while torch's current stream is being captured.
+
+    A compiled graph and what holds it refer to each other, so a dropped one goes whenever Python collects garbage, also in the middle of a
+    capture of the caller's. Destroying a HIP graph waits for the GPU, an error then that ends the process: the graph is put aside until
+    another recording is made or goes.
+    """
+    _put_aside = []
+
+    def __init__(self, graph):
+        import torch
+        self.graph, self._capturing = graph, torch.cuda.is_current_stream_capturing
+        self._put_aside.clear()
+
+    def __del__(self):
+        if self._capturing():
+            self._put_aside.append(self.graph)
+        else:
+            self._put_aside.clear()
+
+
 class CompiledSDFG:
     """Executable form of an expanded SDFG: a flat list of kernel launches.
 
@@ -949,13 +970,13 @@ class CompiledSDFG:
         torch.cuda.synchronize()
         with torch.cuda.graph(g):
             self._run(launches)
-        self._graph = g
+        self._graph = _Recording(g)
         return g
 
     def replay(self):
         if self._graph is None:
             raise RuntimeError("capture_graph() has not been called for the current buffers")
-        self._graph.replay()
+        self._graph.graph.replay()
 
     @property
     def num_launches(self):

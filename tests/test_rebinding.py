@@ -48,3 +48,30 @@ def test_rebinding_equals_binding(graph, fuse):
     assert [_plain(item[3]) for item in again] == [_plain(item[3]) for item in expected] != before
     assert [_plain(item[3]) for item in launches] == before   # another thread may be walking it
     assert [(i[0], i[1], i[2], i[4], i[6]) for i in again] == [(i[0], i[1], i[2], i[4], i[6]) for i in expected]
+
+
+def test_recordings_are_not_destroyed_during_a_capture(monkeypatch):
+    """A dropped model's recording goes when garbage is collected; not while the caller captures a stream."""
+    import gc
+    from dace_onnx_amd.sdfg import _Recording
+    capturing, destroyed = [], []
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: bool(capturing))
+
+    class Graph:
+        def __init__(self, name):
+            self.name = name
+
+        def __del__(self):
+            destroyed.append(self.name)
+
+    holder = {"recording": _Recording(Graph("first"))}
+    holder["itself"] = holder   # as a model and its compiled graph are
+    del holder
+    capturing.append(1)
+    gc.collect()
+    assert not destroyed
+    capturing.clear()
+    second = _Recording(Graph("second"))
+    assert destroyed == ["first"]
+    del second
+    assert destroyed == ["first", "second"]
