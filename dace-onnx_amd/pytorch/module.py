@@ -384,7 +384,7 @@ class DaceModule(nn.Module):
         state = {"compiled": None}
 
         def forward(*args):
-            if tuple(tuple(a.shape) for a in args) != self._input_shapes:
+            if tuple(a.shape for a in args) != self._input_shapes:   # (a torch.Size is a tuple)
                 raise TypeError(f"{self.sdfg_name} was built for inputs of shapes {self._input_shapes}")
             if state["compiled"] is None:     # needs the GPU: done on the first call, not at construction
                 state["compiled"] = self.dace_model.compile_and_init()

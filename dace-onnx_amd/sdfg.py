@@ -24,7 +24,10 @@ node; a library node that was not expanded to kernels cannot run.
 import array
 import collections
 import ctypes
+import functools
+import importlib.util
 import itertools
+import os
 import struct
 import typing
 
@@ -590,6 +593,31 @@ class SDFG:
 # --------------------------------------------------------------------------- executor
 
 
+def _host_call():
+    """The extension module that ``csrc/host_call.cpp`` is built into, next to the library."""
+    global _host_call_module
+    if _host_call_module is None:
+        import torch  # noqa: F401  (whose libraries it is linked against)
+        path = os.path.join(os.path.dirname(_lib.LIBRARY_PATH), "_host_call.so")
+        if not os.path.isfile(path):
+            raise _lib.LibraryNotBuilt(f"{path} not found; build it with `make -C {os.path.join(os.path.dirname(path), 'csrc')}`")
+        spec = importlib.util.spec_from_file_location("_host_call", path)
+        _host_call_module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(_host_call_module)
+    return _host_call_module
+
+
+_host_call_module = None
+
+
+@functools.lru_cache(maxsize=None)
+def _example(dtype, device="cpu", inference=False):
+    """A tensor of that kind, made for its attributes."""
+    import torch
+    with torch.inference_mode(inference):
+        return torch.empty(1, dtype=dtype, device=device)
+
+
 class _Program:
     """A launch list as the words ``mi355x_program_run`` takes: one call into the library issues all launches, with the addresses of a
     call's buffers put in place there."""
@@ -682,7 +710,8 @@ class CompiledSDFG:
         self._transients = {}   # flattened key -> descriptor
         self._transient_tensors = {}   # flattened key -> its allocation (made on first use, kept)
         self._plan = []         # ("call", node, connector -> key) | ("alias", src key, dst key, dst descriptor)
-        self._bound_key = None
+        self._bound = None      # the tensors of the last call in the order of _external (None: a packed copy that was left out), and their addresses:
+        self._bound_words = b""   # they live as long as the launch list points to them
         self._patches = None    # per launch, the pointer arguments that follow the caller's arrays (see _rebind)
         self._program = None    # the launch list as one native call (None: it holds device copies, or functions that cannot be part of one)
         self._launches, self._listed_key = [], None
@@ -843,11 +872,21 @@ class CompiledSDFG:
         return result
 
     @property
+    def _bound_key(self):
+        """The addresses of the last call's tensors."""
+        return None if self._bound is None else array.array("q", self._bound_words).tolist()
+
+    @property
+    def _env(self):
+        return dict(zip(self._external, self._bound))
+
+    @property
     def _launch_list(self):
         """The launches for the buffers of the last call (those of the program, which replaces addresses itself, are brought up to date)."""
-        if self._listed_key != self._bound_key:
-            self._launches = self._rebind(self._launches, dict(zip(self._external, self._bound_key)))
-            self._listed_key = self._bound_key
+        key = self._bound_key
+        if self._listed_key != key:
+            self._launches = self._rebind(self._launches, dict(zip(self._external, key)))
+            self._listed_key = key
         return self._launches
 
     def _tensor(self, env, key):
@@ -930,8 +969,7 @@ class CompiledSDFG:
                 else:
                     self._launches = self._rebind(self._launches, dict(zip(self._external, key)))
                 self._listed_key = key
-            self._env = env   # the caller's arrays live as long as the launch list points to them
-            self._bound_key = key
+            self._bound, self._bound_words = list(env.values()), array.array("q", key).tobytes()
             self._graph = None
         if self._program is None:
             self._run(self._launches)
@@ -947,6 +985,38 @@ class CompiledSDFG:
             outs = [env[n] if any_torch else env[n].cpu().numpy() for n in self._returned]
             return outs[0] if len(outs) == 1 else tuple(outs)
         return None
+
+    # -- the whole of a call in native code ----------------------------------------------
+    def host_plan(self, inputs, outputs, weights, packed):
+        """What :meth:`run_plan` calls (``csrc/host_call.cpp``), None where the launches are no program or an array is none of these: input and
+        output arrays by their places, weights by their names (array -> key of the dict that a call gets), packed copies by their places."""
+        import torch
+        if self._program is None or self.device.type != "cuda" or self.device.index is None:
+            return None
+        slots = []
+        for name in self._external:
+            desc = self.sdfg.arrays[name]
+            kind = next((k for k, places in ((0, inputs), (1, outputs), (3, packed), (2, weights)) if name in places), None)
+            if kind is None:
+                return None
+            index, key = (0, weights[name]) if kind == 2 else ((inputs, outputs, weights, packed)[kind][name], None)
+            slots.append((kind, index, key, _example(self._torch_types[name]), tuple(desc.shape)))
+        plain = [_example(torch.float32, self.device, inference) for inference in (False, True)]
+        return _host_call().plan(ctypes.cast(self._program._run, ctypes.c_void_p).value, self._program._fixed, self._program, slots, len(inputs), len(outputs),
+                                 len(weights), self.device.index, *plain)
+
+    def run_plan(self, plan, weights, copies, inputs):
+        """One call on torch's current stream: its outputs, in fresh tensors; None, with nothing launched, where an argument is no plain tensor as declared."""
+        import torch
+        if self._graph is not None:
+            return None
+        done = plan.call(weights, weights._made, weights._handed_out, copies, inputs, torch._C._cuda_getCurrentRawStream(self.device.index))
+        if done is None:
+            return None
+        status, outputs, self._bound, self._bound_words = done
+        if status:
+            _lib.check(status & 0xff, self._program._names[status >> 8])
+        return outputs
 
     # -- HIP graph -------------------------------------------------------------------
     def capture_graph(self, with_packed=False):

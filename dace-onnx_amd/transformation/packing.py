@@ -23,6 +23,7 @@ class PackedOperand:
         self.shape, self.function, self.geometry, self.offset = shape, function, geometry, offset
         self.derived = model.weights.derived(weight_name)
         self.device, self.weight, self.version, self.packed, self.declared = model.device, None, None, None, False
+        self.record = None   # what csrc/host_call.cpp decides current() by
         if now and model.weights.private(weight_name):
             self.pack()
 
@@ -37,6 +38,7 @@ class PackedOperand:
         self.version = None if weight.is_inference() else weight._version
         if self.packed is None:
             self.packed = torch.empty(self.shape, dtype=torch.int32, device=self.device)
+        self.record = (self.weight_name, weight, self.version, self.derived or declared, self.packed)
         start = weight.data_ptr() + 4 * self.offset
         _lib.check(getattr(_lib.library(), self.function)(start, self.packed.data_ptr(), *self.geometry, _lib.current_stream()), self.function)
 
