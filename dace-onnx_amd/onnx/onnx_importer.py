@@ -430,14 +430,20 @@ class ONNXModel:
         return inputs
 
     def _host_plan(self):
-        """What further calls with tensors on the GPU take; False where there is no such way for this model."""
+        """What calls with tensors on the GPU take from the second on; False where there is no such way for this model."""
+        if self._compiled._bound is None:
+            return None
         clean = clean_onnx_name
         return self._compiled.host_plan({clean(n): i for i, n in enumerate(self.inputs)}, {clean(n): i for i, n in enumerate(self.outputs)},
                                         {clean(n): n for n in self.weights}, {c.array: i for i, c in enumerate(self._packed)}) or False
 
     def _call_by_plan(self, args):
         """The outputs of a call in which every argument is as the graph takes it; None, with nothing done, for :meth:`__call__` to look into it."""
-        if not self._plan or self.use_hip_graph or self.save_transients is not None or type(self.weights) is not Weights or self._capturing():
+        if self.use_hip_graph or self.save_transients is not None or type(self.weights) is not Weights or self._capturing():
+            return None
+        if self._plan is None:
+            self._plan = self._host_plan()
+        if not self._plan:
             return None
         return self._compiled.run_plan(self._plan, self.weights, self._packed, args)
 
@@ -449,7 +455,7 @@ class ONNXModel:
         :return: the output (or a tuple of outputs): torch tensors on the GPU if any
                  input was a torch tensor, numpy arrays otherwise.
         """
-        if self._plan is not None and not kwargs:
+        if self._compiled is not None and not kwargs:
             results = self._call_by_plan(args)
             if results is not None:
                 return results[0] if len(results) == 1 else tuple(results)
@@ -502,8 +508,6 @@ class ONNXModel:
                                                                           device=self.device)
             weights = self._own_weights()
             compiled(**call, **out_kwargs, **(self._weight_args(weights, packed) if packed else weights))
-            if self._plan is None and self.save_transients is None:
-                self._plan = self._host_plan()
         results = [t if use_torch else t.cpu().numpy() for t in outputs.values()]
         return results[0] if len(results) == 1 else tuple(results)
 
