@@ -56,6 +56,10 @@ SIGNATURES: typing.Dict[str, typing.Tuple[typing.Any, typing.List[typing.Any]]] 
                                      _c_i64_p, _c_i64_p, _c_i64_p, _int, _vp]),
     "mi355x_conv2d_packed_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                                         _c_i64_p, _c_i64_p, _c_i64_p, _int, _vp]),
+    "mi355x_conv2d_pool_packed_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _c_i64_p, _c_i64_p, _c_i64_p, _int,
+                                             _i64, _i64, _c_i64_p, _c_i64_p, _c_i64_p, _vp]),
+    "mi355x_conv2d_pool_packed_pays": (_i64, [_i64, _i64, _i64, _i64, _i64, _i64, _i64, _c_i64_p, _c_i64_p, _c_i64_p, _i64, _i64, _c_i64_p, _c_i64_p, _c_i64_p]),
+    "mi355x_pack_conv_pool_f32": (_int, [_vp, _vp, _i64, _i64, _i64, _i64, _vp]),
     "mi355x_pack_conv_f32": (_int, [_vp, _vp, _i64, _i64, _i64, _i64, _vp]),
     "mi355x_conv2d_packed_pays": (_i64, [_i64, _i64, _i64, _i64, _i64, _i64, _i64, _c_i64_p, _c_i64_p, _c_i64_p, _int]),
     "mi355x_matmul_integer": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _int, _i64, _i64, _vp]),

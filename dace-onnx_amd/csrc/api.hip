@@ -68,6 +68,7 @@ static void parse_tuning(Tuning& t) {
     t.conv_per_cu = env_int("MI355X_CONV_PER_CU", 0);
     t.conv_direct = env_int("MI355X_CONV_DIRECT", -1);
     t.conv_packed = env_int("MI355X_CONV_PACKED", -1);
+    t.conv_pool = env_int("MI355X_CONV_POOL", -1);
     t.mmi_generic = getenv("MI355X_MMI_GENERIC") != nullptr;
     t.mmi_wgs_per_cu = env_int("MI355X_MMI_WGS_PER_CU", 0);
     t.mmi_tile = env_int("MI355X_MMI_TILE", 0);

@@ -29,7 +29,7 @@ static inline bool grid_fits(int64_t workgroups, int64_t threads) { return workg
 // and again on mi355x_reload_tuning(); CU count of the current device, asked of the runtime once per device.
 struct Tuning {
     int gemm_config = -1, gemm_nt_bn = 0, gemm_nt_bm = 0, gemm_nt_bk = 0, gemm_nt_per_cu = 0, gemm_nt_waves = 0, gemm_group_m = 0, gemm_ksplit = -1, gemm_split = -1, gemm_direct = -1, gemm_packed = -1;
-    int conv_config = -1, conv_gather_bn = 0, conv_tail = -1, conv_static_taps = 1, conv_per_cu = 0, conv_direct = -1, conv_packed = -1;
+    int conv_config = -1, conv_gather_bn = 0, conv_tail = -1, conv_static_taps = 1, conv_per_cu = 0, conv_direct = -1, conv_packed = -1, conv_pool = -1;
     bool mmi_generic = false;
     int mmi_wgs_per_cu = 0, mmi_tile = 0;
     int attn_waves = 0, attn_split = -1, attn_few = -1;

@@ -374,9 +374,10 @@ class ONNXModel:
             if self.device.type != "cuda":
                 raise RuntimeError("ONNXModel executes on the MI355X only: no HIP device is visible")
             self.expand()
-            from ..transformation.packing import pack_constant_operands, pack_variable_filters
+            from ..transformation.packing import pack_constant_operands, pack_variable_filters, pool_in_convolutions
             from ..transformation.partial_sums import split_products
             split_products(self)
+            pool_in_convolutions(self)
             self._packed = pack_constant_operands(self)
             pack_variable_filters(self.sdfg)
             self._compiled = self.sdfg.compile()

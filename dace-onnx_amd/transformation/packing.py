@@ -8,7 +8,8 @@ library as they are.
 import torch
 
 from .. import _lib
-from ..sdfg import AccessNode, KernelCall, PackedCopy, Ptr, Stream, int32
+from ..sdfg import AccessNode, I64Array, KernelCall, PackedCopy, Ptr, Stream, int32
+from .fusion import _in_edge, _out_edge, _single_consumer
 
 
 class PackedOperand:
@@ -88,6 +89,44 @@ def _packed_conv(call, desc):
     return ("filters", shape, "mi355x_pack_conv_f32", geometry, 0), packed_call
 
 
+def _packed_stem(call, desc):
+    """As :func:`_packed_gemm`, for a convolution with its pooling."""
+    geometry = call.args[6:16] + call.args[17:22]
+    N, C, H, Wd, M, KH, KW = geometry[:7]
+    size = _lib.library().mi355x_conv2d_pool_packed_pays(*[_lib.i64_array(a.values) if isinstance(a, I64Array) else a for a in geometry])
+    if not size or call.args[1].offset or desc.shape != (M, C, KH, KW) or not desc.is_contiguous():
+        return None
+    return ("stem_filters", [size // 3072, 3, 64, 4], "mi355x_pack_conv_pool_f32", (M, C, KH, KW), 0), (call.function, call.args[:2] + [Ptr("_packed")] + call.args[3:])
+
+
+def pool_in_convolutions(model):
+    """A convolution by constant filters whose result only a MaxPool reads becomes one call with it, where the library has a kernel for both."""
+    from ..onnx.onnx_importer import clean_onnx_name
+    sdfg, weights = model.sdfg, {clean_onnx_name(k) for k in model.weights}
+    for state in sdfg.nodes():
+        for call in state.nodes():
+            if not isinstance(call, KernelCall) or call.function != "mi355x_conv2d_f32" or call.args[14] & ~(_lib.EPI_BIAS | _lib.EPI_RELU):
+                continue
+            X, W, bias, Y = call.args[:4]
+            out = _out_edge(state, call, Y.connector)
+            read = out and isinstance(out.dst, AccessNode) and _single_consumer(sdfg, state, out.dst)
+            pool = read and read.dst
+            filters = sdfg.arrays[_in_edge(state, call, W.connector).data.data] if read else None
+            if not isinstance(pool, KernelCall) or pool.function != "mi355x_maxpool2d_f32" or pool.args[0].connector != read.dst_conn \
+                    or pool.args[0].offset or Y.offset or _in_edge(state, call, W.connector).data.data not in weights:
+                continue
+            both = KernelCall(call.label, "mi355x_conv2d_pool_packed_f32", [X, W, Ptr(None), bias, Ptr("_scratch"), Ptr("_pooled", pool.args[1].offset)] + call.args[4:15]
+                              + pool.args[6:11] + [Stream()], call.in_connectors, ["_scratch", "_pooled"])
+            if _packed_stem(both, filters) is None:
+                continue
+            result = _out_edge(state, pool, pool.args[1].connector)
+            state.remove_edge(out)
+            state.remove_node(pool)
+            state.replace_node(call, both, sdfg)
+            state.add_edge(both, "_scratch", out.dst, None, out.data)
+            state.add_edge(both, "_pooled", result.dst, None, result.data)
+
+
 def pack_variable_filters(sdfg):
     """Pack the filters of the remaining convolutions on every call, where the library says that this pays too."""
     for state in sdfg.nodes():
@@ -108,7 +147,8 @@ def pack_variable_filters(sdfg):
             state.add_edge(access, None, packed_call, "_packed", sdfg.make_array_memlet(clean))
 
 
-_PACKED = {"mi355x_gemm_f32": _packed_gemm, "mi355x_gemm_parts_f32": _packed_gemm, "mi355x_conv2d_f32": _packed_conv, "mi355x_conv2d_res_f32": _packed_conv}
+_PACKED = {"mi355x_gemm_f32": _packed_gemm, "mi355x_gemm_parts_f32": _packed_gemm, "mi355x_conv2d_f32": _packed_conv, "mi355x_conv2d_res_f32": _packed_conv,
+           "mi355x_conv2d_pool_packed_f32": _packed_stem}
 
 
 def pack_constant_operands(model):

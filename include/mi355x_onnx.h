@@ -173,6 +173,20 @@ int mi355x_conv2d_packed_f32(const float* X, const void* packed, const float* W,
                              const int64_t* pads, const int64_t* strides,
                              const int64_t* dilations, int epilogue, void* stream);
 
+/* Conv, Relu (or not) and MaxPool of an image classifier's stem in one launch, by W and its packed copy: 7 x 7 filters by two over three channels,
+ * pooled 3 x 3 by two, no dilation. `epilogue`: MI355X_EPI_BIAS and MI355X_EPI_RELU. Elsewhere, and with a null `packed`, mi355x_conv2d_f32
+ * into `scratch` [N, M, OH, OW], which is not written otherwise, and mi355x_maxpool2d_f32. mi355x_conv2d_pool_packed_pays: bytes of the
+ * packed copy, which mi355x_pack_conv_pool_f32 writes; 0 where there is none. (MI355X_CONV_POOL=n: the n-th form takes it, 0: none.) */
+int64_t mi355x_conv2d_pool_packed_pays(int64_t N, int64_t C, int64_t H, int64_t Wd, int64_t M, int64_t KH, int64_t KW,
+                                       const int64_t* pads, const int64_t* strides, const int64_t* dilations, int64_t PKH, int64_t PKW,
+                                       const int64_t* pool_pads, const int64_t* pool_strides, const int64_t* pool_dilations);
+int mi355x_pack_conv_pool_f32(const float* w, void* packed, int64_t M, int64_t C, int64_t KH, int64_t KW, void* stream);
+int mi355x_conv2d_pool_packed_f32(const float* X, const float* W, const void* packed, const float* bias, float* scratch, float* Y,
+                                  int64_t N, int64_t C, int64_t H, int64_t Wd, int64_t M, int64_t KH, int64_t KW,
+                                  const int64_t* pads, const int64_t* strides, const int64_t* dilations, int epilogue,
+                                  int64_t PKH, int64_t PKW, const int64_t* pool_pads, const int64_t* pool_strides,
+                                  const int64_t* pool_dilations, void* stream);
+
 /* Several launches in one call. `program` holds `calls` calls one after the other, each the number of its function
  * (mi355x_program_function of its name, -1 if it cannot be one) and its arguments but the stream in 64-bit words (a float in the
  * low half), and anything behind them. On a copy of it, every patch {word, source, offset} puts addresses[source] + offset, or for
