@@ -257,6 +257,10 @@ int mi355x_log_softmax_f32(const float* X, float* Y,
                            int64_t outer, int64_t axis_len, int64_t inner,
                            void* stream);
 
+/* mi355x_softmax_f32 along the last axis with the largest value of each row beside it (what ReduceMax gives: NaN wins), [rows]: both read
+ * the same input. cols >= 1. */
+int mi355x_softmax_max_f32(const float* X, float* Y, float* largest, int64_t rows, int64_t cols, void* stream);
+
 /* Scaled-dot-product attention core, fp32, one launch:
  *   O[b0,b1] = softmax(scale * Q[b0,b1] K[b0,b1]^T, over keys) V[b0,b1]
  * Q, O are [Sq, D], K, V are [Sk, D] per (b0, b1) slice; the last dimension is
