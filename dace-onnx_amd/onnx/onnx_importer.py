@@ -24,7 +24,7 @@ import numpy as np
 import torch
 
 from .. import sdfg as dace
-from ..sdfg import SDFG, SDFGState, AccessNode
+from ..sdfg import SDFG, SDFGState, AccessNode, KernelCall
 from . import proto
 from .proto import ModelProto, TensorProto
 from .schema import ONNXParameterType
@@ -376,8 +376,15 @@ class ONNXModel:
             self.expand()
             from ..transformation.packing import pack_constant_operands, pack_variable_filters, pool_in_convolutions
             from ..transformation.partial_sums import split_products
-            split_products(self)
-            pool_in_convolutions(self)
+            from ..transformation.row_maxima import softmax_with_maxima
+            if self.fuse:
+                functions = {n.function for state in self.sdfg.nodes() for n in state.nodes() if isinstance(n, KernelCall)}
+                if "mi355x_layernorm_f32" in functions:
+                    split_products(self)
+                if "mi355x_maxpool2d_f32" in functions:
+                    pool_in_convolutions(self)
+                if "mi355x_reduce_f32" in functions:
+                    softmax_with_maxima(self.sdfg)
             self._packed = pack_constant_operands(self)
             pack_variable_filters(self.sdfg)
             self._compiled = self.sdfg.compile()
