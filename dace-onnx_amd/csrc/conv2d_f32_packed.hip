@@ -40,7 +40,11 @@ struct PackedConvArgs {
     int strips, strip_w, patch_h, patch_w, taps_h, step_h, step_w, sample_h, sample_w, pixels;
     FastDiv div_strips, div_strip, div_strip_w, div_patch_h, div_patch_w;
     int groups, stages;   // of 16 channels; of 16 CHUNK WAVES_K
+    // SKIP: a 1 x 1 convolution of another input with the same result, summed into the same sums
+    const float* X2; const float* W2; const float* bias2; const char* packed2;
+    int C2, H2, Wd2, stride2_h, stride2_w, groups2, stages2;   // (of 16 SKIP_CHUNK WAVES_K)
 };
+constexpr int SKIP_CHUNK = 2;
 
 // ROWS x COLUMNS: taps of the filter; PIXELS: C <= 4
 template <int ROWS, int COLUMNS, bool PIXELS>
@@ -49,7 +53,7 @@ struct PackedFilter {
     static constexpr int STEPS = ROWS * PER_ROW;   // MFMA steps of 16 k: of a group of channels, or of the whole filter
 };
 
-template <class FILTER, bool PIXELS, int TP, int WAVES_M, int WAVES_P, int WAVES_K, int CHUNK, int PER_T>
+template <class FILTER, bool PIXELS, int TP, int WAVES_M, int WAVES_P, int WAVES_K, int CHUNK, int PER_T, bool SKIP>
 __global__ __launch_bounds__(WAVES_M * WAVES_P * WAVES_K * WAVE, 2) void conv2d_f32_packed_kernel(PackedConvArgs pa) {
     const ConvArgs& p = pa.c;
     constexpr int THREADS = WAVES_M * WAVES_P * WAVES_K * WAVE, BP = 32 * TP * WAVES_P;
@@ -169,6 +173,42 @@ __global__ __launch_bounds__(WAVES_M * WAVES_P * WAVES_K * WAVE, 2) void conv2d_
         });
     };
 
+    // SKIP: the other input at the tile's positions, SKIP_CHUNK times 16 channels to a group of waves at a time: loaded under the products before,
+    // split into LDS (position by position, halves of 16 channels apart) when everyone has read what was there. (With the first of them loaded
+    // ahead of the taps, where there are registers for that, 8 images of 128 x 28 x 28 take 20.3 us instead of 19.0, one of 512 x 7 x 7 22.3
+    // instead of 22.6.) Bound by the loads and their latency: 3 us for 32 channels of a tile of 64 x 256, a fifth of it products.
+    constexpr int SKIP_THREADS = THREADS / WAVES_K, SKIP_UNITS = 2 * SKIP_CHUNK * BP, PER_2 = SKIP ? SKIP_UNITS / SKIP_THREADS : 1;
+    static_assert(!SKIP || SKIP_UNITS % SKIP_THREADS == 0, "whole units per thread");
+    const __amdgpu_buffer_rsrc_t x2_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(pa.X2), 0, 0x7fffffff, 0x00020000);
+    const __amdgpu_buffer_rsrc_t w2_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(pa.packed2), 0, 0x7fffffff, 0x00020000);
+    const int id2 = tid % SKIP_THREADS, plane2 = pa.H2 * pa.Wd2 * 4;
+    const uint32_t w2_block = (uint32_t)min(m0 / 32 + wm, blocks - 1) * (uint32_t)pa.groups2 * (uint32_t)PK_FRAGMENT;
+    f32x4 v2[PER_2][2];
+    bf16x8 fw2[SKIP_CHUNK][SP_PLANES];
+    auto load_w2 = [&](int stage) {
+        const int first = (stage * WAVES_K + wk) * SKIP_CHUNK;   // group of 16 channels
+#pragma unroll
+        for (int g = 0; g < SKIP_CHUNK; ++g)
+#pragma unroll
+            for (int q = 0; q < SP_PLANES; ++q)
+                fw2[g][q] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(w2_rsrc, lane * 16 + q * PK_PLANE,
+                                                                                           (int)(w2_block + (uint32_t)min(first + g, pa.groups2 - 1) * (uint32_t)PK_FRAGMENT), 0));
+    };
+    auto load_x2 = [&](int stage) {
+        const int first = (stage * WAVES_K + wk) * SKIP_CHUNK;
+#pragma unroll
+        for (int it = 0; it < PER_2; ++it) {
+            const int unit = id2 + it * SKIP_THREADS, c = 16 * first + 8 * (unit / BP);
+            uint32_t n, oy, ox;
+            output_of(min(p0 + unit % BP, (int)p.P - 1), n, oy, ox);
+            const uint32_t at_0 = 4u * (uint32_t)((((int)n * pa.C2 + c) * pa.H2 + (int)oy * pa.stride2_h) * pa.Wd2 + (int)ox * pa.stride2_w);
+            const uint32_t off = c < pa.C2 ? at_0 : OUT;   // C2 is a multiple of eight
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                v2[it][e / 4][e % 4] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(x2_rsrc, (int)off, e * plane2, 0));
+        }
+    };
+
 #pragma unroll
     for (int s = 0; s < RING; ++s) load_w(s, 0, s);
     if constexpr (PIXELS) {
@@ -244,6 +284,38 @@ __global__ __launch_bounds__(WAVES_M * WAVES_P * WAVES_K * WAVE, 2) void conv2d_
             multiply(stage);
         }
         if (WAVES_K > 1 && !late) sync();   // as many barriers for every wave
+    }
+
+    if constexpr (SKIP) {
+        load_x2(0);
+        load_w2(0);
+        for (int stage = 0; stage < pa.stages2; ++stage) {
+            __syncthreads();   // everyone has read its last units
+#pragma unroll
+            for (int it = 0; it < PER_2; ++it) {
+                u32x4 part[SP_PLANES];
+                split_unit8(v2[it][0], v2[it][1], part);
+#pragma unroll
+                for (int q = 0; q < SP_PLANES; ++q) *reinterpret_cast<u32x4*>(lds + (wk * SKIP_UNITS + id2 + it * SKIP_THREADS) * 48 + q * 16) = part[q];
+            }
+            __syncthreads();
+            if (stage + 1 < pa.stages2) load_x2(stage + 1);
+#pragma unroll
+            for (int g = 0; g < SKIP_CHUNK; ++g)
+#pragma unroll
+                for (int j = 0; j < TP; ++j) {
+                    const char* from = lds + (wk * SKIP_UNITS + (2 * g + lh) * BP + 32 * (wp * TP + j) + li) * 48;
+                    bf16x8 x[SP_PLANES];
+#pragma unroll
+                    for (int q = 0; q < SP_PLANES; ++q) x[q] = *reinterpret_cast<const bf16x8*>(from + q * 16);
+#pragma unroll
+                    for (int u = 0; u < PK_PRODUCTS; ++u) {
+                        f32x16& sum = u == 0 ? acc[j] : small[j];
+                        sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw2[g][PK_QA[u]], x[PK_QB[u]], sum, 0, 0, 0);
+                    }
+                }
+            if (stage + 1 < pa.stages2) load_w2(stage + 1);
+        }
     }
 
     // the sums of the groups, in order, into those of the first
@@ -352,6 +424,14 @@ __global__ __launch_bounds__(WAVES_M * WAVES_P * WAVES_K * WAVE, 2) void conv2d_
 #pragma unroll
                     for (int i = 0; i < CHANNELS * TAPS; ++i) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[i / 4][i % 4], xv[i], sum, 0, 0, 0);
                 }
+                if constexpr (SKIP) {   // eight channels at a time, the upper lanes' four further on
+                    const float* w2 = pa.W2 + (int64_t)m * pa.C2 + 4 * lh;
+                    const float* x2 = pa.X2 + (((int64_t)n * pa.C2 + 4 * lh) * pa.H2 + (int)oy * pa.stride2_h) * pa.Wd2 + (int)ox * pa.stride2_w;
+                    for (int c = 8 * wk; c < pa.C2; c += 8 * WAVES_K)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            sum = __builtin_amdgcn_mfma_f32_32x32x2f32(w2[c + e], x2[(int64_t)(c + e) * pa.H2 * pa.Wd2], sum, 0, 0, 0);
+                }
             }
             acc[j] = sum;
         }
@@ -368,6 +448,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_P * WAVES_K * WAVE, 2) void conv2d_
     for (int r = 0; r < 16; ++r) {
         const int m = mb + 8 * (r / 4) + 4 * lh + r % 4;
         bias[r] = (p.epi & MI355X_EPI_BIAS) && m < p.M ? p.bias[m] : 0.f;
+        if constexpr (SKIP) bias[r] += pa.bias2 && m < p.M ? pa.bias2[m] : 0.f;
     }
 #pragma unroll
     for (int j = 0; j < TP; ++j) {
@@ -424,17 +505,18 @@ __global__ void pack_conv_f32_kernel(const float* w, u32x4* packed, int M, int C
 // gemm_f32_packed.hip). Fitted over 370 layers of 1 to 32 images, 5 to 256 columns, 1 to 512 channels and 16 to 768 filters, 3 % off on
 // average; the pick is 2.5 % behind the fastest form over 144 others, up to 1.6 times for 1 x 1 and for few 7 x 7 filters.
 struct PackedConvCost { int per_t; double fixed, per_step, per_pixel, again, again_step, again_pixel; };
-struct PackedConvForm { int bm, bp, waves, waves_k; PackedConvCost kinds[3]; };
+// `skip`: nanoseconds of a stage of a 1 x 1 convolution that is summed too, from 21 ends of residual blocks.
+struct PackedConvForm { int bm, bp, waves, waves_k; double skip; PackedConvCost kinds[3]; };
 constexpr PackedConvForm kPackedConvForms[] = {
-    {64, 256, 4, 1, {{4, 6690, 3100, 328, 4980, 3590, 0}, {}, {6, 5450, 475, 84.5, 3160, 339, 59.9}}},
-    {64, 256, 8, 2, {{4, 7300, 6020, 355, 6280, 9650, 0}, {}, {}}},
-    {64, 128, 8, 2, {{4, 5760, 3210, 360, 3730, 5250, 0}, {}, {}}},
-    {64, 128, 4, 1, {{6, 4760, 1700, 312, 1870, 2250, 0}, {4, 4930, 499, 691, 3020, 263, 0}, {4, 4390, 241, 78, 1390, 212, 23.6}}},
-    {64, 64, 8, 4, {{6, 6010, 3150, 704, 3980, 5100, 0}, {}, {}}},
-    {32, 128, 8, 4, {{6, 5940, 3110, 706, 4130, 5550, 0}, {}, {}}},
-    {32, 64, 8, 4, {{6, 4570, 1700, 730, 2770, 3050, 107}, {4, 4780, 268, 1540, 2400, 93.3, 1720}, {}}},
-    {32, 32, 8, 8, {{8, 5450, 1250, 1730, 4090, 2660, 372}, {4, 4970, 0, 3640, 0, 0, 7770}, {}}},
-    {64, 64, 4, 1, {{6, 3640, 1070, 281, 1380, 1220, 20.4}, {4, 3520, 477, 549, 1090, 357, 88.1}, {4, 4380, 111, 0, 777, 129, 26.9}}}};
+    {64, 256, 4, 1, 3000, {{4, 6690, 3100, 328, 4980, 3590, 0}, {}, {6, 5450, 475, 84.5, 3160, 339, 59.9}}},
+    {64, 256, 8, 2, 3000, {{4, 7300, 6020, 355, 6280, 9650, 0}, {}, {}}},
+    {64, 128, 8, 2, 3000, {{4, 5760, 3210, 360, 3730, 5250, 0}, {}, {}}},
+    {64, 128, 4, 1, 1900, {{6, 4760, 1700, 312, 1870, 2250, 0}, {4, 4930, 499, 691, 3020, 263, 0}, {4, 4390, 241, 78, 1390, 212, 23.6}}},
+    {64, 64, 8, 4, 3000, {{6, 6010, 3150, 704, 3980, 5100, 0}, {}, {}}},
+    {32, 128, 8, 4, 4800, {{6, 5940, 3110, 706, 4130, 5550, 0}, {}, {}}},
+    {32, 64, 8, 4, 2900, {{6, 4570, 1700, 730, 2770, 3050, 107}, {4, 4780, 268, 1540, 2400, 93.3, 1720}, {}}},
+    {32, 32, 8, 8, 3500, {{8, 5450, 1250, 1730, 4090, 2660, 372}, {4, 4970, 0, 3640, 0, 0, 7770}, {}}},
+    {64, 64, 4, 1, 1150, {{6, 3640, 1070, 281, 1380, 1220, 20.4}, {4, 3520, 477, 549, 1090, 357, 88.1}, {4, 4380, 111, 0, 777, 129, 26.9}}}};
 constexpr int kNumPackedConvForms = sizeof(kPackedConvForms) / sizeof(kPackedConvForms[0]);
 
 enum { PC_3X3, PC_1X1, PC_7X7, PC_NONE };
@@ -447,12 +529,12 @@ static int packed_conv_kind(int64_t C, int64_t KH, int64_t KW, const int64_t* di
 static int packed_conv_chunk(int kind) { return kind == PC_1X1 ? 2 : 1; }
 static int packed_conv_steps(int kind) { return kind == PC_3X3 ? 9 : kind == PC_1X1 ? 1 : 14; }
 
-template <class FILTER, bool PIXELS, int CHUNK, int KIND>
+template <class FILTER, bool PIXELS, int CHUNK, int KIND, bool SKIP = false>
 static void launch_packed_conv(int form, const PackedConvArgs& pa, int lds, hipStream_t st) {
 #define MI355X_FORM(index, tp, wm, wp, wk)                                                                                             \
     case index:                                                                                                                        \
         if constexpr (kPackedConvForms[index].kinds[KIND].per_t > 0)                                                                   \
-            hipLaunchKernelGGL((conv2d_f32_packed_kernel<FILTER, PIXELS, tp, wm, wp, wk, CHUNK, kPackedConvForms[index].kinds[KIND].per_t>), \
+            hipLaunchKernelGGL((conv2d_f32_packed_kernel<FILTER, PIXELS, tp, wm, wp, wk, CHUNK, kPackedConvForms[index].kinds[KIND].per_t, SKIP>), \
                                dim3((unsigned)pa.c.nwg), dim3(wm * wp * wk * WAVE), lds, st, pa);                                      \
         break;
     switch (form) {
@@ -509,7 +591,7 @@ static void set_strips(PackedConvArgs& pa, int kind, int strip_w, int64_t pixels
 }
 
 // Bytes of LDS that a form needs for patches of `pixels`, 0 where it does not fit.
-static int packed_conv_lds(int kind, const PackedConvForm& f, int64_t pixels) {
+static int packed_conv_lds(int kind, const PackedConvForm& f, int64_t pixels, bool skip = false) {
     constexpr int64_t LDS_BYTES = 160 * 1024;
     const int per_t = f.kinds[kind].per_t;
     if (per_t == 0) return 0;
@@ -520,6 +602,7 @@ static int packed_conv_lds(int kind, const PackedConvForm& f, int64_t pixels) {
         bytes = halves * f.waves_k * pixels * 48;
     }
     bytes = std::max(bytes, (int64_t)(f.waves_k - 1) * f.bm * f.bp * 4);
+    if (skip) bytes = std::max(bytes, (int64_t)f.waves_k * 2 * SKIP_CHUNK * f.bp * 48);
     return bytes <= LDS_BYTES ? (int)bytes : 0;
 }
 
@@ -560,6 +643,8 @@ static bool packed_conv_args(PackedConvArgs& pa, int& kind, int64_t N, int64_t C
     return ceil_div(M, (int64_t)32) * pa.groups * packed_conv_steps(kind) * PK_FRAGMENT < ((int64_t)1 << 31);
 }
 
+static int64_t skip_stages(const PackedConvArgs& pa, const PackedConvForm& f) { return ceil_div((int64_t)pa.groups2, (int64_t)SKIP_CHUNK * f.waves_k); }
+
 static int64_t packed_conv_stages(const PackedConvArgs& pa, int kind, const PackedConvForm& f) {
     return ceil_div((int64_t)pa.groups, (int64_t)packed_conv_chunk(kind) * f.waves_k);
 }
@@ -591,10 +676,12 @@ static double unpacked_conv_cost(const ConvArgs& p, int cus, bool& summed_apart)
 // the gather kernel's estimate is up to a third too long for 1 x 1 filters, most for few of them). A form whose waves all sum the
 // same channels does not take over from the kernel that sums them apart: its error was up to 1.3 times as large there, everywhere else and
 // of the other forms it is 0.2 to 0.9 of the kernels' before.
-static int choose_packed_conv(PackedConvArgs& pa, int kind, int cus, double besides) {
+// `best_cost`: of what is chosen, either way. `skip`: the fastest form that sums a 1 x 1 convolution too, with that, whatever the kernels before take.
+static int choose_packed_conv(PackedConvArgs& pa, int kind, int cus, double besides, double& best_cost, bool skip = false) {
     const ConvArgs& p = pa.c;
     bool summed_apart;
-    double best_cost = (kind != PC_1X1 ? 0.9 : p.M > 64 ? 0.85 : 0.7) * unpacked_conv_cost(p, cus, summed_apart) - besides;
+    best_cost = (kind != PC_1X1 ? 0.9 : p.M > 64 ? 0.85 : 0.7) * unpacked_conv_cost(p, cus, summed_apart) - besides;
+    if (skip) best_cost = 1e300;
     int best = -1, last_bp = 0, strip_w = 0;
     int64_t pixels = 0;
     for (int bp : {256, 128, 64, 32})
@@ -603,14 +690,15 @@ static int choose_packed_conv(PackedConvArgs& pa, int kind, int cus, double besi
             if (f.bp != bp || (summed_apart && f.waves_k == 1)) continue;
             if (bp != last_bp) pixels = choose_strips(pa, kind, bp, strip_w);
             last_bp = bp;
-            if (!packed_conv_lds(kind, f, pixels)) continue;
+            if (!packed_conv_lds(kind, f, pixels, skip)) continue;
             const PackedConvCost& c = f.kinds[kind];
             const int64_t nwg = ceil_div((int64_t)p.M, (int64_t)f.bm) * ceil_div(p.P, (int64_t)f.bp), up = ceil_div(nwg, (int64_t)cus);
             const double more = up <= 6 ? (double)(up - 1) : (double)nwg / cus - 0.5;
             const bool few = kind == PC_7X7;
             const double stages = few ? 1 : (double)packed_conv_stages(pa, kind, f), steps = few ? packed_conv_steps(kind) : stages;
             const double patch = stages * (double)pixels / 100;
-            const double cost = c.fixed + c.per_step * steps + c.per_pixel * patch + more * (c.again + c.again_step * steps + c.again_pixel * patch);
+            double cost = c.fixed + c.per_step * steps + c.per_pixel * patch + more * (c.again + c.again_step * steps + c.again_pixel * patch);
+            if (skip) cost += (double)skip_stages(pa, f) * f.skip * (1 + 0.65 * more);
             if (cost < best_cost) { best = i; best_cost = cost; }
         }
     return best;
@@ -618,12 +706,27 @@ static int choose_packed_conv(PackedConvArgs& pa, int kind, int cus, double besi
 
 // The form that takes a call, -1 where mi355x_conv2d_res_f32 does: the fastest, or the one that is forced (MI355X_CONV_PACKED) if its
 // patch fits. With its strips, its patch's pixels and its LDS.
-static int packed_conv_form(PackedConvArgs& pa, int kind, int cus, double besides, int& strip_w, int64_t& pixels, int& lds) {
-    const int force = tuning().conv_packed, form = force >= 0 ? force - 1 : choose_packed_conv(pa, kind, cus, besides);
+static int packed_conv_form(PackedConvArgs& pa, int kind, int cus, double besides, int& strip_w, int64_t& pixels, int& lds, bool skip = false) {
+    double cost;
+    const int force = tuning().conv_packed, form = force >= 0 ? force - 1 : choose_packed_conv(pa, kind, cus, besides, cost, skip);
     if (form < 0 || form >= kNumPackedConvForms) return -1;
     pixels = choose_strips(pa, kind, kPackedConvForms[form].bp, strip_w);
-    lds = packed_conv_lds(kind, kPackedConvForms[form], pixels);
+    lds = packed_conv_lds(kind, kPackedConvForms[form], pixels, skip);
     return lds > 0 ? form : -1;
+}
+
+// The other input of a call with a 1 x 1 convolution summed too; false where the kernel does not take it. (After packed_conv_args.)
+static bool skip_args(PackedConvArgs& pa, int kind, int64_t C2, int64_t H2, int64_t Wd2, const int64_t* strides2) {
+    const ConvArgs& p = pa.c;
+    if (kind != PC_3X3 || C2 < 8 || C2 % 8 || C2 >= (1 << 24) || H2 < 1 || H2 >= (1 << 20) || Wd2 < 1 || Wd2 >= (1 << 20)) return false;
+    for (int i = 0; i < 2; ++i)
+        if (strides2[i] < 1 || strides2[i] >= (1 << 10)) return false;
+    if ((H2 - 1) / strides2[0] + 1 != p.OH || (Wd2 - 1) / strides2[1] + 1 != p.OW) return false;
+    const int64_t limit = (int64_t)1 << 29;
+    if (p.N * C2 >= limit || p.N * C2 * H2 >= limit || p.N * C2 * H2 * Wd2 >= limit) return false;
+    pa.C2 = (int)C2; pa.H2 = (int)H2; pa.Wd2 = (int)Wd2; pa.stride2_h = (int)strides2[0]; pa.stride2_w = (int)strides2[1];
+    pa.groups2 = (int)ceil_div(C2, (int64_t)16);
+    return ceil_div((int64_t)p.M, (int64_t)32) * pa.groups2 * PK_FRAGMENT < ((int64_t)1 << 31);
 }
 
 // Nanoseconds of mi355x_pack_conv_f32 before the convolution (512 x 256 filters of one tap 3.8 us, 768 x 512 of nine 16.5).
@@ -697,4 +800,68 @@ extern "C" int mi355x_conv2d_packed_f32(const float* X, const void* packed, cons
         }
     }
     return mi355x_conv2d_res_f32(X, W, bias, residual, Y, N, C, H, Wd, M, KH, KW, pads, strides, dilations, epilogue, stream);
+}
+
+extern "C" int mi355x_conv2d_skip_pays(int64_t N, int64_t C, int64_t H, int64_t Wd, int64_t M, int64_t KH, int64_t KW, const int64_t* pads,
+                                       const int64_t* strides, const int64_t* dilations, int64_t C2, int64_t H2, int64_t Wd2, const int64_t* strides2) {
+    using namespace mi355x;
+    PackedConvArgs pa = {}, pointwise = {};
+    int kind, kind2;
+    const int64_t none[4] = {0, 0, 0, 0}, ones[2] = {1, 1};
+    if (!pads || !strides || !dilations || !strides2 || !packed_conv_args(pa, kind, N, C, H, Wd, M, KH, KW, pads, strides, dilations) ||
+        !skip_args(pa, kind, C2, H2, Wd2, strides2) || !packed_conv_args(pointwise, kind2, N, C2, H2, Wd2, M, 1, 1, none, strides2, ones)) return 0;
+    int cus = device_cus();
+    if (cus <= 0) cus = 256;
+    if (tuning().conv_packed >= 0) {
+        int strip_w, lds;
+        int64_t pixels;
+        return packed_conv_form(pa, kind, cus, 0, strip_w, pixels, lds, true) >= 0;
+    }
+    double both, conv, alone;
+    if (choose_packed_conv(pa, kind, cus, 0, both, true) < 0) return 0;
+    choose_packed_conv(pa, kind, cus, 0, conv);
+    choose_packed_conv(pointwise, kind2, cus, 0, alone);
+    return both < conv + alone - 500;   // (one image: 128 x 28 x 28 13.5 us as two launches, 12.7 as one, 256 x 14 x 14 14.8 and 16.6; 32 images 57 and 49, 54 and 48)
+}
+
+extern "C" int mi355x_conv2d_skip_f32(const float* X, const float* W, const void* packed, const float* bias, const float* X2, const float* W2, const void* packed2,
+                                      const float* bias2, float* scratch, float* Y, int64_t N, int64_t C, int64_t H, int64_t Wd, int64_t M, int64_t KH, int64_t KW,
+                                      const int64_t* pads, const int64_t* strides, const int64_t* dilations, int64_t C2, int64_t H2, int64_t Wd2,
+                                      const int64_t* strides2, int epilogue, void* stream) {
+    using namespace mi355x;
+    MI355X_REQUIRE((epilogue & ~(MI355X_EPI_BIAS | MI355X_EPI_RELU_AFTER)) == 0, "conv2d_skip: unknown epilogue bits 0x%x", epilogue);
+    auto al16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+    PackedConvArgs pa = {};
+    ConvArgs& p = pa.c;
+    int kind;
+    if (X && W && Y && packed && X2 && W2 && packed2 && al16(packed) && al16(packed2) && pads && strides && dilations && strides2 &&
+        (!(epilogue & MI355X_EPI_BIAS) || bias) && packed_conv_args(pa, kind, N, C, H, Wd, M, KH, KW, pads, strides, dilations) &&
+        skip_args(pa, kind, C2, H2, Wd2, strides2)) {
+        const int cus = device_cus();
+        if (cus <= 0) return set_error(MI355X_ERR_NOT_INITIALIZED, "conv2d: no usable HIP device");
+        int strip_w, lds;
+        int64_t pixels;
+        const int form = packed_conv_form(pa, kind, cus, 0, strip_w, pixels, lds, true);
+        if (form >= 0) {
+            const PackedConvForm& f = kPackedConvForms[form];
+            p.X = X; p.W = W; p.bias = bias; p.Y = Y; p.epi = epilogue;
+            pa.X2 = X2; pa.W2 = W2; pa.packed2 = static_cast<const char*>(packed2); pa.bias2 = bias2;
+            p.tiles_m = ceil_div(M, (int64_t)f.bm);
+            p.tiles_p = ceil_div(p.P, (int64_t)f.bp);
+            p.nwg = p.tiles_m * p.tiles_p;
+            pa.packed = static_cast<const char*>(packed);
+            pa.stages = (int)packed_conv_stages(pa, kind, f);
+            pa.stages2 = (int)skip_stages(pa, f);
+            if (grid_fits(p.nwg, f.waves * WAVE)) {
+                set_strips(pa, kind, strip_w, pixels);
+                launch_packed_conv<PackedFilter<3, 3, false>, false, 1, 0, true>(form, pa, lds, static_cast<hipStream_t>(stream));
+                return check_launch("conv2d_f32_packed_kernel");
+            }
+        }
+    }
+    MI355X_REQUIRE(strides2 && scratch, "conv2d_skip: null pointer");
+    const int64_t none[4] = {0, 0, 0, 0}, ones[2] = {1, 1};
+    const int status = mi355x_conv2d_packed_f32(X2, packed2, W2, bias2, nullptr, scratch, N, C2, H2, Wd2, M, 1, 1, none, strides2, ones, bias2 ? MI355X_EPI_BIAS : 0, stream);
+    if (status != MI355X_OK) return status;
+    return mi355x_conv2d_packed_f32(X, packed, W, bias, scratch, Y, N, C, H, Wd, M, KH, KW, pads, strides, dilations, epilogue | MI355X_EPI_RESIDUAL, stream);
 }

@@ -99,6 +99,72 @@ def _packed_stem(call, desc):
     return ("stem_filters", [size // 3072, 3, 64, 4], "mi355x_pack_conv_pool_f32", (M, C, KH, KW), 0), (call.function, call.args[:2] + [Ptr("_packed")] + call.args[3:])
 
 
+def _packed_filters(call, desc, argument, connector, size, geometry):
+    """The packed copy of the filters that ``call`` takes as an argument, and the call that multiplies by it."""
+    if call.args[argument].offset or desc.shape != geometry or not desc.is_contiguous():
+        return None
+    args = call.args[:argument + 1] + [Ptr(connector)] + call.args[argument + 2:]
+    return ("filters", [size // 3072, 3, 64, 4], "mi355x_pack_conv_f32", geometry, 0), (call.function, args)
+
+
+def _packed_block(call, desc):
+    C, M = call.args[11], call.args[14]
+    return _packed_filters(call, desc, 1, "_packed", -(-M // 32) * -(-C // 16) * 9 * 3072, (M, C, 3, 3))
+
+
+def _packed_skip(call, desc):
+    C, M = call.args[20], call.args[14]
+    return _packed_filters(call, desc, 5, "_packed_skip", -(-M // 32) * -(-C // 16) * 3072, (M, C, 1, 1))
+
+
+def skip_in_convolutions(model):
+    """A convolution by constant filters whose residual is a 1 x 1 convolution by constant filters becomes one call with it, where the library says that
+    this pays."""
+    from ..onnx.onnx_importer import clean_onnx_name
+    sdfg, weights = model.sdfg, {clean_onnx_name(k) for k in model.weights}
+    constant = lambda state, call: _in_edge(state, call, call.args[1].connector).data.data in weights   # noqa: E731
+    for state in sdfg.nodes():
+        for call in state.nodes():
+            if not isinstance(call, KernelCall) or call.function != "mi355x_conv2d_res_f32":
+                continue
+            X, W, bias, residual, Y = call.args[:5]
+            epilogue = call.args[15]
+            source = _in_edge(state, call, residual.connector).src
+            made = _in_edge_of(state, source)
+            skip = made and made.src
+            if epilogue & ~(_lib.EPI_BIAS | _lib.EPI_RESIDUAL | _lib.EPI_RELU_AFTER) or not epilogue & _lib.EPI_RESIDUAL or residual.offset or Y.offset \
+                    or not isinstance(skip, KernelCall) or skip.function != "mi355x_conv2d_f32" or _single_consumer(sdfg, state, source) is None:
+                continue
+            X2, W2, bias2, Y2 = skip.args[:4]
+            N2, C2, H2, Wd2, M2, KH2, KW2, pads2, strides2, _, epilogue2 = skip.args[4:15]
+            geometry = call.args[5:15]
+            if (N2, M2, KH2, KW2) != (geometry[0], geometry[4], 1, 1) or any(pads2.values) or epilogue2 & ~_lib.EPI_BIAS or Y2.offset or X2.offset \
+                    or not constant(state, call) or not constant(state, skip):
+                continue
+            arrays = [_lib.i64_array(a.values) if isinstance(a, I64Array) else a for a in geometry]
+            if not _lib.library().mi355x_conv2d_skip_pays(*arrays, C2, H2, Wd2, _lib.i64_array(strides2.values)):
+                continue
+            moved = {"_skip_X": X2, "_skip_W": W2}
+            if epilogue2 & _lib.EPI_BIAS:
+                moved["_skip_B"] = bias2
+            edges = {new: _in_edge(state, skip, old.connector) for new, old in moved.items()}
+            both = KernelCall(call.label, "mi355x_conv2d_skip_f32",
+                              [X, W, Ptr(None), bias, Ptr("_skip_X"), Ptr("_skip_W", W2.offset), Ptr(None), Ptr("_skip_B", bias2.offset) if "_skip_B" in moved else Ptr(None),
+                               Ptr("_scratch"), Y] + geometry + [C2, H2, Wd2, strides2, epilogue & ~_lib.EPI_RESIDUAL, Stream()],
+                              [c for c in call.in_connectors if c != residual.connector] + list(moved), list(call.out_connectors) + ["_scratch"])
+            state.remove_edge(_in_edge(state, call, residual.connector))
+            state.remove_node(skip)
+            state.replace_node(call, both, sdfg)
+            for new, edge in edges.items():
+                state.add_edge(edge.src, None, both, new, edge.data)
+            state.add_edge(both, "_scratch", source, None, made.data)
+
+
+def _in_edge_of(state, access):
+    edges = state.in_edges(access) if isinstance(access, AccessNode) else []
+    return edges[0] if len(edges) == 1 else None
+
+
 def pool_in_convolutions(model):
     """A convolution by constant filters whose result only a MaxPool reads becomes one call with it, where the library has a kernel for both."""
     from ..onnx.onnx_importer import clean_onnx_name
@@ -131,7 +197,7 @@ def pack_variable_filters(sdfg):
     """Pack the filters of the remaining convolutions on every call, where the library says that this pays too."""
     for state in sdfg.nodes():
         for call in state.nodes():
-            packed = _by_packed_filters(call, False) if isinstance(call, KernelCall) and _PACKED.get(call.function) is _packed_conv else None
+            packed = _by_packed_filters(call, False) if isinstance(call, KernelCall) and call.function in ("mi355x_conv2d_f32", "mi355x_conv2d_res_f32") else None
             if packed is None:
                 continue
             shape, geometry, (function, args) = packed
@@ -147,8 +213,10 @@ def pack_variable_filters(sdfg):
             state.add_edge(access, None, packed_call, "_packed", sdfg.make_array_memlet(clean))
 
 
-_PACKED = {"mi355x_gemm_f32": _packed_gemm, "mi355x_gemm_parts_f32": _packed_gemm, "mi355x_conv2d_f32": _packed_conv, "mi355x_conv2d_res_f32": _packed_conv,
-           "mi355x_conv2d_pool_packed_f32": _packed_stem}
+# function -> of each operand that may be packed: the argument that is the weight, the name of the packed copy's connector, the function above
+_PACKED = {"mi355x_gemm_f32": [(1, "_packed", _packed_gemm)], "mi355x_gemm_parts_f32": [(1, "_packed", _packed_gemm)], "mi355x_conv2d_f32": [(1, "_packed", _packed_conv)],
+           "mi355x_conv2d_res_f32": [(1, "_packed", _packed_conv)], "mi355x_conv2d_pool_packed_f32": [(1, "_packed", _packed_stem)],
+           "mi355x_conv2d_skip_f32": [(1, "_packed", _packed_block), (5, "_packed_skip", _packed_skip)]}
 
 
 def pack_constant_operands(model):
@@ -164,29 +232,38 @@ def pack_constant_operands(model):
     for state in sdfg.nodes():
         written = {e.dst.data for e in state.edges() if isinstance(e.dst, AccessNode)}
         for call in state.nodes():
-            if not isinstance(call, KernelCall) or call.function not in _PACKED:
+            if not isinstance(call, KernelCall):
                 continue
-            edge = next(e for e in state.in_edges(call) if e.dst_conn == call.args[1].connector)
-            if edge.src.data not in by_clean or edge.src.data in written:
-                continue
-            weight_name = by_clean[edge.src.data]
-            desc = sdfg.arrays[edge.src.data]
-            if desc.dtype.name != "float32":
-                continue
-            packed = _PACKED[call.function](call, desc)
-            if packed is None:
-                continue
-            (suffix, *copy), (function, args) = packed
-            name = f"{weight_name}_packed_{suffix}"
-            clean = clean_onnx_name(name)
-            if clean not in sdfg.arrays:
-                copies.append(PackedOperand(model, weight_name, desc, now, clean, *copy))
-                sdfg.add_datadesc(clean, PackedCopy(int32, copies[-1].shape, copies[-1].derived))
-                if copies[-1].derived and copies[-1].packed is not None:
-                    model.weights.make(name, copies[-1].packed, derived=True)
-            packed_call = KernelCall(call.label, function, args, list(call.in_connectors) + ["_packed"], list(call.out_connectors))
-            state.replace_node(call, packed_call, sdfg)
-            state.add_edge(state.add_access(clean), None, packed_call, "_packed", sdfg.make_array_memlet(clean))
+            for argument, connector, packed_operand in _PACKED.get(call.function, ()):
+                call = _pack_operand(model, state, call, by_clean, written, argument, connector, packed_operand, now, copies)
     if copies and now:
         torch.cuda.current_stream().synchronize()   # later calls may come on other streams
     return copies
+
+
+def _pack_operand(model, state, call, by_clean, written, argument, connector, packed_operand, now, copies):
+    """``call``, or what stands in its place and multiplies by a packed copy of its operand; a copy that there was none of yet is added to ``copies``."""
+    from ..onnx.onnx_importer import clean_onnx_name
+    sdfg = model.sdfg
+    edge = next(e for e in state.in_edges(call) if e.dst_conn == call.args[argument].connector)
+    if edge.src.data not in by_clean or edge.src.data in written:
+        return call
+    weight_name = by_clean[edge.src.data]
+    desc = sdfg.arrays[edge.src.data]
+    if desc.dtype.name != "float32":
+        return call
+    packed = packed_operand(call, desc)
+    if packed is None:
+        return call
+    (suffix, *copy), (function, args) = packed
+    name = f"{weight_name}_packed_{suffix}"
+    clean = clean_onnx_name(name)
+    if clean not in sdfg.arrays:
+        copies.append(PackedOperand(model, weight_name, desc, now, clean, *copy))
+        sdfg.add_datadesc(clean, PackedCopy(int32, copies[-1].shape, copies[-1].derived))
+        if copies[-1].derived and copies[-1].packed is not None:
+            model.weights.make(name, copies[-1].packed, derived=True)
+    packed_call = KernelCall(call.label, function, args, list(call.in_connectors) + [connector], list(call.out_connectors))
+    state.replace_node(call, packed_call, sdfg)
+    state.add_edge(state.add_access(clean), None, packed_call, connector, sdfg.make_array_memlet(clean))
+    return packed_call

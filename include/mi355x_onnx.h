@@ -173,6 +173,19 @@ int mi355x_conv2d_packed_f32(const float* X, const void* packed, const float* W,
                              const int64_t* pads, const int64_t* strides,
                              const int64_t* dilations, int epilogue, void* stream);
 
+/* The end of a residual block whose other branch is a 1 x 1 convolution: mi355x_conv2d_packed_f32 by W plus the one by W2 [M, C2, 1, 1] of X2
+ * [N, C2, H2, Wd2] with strides2 and bias2 (or NULL), in one launch by both packed copies (mi355x_pack_conv_f32). `epilogue`: MI355X_EPI_BIAS
+ * (of W) and MI355X_EPI_RELU_AFTER. With a null copy, and where the kernel takes no such layer, two launches by way of `scratch`, laid out
+ * like Y. mi355x_conv2d_skip_pays: 1 where one launch is ahead of two. */
+int mi355x_conv2d_skip_pays(int64_t N, int64_t C, int64_t H, int64_t Wd, int64_t M, int64_t KH, int64_t KW,
+                            const int64_t* pads, const int64_t* strides, const int64_t* dilations,
+                            int64_t C2, int64_t H2, int64_t Wd2, const int64_t* strides2);
+int mi355x_conv2d_skip_f32(const float* X, const float* W, const void* packed, const float* bias, const float* X2, const float* W2,
+                           const void* packed2, const float* bias2, float* scratch, float* Y,
+                           int64_t N, int64_t C, int64_t H, int64_t Wd, int64_t M, int64_t KH, int64_t KW,
+                           const int64_t* pads, const int64_t* strides, const int64_t* dilations,
+                           int64_t C2, int64_t H2, int64_t Wd2, const int64_t* strides2, int epilogue, void* stream);
+
 /* Conv, Relu (or not) and MaxPool of an image classifier's stem in one launch, by W and its packed copy: 7 x 7 filters by two over three channels,
  * pooled 3 x 3 by two, no dilation. `epilogue`: MI355X_EPI_BIAS and MI355X_EPI_RELU. Elsewhere, and with a null `packed`, mi355x_conv2d_f32
  * into `scratch` [N, M, OH, OW], which is not written otherwise, and mi355x_maxpool2d_f32. mi355x_conv2d_pool_packed_pays: bytes of the
