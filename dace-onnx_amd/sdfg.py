@@ -458,9 +458,8 @@ class SDFGState:
         self._prune_dangling_reads()
 
     def _prune_dangling_reads(self):
-        for n in list(self._nodes):
-            if isinstance(n, AccessNode) and not self.in_edges(n) and not self.out_edges(n):
-                self._nodes.remove(n)
+        used = {id(n) for e in self._edges for n in (e.src, e.dst)}
+        self._nodes = [n for n in self._nodes if not isinstance(n, AccessNode) or id(n) in used]
 
     def topological_nodes(self):
         """Nodes in dependency order. Two access nodes of the same array are
