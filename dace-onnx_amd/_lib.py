@@ -45,6 +45,8 @@ SIGNATURES: typing.Dict[str, typing.Tuple[typing.Any, typing.List[typing.Any]]] 
     "mi355x_gemm_packed_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,
                                       _c_i64_p, _c_i64_p, _c_i64_p, _c_i64_p, _f32, _int, _vp]),
     "mi355x_pack_f32": (_int, [_vp, _vp, _i64, _i64, _i64, _i64, _vp]),
+    "mi355x_gemm_softmax_pays": (_int, [_i64, _i64, _i64, _int]),
+    "mi355x_gemm_softmax_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _int, _vp]),
     "mi355x_gemm_parts_f32": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _vp]),
     "mi355x_gemm_parts_packed_pays": (_int, [_i64, _i64, _i64, _i64, _int]),
     "mi355x_gemm_parts": (_i64, [_i64, _i64, _i64, _int, _int]),

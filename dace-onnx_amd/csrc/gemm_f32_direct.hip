@@ -16,9 +16,12 @@ namespace mi355x {
 constexpr int GD_WAVES = 16;
 
 // B_KC: B contiguous along k, columns n0 + 16 j + li. Otherwise along n, TN = 4: columns n0 + 4 li + j.
-template <int TM, int TN, bool B_KC>
+// SOFTMAX: N <= 16, the end of a classifier of few classes: the sixteen lanes that hold a row's results make its probabilities of them, and the launch
+// that would read them again (2.3 us and 3 of the host's for 5 x 10) is left out.
+template <int TM, int TN, bool B_KC, bool SOFTMAX = false>
 __global__ __launch_bounds__(WAVE * GD_WAVES) void gemm_f32_direct_kernel(GemmArgs p) {
     static_assert(B_KC || TN == 4, "one 16-byte load along n is four columns");
+    static_assert(!SOFTMAX || (TM == 1 && TN == 1 && B_KC), "whole rows in a tile");
     constexpr int TILES = TM * TN;
     constexpr int RING = TILES >= 8 ? 2 : B_KC ? 4 : 3;
     constexpr int NB = B_KC ? TN : 4;
@@ -130,10 +133,19 @@ __global__ __launch_bounds__(WAVE * GD_WAVES) void gemm_f32_direct_kernel(GemmAr
 #pragma unroll
         for (int j = 0; j < TN; ++j) red[wave][i * TN + j][lane] = acc[i][j];
     __syncthreads();
-    if (!stored) return;
+    if (SOFTMAX ? !sums : !stored) return;   // (a whole wave where its lanes go on together)
     f32x4 v = red[0][tile][lane];
 #pragma unroll
     for (int w = 1; w < GD_WAVES; ++w) v += red[w][tile][lane];
+    if constexpr (SOFTMAX) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float x = stored ? apply_epilogue(v[r] * p.alpha, p.epi, bias) : -INFINITY;
+            const float e = expf(x - row16_max(x)), s = row16_sum(e);   // (e of a column that is not there: 0)
+            if (stored && om + r < M) p.C[(int64_t)(om + r) * N + on] = e * (1.0f / s);
+        }
+        return;
+    }
     float* C = p.C + b0 * p.c_sb0 + b1 * p.c_sb1 + on;
 #pragma unroll
     for (int r = 0; r < 4; ++r)
@@ -202,3 +214,30 @@ bool launch_gemm_f32_direct(GemmArgs p, bool b_kc, double other_cost, int cus, h
 }
 
 }  // namespace mi355x
+
+// Up to 4096 rows: as many workgroups as CUs, which the kernel for few tiles is made for.
+extern "C" int mi355x_gemm_softmax_pays(int64_t M, int64_t N, int64_t K, int b_kc) { return M > 0 && M <= 4096 && N > 0 && N <= 16 && K >= 4 && b_kc; }
+
+extern "C" int mi355x_gemm_softmax_f32(const float* A, const float* B, const float* bias, float* scratch, float* Y, int64_t M, int64_t N, int64_t K,
+                                       int64_t a_row_stride, int64_t b_k_stride, int64_t b_column_stride, float alpha, int epilogue, void* stream) {
+    using namespace mi355x;
+    MI355X_REQUIRE(M >= 0 && N >= 0 && K >= 0, "gemm_softmax: negative extent (M=%lld N=%lld K=%lld)", (long long)M, (long long)N, (long long)K);
+    MI355X_REQUIRE((epilogue & ~(MI355X_EPI_BIAS | MI355X_EPI_RELU | MI355X_EPI_GELU)) == 0, "gemm_softmax: unknown epilogue bits 0x%x", epilogue);
+    MI355X_REQUIRE(!(epilogue & MI355X_EPI_BIAS) || bias, "gemm_softmax: MI355X_EPI_BIAS without bias");
+    if (M == 0 || N == 0) return MI355X_OK;
+    if (A && B && Y && a_row_stride >= 0 && b_column_stride >= 0 && mi355x_gemm_softmax_pays(M, N, K, b_k_stride == 1) &&
+        (M - 1) * a_row_stride + K < ((int64_t)1 << 29) && (N - 1) * b_column_stride + K < ((int64_t)1 << 29)) {
+        GemmArgs p = {};
+        MI355X_TRACE_INIT(p);
+        p.A = A; p.B = B; p.C = Y; p.bias = bias;
+        p.batch = p.batch1 = 1; p.M = M; p.N = N; p.K = K;
+        p.a_sm = a_row_stride; p.a_sk = 1; p.b_sk = 1; p.b_sn = b_column_stride; p.c_sm = N;
+        p.alpha = alpha; p.epi = epilogue;
+        p.tiles_m = ceil_div(M, (int64_t)16); p.tiles_n = 1; p.nwg = p.tiles_m;
+        hipLaunchKernelGGL((gemm_f32_direct_kernel<1, 1, true, true>), dim3((unsigned)p.nwg), dim3(WAVE * GD_WAVES), 0, static_cast<hipStream_t>(stream), p);
+        return check_launch("gemm_f32_direct_kernel");
+    }
+    const int64_t a[4] = {0, 0, a_row_stride, 1}, b[4] = {0, 0, b_k_stride, b_column_stride}, c[3] = {0, 0, N};
+    const int status = mi355x_gemm_f32(A, B, scratch, bias, nullptr, 1, 1, M, N, K, a, b, c, nullptr, alpha, epilogue, stream);
+    return status != MI355X_OK ? status : mi355x_softmax_f32(scratch, Y, M, N, 1, stream);
+}

@@ -376,7 +376,7 @@ class ONNXModel:
             self.expand()
             from ..transformation.packing import pack_constant_operands, pack_variable_filters, pool_in_convolutions, skip_in_convolutions
             from ..transformation.partial_sums import split_products
-            from ..transformation.row_maxima import softmax_with_maxima
+            from ..transformation.softmax_fusion import softmax_of_products, softmax_with_maxima
             if self.fuse:
                 functions = {n.function for state in self.sdfg.nodes() for n in state.nodes() if isinstance(n, KernelCall)}
                 if "mi355x_layernorm_f32" in functions:
@@ -385,8 +385,10 @@ class ONNXModel:
                     skip_in_convolutions(self)
                 if "mi355x_maxpool2d_f32" in functions:
                     pool_in_convolutions(self)
-                if "mi355x_reduce_f32" in functions:
-                    softmax_with_maxima(self.sdfg)
+                if "mi355x_softmax_f32" in functions:
+                    softmax_of_products(self)
+                    if "mi355x_reduce_f32" in functions:
+                        softmax_with_maxima(self.sdfg)
             self._packed = pack_constant_operands(self)
             pack_variable_filters(self.sdfg)
             self._compiled = self.sdfg.compile()

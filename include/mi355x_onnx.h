@@ -102,6 +102,13 @@ int mi355x_gemm_f32(const float* A, const float* B, float* C,
                     const int64_t* c_strides, const int64_t* r_strides,
                     float alpha, int epilogue, void* stream);
 
+/* Y = softmax(epilogue(alpha A B)) over each row, [M, N] contiguous, A contiguous along k; `epilogue` of MI355X_EPI_BIAS, MI355X_EPI_RELU and
+ * MI355X_EPI_GELU. One launch where mi355x_gemm_softmax_pays says 1 (few classes; b_kc: B contiguous along k), elsewhere mi355x_gemm_f32 into
+ * `scratch` [M, N], which is not written otherwise, and mi355x_softmax_f32. */
+int mi355x_gemm_softmax_pays(int64_t M, int64_t N, int64_t K, int b_kc);
+int mi355x_gemm_softmax_f32(const float* A, const float* B, const float* bias, float* scratch, float* Y, int64_t M, int64_t N, int64_t K,
+                            int64_t a_row_stride, int64_t b_k_stride, int64_t b_column_stride, float alpha, int epilogue, void* stream);
+
 /* The same product with a B that is constant, [K, N] without batch dimensions, and was packed beforehand for the bf16
  * matrix unit (three bf16 parts of every value, in the order the kernel's registers take them; ONNX nodes do it once when the
  * graph is prepared, transformation/packing.py, and the reference has no counterpart). `packed` holds, 6144 bytes each,
