@@ -15,6 +15,8 @@
 // 180 -> 144 us (201 TFLOP/s), 8192 x 768 x 768 65 -> 52, 8192 x 3072 x 768 222 -> 178, 8192 x 768 x 3072 228 -> 187,
 // 1024 x 30522 x 768 297 -> 235, 1500 x 1024 x 4096 135 -> 74, 1024 x 2304 x 768 36.5 -> 28.8, 1024 x 3072 x 768 42.4 -> 31.4,
 // 1024 x 768 x 3072 41.5 -> 37.5, 128 x 2304 x 768 12.3 -> 8.6, 373 x 1024 x 256 7.4 -> 6.1; 187 products of 8 to 16384 rows 0.84 of the time.
+// Twelve waves over 128 x 192 fill the chip evenly where the wider tiles do not (192 columns divide 768, 2304 and 3072): 8192 x 768 x 768 51.5 -> 47.7 us,
+// 8192 x 2304 x 768 144 -> 138, 2151 x 2304 x 768 46.1 -> 41.5, 1505 x 3072 x 768 45.3 -> 39.5.
 // Its error against float64 is smaller than theirs: 0.8e-7 (2-norm) where the fp32 MFMA has 5.0e-7 and 16 x 16 x 32 1.6e-7 (K = 768).
 // Tried: B two steps ahead instead of one and A two (even), B's fragments through LDS, A packed beforehand too (its loads are half as
 // long again: even), loads and splits placed between the MFMAs by hand (even or behind).
@@ -43,8 +45,8 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * WAVES_K * WAVE, PER_SIMD) void 
     constexpr int GROUP = BM / 32 * 2 * PK_FRAGMENT, STAGE = WAVES_K * GROUP;      // bytes of a 32-k tile of A; of all groups' tiles
     constexpr int BLOCKS = BM * BN / 1024;                                        // 32 x 32 blocks of the workgroup's tile
     constexpr int SUMS = WAVES_K > 1 ? WAVES_K * BLOCKS * 4096 : 0;
-    constexpr int UNITS = BM * 4 * WAVES_K, PER_T = UNITS / THREADS;
-    static_assert(UNITS % THREADS == 0 && THREADS % (4 * WAVE) == 0, "whole units per thread");
+    constexpr int UNITS = BM * 4 * WAVES_K, PER_T = (UNITS + THREADS - 1) / THREADS;
+    static_assert((UNITS % THREADS == 0 || UNITS < THREADS) && UNITS % WAVE == 0 && THREADS % (4 * WAVE) == 0, "whole units per thread, or one for some waves");
     __shared__ __attribute__((aligned(16))) char lds[2 * STAGE > SUMS ? 2 * STAGE : SUMS];
 
     const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
@@ -80,7 +82,9 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * WAVES_K * WAVE, PER_SIMD) void 
     }
     const int steps = (pa.kt + WAVES_K - 1) / WAVES_K;
     f32x4 va[PER_T][2];
+    const bool loads = UNITS >= THREADS || tid < UNITS;   // (uniform)
     auto load_a = [&](int it, int st) {
+        if (!loads) return;
         uint32_t off = a_off[it];
         if constexpr (WAVES_K > 1) {   // a group that has no tile in the last step multiplies zeros
             const int kg = (tid + it * THREADS) / 4 / BM;
@@ -91,6 +95,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * WAVES_K * WAVE, PER_SIMD) void 
         for (int h = 0; h < 2; ++h) va[it][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, (int)(off + 64u * h), base, 0));
     };
     auto store_a = [&](char* stage, int it) {
+        if (!loads) return;
         u32x4 part[SP_PLANES];
         split_unit8(va[it][0], va[it][1], part);
 #pragma unroll
@@ -377,7 +382,10 @@ static const PackedForm kPackedForms[] = {
     {128, 256, 512, 1, 8440, 56.0, 7580, 64.7}, {64, 256, 256, 2, 5220, 35.8, 3290, 30.8}, {64, 192, 512, 1, 7490, 25.8, 5920, 29.7},
     {64, 128, 512, 1, 4900, 16.5, 2570, 17.5},  {64, 64, 512, 1, 5180, 8.85, 3530, 12.1},  {64, 64, 256, 3, 3870, 15.0, 860, 10.6},
     {32, 64, 512, 1, 4260, 5.5, 1290, 6.25},    {32, 32, 512, 1, 4730, 3.69, 2050, 5.7},   {128, 128, 256, 2, 6040, 35.6, 3120, 31.7},
-    {64, 128, 256, 2, 3660, 21.0, 1900, 16.2}};
+    {64, 128, 256, 2, 3660, 21.0, 1900, 16.2},
+    {128, 192, 768, 1, 7600, 52.0, 2800, 53.5}};
+constexpr int TWELVE_WAVES = 10;
+constexpr int kPackedGroups[] = {1, 1, 2, 2, 4, 1, 4, 8, 1, 1, 1};   // of waves that share K
 constexpr int kNumPackedForms = sizeof(kPackedForms) / sizeof(kPackedForms[0]);
 
 static void launch_packed(int form, const PackedGemmArgs& p, hipStream_t st) {
@@ -392,6 +400,7 @@ static void launch_packed(int form, const PackedGemmArgs& p, hipStream_t st) {
         case 6: hipLaunchKernelGGL((gemm_f32_packed_kernel<1, 1, 1, 2, 4, 2>), grid, block, 0, st, p); break;
         case 8: hipLaunchKernelGGL((gemm_f32_packed_kernel<2, 2, 2, 2, 1, 2>), grid, block, 0, st, p); break;
         case 9: hipLaunchKernelGGL((gemm_f32_packed_kernel<2, 1, 1, 4, 1, 2>), grid, block, 0, st, p); break;
+        case 10: hipLaunchKernelGGL((gemm_f32_packed_kernel<2, 1, 2, 6, 1, 3>), grid, block, 0, st, p); break;
         default: hipLaunchKernelGGL((gemm_f32_packed_kernel<1, 1, 1, 1, 8, 2>), grid, block, 0, st, p); break;
     }
 }
@@ -440,6 +449,9 @@ static int choose_packed(const GemmArgs& p, int cus, double& best_cost) {
     if (p.M <= 32) best_cost *= 0.8;
     int best = -1;
     for (int f = 0; f < kNumPackedForms; ++f) {
+        // Twelve waves sum K in one go. In place of groups that share it their error is up to 1.4 times as large (a layer of 8192 x 768 x 3072 that is
+        // 7 % faster so stays with two groups for it).
+        if (f == TWELVE_WAVES && (best < 0 || kPackedGroups[best] > 1 || p.K < 512)) continue;   // (2048 x 13720 x 256 91 us so, 80)
         const PackedForm& form = kPackedForms[f];
         const double cost = packed_cost(form, p.batch * ceil_div(p.M, (int64_t)form.bm) * ceil_div(p.N, (int64_t)form.bn), p.K, cus);
         if (cost < best_cost) { best = f; best_cost = cost; }
@@ -463,6 +475,7 @@ static int choose_part(const GemmArgs& p, bool packed, int cus, double& best_cos
     if (!packed || !packed_takes(p) || force >= 0 || p.M <= 16) return -1;
     int best = -1;
     for (int f = 0; f < kNumPackedForms; ++f) {
+        if (f == TWELVE_WAVES) continue;   // (parts are for few tiles)
         const PackedForm& form = kPackedForms[f];
         const double cost = packed_cost(form, p.batch * ceil_div(p.M, (int64_t)form.bm) * ceil_div(p.N, (int64_t)form.bn), p.K, cus) * (p.M <= 32 ? 1.25 : 1);
         if (cost < best_cost) { best = f; best_cost = cost; }
@@ -541,9 +554,10 @@ extern "C" int mi355x_gemm_packed_f32(const float* A, const void* packed, const 
 }
 
 // Between one and eight parts, of at least 256 k each, by the estimates of the kernels and what the normalization takes longer to read them.
-// Over 49 products of 1 to 2048 rows the pick takes 0.82 of the time in one part, normalization included, and is nowhere more than 2 % behind it.
+// What the sums' bytes cost is three times what a warm measurement says: a program whose weights do not fit the memory-side cache pays for every further
+// byte there (an encoder layer over 1024 tokens with FFN2 in four parts 117 us over one set of weights, 122 in one part, but 131 against 128 over three).
 // Both launches, weights from beyond the L2: 16 x 768 x 3072 16.0 us in one part, 8.9 in eight; 128 rows 21.7, 12.9 in four; 512 rows 28.9, 22.5 in
-// four; 865 rows 39.7, 30.3 in three; 1024 rows 40.3, 35.2 in four; 16 x 1024 x 4096 19.6, 9.9 in eight; 128 x 768 x 768 9.9, 9.3 in three.
+// four; 865 rows 39.7, 30.3 in three; 16 x 1024 x 4096 19.6, 9.9 in eight; 16 x 768 x 768 8.0, 7.1 in three. None of 49 products is behind one part.
 extern "C" int64_t mi355x_gemm_parts(int64_t M, int64_t N, int64_t K, int b_kc, int packed) {
     using namespace mi355x;
     if (M <= 0 || N <= 0 || K <= 0 || N % 4 || N > 1024) return 1;
@@ -562,7 +576,7 @@ extern "C" int64_t mi355x_gemm_parts(int64_t M, int64_t N, int64_t K, int b_kc, 
         p.batch = parts; p.K = K / parts;
         double cost;
         choose_part(p, packed, cus, cost);
-        cost += 200.0 + 50.0 * (double)parts + 4.0 * (double)parts * (double)M * (double)N / 10000.0;
+        cost += 200.0 + 50.0 * (double)parts + 4.0 * (double)parts * (double)M * (double)N / 3000.0;
         if (cost < best_cost) { best = parts; best_cost = cost; }
     }
     return best;

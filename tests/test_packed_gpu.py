@@ -267,3 +267,14 @@ def test_a_first_call_under_stream_capture():
         graph.replay()
         assert close(y, x, weight)
     assert close(model(x), x, weight)
+
+
+@pytest.mark.parametrize("kc", [True, False])
+@pytest.mark.parametrize("batch, M, N, K, epi", [(1, 1, 1, 32, 0), (1, 127, 193, 64, 1), (2, 129, 191, 160, 13), (1, 300, 400, 768, 9), (3, 96, 577, 1056, 8)])
+def test_gemm_by_twelve_waves(tuning, kc, batch, M, N, K, epi):
+    """128 x 192 tiles, whose rows eight of the twelve waves load."""
+    test_gemm_by_a_packed_constant(tuning, 11, kc, batch, M, N, K, epi)
+
+
+def test_gemm_by_twelve_waves_keeps_infinities_nan_and_the_largest_values(tuning):
+    test_gemm_by_a_packed_constant_keeps_infinities_nan_and_the_largest_values(tuning, 11)
