@@ -39,7 +39,8 @@ struct PackedConvArgs {
     // samples the input at `sample` times its place, positions are `step` pixels apart; `pixels` is the most that a tile's patch has.
     int strips, strip_w, patch_h, patch_w, taps_h, step_h, step_w, sample_h, sample_w, pixels;
     FastDiv div_strips, div_strip, div_strip_w, div_patch_h, div_patch_w;
-    int groups, stages;   // of 16 channels; of 16 CHUNK WAVES_K
+    int groups, stages;   // of 16 channels; of 16 CHUNK WAVES_K (in a part of the channels, if they are summed in parts)
+    int64_t part_size;    // outputs of a part, one after the other
     // SKIP: a 1 x 1 convolution of another input with the same result, summed into the same sums
     const float* X2; const float* W2; const float* bias2; const char* packed2;
     int C2, H2, Wd2, stride2_h, stride2_w, groups2, stages2;   // (of 16 SKIP_CHUNK WAVES_K)
@@ -65,7 +66,8 @@ __global__ __launch_bounds__(WAVES_M * WAVES_P * WAVES_K * WAVE, 2) void conv2d_
     const int li = lane % 32, lh = lane / 32;
     const int wm = wave % WAVES_M, wp = wave / WAVES_M % WAVES_P, wk = wave / (WAVES_M * WAVES_P);
     // consecutive tiles share their positions
-    const uint32_t logical = (uint32_t)xcd_remap(blockIdx.x, p.nwg);
+    const uint32_t number = (uint32_t)xcd_remap(blockIdx.x, p.nwg), tiles = (uint32_t)(p.tiles_m * p.tiles_p), part = number / tiles, logical = number - part * tiles;
+    const int stage0 = PIXELS ? 0 : (int)part * pa.stages, stage_end = stage0 + pa.stages;
     const int m0 = (int)(logical % (uint32_t)p.tiles_m) * 32 * WAVES_M;
     const int p0 = (int)(logical / (uint32_t)p.tiles_m) * BP;
 
@@ -210,7 +212,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_P * WAVES_K * WAVE, 2) void conv2d_
     };
 
 #pragma unroll
-    for (int s = 0; s < RING; ++s) load_w(s, 0, s);
+    for (int s = 0; s < RING; ++s) load_w(s, stage0, s);
     if constexpr (PIXELS) {
         // the whole patch at once, in turns of PER_T units per thread
         for (int first = tid; first < pixels; first += PER_T * THREADS) {
@@ -265,10 +267,10 @@ __global__ __launch_bounds__(WAVES_M * WAVES_P * WAVES_K * WAVE, 2) void conv2d_
                     v[it][e / 4][e % 4] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(x_rsrc, (int)off, (first + e) * plane, 0));
             }
         };
-        load_x(0);
+        load_x(stage0);
         if (late) sync();
-        for (int stage = 0; stage < pa.stages; ++stage) {
-            if (stage) sync();   // the group has read its last channels
+        for (int stage = stage0; stage < stage_end; ++stage) {
+            if (stage != stage0) sync();   // the group has read its last channels
 #pragma unroll
             for (int it = 0; it < PER_T; ++it) {
                 if (it * GROUP_THREADS >= units) break;
@@ -280,7 +282,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_P * WAVES_K * WAVE, 2) void conv2d_
                 }
             }
             sync();
-            if (stage + 1 < pa.stages) load_x(stage + 1);
+            if (stage + 1 < stage_end) load_x(stage + 1);
             multiply(stage);
         }
         if (WAVES_K > 1 && !late) sync();   // as many barriers for every wave
@@ -407,7 +409,8 @@ __global__ __launch_bounds__(WAVES_M * WAVES_P * WAVES_K * WAVE, 2) void conv2d_
                     const bool in = (unsigned)y < (unsigned)p.H && (unsigned)x < (unsigned)p.Wd;
                     x_first[t] = in ? 4u * (uint32_t)(((int)n * p.C * p.H + y) * p.Wd + x) + (uint32_t)(lh * CHANNELS) * (uint32_t)plane : OUT;
                 }
-                for (int c = 2 * CHANNELS * wk; c < p.C; c += 2 * CHANNELS * WAVES_K) {
+                const int c_end = min(p.C, stage_end * 16 * CHUNK * WAVES_K);
+                for (int c = stage0 * 16 * CHUNK * WAVES_K + 2 * CHANNELS * wk; c < c_end; c += 2 * CHANNELS * WAVES_K) {
                     f32x4 wv[CHANNELS * TAPS / 4];
                     float xv[CHANNELS * TAPS];
 #pragma unroll
@@ -440,7 +443,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_P * WAVES_K * WAVE, 2) void conv2d_
     if (wk > 0) return;
 
     // acc[j][r]: filter 8 (r / 4) + 4 lh + r % 4 of the block, position li
-    const __amdgpu_buffer_rsrc_t y_rsrc = __builtin_amdgcn_make_buffer_rsrc(p.Y, 0, 0x7fffffff, 0x00020000);
+    const __amdgpu_buffer_rsrc_t y_rsrc = __builtin_amdgcn_make_buffer_rsrc(p.Y + part * pa.part_size, 0, 0x7fffffff, 0x00020000);
     const __amdgpu_buffer_rsrc_t r_rsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.epi & MI355X_EPI_RESIDUAL ? p.residual : p.Y), 0, 0x7fffffff, 0x00020000);
     float bias[16];
@@ -474,6 +477,34 @@ __global__ __launch_bounds__(WAVES_M * WAVES_P * WAVES_K * WAVE, 2) void conv2d_
             if (p.epi & MI355X_EPI_RELU_AFTER) o = fmaxf(o, 0.f);
             __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, o), y_rsrc, (int)off[r], 0, 0);
         }
+    }
+}
+
+// The sums of a convolution that was computed in parts of its channels, with its epilogue; MEAN: and the mean over the positions, all that a
+// global pooling after it keeps. One wave to a row of positions; bound by the launch and one trip to memory (512 rows of 49 in four parts 2.9 us).
+template <bool MEAN>
+__global__ __launch_bounds__(256) void conv_parts_kernel(const float* __restrict__ P, int parts, const float* __restrict__ bias, const float* __restrict__ residual,
+                                                         float* __restrict__ Y, int64_t rows, int M, int positions, int epi) {
+    const int lane = threadIdx.x % WAVE;
+    const int64_t row = (int64_t)blockIdx.x * (256 / WAVE) + threadIdx.x / WAVE, size = rows * positions;
+    if (row >= rows) return;   // (a whole wave)
+    const float b = epi & MI355X_EPI_BIAS ? bias[row % M] : 0.f;
+    float total = 0.f;
+    for (int at = lane; at < positions; at += WAVE) {
+        const int64_t i = row * positions + at;
+        float v[4], res = epi & MI355X_EPI_RESIDUAL ? residual[i] : 0.f;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) v[s] = s < parts ? P[s * size + i] : 0.f;
+        float o = (v[0] + v[1]) + (v[2] + v[3]) + b;
+        if (epi & MI355X_EPI_RELU) o = fmaxf(o, 0.f);
+        o += res;
+        if (epi & MI355X_EPI_RELU_AFTER) o = fmaxf(o, 0.f);
+        if constexpr (MEAN) total += o;
+        else Y[i] = o;
+    }
+    if constexpr (MEAN) {
+        total = wave_sum(total);
+        if (lane == 0) Y[row] = total * (1.0f / (float)positions);
     }
 }
 
@@ -729,6 +760,32 @@ static bool skip_args(PackedConvArgs& pa, int kind, int64_t C2, int64_t H2, int6
     return ceil_div((int64_t)p.M, (int64_t)32) * pa.groups2 * PK_FRAGMENT < ((int64_t)1 << 31);
 }
 
+// The same in parts of the channels, whose sums a launch of its own adds up (`mean`: in place of one that takes their mean): the form, its parts and their time.
+// For one or a few images, of which the last layers are a few tiles with long sums; up to 256 positions, which a wave of the launch that adds up goes
+// through in turns. Weights from beyond the L2: 1 x 512 x 7 x 7 -> 512 18.5 us in one part, 12.5 in four (with the mean after it 20.7 and 12.7), 1 x 256 x
+// 14 x 14 -> 512 by two 12.7 and 11.3, 2 x 256 x 14 x 14 -> 256 13.2 and 11.8, 4 x 512 x 7 x 7 22.8 and 14.4. Of 20 layers none is behind.
+static int choose_conv_parts(PackedConvArgs& pa, int kind, int cus, bool mean, int& parts, double& best_cost) {
+    const ConvArgs& p = pa.c;
+    int best = -1, strip_w = 0;
+    best_cost = 1e300;
+    if (kind != PC_3X3 || p.OHW > 256) return -1;
+    for (int i = 0; i < kNumPackedConvForms; ++i) {
+        const PackedConvForm& f = kPackedConvForms[i];
+        const int64_t pixels = choose_strips(pa, kind, f.bp, strip_w), all = packed_conv_stages(pa, kind, f);
+        if (f.waves_k == 1 || !packed_conv_lds(kind, f, pixels)) continue;   // (forms whose groups share the channels: no more error than the kernels before)
+        for (const int n : {2, 4}) {
+            if (all % n || pa.groups % (n * f.waves_k)) continue;
+            const PackedConvCost& c = f.kinds[kind];
+            const int64_t nwg = n * ceil_div((int64_t)p.M, (int64_t)f.bm) * ceil_div(p.P, (int64_t)f.bp), up = ceil_div(nwg, (int64_t)cus);
+            const double more = up <= 6 ? (double)(up - 1) : (double)nwg / cus - 0.5, stages = (double)(all / n), patch = stages * (double)pixels / 100;
+            const double sums = (mean ? 300 : 2300) + 4.0 * (n + 2) * (double)p.M * (double)p.P / 2000.0;
+            const double cost = c.fixed + c.per_step * stages + c.per_pixel * patch + more * (c.again + c.again_step * stages + c.again_pixel * patch) + sums;
+            if (cost < best_cost) { best = i; parts = n; best_cost = cost; }
+        }
+    }
+    return best;
+}
+
 // Nanoseconds of mi355x_pack_conv_f32 before the convolution (512 x 256 filters of one tap 3.8 us, 768 x 512 of nine 16.5).
 constexpr double PACKING = 3000, PACKING_PER_WEIGHT = 0.004;
 
@@ -864,4 +921,65 @@ extern "C" int mi355x_conv2d_skip_f32(const float* X, const float* W, const void
     const int status = mi355x_conv2d_packed_f32(X2, packed2, W2, bias2, nullptr, scratch, N, C2, H2, Wd2, M, 1, 1, none, strides2, ones, bias2 ? MI355X_EPI_BIAS : 0, stream);
     if (status != MI355X_OK) return status;
     return mi355x_conv2d_packed_f32(X, packed, W, bias, scratch, Y, N, C, H, Wd, M, KH, KW, pads, strides, dilations, epilogue | MI355X_EPI_RESIDUAL, stream);
+}
+
+extern "C" int64_t mi355x_conv2d_parts(int64_t N, int64_t C, int64_t H, int64_t Wd, int64_t M, int64_t KH, int64_t KW, const int64_t* pads,
+                                       const int64_t* strides, const int64_t* dilations, int mean) {
+    using namespace mi355x;
+    PackedConvArgs pa = {};
+    int kind, parts = 1;
+    if (!pads || !strides || !dilations || !packed_conv_args(pa, kind, N, C, H, Wd, M, KH, KW, pads, strides, dilations) || tuning().conv_packed >= 0) return 1;
+    int cus = device_cus();
+    if (cus <= 0) cus = 256;
+    double apart, whole;
+    if (choose_conv_parts(pa, kind, cus, mean, parts, apart) < 0) return 1;
+    choose_packed_conv(pa, kind, cus, 0, whole);
+    return apart < whole ? parts : 1;
+}
+
+extern "C" int mi355x_conv2d_parts_f32(const float* X, const float* W, const void* packed, const float* bias, const float* residual, float* P, float* Y, int64_t N,
+                                       int64_t C, int64_t H, int64_t Wd, int64_t M, int64_t KH, int64_t KW, const int64_t* pads, const int64_t* strides,
+                                       const int64_t* dilations, int epilogue, int mean, void* stream) {
+    using namespace mi355x;
+    MI355X_REQUIRE((epilogue & ~(MI355X_EPI_BIAS | MI355X_EPI_RELU | MI355X_EPI_RESIDUAL | MI355X_EPI_RELU_AFTER)) == 0, "conv2d_parts: unknown epilogue bits 0x%x", epilogue);
+    MI355X_REQUIRE((!(epilogue & MI355X_EPI_BIAS) || bias) && (!(epilogue & MI355X_EPI_RESIDUAL) || residual), "conv2d_parts: null bias or residual");
+    PackedConvArgs pa = {};
+    ConvArgs& p = pa.c;
+    int kind;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (X && W && P && Y && packed && pads && strides && dilations && (reinterpret_cast<uintptr_t>(packed) & 15) == 0 &&
+        packed_conv_args(pa, kind, N, C, H, Wd, M, KH, KW, pads, strides, dilations)) {
+        const int cus = device_cus();
+        if (cus <= 0) return set_error(MI355X_ERR_NOT_INITIALIZED, "conv2d: no usable HIP device");
+        int parts = 1, strip_w;
+        double cost;
+        const int form = choose_conv_parts(pa, kind, cus, mean, parts, cost);
+        const int64_t rows = N * M, positions = p.OHW;
+        if (form >= 0 && grid_fits(ceil_div(rows, (int64_t)4), 256)) {
+            const PackedConvForm& f = kPackedConvForms[form];
+            const int64_t pixels = choose_strips(pa, kind, f.bp, strip_w);
+            p.X = X; p.W = W; p.Y = P; p.epi = 0;
+            p.tiles_m = ceil_div(M, (int64_t)f.bm);
+            p.tiles_p = ceil_div(p.P, (int64_t)f.bp);
+            p.nwg = parts * p.tiles_m * p.tiles_p;
+            pa.packed = static_cast<const char*>(packed);
+            pa.stages = (int)(packed_conv_stages(pa, kind, f) / parts);
+            pa.part_size = rows * positions;
+            if (grid_fits(p.nwg, f.waves * WAVE)) {
+                set_strips(pa, kind, strip_w, pixels);
+                launch_packed_conv<PackedFilter<3, 3, false>, false, 1, 0>(form, pa, packed_conv_lds(kind, f, pixels), st);
+                const int status = check_launch("conv2d_f32_packed_kernel");
+                if (status != MI355X_OK) return status;
+                const dim3 grid((unsigned)ceil_div(rows, (int64_t)4));
+                if (mean) hipLaunchKernelGGL(conv_parts_kernel<true>, grid, dim3(256), 0, st, P, parts, bias, residual, Y, rows, (int)M, (int)positions, epilogue);
+                else hipLaunchKernelGGL(conv_parts_kernel<false>, grid, dim3(256), 0, st, P, parts, bias, residual, Y, rows, (int)M, (int)positions, epilogue);
+                return check_launch("conv_parts_kernel");
+            }
+        }
+    }
+    MI355X_REQUIRE(!mean || P, "conv2d_parts: null pointer");
+    const int status = mi355x_conv2d_packed_f32(X, packed, W, bias, residual, mean ? P : Y, N, C, H, Wd, M, KH, KW, pads, strides, dilations, epilogue, stream);
+    if (status != MI355X_OK || !mean) return status;
+    const int64_t OH = (H + pads[0] + pads[2] - (KH - 1) * dilations[0] - 1) / strides[0] + 1, OW = (Wd + pads[1] + pads[3] - (KW - 1) * dilations[1] - 1) / strides[1] + 1;
+    return mi355x_reduce_mean_f32(P, Y, N * M, OH * OW, 1, stream);
 }

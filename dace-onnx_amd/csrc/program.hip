@@ -58,7 +58,7 @@ struct Function {
 constexpr Function kFunctions[] = {
     MI355X_FUNCTION(mi355x_gemm_f32), MI355X_FUNCTION(mi355x_gemm_packed_f32), MI355X_FUNCTION(mi355x_conv2d_f32),
     MI355X_FUNCTION(mi355x_conv2d_res_f32), MI355X_FUNCTION(mi355x_pack_conv_f32), MI355X_FUNCTION(mi355x_pack_conv_pool_f32),
-    MI355X_FUNCTION(mi355x_conv2d_packed_f32), MI355X_FUNCTION(mi355x_conv2d_pool_packed_f32), MI355X_FUNCTION(mi355x_conv2d_skip_f32), MI355X_FUNCTION(mi355x_matmul_integer),
+    MI355X_FUNCTION(mi355x_conv2d_packed_f32), MI355X_FUNCTION(mi355x_conv2d_pool_packed_f32), MI355X_FUNCTION(mi355x_conv2d_skip_f32), MI355X_FUNCTION(mi355x_conv2d_parts_f32), MI355X_FUNCTION(mi355x_matmul_integer),
     MI355X_FUNCTION(mi355x_matmul_integer_i8), MI355X_FUNCTION(mi355x_softmax_f32), MI355X_FUNCTION(mi355x_log_softmax_f32), MI355X_FUNCTION(mi355x_softmax_max_f32),
     MI355X_FUNCTION(mi355x_attention_f32), MI355X_FUNCTION(mi355x_attention_masked_f32), MI355X_FUNCTION(mi355x_layernorm_f32), MI355X_FUNCTION(mi355x_layernorm_parts_f32), MI355X_FUNCTION(mi355x_gemm_parts_f32), MI355X_FUNCTION(mi355x_gemm_softmax_f32),
     MI355X_FUNCTION(mi355x_reduce_mean_f32), MI355X_FUNCTION(mi355x_reduce_f32), MI355X_FUNCTION(mi355x_reduce_nd_f32),

@@ -374,13 +374,15 @@ class ONNXModel:
             if self.device.type != "cuda":
                 raise RuntimeError("ONNXModel executes on the MI355X only: no HIP device is visible")
             self.expand()
-            from ..transformation.packing import pack_constant_operands, pack_variable_filters, pool_in_convolutions, skip_in_convolutions
+            from ..transformation.packing import convolutions_in_parts, pack_constant_operands, pack_variable_filters, pool_in_convolutions, skip_in_convolutions
             from ..transformation.partial_sums import split_products
             from ..transformation.softmax_fusion import softmax_of_products, softmax_with_maxima
             if self.fuse:
                 functions = {n.function for state in self.sdfg.nodes() for n in state.nodes() if isinstance(n, KernelCall)}
                 if "mi355x_layernorm_f32" in functions:
                     split_products(self)
+                if {"mi355x_conv2d_f32", "mi355x_conv2d_res_f32"} & functions:
+                    convolutions_in_parts(self)
                 if "mi355x_conv2d_res_f32" in functions:
                     skip_in_convolutions(self)
                 if "mi355x_maxpool2d_f32" in functions:

@@ -5,10 +5,11 @@ A packed copy holds three bf16 parts of every value in the order in which the ma
 made once, on the GPU. The reference has no counterpart: its constants are handed to a BLAS
 library as they are.
 """
+import numpy as np
 import torch
 
 from .. import _lib
-from ..sdfg import AccessNode, I64Array, KernelCall, PackedCopy, Ptr, Stream, int32
+from ..sdfg import AccessNode, I64Array, KernelCall, PackedCopy, Ptr, Stream, float32, int32
 from .fusion import _in_edge, _out_edge, _single_consumer
 
 
@@ -117,6 +118,51 @@ def _packed_skip(call, desc):
     return _packed_filters(call, desc, 5, "_packed_skip", -(-M // 32) * -(-C // 16) * 3072, (M, C, 1, 1))
 
 
+def _packed_part(call, desc):
+    C, M = call.args[8], call.args[11]
+    return _packed_filters(call, desc, 1, "_packed", -(-M // 32) * -(-C // 16) * 9 * 3072, (M, C, 3, 3))
+
+
+def convolutions_in_parts(model):
+    """A convolution by constant filters of few tiles and many channels is computed in parts of them, where the library says that this pays; with a
+    global pooling that is all that reads it, the launch that adds the parts up takes its means."""
+    from ..onnx.onnx_importer import clean_onnx_name
+    sdfg, weights, lib = model.sdfg, {clean_onnx_name(k): k for k in model.weights}, _lib.library()
+    for state in sdfg.nodes():
+        for call in state.nodes():
+            if not isinstance(call, KernelCall) or call.function not in ("mi355x_conv2d_f32", "mi355x_conv2d_res_f32"):
+                continue
+            X, W, bias = call.args[:3]
+            residual, Y = call.args[3:5] if call.function == "mi355x_conv2d_res_f32" else (Ptr(None), call.args[3])
+            geometry, epilogue = call.args[-12:-2], call.args[-2]
+            weight = weights.get(_in_edge(state, call, W.connector).data.data)
+            if weight is None or not model.weights.private(weight) or geometry[5:7] != [3, 3] or Y.offset or W.offset:
+                continue
+            out = _out_edge(state, call, Y.connector)
+            read = _single_consumer(sdfg, state, out.dst) if isinstance(out.dst, AccessNode) else None
+            pool = read and read.dst
+            rows, positions = geometry[0] * geometry[4], int(np.prod(sdfg.arrays[out.data.data].shape)) // (geometry[0] * geometry[4])
+            mean = isinstance(pool, KernelCall) and pool.function == "mi355x_reduce_mean_f32" and list(pool.args[2:5]) == [rows, positions, 1] and not pool.args[0].offset
+            arrays = [_lib.i64_array(a.values) if isinstance(a, I64Array) else a for a in geometry]
+            parts = lib.mi355x_conv2d_parts(*arrays, int(mean))
+            if parts <= 1:
+                continue
+            result = _out_edge(state, pool, pool.args[1].connector) if mean else out
+            sums = f"{out.data.data}_parts"
+            sdfg.add_transient(sums, [parts, rows, positions], float32)
+            target = Ptr("_summed", pool.args[1].offset if mean else 0)
+            summed = KernelCall(call.label, "mi355x_conv2d_parts_f32", [X, W, Ptr(None), bias, residual, Ptr("_parts"), target] + geometry + [epilogue, int(mean), Stream()],
+                                call.in_connectors, ["_parts", "_summed"])
+            state.remove_edge(out)
+            if mean:
+                state.remove_node(pool)
+                state.remove_node(out.dst)
+                del sdfg.arrays[out.data.data]
+            state.replace_node(call, summed, sdfg)
+            state.add_edge(summed, "_parts", state.add_access(sums), None, sdfg.make_array_memlet(sums))
+            state.add_edge(summed, "_summed", result.dst, None, result.data)
+
+
 def skip_in_convolutions(model):
     """A convolution by constant filters whose residual is a 1 x 1 convolution by constant filters becomes one call with it, where the library says that
     this pays."""
@@ -216,6 +262,7 @@ def pack_variable_filters(sdfg):
 # function -> of each operand that may be packed: the argument that is the weight, the name of the packed copy's connector, the function above
 _PACKED = {"mi355x_gemm_f32": [(1, "_packed", _packed_gemm)], "mi355x_gemm_parts_f32": [(1, "_packed", _packed_gemm)], "mi355x_conv2d_f32": [(1, "_packed", _packed_conv)],
            "mi355x_conv2d_res_f32": [(1, "_packed", _packed_conv)], "mi355x_conv2d_pool_packed_f32": [(1, "_packed", _packed_stem)],
+           "mi355x_conv2d_parts_f32": [(1, "_packed", _packed_part)],
            "mi355x_conv2d_skip_f32": [(1, "_packed", _packed_block), (5, "_packed_skip", _packed_skip)]}
 
 

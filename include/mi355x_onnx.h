@@ -180,6 +180,15 @@ int mi355x_conv2d_packed_f32(const float* X, const void* packed, const float* W,
                              const int64_t* pads, const int64_t* strides,
                              const int64_t* dilations, int epilogue, void* stream);
 
+/* mi355x_conv2d_packed_f32 with the channels in parts, P being their sums [parts, N, M, OH, OW], and a launch that adds them up and applies the epilogue;
+ * with `mean` that takes the mean over the positions too, Y being [N, M]. Elsewhere, and with a null `packed`, mi355x_conv2d_packed_f32 (into
+ * P and mi355x_reduce_mean_f32 after it with `mean`). mi355x_conv2d_parts: how many parts pay, 1 where none do. */
+int64_t mi355x_conv2d_parts(int64_t N, int64_t C, int64_t H, int64_t Wd, int64_t M, int64_t KH, int64_t KW,
+                            const int64_t* pads, const int64_t* strides, const int64_t* dilations, int mean);
+int mi355x_conv2d_parts_f32(const float* X, const float* W, const void* packed, const float* bias, const float* residual, float* P, float* Y,
+                            int64_t N, int64_t C, int64_t H, int64_t Wd, int64_t M, int64_t KH, int64_t KW,
+                            const int64_t* pads, const int64_t* strides, const int64_t* dilations, int epilogue, int mean, void* stream);
+
 /* The end of a residual block whose other branch is a 1 x 1 convolution: mi355x_conv2d_packed_f32 by W plus the one by W2 [M, C2, 1, 1] of X2
  * [N, C2, H2, Wd2] with strides2 and bias2 (or NULL), in one launch by both packed copies (mi355x_pack_conv_f32). `epilogue`: MI355X_EPI_BIAS
  * (of W) and MI355X_EPI_RELU_AFTER. With a null copy, and where the kernel takes no such layer, two launches by way of `scratch`, laid out
