@@ -990,8 +990,8 @@ class CompiledSDFG:
         """What :meth:`run_plan` calls (``csrc/host_call.cpp``), None where the launches are no program or an array is none of these: input and
         output arrays by their places, weights by their names (array -> key of the dict that a call gets), packed copies by their places."""
         import torch
-        if self._program is None or self.device.type != "cuda" or self.device.index is None:
-            return None
+        if self._program is None or self.device.type != "cuda" or self.device.index is None or not inputs:
+            return None   # (without inputs there is no tensor among them: results are numpy arrays then)
         slots = []
         for name in self._external:
             desc = self.sdfg.arrays[name]

@@ -139,3 +139,17 @@ def test_streams_threads_and_recordings(x, by_plan):
         graph.replay()
         torch.cuda.synchronize()
         assert all(torch.allclose(r, e, rtol=1e-5, atol=1e-6) for r, e in zip(recorded, expected))
+
+
+def test_nothing_outlives_a_dropped_model(x):
+    import gc
+    gc.collect()
+    before = torch.cuda.memory_allocated()
+    for _ in range(3):
+        model = _model()
+        for _ in range(3):
+            model(x)
+        model.compile_and_init().bound_launches()
+        del model
+        gc.collect()
+    assert torch.cuda.memory_allocated() <= before + 4096   # (the two tensors of _example, once)
