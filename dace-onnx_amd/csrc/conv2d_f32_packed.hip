@@ -18,6 +18,8 @@
 // (MI355X_CONV_PACKED=0), 32 images, 3 x 3: 64 x 56 x 56 -> 64 67 -> 45 us (164 TFLOP/s), 128 x 28 x 28 -> 128 69 -> 42,
 // 256 x 14 x 14 -> 256 73 -> 44, 512 x 7 x 7 -> 512 78 -> 48, 64 x 56 x 56 -> 128 by two 46 -> 36; 1 x 1 128 x 28 x 28 -> 256 by two
 // 14.7 -> 10.3; 7 x 7 by two over 3 x 224 x 224 -> 64 140 -> 65, one image 13.7 -> 5.9; 131 random layers take 0.63 of the time.
+// Tiles of 128 filters split a patch half as often, which shows where it is large, by two (against tiles of 64): 32 images 64 x 56 x 56 -> 128
+// 37.0 -> 28 us, 128 x 28 x 28 -> 256 32.9 -> 26, 16 images 64 x 49 x 49 -> 128 18.1 -> 15.7; by one at most 5 % ahead, where the rule seldom takes them.
 // Tried: no strips (the first layer 104 us, patches of 99 KB where 34 do); all groups splitting at once (2 % behind over 8 x 256 x
 // 28 x 28, 11 % over 1 x 512 x 7 x 7); loads placed by the compiler, which puts them before their uses (82 us where it is 45 now);
 // 128 x 256 tiles (never ahead for 3 x 3); a second set of accumulators in turn for the five small products (even).
@@ -536,8 +538,9 @@ __global__ void pack_conv_f32_kernel(const float* w, u32x4* packed, int M, int C
 // gemm_f32_packed.hip). Fitted over 370 layers of 1 to 32 images, 5 to 256 columns, 1 to 512 channels and 16 to 768 filters, 3 % off on
 // average; the pick is 2.5 % behind the fastest form over 144 others, up to 1.6 times for 1 x 1 and for few 7 x 7 filters.
 struct PackedConvCost { int per_t; double fixed, per_step, per_pixel, again, again_step, again_pixel; };
-// `skip`: nanoseconds of a stage of a 1 x 1 convolution that is summed too, from 21 ends of residual blocks.
+// `skip`: nanoseconds of a stage of a 1 x 1 convolution that is summed too, from 21 ends of residual blocks (0: no such kernel).
 struct PackedConvForm { int bm, bp, waves, waves_k; double skip; PackedConvCost kinds[3]; };
+constexpr int WIDE = 128;   // filters of a tile, for which a patch is split half as often
 constexpr PackedConvForm kPackedConvForms[] = {
     {64, 256, 4, 1, 3000, {{4, 6690, 3100, 328, 4980, 3590, 0}, {}, {6, 5450, 475, 84.5, 3160, 339, 59.9}}},
     {64, 256, 8, 2, 3000, {{4, 7300, 6020, 355, 6280, 9650, 0}, {}, {}}},
@@ -547,7 +550,9 @@ constexpr PackedConvForm kPackedConvForms[] = {
     {32, 128, 8, 4, 4800, {{6, 5940, 3110, 706, 4130, 5550, 0}, {}, {}}},
     {32, 64, 8, 4, 2900, {{6, 4570, 1700, 730, 2770, 3050, 107}, {4, 4780, 268, 1540, 2400, 93.3, 1720}, {}}},
     {32, 32, 8, 8, 3500, {{8, 5450, 1250, 1730, 4090, 2660, 372}, {4, 4970, 0, 3640, 0, 0, 7770}, {}}},
-    {64, 64, 4, 1, 1150, {{6, 3640, 1070, 281, 1380, 1220, 20.4}, {4, 3520, 477, 549, 1090, 357, 88.1}, {4, 4380, 111, 0, 777, 129, 26.9}}}};
+    {64, 64, 4, 1, 1150, {{6, 3640, 1070, 281, 1380, 1220, 20.4}, {4, 3520, 477, 549, 1090, 357, 88.1}, {4, 4380, 111, 0, 777, 129, 26.9}}},
+    {WIDE, 128, 8, 1, 0, {{4, 7200, 3200, 155, 6000, 4700, 200}, {}, {}}},
+    {WIDE, 64, 8, 2, 0, {{6, 5900, 3850, 245, 6000, 4300, 100}, {}, {}}}};
 constexpr int kNumPackedConvForms = sizeof(kPackedConvForms) / sizeof(kPackedConvForms[0]);
 
 enum { PC_3X3, PC_1X1, PC_7X7, PC_NONE };
@@ -564,7 +569,7 @@ template <class FILTER, bool PIXELS, int CHUNK, int KIND, bool SKIP = false>
 static void launch_packed_conv(int form, const PackedConvArgs& pa, int lds, hipStream_t st) {
 #define MI355X_FORM(index, tp, wm, wp, wk)                                                                                             \
     case index:                                                                                                                        \
-        if constexpr (kPackedConvForms[index].kinds[KIND].per_t > 0)                                                                   \
+        if constexpr (kPackedConvForms[index].kinds[KIND].per_t > 0 && !(SKIP && kPackedConvForms[index].skip == 0))                   \
             hipLaunchKernelGGL((conv2d_f32_packed_kernel<FILTER, PIXELS, tp, wm, wp, wk, CHUNK, kPackedConvForms[index].kinds[KIND].per_t, SKIP>), \
                                dim3((unsigned)pa.c.nwg), dim3(wm * wp * wk * WAVE), lds, st, pa);                                      \
         break;
@@ -578,6 +583,8 @@ static void launch_packed_conv(int form, const PackedConvArgs& pa, int lds, hipS
         MI355X_FORM(6, 1, 1, 2, 4)
         MI355X_FORM(7, 1, 1, 1, 8)
         MI355X_FORM(8, 1, 2, 2, 1)
+        MI355X_FORM(9, 2, 4, 2, 1)
+        MI355X_FORM(10, 2, 4, 1, 2)
     }
 #undef MI355X_FORM
 }
@@ -625,7 +632,7 @@ static void set_strips(PackedConvArgs& pa, int kind, int strip_w, int64_t pixels
 static int packed_conv_lds(int kind, const PackedConvForm& f, int64_t pixels, bool skip = false) {
     constexpr int64_t LDS_BYTES = 160 * 1024;
     const int per_t = f.kinds[kind].per_t;
-    if (per_t == 0) return 0;
+    if (per_t == 0 || (skip && f.skip == 0)) return 0;
     int64_t bytes = pixels * 8 * SP_PLANES + 16;
     if (kind == PC_3X3 || kind == PC_1X1) {
         const int64_t halves = 2 * packed_conv_chunk(kind);
@@ -706,7 +713,8 @@ static double unpacked_conv_cost(const ConvArgs& p, int cus, bool& summed_apart)
 // 3 of 131 layers were 5 to 14 % slower, 32 x 256 x 56 x 56 -> 64, 1 x 1, 38.2 -> 43.5 us; as it is 1 of 438, 4 x 1 x 244 x 244 -> 100, 63.6 -> 66.7;
 // the gather kernel's estimate is up to a third too long for 1 x 1 filters, most for few of them). A form whose waves all sum the
 // same channels does not take over from the kernel that sums them apart: its error was up to 1.3 times as large there, everywhere else and
-// of the other forms it is 0.2 to 0.9 of the kernels' before.
+// of the other forms it is 0.2 to 0.9 of the kernels' before. Nor does a wide form from one whose channels more groups share (64 x 56 x 56 -> 128 by two
+// 1.35e-7 of the outputs' norm by one group, 1.0e-7 by two; 128 x 25 x 25 -> 256 would go from 1.0e-7 to 1.4e-7 with 33.6 -> 23.7 us).
 // `best_cost`: of what is chosen, either way. `skip`: the fastest form that sums a 1 x 1 convolution too, with that, whatever the kernels before take.
 static int choose_packed_conv(PackedConvArgs& pa, int kind, int cus, double besides, double& best_cost, bool skip = false) {
     const ConvArgs& p = pa.c;
@@ -715,10 +723,12 @@ static int choose_packed_conv(PackedConvArgs& pa, int kind, int cus, double besi
     if (skip) best_cost = 1e300;
     int best = -1, last_bp = 0, strip_w = 0;
     int64_t pixels = 0;
-    for (int bp : {256, 128, 64, 32})
+    for (int turn = 0; turn < 6; ++turn)   // (the wide forms last: they are held against the pick of the others)
         for (int i = 0; i < kNumPackedConvForms; ++i) {
             const PackedConvForm& f = kPackedConvForms[i];
-            if (f.bp != bp || (summed_apart && f.waves_k == 1)) continue;
+            const int bp = turn < 4 ? 256 >> turn : 128 >> (turn - 4);
+            if (f.bp != bp || (f.bm == WIDE) != (turn >= 4) || (summed_apart && f.waves_k == 1)) continue;
+            if (f.bm == WIDE && best >= 0 && kPackedConvForms[best].waves_k > f.waves_k) continue;
             if (bp != last_bp) pixels = choose_strips(pa, kind, bp, strip_w);
             last_bp = bp;
             if (!packed_conv_lds(kind, f, pixels, skip)) continue;
@@ -772,7 +782,7 @@ static int choose_conv_parts(PackedConvArgs& pa, int kind, int cus, bool mean, i
     for (int i = 0; i < kNumPackedConvForms; ++i) {
         const PackedConvForm& f = kPackedConvForms[i];
         const int64_t pixels = choose_strips(pa, kind, f.bp, strip_w), all = packed_conv_stages(pa, kind, f);
-        if (f.waves_k == 1 || !packed_conv_lds(kind, f, pixels)) continue;   // (forms whose groups share the channels: no more error than the kernels before)
+        if (f.bm == WIDE || f.waves_k == 1 || !packed_conv_lds(kind, f, pixels)) continue;   // (forms whose groups share the channels: no more error than the kernels before)
         for (const int n : {2, 4}) {
             if (all % n || pa.groups % (n * f.waves_k)) continue;
             const PackedConvCost& c = f.kinds[kind];

@@ -135,6 +135,29 @@ def test_convolution_by_packed_filters_keeps_small_values(tuning, form, C, kerne
     assert bool(((expected - got.double()).abs() <= size * (C * kernel * kernel // 4 + 9) * 2.0**-23 + 2.0**-149).all())
 
 
+@pytest.mark.parametrize("N, C, H, W, M, kernel, pads, strides, dilations, epi, form",
+                         [(*layer, form) for layer in LAYERS if layer[1] > 4 and layer[5] == 3 and layer[:4] != (3, 24, 19, 17) for form in (10, 11)])
+def test_tiles_of_128_filters(tuning, form, N, C, H, W, M, kernel, pads, strides, dilations, epi):
+    """The edges above (one patch does not fit), and values that are not finite."""
+    test_convolution_by_packed_filters(tuning, form, N, C, H, W, M, kernel, pads, strides, dilations, epi)
+    test_convolution_by_packed_filters_keeps_infinities_nan_and_the_largest_values(tuning, form, 24, 3)
+
+
+@pytest.mark.parametrize("low, high", [(-100, 90), (-148, 105), (90, -3)])
+@pytest.mark.parametrize("form", [10, 11])
+def test_tiles_of_128_filters_keep_small_values(tuning, form, low, high):
+    test_convolution_by_packed_filters_keeps_small_values(tuning, form, 32, 3, low, high)
+
+
+@pytest.mark.parametrize("N, C, H, M", [(32, 64, 56, 128), (30, 128, 28, 256), (17, 64, 49, 130)])
+def test_layers_that_take_tiles_of_128_filters(N, C, H, M):
+    """By the rule: no more error than by tiles of 64, whose sums they have in the same order; 1.6e-7 of the norm leaves a tenth over the largest seen."""
+    torch.manual_seed(N)
+    x, w = torch.randn(N, C, H, H, device="cuda"), torch.randn(M, C, 3, 3, device="cuda")
+    got, wide = packed_conv(x, w, pads=(1, 1, 1, 1), strides=(2, 2)), exact_conv(x, w, (1, 1, 1, 1), (2, 2))
+    assert float((got.double() - wide).norm() / wide.norm()) < 1.6e-7
+
+
 def test_a_packed_convolution_follows_its_filters():
     """A block of a residual network: filters written in place after the first call; the next call multiplies by the new ones."""
     conv = nn.Conv2d(64, 64, 3, padding=1).cuda()
