@@ -464,6 +464,9 @@ class ONNXModel:
     def __call__(self, *args, **kwargs):
         """Execute the model.
 
+        Calls of one model share its intermediate arrays: they follow one another on one stream, or the caller makes one wait for the other. Calls
+        of a model without any (one node, or what fuses into one launch) may overlap on several streams and threads.
+
         :param args: positional arguments; the i-th is the i-th graph input.
         :param kwargs: named arguments matching the ONNX input names.
         :return: the output (or a tuple of outputs): torch tensors on the GPU if any

@@ -9,7 +9,7 @@ import numpy as np
 import torch
 
 from .. import _lib
-from ..sdfg import AccessNode, I64Array, KernelCall, PackedCopy, Ptr, Stream, float32, int32
+from ..sdfg import AccessNode, AliasNode, I64Array, KernelCall, PackedCopy, Ptr, Stream, float32, int32
 from .fusion import _in_edge, _out_edge, _single_consumer
 
 
@@ -123,12 +123,27 @@ def _packed_part(call, desc):
     return _packed_filters(call, desc, 1, "_packed", -(-M // 32) * -(-C // 16) * 9 * 3072, (M, C, 3, 3))
 
 
+def _shared_by_calls(sdfg, state):
+    """The arrays of which a compiled graph keeps one for all of its calls: transients, but for views of an array of the caller's."""
+    shared = {name for name, desc in sdfg.arrays.items() if desc.transient}
+    views = [{_in_edge(state, n, n.in_conn).data.data, _out_edge(state, n, n.out_conn).data.data} for n in state.nodes() if isinstance(n, AliasNode)]
+    for _ in views:   # (a chain of them is no longer than that)
+        for view in views:
+            if not view <= shared:
+                shared -= view
+    return shared
+
+
 def convolutions_in_parts(model):
     """A convolution by constant filters of few tiles and many channels is computed in parts of them, where the library says that this pays; with a
-    global pooling that is all that reads it, the launch that adds the parts up takes its means."""
+    global pooling that is all that reads it, the launch that adds the parts up takes its means.
+
+    The parts are an array that all calls of the compiled graph share, so that calls on two streams or from two threads must not overlap. A convolution
+    from one array of the caller's into another, which they may, stays whole."""
     from ..onnx.onnx_importer import clean_onnx_name
     sdfg, weights, lib = model.sdfg, {clean_onnx_name(k): k for k in model.weights}, _lib.library()
     for state in sdfg.nodes():
+        shared = _shared_by_calls(sdfg, state)
         for call in state.nodes():
             if not isinstance(call, KernelCall) or call.function not in ("mi355x_conv2d_f32", "mi355x_conv2d_res_f32"):
                 continue
@@ -139,6 +154,8 @@ def convolutions_in_parts(model):
             if weight is None or not model.weights.private(weight) or geometry[5:7] != [3, 3] or Y.offset or W.offset:
                 continue
             out = _out_edge(state, call, Y.connector)
+            if not {_in_edge(state, call, X.connector).data.data, out.data.data} & shared:
+                continue
             read = _single_consumer(sdfg, state, out.dst) if isinstance(out.dst, AccessNode) else None
             pool = read and read.dst
             rows, positions = geometry[0] * geometry[4], int(np.prod(sdfg.arrays[out.data.data].shape)) // (geometry[0] * geometry[4])

@@ -1,0 +1,52 @@
+"""Arrays that all calls of a compiled graph share: a graph whose calls may overlap (no GPU: launch lists only)."""
+import numpy as np
+import pytest
+
+import dace_onnx_amd.onnx as donnx
+from dace_onnx_amd.onnx.proto import TensorProto, helper, numpy_helper
+from dace_onnx_amd.sdfg import KernelCall
+from dace_onnx_amd.transformation import packing
+
+SHAPE = [1, 512, 7, 7]   # parts pay here
+
+
+def _conv_graph(before=(), after=(), source="x", result="y", outputs=(("y", SHAPE), ), input_shape=SHAPE):
+    rng = np.random.default_rng(2)
+    info = lambda n, s: helper.make_tensor_value_info(n, TensorProto.FLOAT, s)   # noqa: E731
+    nodes = [*before, helper.make_node("Conv", [source, "w"], [result], kernel_shape=[3, 3], pads=[1] * 4), *after]
+    weights = [numpy_helper.from_array(rng.standard_normal((512, 512, 3, 3), dtype=np.float32), "w"), numpy_helper.from_array(np.array(SHAPE, np.int64), "image"),
+               numpy_helper.from_array(np.array([512, 49], np.int64), "rows")]
+    graph = helper.make_graph(nodes, "g", [info("x", input_shape)], [info(*o) for o in outputs], initializer=weights)
+    return helper.make_model(graph, opset_imports=[helper.make_opsetid("", 12)])
+
+
+def _functions_and_transients(model):
+    model = donnx.ONNXModel("shared", model)
+    model.expand()
+    packing.convolutions_in_parts(model)
+    return [n.function for s in model.sdfg.nodes() for n in s.nodes() if isinstance(n, KernelCall)], [d for d in model.sdfg.arrays.values() if d.transient]
+
+
+node = helper.make_node
+
+
+@pytest.mark.parametrize("graph", [
+    lambda: _conv_graph(),
+    lambda: _conv_graph(after=[node("Add", ["c", "x"], ["s"]), node("Relu", ["s"], ["y"])], result="c"),
+    lambda: _conv_graph(before=[node("Reshape", ["x", "image"], ["i"])], after=[node("Reshape", ["c", "rows"], ["y"])], source="i", result="c",
+                        outputs=[("y", [512, 49])], input_shape=[512, 49]),
+])
+def test_a_convolution_between_arrays_of_the_caller_keeps_none_of_its_own(graph):
+    functions, transients = _functions_and_transients(graph())
+    assert len(functions) == 1 and functions[0] in ("mi355x_conv2d_f32", "mi355x_conv2d_res_f32")
+    assert not any(np.prod(d.shape) > np.prod(SHAPE) for d in transients)
+
+
+@pytest.mark.parametrize("graph", [
+    lambda: _conv_graph(after=[node("Exp", ["c"], ["y"])], result="c"),
+    lambda: _conv_graph(before=[node("Exp", ["x"], ["e"])], source="e"),
+    lambda: _conv_graph(after=[node("GlobalAveragePool", ["c"], ["y"])], result="c", outputs=[("y", [1, 512, 1, 1])]),
+])
+def test_one_that_reads_or_writes_an_array_of_the_graph_is_computed_in_parts(graph):
+    functions, _ = _functions_and_transients(graph())
+    assert "mi355x_conv2d_parts_f32" in functions
