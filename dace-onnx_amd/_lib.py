@@ -59,7 +59,7 @@ SIGNATURES: typing.Dict[str, typing.Tuple[typing.Any, typing.List[typing.Any]]] 
     "mi355x_conv2d_packed_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                                         _c_i64_p, _c_i64_p, _c_i64_p, _int, _vp]),
     "mi355x_conv2d_parts": (_i64, [_i64, _i64, _i64, _i64, _i64, _i64, _i64, _c_i64_p, _c_i64_p, _c_i64_p, _int]),
-    "mi355x_conv2d_parts_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _c_i64_p, _c_i64_p, _c_i64_p, _int, _int, _vp]),
+    "mi355x_conv2d_parts_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _c_i64_p, _c_i64_p, _c_i64_p, _int, _int, _vp]),
     "mi355x_conv2d_skip_pays": (_int, [_i64, _i64, _i64, _i64, _i64, _i64, _i64, _c_i64_p, _c_i64_p, _c_i64_p, _i64, _i64, _i64, _c_i64_p]),
     "mi355x_conv2d_skip_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _c_i64_p, _c_i64_p, _c_i64_p,
                                       _i64, _i64, _i64, _c_i64_p, _int, _vp]),

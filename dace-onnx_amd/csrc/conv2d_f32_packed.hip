@@ -774,8 +774,10 @@ static bool skip_args(PackedConvArgs& pa, int kind, int64_t C2, int64_t H2, int6
 // For one or a few images, of which the last layers are a few tiles with long sums; up to 256 positions, which a wave of the launch that adds up goes
 // through in turns. Weights from beyond the L2: 1 x 512 x 7 x 7 -> 512 18.5 us in one part, 12.5 in four (with the mean after it 20.7 and 12.7), 1 x 256 x
 // 14 x 14 -> 512 by two 12.7 and 11.3, 2 x 256 x 14 x 14 -> 256 13.2 and 11.8, 4 x 512 x 7 x 7 22.8 and 14.4. Of 20 layers none is behind.
-static int choose_conv_parts(PackedConvArgs& pa, int kind, int cus, bool mean, int& parts, double& best_cost) {
+// `parts`: 0 for as many as pay, which it is set to, or how many are asked for.
+static int choose_conv_parts(PackedConvArgs& pa, int kind, int cus, bool mean, int64_t& parts, double& best_cost) {
     const ConvArgs& p = pa.c;
+    const int64_t asked = parts;
     int best = -1, strip_w = 0;
     best_cost = 1e300;
     if (kind != PC_3X3 || p.OHW > 256) return -1;
@@ -784,7 +786,7 @@ static int choose_conv_parts(PackedConvArgs& pa, int kind, int cus, bool mean, i
         const int64_t pixels = choose_strips(pa, kind, f.bp, strip_w), all = packed_conv_stages(pa, kind, f);
         if (f.bm == WIDE || f.waves_k == 1 || !packed_conv_lds(kind, f, pixels)) continue;   // (forms whose groups share the channels: no more error than the kernels before)
         for (const int n : {2, 4}) {
-            if (all % n || pa.groups % (n * f.waves_k)) continue;
+            if ((asked && n != asked) || all % n || pa.groups % (n * f.waves_k)) continue;
             const PackedConvCost& c = f.kinds[kind];
             const int64_t nwg = n * ceil_div((int64_t)p.M, (int64_t)f.bm) * ceil_div(p.P, (int64_t)f.bp), up = ceil_div(nwg, (int64_t)cus);
             const double more = up <= 6 ? (double)(up - 1) : (double)nwg / cus - 0.5, stages = (double)(all / n), patch = stages * (double)pixels / 100;
@@ -937,7 +939,8 @@ extern "C" int64_t mi355x_conv2d_parts(int64_t N, int64_t C, int64_t H, int64_t 
                                        const int64_t* strides, const int64_t* dilations, int mean) {
     using namespace mi355x;
     PackedConvArgs pa = {};
-    int kind, parts = 1;
+    int kind;
+    int64_t parts = 0;
     if (!pads || !strides || !dilations || !packed_conv_args(pa, kind, N, C, H, Wd, M, KH, KW, pads, strides, dilations) || tuning().conv_packed >= 0) return 1;
     int cus = device_cus();
     if (cus <= 0) cus = 256;
@@ -947,12 +950,13 @@ extern "C" int64_t mi355x_conv2d_parts(int64_t N, int64_t C, int64_t H, int64_t 
     return apart < whole ? parts : 1;
 }
 
-extern "C" int mi355x_conv2d_parts_f32(const float* X, const float* W, const void* packed, const float* bias, const float* residual, float* P, float* Y, int64_t N,
-                                       int64_t C, int64_t H, int64_t Wd, int64_t M, int64_t KH, int64_t KW, const int64_t* pads, const int64_t* strides,
+extern "C" int mi355x_conv2d_parts_f32(const float* X, const float* W, const void* packed, const float* bias, const float* residual, float* P, int64_t parts, float* Y,
+                                       int64_t N, int64_t C, int64_t H, int64_t Wd, int64_t M, int64_t KH, int64_t KW, const int64_t* pads, const int64_t* strides,
                                        const int64_t* dilations, int epilogue, int mean, void* stream) {
     using namespace mi355x;
     MI355X_REQUIRE((epilogue & ~(MI355X_EPI_BIAS | MI355X_EPI_RELU | MI355X_EPI_RESIDUAL | MI355X_EPI_RELU_AFTER)) == 0, "conv2d_parts: unknown epilogue bits 0x%x", epilogue);
     MI355X_REQUIRE((!(epilogue & MI355X_EPI_BIAS) || bias) && (!(epilogue & MI355X_EPI_RESIDUAL) || residual), "conv2d_parts: null bias or residual");
+    MI355X_REQUIRE(parts >= 1, "conv2d_parts: %lld parts", (long long)parts);
     PackedConvArgs pa = {};
     ConvArgs& p = pa.c;
     int kind;
@@ -961,9 +965,9 @@ extern "C" int mi355x_conv2d_parts_f32(const float* X, const float* W, const voi
         packed_conv_args(pa, kind, N, C, H, Wd, M, KH, KW, pads, strides, dilations)) {
         const int cus = device_cus();
         if (cus <= 0) return set_error(MI355X_ERR_NOT_INITIALIZED, "conv2d: no usable HIP device");
-        int parts = 1, strip_w;
+        int strip_w;
         double cost;
-        const int form = choose_conv_parts(pa, kind, cus, mean, parts, cost);
+        const int form = choose_conv_parts(pa, kind, cus, mean, parts, cost);   // (P has room for that many)
         const int64_t rows = N * M, positions = p.OHW;
         if (form >= 0 && grid_fits(ceil_div(rows, (int64_t)4), 256)) {
             const PackedConvForm& f = kPackedConvForms[form];
@@ -981,8 +985,8 @@ extern "C" int mi355x_conv2d_parts_f32(const float* X, const float* W, const voi
                 const int status = check_launch("conv2d_f32_packed_kernel");
                 if (status != MI355X_OK) return status;
                 const dim3 grid((unsigned)ceil_div(rows, (int64_t)4));
-                if (mean) hipLaunchKernelGGL(conv_parts_kernel<true>, grid, dim3(256), 0, st, P, parts, bias, residual, Y, rows, (int)M, (int)positions, epilogue);
-                else hipLaunchKernelGGL(conv_parts_kernel<false>, grid, dim3(256), 0, st, P, parts, bias, residual, Y, rows, (int)M, (int)positions, epilogue);
+                if (mean) hipLaunchKernelGGL(conv_parts_kernel<true>, grid, dim3(256), 0, st, P, (int)parts, bias, residual, Y, rows, (int)M, (int)positions, epilogue);
+                else hipLaunchKernelGGL(conv_parts_kernel<false>, grid, dim3(256), 0, st, P, (int)parts, bias, residual, Y, rows, (int)M, (int)positions, epilogue);
                 return check_launch("conv_parts_kernel");
             }
         }

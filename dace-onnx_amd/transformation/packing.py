@@ -119,7 +119,7 @@ def _packed_skip(call, desc):
 
 
 def _packed_part(call, desc):
-    C, M = call.args[8], call.args[11]
+    C, M = call.args[9], call.args[12]
     return _packed_filters(call, desc, 1, "_packed", -(-M // 32) * -(-C // 16) * 9 * 3072, (M, C, 3, 3))
 
 
@@ -168,7 +168,7 @@ def convolutions_in_parts(model):
             sums = f"{out.data.data}_parts"
             sdfg.add_transient(sums, [parts, rows, positions], float32)
             target = Ptr("_summed", pool.args[1].offset if mean else 0)
-            summed = KernelCall(call.label, "mi355x_conv2d_parts_f32", [X, W, Ptr(None), bias, residual, Ptr("_parts"), target] + geometry + [epilogue, int(mean), Stream()],
+            summed = KernelCall(call.label, "mi355x_conv2d_parts_f32", [X, W, Ptr(None), bias, residual, Ptr("_parts"), parts, target] + geometry + [epilogue, int(mean), Stream()],
                                 call.in_connectors, ["_parts", "_summed"])
             state.remove_edge(out)
             if mean:

@@ -180,12 +180,12 @@ int mi355x_conv2d_packed_f32(const float* X, const void* packed, const float* W,
                              const int64_t* pads, const int64_t* strides,
                              const int64_t* dilations, int epilogue, void* stream);
 
-/* mi355x_conv2d_packed_f32 with the channels in parts, P being their sums [parts, N, M, OH, OW], and a launch that adds them up and applies the epilogue;
- * with `mean` that takes the mean over the positions too, Y being [N, M]. Elsewhere, and with a null `packed`, mi355x_conv2d_packed_f32 (into
- * P and mi355x_reduce_mean_f32 after it with `mean`). mi355x_conv2d_parts: how many parts pay, 1 where none do. */
+/* mi355x_conv2d_packed_f32 with the channels in `parts` parts (2 or 4), P being their sums [parts, N, M, OH, OW], and a launch that adds them up and
+ * applies the epilogue; with `mean` that takes the mean over the positions too, Y being [N, M]. Where the channels do not divide so, and with a null
+ * `packed`, mi355x_conv2d_packed_f32 (into P and mi355x_reduce_mean_f32 after it with `mean`). mi355x_conv2d_parts: how many parts pay, 1 where none do. */
 int64_t mi355x_conv2d_parts(int64_t N, int64_t C, int64_t H, int64_t Wd, int64_t M, int64_t KH, int64_t KW,
                             const int64_t* pads, const int64_t* strides, const int64_t* dilations, int mean);
-int mi355x_conv2d_parts_f32(const float* X, const float* W, const void* packed, const float* bias, const float* residual, float* P, float* Y,
+int mi355x_conv2d_parts_f32(const float* X, const float* W, const void* packed, const float* bias, const float* residual, float* P, int64_t parts, float* Y,
                             int64_t N, int64_t C, int64_t H, int64_t Wd, int64_t M, int64_t KH, int64_t KW,
                             const int64_t* pads, const int64_t* strides, const int64_t* dilations, int epilogue, int mean, void* stream);
 

@@ -20,17 +20,18 @@ def normal(seed, *shapes):
     return [torch.from_numpy(rng.standard_normal(s, dtype=np.float32)).cuda() for s in shapes]
 
 
-def conv(x, w, bias, residual, stride, epilogue, mean, packed=True):
+def conv(x, w, bias, residual, stride, epilogue, mean, packed=True, count=4):
     (N, C, H, Wd), M, i64 = x.shape, w.shape[0], _lib.i64_array
     OH, OW = (H - 1) // stride + 1, (Wd - 1) // stride + 1
     geometry = (N, C, H, Wd, M, 3, 3, i64([1] * 4), i64([stride] * 2), i64([1, 1]))
     copy = torch.empty(-(-M // 32) * -(-C // 16) * 9 * 768, dtype=torch.int32, device="cuda") if packed else None
     if packed:
         call("mi355x_pack_conv_f32", w.data_ptr(), copy.data_ptr(), M, C, 3, 3)
-    parts = torch.full((4 * N * M * OH * OW + 64, ), -7.0, device="cuda")
+    outputs = N * M * OH * OW
+    parts = torch.full((count * outputs + 64, ), -7.0, device="cuda")
     y = torch.full((N * M * (1 if mean else OH * OW) + 64, ), -7.0, device="cuda")
-    call("mi355x_conv2d_parts_f32", x.data_ptr(), w.data_ptr(), _lib.ptr(copy), _lib.ptr(bias), _lib.ptr(residual), parts.data_ptr(), y.data_ptr(), *geometry, epilogue, int(mean))
-    assert bool((y[-64:] == -7).all()) and bool((parts[-64:] == -7).all()) and bool((parts[N * M * OH * OW:2 * N * M * OH * OW] != -7).any()) == packed
+    call("mi355x_conv2d_parts_f32", x.data_ptr(), w.data_ptr(), _lib.ptr(copy), _lib.ptr(bias), _lib.ptr(residual), parts.data_ptr(), count, y.data_ptr(), *geometry, epilogue, int(mean))
+    assert bool((y[-64:] == -7).all()) and bool((parts[-64:] == -7).all()) and bool((parts[(count - 1) * outputs:-64] != -7).any()) == (packed or (mean and count == 1))
     return y[:-64].reshape((N, M) if mean else (N, M, OH, OW))
 
 
@@ -58,8 +59,8 @@ def test_convolution_in_parts(N, C, H, Wd, M, stride, epilogue, mean):
     expected, bound = wide_conv(x, w, bias, residual, stride, epilogue)
     if mean:
         expected, bound = expected.mean((2, 3)), bound.mean((2, 3)) * 1.1
-    for packed in (C >= 256, False):
-        got = conv(x, w, bias, residual, stride, epilogue, mean, packed)
+    for packed, count in ((C >= 256, 4), (C >= 256, 2), (False, 2)):   # (no more parts than there is room for, whatever would pay)
+        got = conv(x, w, bias, residual, stride, epilogue, mean, packed, count)
         assert bool(((got.double() - expected).abs() <= bound + 1e-30).all())
 
 

@@ -3,8 +3,9 @@ import numpy as np
 import pytest
 
 import dace_onnx_amd.onnx as donnx
+from dace_onnx_amd import _lib
 from dace_onnx_amd.onnx.proto import TensorProto, helper, numpy_helper
-from dace_onnx_amd.sdfg import KernelCall
+from dace_onnx_amd.sdfg import I64Array, KernelCall, Ptr, Stream
 from dace_onnx_amd.transformation import packing
 
 SHAPE = [1, 512, 7, 7]   # parts pay here
@@ -50,3 +51,18 @@ def test_a_convolution_between_arrays_of_the_caller_keeps_none_of_its_own(graph)
 def test_one_that_reads_or_writes_an_array_of_the_graph_is_computed_in_parts(graph):
     functions, _ = _functions_and_transients(graph())
     assert "mi355x_conv2d_parts_f32" in functions
+
+
+def test_the_launch_is_told_how_many_parts_its_array_holds():
+    """However many pay where it is launched: the kernel writes as many as there is room for."""
+    model = donnx.ONNXModel("parts", _conv_graph(before=[node("Exp", ["x"], ["e"])], source="e"))
+    model.expand()
+    packing.convolutions_in_parts(model)
+    (call, sums), = [(n, model.sdfg.arrays[e.data.data]) for s in model.sdfg.nodes() for n in s.nodes() if isinstance(n, KernelCall) for e in s.out_edges(n)
+                     if e.src_conn == "_parts"]
+    place = [a.connector if isinstance(a, Ptr) else None for a in call.args].index("_parts")
+    assert call.args[place + 1] == sums.shape[0] > 1
+    values = [_lib.i64_array(a.values) if isinstance(a, I64Array) else 0 if isinstance(a, Stream) else 16 if isinstance(a, Ptr) else a for a in call.args]
+    values[place + 1] = 0
+    with pytest.raises(_lib.MI355XError, match="0 parts"):
+        _lib.check(_lib.library().mi355x_conv2d_parts_f32(*values), "mi355x_conv2d_parts_f32")
