@@ -224,5 +224,7 @@ PyMODINIT_FUNC PyInit__host_call() {
     plan_type.tp_flags = Py_TPFLAGS_DEFAULT;
     plan_type.tp_methods = plan_methods;
     if (PyType_Ready(&plan_type) < 0) return nullptr;
-    return PyModule_Create(&module);
+    PyObject* made = PyModule_Create(&module);
+    if (made && PyModule_AddStringConstant(made, "built_against", BUILT_AGAINST) < 0) Py_CLEAR(made);   // torch, whose tensors are read by its inline functions
+    return made;
 }

@@ -27,13 +27,17 @@ import ctypes
 import functools
 import importlib.util
 import itertools
+import logging
 import os
 import struct
+import sysconfig
 import typing
 
 import numpy as np
 
 from . import _lib
+
+log = logging.getLogger(__name__)
 
 # --------------------------------------------------------------------------- dtypes
 
@@ -592,21 +596,28 @@ class SDFG:
 # --------------------------------------------------------------------------- executor
 
 
+def _load_host_call(path):
+    import torch   # whose libraries it is linked against
+    spec = importlib.util.spec_from_file_location("_host_call", path)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    running = f"{torch.version.__version__} {torch.version.git_version}"
+    if module.built_against != running:
+        raise ImportError(f"built against torch {module.built_against}, this is {running}")
+    return module
+
+
+@functools.lru_cache(maxsize=None)
 def _host_call():
-    """The extension module that ``csrc/host_call.cpp`` is built into, next to the library."""
-    global _host_call_module
-    if _host_call_module is None:
-        import torch  # noqa: F401  (whose libraries it is linked against)
-        path = os.path.join(os.path.dirname(_lib.LIBRARY_PATH), "_host_call.so")
-        if not os.path.isfile(path):
-            raise _lib.LibraryNotBuilt(f"{path} not found; build it with `make -C {os.path.join(os.path.dirname(path), 'csrc')}`")
-        spec = importlib.util.spec_from_file_location("_host_call", path)
-        _host_call_module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(_host_call_module)
-    return _host_call_module
-
-
-_host_call_module = None
+    """The extension module that ``csrc/host_call.cpp`` is built into, next to the library; None where there is none for this interpreter and torch:
+    calls take the general way then, as they do for arguments that it does not take."""
+    path = os.path.join(os.path.dirname(_lib.LIBRARY_PATH), "_host_call" + sysconfig.get_config_var("EXT_SUFFIX"))
+    try:
+        return _load_host_call(path)
+    except (ImportError, OSError) as error:
+        log.warning("calls take the general way, up to 3 times as long on the host (%s: %s); build it with `make -B -C %s`", path, error,
+                    os.path.join(os.path.dirname(path), "csrc"))
+        return None
 
 
 @functools.lru_cache(maxsize=None)
@@ -990,7 +1001,7 @@ class CompiledSDFG:
         """What :meth:`run_plan` calls (``csrc/host_call.cpp``), None where the launches are no program or an array is none of these: input and
         output arrays by their places, weights by their names (array -> key of the dict that a call gets), packed copies by their places."""
         import torch
-        if self._program is None or self.device.type != "cuda" or self.device.index is None or not inputs:
+        if self._program is None or self.device.type != "cuda" or self.device.index is None or not inputs or _host_call() is None:
             return None   # (without inputs there is no tensor among them: results are numpy arrays then)
         slots = []
         for name in self._external:
