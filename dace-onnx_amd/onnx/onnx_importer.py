@@ -85,7 +85,8 @@ class ONNXModel:
         :param auto_optimize: apply the graph-level fusion pass before expanding (first call).
         :param parent_pytorch_module: when not None, weights whose names match parameters of this
                                       module are taken from it rather than from the ONNX graph.
-        :param fuse: with ``auto_optimize``, fold bias/activation/residual/transposes into contractions.
+        :param fuse: with ``auto_optimize``, fold bias/activation/residual/transposes into contractions, and make one
+                     launch of two where there is a kernel for both.
         :param use_hip_graph: replay the launch sequence as one HIP graph from the second call on.
         :param storage: kept for signature compatibility (``onnx_importer.py:104``): parameters, inputs and
                         outputs always live in GPU global memory; anything else named here is an error.
@@ -369,28 +370,35 @@ class ONNXModel:
         expand_onnx_nodes(self.sdfg)
         self._expanded = True
 
+    def _merge_launches(self):
+        """Make one launch of two where the library has one, or parts of a launch that the next adds up: what fusion does after the expansion.
+        Graphs that were expanded without it stay as they are."""
+        if not self.sdfg.fused:
+            return
+        from ..transformation.packing import convolutions_in_parts, pool_in_convolutions, skip_in_convolutions
+        from ..transformation.partial_sums import split_products
+        from ..transformation.softmax_fusion import softmax_of_products, softmax_with_maxima
+        functions = {n.function for state in self.sdfg.nodes() for n in state.nodes() if isinstance(n, KernelCall)}
+        if "mi355x_layernorm_f32" in functions:
+            split_products(self)
+        if {"mi355x_conv2d_f32", "mi355x_conv2d_res_f32"} & functions:
+            convolutions_in_parts(self)
+        if "mi355x_conv2d_res_f32" in functions:
+            skip_in_convolutions(self)
+        if "mi355x_maxpool2d_f32" in functions:
+            pool_in_convolutions(self)
+        if "mi355x_softmax_f32" in functions:
+            softmax_of_products(self)
+            if "mi355x_reduce_f32" in functions:
+                softmax_with_maxima(self.sdfg)
+
     def compile_and_init(self):
         if self._compiled is None:
             if self.device.type != "cuda":
                 raise RuntimeError("ONNXModel executes on the MI355X only: no HIP device is visible")
             self.expand()
-            from ..transformation.packing import convolutions_in_parts, pack_constant_operands, pack_variable_filters, pool_in_convolutions, skip_in_convolutions
-            from ..transformation.partial_sums import split_products
-            from ..transformation.softmax_fusion import softmax_of_products, softmax_with_maxima
-            if self.fuse:
-                functions = {n.function for state in self.sdfg.nodes() for n in state.nodes() if isinstance(n, KernelCall)}
-                if "mi355x_layernorm_f32" in functions:
-                    split_products(self)
-                if {"mi355x_conv2d_f32", "mi355x_conv2d_res_f32"} & functions:
-                    convolutions_in_parts(self)
-                if "mi355x_conv2d_res_f32" in functions:
-                    skip_in_convolutions(self)
-                if "mi355x_maxpool2d_f32" in functions:
-                    pool_in_convolutions(self)
-                if "mi355x_softmax_f32" in functions:
-                    softmax_of_products(self)
-                    if "mi355x_reduce_f32" in functions:
-                        softmax_with_maxima(self.sdfg)
+            from ..transformation.packing import pack_constant_operands, pack_variable_filters
+            self._merge_launches()
             self._packed = pack_constant_operands(self)
             pack_variable_filters(self.sdfg)
             self._compiled = self.sdfg.compile()

@@ -506,6 +506,7 @@ class SDFG:
         self.arrays: typing.Dict[str, Array] = collections.OrderedDict()
         self._states: typing.List[SDFGState] = []
         self._compiled = None
+        self.fused = False   #: whether graph-level fusion went over it before its nodes were expanded
 
     # -- construction ------------------------------------------------------------
     def add_array(self, name, shape, dtype, strides=None, transient=False, storage=StorageType.GPU_Global):

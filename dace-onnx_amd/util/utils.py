@@ -86,4 +86,5 @@ def auto_optimize(sdfg: SDFG, cuda: bool = True, apply_strict: bool = False, fus
     if fuse:
         from ..transformation import fuse_onnx_graph
         fuse_onnx_graph(sdfg)
+        sdfg.fused = True
     expand_onnx_nodes(sdfg)
