@@ -172,9 +172,9 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(AttnArgs p) {
 // Any number of keys: the same workgroup walks the keys in blocks of 128 with a running row maximum and
 // row sum (the probabilities of a block are exp(s - running max); when the maximum grows, the sums and the
 // output accumulators are rescaled by exp(old max - new max); the division by the row sum happens once, at
-// the end). Keys beyond Sk in the last block are loaded from the last valid row and their scores set to
-// -inf. Every wave takes part in the barriers of every block, so there is no early exit for query rows
-// beyond Sq: they are computed on the clamped last row and not stored.
+// the end). Keys beyond Sk in the last block are loaded from the last valid row, their scores set to -inf
+// and their values to zero. Every wave takes part in the barriers of every block, so there is no early exit
+// for query rows beyond Sq: they are computed on the clamped last row and not stored.
 //
 // MASKED: scale * Q K^T + mask, the padding mask of a batch of unequal sentences (or any mask of the scores' shape up to
 // broadcasting). The scores stay in natural units then and the difference to the maximum is scaled by log2(e): a mask of the
@@ -228,6 +228,10 @@ __device__ __forceinline__ void attention_blocks(const AttnArgs& p, int64_t slic
             rk[it] = *reinterpret_cast<const f32x4*>(K + row * p.k_sr + 4 * c4);
             rv[it] = *reinterpret_cast<const f32x4*>(V + row * p.v_sr + 4 * c4);
         }
+        if (key0 + SK > p.Sk)   // (zero times an infinity of the last key's would be NaN)
+#pragma unroll
+            for (int it = 0; it < 8; ++it)
+                if (key0 + (tid + it * 256) / (D / 4) >= p.Sk) rv[it] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (key0 > 0) __syncthreads();   // the previous block's operands have been read by everyone
 #pragma unroll
         for (int it = 0; it < 8; ++it) {
@@ -466,6 +470,10 @@ __global__ __launch_bounds__(WAVE * WAVES) void attention_few_kernel(AttnArgs p)
 #pragma unroll
         for (int r = 0; r < 4; ++r) s[r] = power(s[r]);
         const float sum = quad_lanes_sum((s[0] + s[1]) + (s[2] + s[3]));
+        if (key0 + KEYS > p.Sk)   // (zero times an infinity of the last key's would be NaN)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (key0 + 4 * lq + r >= p.Sk) rv[r] = f32x4{0.f, 0.f, 0.f, 0.f};
         f32x4 product[4];
         {
             bf16x4 fp[SP_PLANES];

@@ -152,3 +152,19 @@ def test_attention_of_few_rows_keeps_infinities_nan_and_the_largest_values(tunin
         assert torch.equal(torch.isnan(results[0]), torch.isnan(results[1])) and torch.equal(torch.isinf(results[0]), torch.isinf(results[1]))
         fine = torch.isfinite(results[0])
         assert bool(((results[0] - results[1]).abs()[fine] <= 1e-5 * results[0].abs()[fine].clamp(min=1)).all())
+
+
+@pytest.mark.parametrize("form", [dict(MI355X_ATTN_FEW=1), dict(MI355X_ATTN_FEW=2), dict(MI355X_ATTN_FEW=4), dict(MI355X_ATTN_FEW=8), dict(MI355X_ATTN_SPLIT=1),
+                                  dict(MI355X_ATTN_SPLIT=0), {}], ids=str)
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("sk", [1, 15, 16, 33, 100, 128, 130, 200])
+def test_an_infinite_value_of_the_last_key(tuning, form, masked, sk):
+    """Keys beyond the last have no probability, and no value that could turn it into NaN: against float64."""
+    tuning(**form)
+    q, k, v = inputs(2, 2, 20, sk)
+    v[1, 0, sk - 1, 9], v[0, 1, sk - 1, 63] = float("inf"), -float("inf")
+    mask = torch.zeros(1, 1, 20, sk, device="cuda") if masked else None
+    expected = torch.softmax(0.125 * (q.double() @ k.double().transpose(-1, -2).contiguous()), -1) @ v.double()
+    got = attention(q, k, v, mask).double()
+    fine = torch.isfinite(expected)
+    assert torch.equal(got[~fine], expected[~fine]) and bool(((got - expected).abs()[fine] <= 2.0**-19 * v[v.isfinite()].abs().max()).all())
