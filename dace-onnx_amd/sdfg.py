@@ -25,6 +25,7 @@ import array
 import collections
 import ctypes
 import functools
+import gc
 import importlib.util
 import itertools
 import logging
@@ -678,8 +679,9 @@ class _Recording:
     """A HIP graph that is never destroyed while torch's current stream is being captured.
 
     A compiled graph and what holds it refer to each other, so a dropped one goes whenever Python collects garbage, also in the middle of a
-    capture of the caller's. Destroying a HIP graph waits for the GPU, an error then that ends the process: the graph is put aside until
-    another recording is made or goes.
+    capture of the caller's. Destroying a HIP graph waits for the GPU, an error then that ends the process: the graph is put aside, with its
+    memory, until the next collection, recording or call of a compiled graph after the capture. (A collection by one thread while another
+    captures is not seen: torch tells a thread about its own stream only.)
     """
     _put_aside = []
 
@@ -690,9 +692,16 @@ class _Recording:
 
     def __del__(self):
         if self._capturing():
-            self._put_aside.append(self.graph)
+            if _Recording.give_back not in gc.callbacks:
+                gc.callbacks.append(_Recording.give_back)
+            self._put_aside.append((self.graph, self._capturing))
         else:
             self._put_aside.clear()
+
+    @staticmethod
+    def give_back(phase="stop", info=None):
+        if phase == "stop" and _Recording._put_aside and not _Recording._put_aside[-1][1]():
+            _Recording._put_aside.clear()
 
 
 class CompiledSDFG:
@@ -927,6 +936,7 @@ class CompiledSDFG:
 
     def __call__(self, **kwargs):
         import torch
+        _Recording.give_back()
         sdfg = self.sdfg
         if not kwargs.keys() <= sdfg.arrays.keys():
             unknown = set(kwargs) - set(sdfg.arrays)
@@ -1021,6 +1031,7 @@ class CompiledSDFG:
         import torch
         if self._graph is not None:
             return None
+        _Recording.give_back()
         done = plan.call(weights, weights._made, weights._handed_out, copies, inputs, torch._C._cuda_getCurrentRawStream(self.device.index))
         if done is None:
             return None
@@ -1057,6 +1068,7 @@ class CompiledSDFG:
     def replay(self):
         if self._graph is None:
             raise RuntimeError("capture_graph() has not been called for the current buffers")
+        _Recording.give_back()
         self._graph.graph.replay()
 
     @property

@@ -70,3 +70,35 @@ def test_recordings_are_not_destroyed_during_a_capture(monkeypatch):
     alive = weakref.ref(second.graph)
     del second
     assert alive() is None
+
+
+@pytest.mark.parametrize("after", ["a collection", "a call", "a replay"])
+def test_a_recording_that_was_put_aside_is_given_back_after_the_capture(monkeypatch, after):
+    """Also where no other recording is ever made or dropped."""
+    import gc
+    import weakref
+    from dace_onnx_amd.sdfg import _Program, _Recording
+    capturing = [1]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: bool(capturing))
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: type("Stream", (), {"cuda_stream": 0})())
+    monkeypatch.setattr(_Program, "run", lambda *a: None)
+    compiled = donnx.ONNXModel("given_back", _chain_model()).expand().compile()
+    compiled.device = torch.device("cpu")
+
+    def use():
+        if after == "a collection":
+            gc.collect()
+        elif after == "a call":
+            compiled(**{k: np.zeros(d.shape, d.dtype.np_dtype) for k, d in compiled.sdfg.arrays.items() if not d.transient})
+        else:
+            compiled._graph = type("Kept", (), {"graph": type("Graph", (), {"replay": lambda self: None})()})()
+            compiled.replay()
+
+    graph = np.zeros(1)
+    alive, recording = weakref.ref(graph), _Recording(graph)
+    del graph, recording
+    use()
+    assert alive() is not None
+    capturing.clear()
+    use()
+    assert alive() is None
