@@ -61,14 +61,14 @@ class _Sub(torch.Tensor):
     pass
 
 
-@pytest.mark.parametrize("make", [lambda x: x.t().contiguous().t(), lambda x: x.cpu(), lambda x: x.cpu().numpy(), lambda x: x.as_subclass(_Sub),
-                                  lambda x: torch.stack([x, -x])[0]])
-def test_arguments_of_other_kinds(x, by_plan, make):
+@pytest.mark.parametrize("make, taken", [(lambda x: x.t().contiguous().t(), False), (lambda x: x.cpu(), False), (lambda x: x.cpu().numpy(), False),
+                                         (lambda x: x.as_subclass(_Sub), False), (lambda x: torch.stack([x, -x])[0], True)])
+def test_arguments_of_other_kinds(x, by_plan, make, taken):
     model, expected = _model(), _model()(x)
     model(x)
     got = model(make(x))
-    assert same([torch.as_tensor(g).cuda() for g in got], expected) and (by_plan == [False] or isinstance(make(x), torch.Tensor))
-    assert same(model(x=x), expected) and same(model(x), expected) and by_plan[-1]
+    assert same([torch.as_tensor(g).cuda() for g in got], expected) and by_plan == [taken]
+    assert same(model(x=x), expected) and same(model(x), expected) and by_plan == [taken, True]
 
 
 @pytest.mark.parametrize("make", [lambda x: x.double(), lambda x: x[:32], lambda x: x.reshape(K, ROWS)])
@@ -119,7 +119,7 @@ def test_streams_threads_and_recordings(x, by_plan):
     results = {}
 
     def work(i):
-        for _ in range(20):   # (one at a time on the GPU: a model has one set of intermediate arrays)
+        for _ in range(20):   # (with one input: calls that overlap write the same into the intermediate array that they share)
             results[i] = model(x)
 
     threads = [threading.Thread(target=work, args=(i, )) for i in range(4)]
@@ -139,6 +139,45 @@ def test_streams_threads_and_recordings(x, by_plan):
         graph.replay()
         torch.cuda.synchronize()
         assert all(torch.allclose(r, e, rtol=1e-5, atol=1e-6) for r, e in zip(recorded, expected))
+
+
+def _tail():
+    return [helper.make_node("Softmax", ["y"], ["p"], axis=1), helper.make_node("ReduceMax", ["y"], ["m"], axes=[1], keepdims=0)], {"y": [4096, N]}, {"p": [4096, N], "m": [4096]}, []
+
+
+def _convolution():
+    w = numpy_helper.from_array(np.random.default_rng(2).standard_normal((512, 512, 3, 3), dtype=np.float32), "w")
+    nodes = [helper.make_node("Conv", ["y", "w"], ["c"], kernel_shape=[3, 3], pads=[1] * 4), helper.make_node("Relu", ["c"], ["p"])]
+    return nodes, {"y": [1, 512, 7, 7]}, {"p": [1, 512, 7, 7]}, [w]
+
+
+@pytest.mark.parametrize("make", [_tail, _convolution])
+@pytest.mark.parametrize("shared_stream", [True, False])
+def test_calls_of_a_model_without_intermediate_arrays_may_overlap(by_plan, make, shared_stream):
+    """From four threads, each with its inputs: on one stream, where their launches come in any order, and on a stream each."""
+    nodes, inputs, outputs, weights = make()
+    infos = lambda of: [helper.make_tensor_value_info(n, TensorProto.FLOAT, s) for n, s in of.items()]   # noqa: E731
+    graph = helper.make_graph(nodes, "g", infos(inputs), infos(outputs), initializer=weights)
+    model = donnx.ONNXModel("overlap", helper.make_model(graph, opset_imports=[helper.make_opsetid("", 12)]))
+    xs = [torch.from_numpy(np.random.default_rng(i).standard_normal(inputs["y"], dtype=np.float32)).cuda() for i in range(4)]
+    call = lambda x: r if isinstance(r := model(x), tuple) else (r, )   # noqa: E731
+    expected, results = [call(x) for x in xs], {}
+    assert not any(d.transient for d in model.sdfg.arrays.values())
+    torch.cuda.synchronize()
+
+    def work(i):
+        stream = torch.cuda.current_stream() if shared_stream else torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            results[i] = [call(xs[i]) for _ in range(20)]
+        stream.synchronize()
+
+    threads = [threading.Thread(target=work, args=(i, )) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(results) == 4 and all(same(r, expected[i]) for i in range(4) for r in results[i])
+    assert by_plan == [True] * 83
 
 
 def test_nothing_outlives_a_dropped_model(x):
