@@ -520,6 +520,12 @@ class SDFG:
     def add_transient(self, name, shape, dtype, strides=None, storage=StorageType.GPU_Global):
         return self.add_array(name, shape, dtype, strides, True, storage)
 
+    def free_name(self, name):
+        """``name``, with underscores behind it if the graph has an array of that name."""
+        while name in self.arrays:
+            name += "_"
+        return name
+
     def add_scalar(self, name, dtype, transient=False):
         return self.add_array(name, (), dtype, None, transient)
 

@@ -165,7 +165,7 @@ def convolutions_in_parts(model):
             if parts <= 1:
                 continue
             result = _out_edge(state, pool, pool.args[1].connector) if mean else out
-            sums = f"{out.data.data}_parts"
+            sums = sdfg.free_name(f"{out.data.data}_parts")
             sdfg.add_transient(sums, [parts, rows, positions], float32)
             target = Ptr("_summed", pool.args[1].offset if mean else 0)
             summed = KernelCall(call.label, "mi355x_conv2d_parts_f32", [X, W, Ptr(None), bias, residual, Ptr("_parts"), parts, target] + geometry + [epilogue, int(mean), Stream()],

@@ -42,7 +42,7 @@ def split_products(model):
             parts = lib.mi355x_gemm_parts(M, N, K, int(b_k == 1), int(weight is not None and model.weights.private(weight)))
             if parts <= 1:
                 continue
-            sums = f"{_out_edge(state, call, C.connector).data.data}_parts"
+            sums = sdfg.free_name(f"{_out_edge(state, call, C.connector).data.data}_parts")
             sdfg.add_transient(sums, [parts, M, N], float32)
             product = KernelCall(call.label, "mi355x_gemm_parts_f32", [A, B, Ptr(None), Ptr("_parts", C.offset), parts, M, N, K, a_strides.values[2], b_k, b_column,
                                                                        call.args[14], Stream()], [A.connector, B.connector], ["_parts"])

@@ -7,6 +7,7 @@ from dace_onnx_amd import _lib
 from dace_onnx_amd.onnx.proto import TensorProto, helper, numpy_helper
 from dace_onnx_amd.sdfg import I64Array, KernelCall, Ptr, Stream
 from dace_onnx_amd.transformation import packing
+from dace_onnx_amd.transformation.partial_sums import split_products
 
 SHAPE = [1, 512, 7, 7]   # parts pay here
 
@@ -66,3 +67,16 @@ def test_the_launch_is_told_how_many_parts_its_array_holds():
     values[place + 1] = 0
     with pytest.raises(_lib.MI355XError, match="0 parts"):
         _lib.check(_lib.library().mi355x_conv2d_parts_f32(*values), "mi355x_conv2d_parts_f32")
+
+
+def test_a_graph_with_an_array_of_that_name_already():
+    """"c_parts" of the caller's, beside the product and the convolution whose results are "c"."""
+    functions, _ = _functions_and_transients(_conv_graph(before=[node("Exp", ["x"], ["c_parts"])], source="c_parts", after=[node("Abs", ["c"], ["y"])], result="c"))
+    assert "mi355x_conv2d_parts_f32" in functions
+    weights = [numpy_helper.from_array(np.ones(s, np.float32), n) for n, s in (("w", (3072, 768)), ("g", (768, )))]
+    infos = [helper.make_tensor_value_info(n, TensorProto.FLOAT, s) for n, s in (("x", [16, 3072]), ("y", [16, 768]))]
+    nodes = [node("Exp", ["x"], ["c_parts"]), node("MatMul", ["c_parts", "w"], ["c"]), node("LayerNormalization", ["c", "g"], ["y"], axis=-1)]
+    graph = helper.make_graph(nodes, "g", infos[:1], infos[1:], initializer=weights)
+    model = donnx.ONNXModel("named", helper.make_model(graph, opset_imports=[helper.make_opsetid("", 17)]))
+    model.expand()
+    assert split_products(model) == 1
