@@ -473,7 +473,7 @@ class ONNXModel:
         """Execute the model.
 
         Calls of one model share its intermediate arrays: they follow one another on one stream, or the caller makes one wait for the other. Calls
-        of a model without any (a graph of one launch) may overlap on several streams and threads.
+        of a model without any (no transient among ``sdfg.arrays`` once it is compiled) may overlap on several streams and threads.
 
         :param args: positional arguments; the i-th is the i-th graph input.
         :param kwargs: named arguments matching the ONNX input names.
